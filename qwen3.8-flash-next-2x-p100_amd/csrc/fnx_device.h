@@ -1,10 +1,12 @@
 // Device-side helpers shared by the gfx950 kernels: wave64 reductions, half conversion, the signed IQ3_S lookup table.
 #pragma once
 
+#include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "../../include/fnx_expf.h"
+#include "../../include/fnx_mi355x.h"
 #include "iq3s_grid.h"
 
 namespace fnx {
@@ -30,6 +32,7 @@ struct SignedGrid {
     }
 };
 constexpr int SGRID_WORDS = 8192;
+static __device__ const SignedGrid g_sgrid{};
 // entry (s, g) from entry (0, g): the bytes whose bit of s is set, negated. No byte of the codebook is zero, so
 // (b ^ 0xFF) + 1 = 256 - b never carries into the next byte and the four bytes go in one xor and one add.
 constexpr bool grid_bytes_nonzero() {
@@ -68,6 +71,18 @@ __device__ __forceinline__ float group_max(float v) {
 // includes the same lines), so that the q8_1 codes of h and the combine's gate come out bit for bit on both sides
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + fnx_expf(-x)); }
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + fnx_expf(-x)); }
+
+// q8_1 quantisation (kernels.cu:131-145), one 32-lane half-wave per block of 32 values
+__device__ __forceinline__ void q8_1_store(float xi, uint8_t* blk, int lane32) {
+    const float amax = group_max<32>(fabsf(xi)), sum = group_sum<32>(xi);
+    const float d = amax / 127.0f;
+    const int8_t qv = amax == 0.0f ? (int8_t) 0 : (int8_t) roundf(xi / d);
+    reinterpret_cast<int8_t*>(blk + 4)[lane32] = qv;
+    if (lane32 == 0) {
+        reinterpret_cast<unsigned short*>(blk)[0] = float_to_half_bits(d);
+        reinterpret_cast<unsigned short*>(blk)[1] = float_to_half_bits(sum);
+    }
+}
 
 // Sums over a weight row's lanes in the reference's order: lane l holds the terms of sub-block l of the row (for rows of 64
 // sub-blocks: l and l + 32 are the two super-blocks a lane of the reference's 32 takes, kernels.cu:209-228, moe.cuh:664-670),

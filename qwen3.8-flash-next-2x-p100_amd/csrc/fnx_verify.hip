@@ -48,24 +48,12 @@ static int env_int(const char* name, int dflt, int lo, int hi) {
 }
 
 // ================================================================ device globals
-__device__ const SignedGrid g_sgrid{};
 // h = silu(gate) * up of every pair of the window as q8_1 rows, made once for moe_down (one MoE in flight per device,
 // as the reference's g_moe_hq, moe.cuh:592-594)
 constexpr int HQ_ROWS = FNX_MAXT * 10 + FNX_MAXT, HQ_MAX_FF = 1024;
 __device__ uint8_t g_moe_hq[HQ_ROWS * (HQ_MAX_FF / 32) * FNX_Q8_1_BLOCK];
 
 // ================================================================ q8_1 quantisation (kernels.cu:131-145)
-// one 32-lane half-wave per block of 32 values
-__device__ __forceinline__ void q8_1_store(float xi, uint8_t* blk, int lane32) {
-    const float amax = group_max<32>(fabsf(xi)), sum = group_sum<32>(xi);
-    const float d = amax / 127.0f;
-    const int8_t qv = amax == 0.0f ? (int8_t) 0 : (int8_t) roundf(xi / d);
-    reinterpret_cast<int8_t*>(blk + 4)[lane32] = qv;
-    if (lane32 == 0) {
-        reinterpret_cast<unsigned short*>(blk)[0] = float_to_half_bits(d);
-        reinterpret_cast<unsigned short*>(blk)[1] = float_to_half_bits(sum);
-    }
-}
 __global__ void __launch_bounds__(256) k_quantize_q8_1(const float* __restrict__ x, uint8_t* __restrict__ q, int n) {
     const int row = blockIdx.y, b = blockIdx.x * 8 + (threadIdx.x >> 5), lane = threadIdx.x & 31;
     if (b >= n / 32) return;
@@ -467,7 +455,7 @@ __global__ void __launch_bounds__(512) k_iq3s_jobs(const RowsArgs a) {
 #include "k_decoder.h"
 #include "k_round.h"
 #include "k_sampler.h"
-#include "k_qtypes.h"
+#include "k_qt_jobs.h"
 #include "k_stream.h"
 namespace fnx {
 
@@ -801,11 +789,13 @@ struct BufferScope {   // enter now, leave when the call returns
     ~BufferScope() { o.leave(s); }
 };
 
+void window_launch_type(uint32_t type, const WindowArgs& a, int blocks, hipStream_t s);   // fnx_window_types.hip
+
 // wide: the jobs are expected to hold many rows each (a dense matrix over the whole window) rather than one or two
 static int rows_launch(const fnx_dw* W, size_t w_stride, const fnx_job* jobs, const int* njobs, int njobs_max, const void* y, float* out,
                        int out_stride, void* st, const char* who, bool wide = false) {
     if (!W || !jobs || !out) return fail(std::string(who) + ": null argument");
-    if (W->type == QT_Q4_0 || W->type == QT_Q5_1 || W->type == QT_Q8_0 || W->type == QT_IQ4_NL || W->type == QT_IQ4_XS || W->type == QT_Q4_K || W->type == QT_Q5_K) {
+    if (qt_type(W->type)) {
         // the other types of kernels.cu:2454-2471 that the reference's own host code can decode (k_qtypes.h)
         gguf::BlockShape bs{};
         gguf::block_shape(W->type, bs);
@@ -888,13 +878,28 @@ static int rows_launch(const fnx_dw* W, size_t w_stride, const fnx_job* jobs, co
 // the shapes and layouts the one-launch window takes (k_moe_window.h)
 // the shared expert as dense split Q8_0 (engine.cu:1600-1604) instead of sh_gu / sh_down
 static bool shared_is_q8(const fnx_moe_layer* L) { return L->sh_gu_q8.q && L->sh_down_q8.q; }
-static bool layer_fused_ok(const fnx_moe_layer* L, int T) {
+static bool layer_shape_ok(const fnx_moe_layer* L, int T) {
     static const int on = env_int("FNX_LAYER_FUSED", 1, 0, 1);
+    return on && L->n == FL_N && (L->ff == 256 || L->ff == 512 || L->ff == 1024) && L->nexp <= 1024 && L->topk <= FL_MAXK &&
+           T * L->topk <= FL_MAXP && cu_count() >= WN_WAVES * T;   // sixteen blocks a row at least (moe_window_plan.h)
+}
+static bool layer_fused_ok(const fnx_moe_layer* L, int T) {
     const auto packed = [](const fnx_dw& w) { return w.type == FNX_T_IQ3S_UNIT64; };
     const bool shared_ok = shared_is_q8(L) || (packed(L->sh_gu) && packed(L->sh_down) && L->sh_gu.p && L->sh_down.p);
-    return on && L->n == FL_N && (L->ff == 256 || L->ff == 512 || L->ff == 1024) && L->nexp <= 1024 && L->topk <= FL_MAXK &&
-           T * L->topk <= FL_MAXP && packed(L->gu) && packed(L->down) && shared_ok && L->gu_stride % UNIT_BYTES == 0 &&
-           L->down_stride % UNIT_BYTES == 0 && cu_count() >= WN_WAVES * T;   // sixteen blocks a row at least (moe_window_plan.h)
+    return layer_shape_ok(L, T) && packed(L->gu) && packed(L->down) && shared_ok && L->gu_stride % UNIT_BYTES == 0 &&
+           L->down_stride % UNIT_BYTES == 0;
+}
+// The same launch over the other expert types, as files hold them: all four matrices of one type (or the shared expert as
+// dense split Q8_0) - a kernel takes one type. Against the nine launches of the operators one by one: Q4_K experts, 7 rows,
+// 143 -> 41 us; Q5_K of width 1024, 14 rows: 327 -> 113.
+static bool layer_types_ok(const fnx_moe_layer* L, int T) {
+    const auto same = [&](const fnx_dw& w) {
+        gguf::BlockShape bs{};
+        return w.type == L->gu.type && gguf::block_shape(w.type, bs) && w.n_in % bs.values == 0 &&
+               w.row_bytes == (size_t) (w.n_in / bs.values) * (size_t) bs.bytes && ((uintptr_t) w.p & 1) == 0;
+    };
+    return layer_shape_ok(L, T) && qt_type(L->gu.type) && same(L->gu) && same(L->down) && (L->gu.p || L->gu.ep) && (L->down.p || L->down.ep) &&
+           L->gu_stride % 2 == 0 && L->down_stride % 2 == 0 && (shared_is_q8(L) || (same(L->sh_gu) && same(L->sh_down) && L->sh_gu.p && L->sh_down.p));
 }
 // timing of the window (fnx_layer_profile): events recorded on the launch stream around the window's launch (and around the
 // dense launches of a split-Q8_0 shared expert before it); the counterpart of the reference's FNX_PROF stamps in its window
@@ -968,7 +973,8 @@ static int layer_fused(const fnx_moe_layer* L, const float* x, int T, float* out
         if (wa.next_x) launch(sbr, std::true_type{});
         else launch(sbr, std::false_type{});
     };
-    if (ff == 256) launch_dec(std::integral_constant<int, 8>{});
+    if (qt_type(L->gu.type)) window_launch_type(L->gu.type, wa, nb, s);
+    else if (ff == 256) launch_dec(std::integral_constant<int, 8>{});
     else if (ff == 512) launch_dec(std::integral_constant<int, 16>{});
     else launch_dec(std::integral_constant<int, 32>{});
     prof_mark(2, s);
@@ -1251,6 +1257,7 @@ static int moe_layer_checked(const fnx_moe_layer* L, const float* x, int T, floa
         if (next_done) *next_done = next && next->x;
         return layer_fused(L, x, T, out, ws, st, live, next);
     }
+    if (layer_types_ok(L, T)) return layer_fused(L, x, T, out, ws, st);
     // operator by operator the pairs' q8_1 rows of h go through the library's pair buffer, rows of ff / 32 blocks
     if (ff <= 0 || ff % 32 || ff > HQ_MAX_FF) return fail("moe_verify_layer: expert width does not fit the pair buffer");
     hipStream_t s = (hipStream_t) st;

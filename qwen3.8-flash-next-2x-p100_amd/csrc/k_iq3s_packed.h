@@ -220,7 +220,7 @@ __device__ __forceinline__ void packed_range(const uint32_t* tab, const uint8_t*
 // ---------------------------------------------------------------- raw ggml blocks -> unit64 (once, at load)
 // One wave per unit. Every lane reads its sub-block's raw fields first, the wave then writes the unit, so src and dst
 // may be the same buffer.
-__global__ void __launch_bounds__(256) k_iq3s_repack(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, long units) {
+static __global__ void __launch_bounds__(256) k_iq3s_repack(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, long units) {
     __shared__ uint32_t stage[4][UNIT_BYTES / 4];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sb = lane >> 3, ib = lane & 7;
     const long u = (long) blockIdx.x * 4 + wave;

@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "k_moe_layer.h"
+#include "k_window_formats.h"
 #include "moe_window_plan.h"
 
 namespace fnx {
@@ -233,15 +234,18 @@ __device__ __forceinline__ void win_next_row(const WindowArgs& a, int t, bool ad
 // RBF: the router's rows are bf16 (a.router_bf16). A template argument, and a row past the block's slice is loaded all the same
 // (the slice's last, its sum thrown away): the number of loads behind the block's row of x is then the same on every path,
 // the compiler knows it, and the block's first meeting does not wait for the router's rows as well.
-template <int SBR, bool DEC = false, bool RBF = false>
+// RBF 2: looked up in a.router_bf16 (the types whose window is not worth a kernel a router type).
+// F: the weights' type (k_window_formats.h)
+template <int SBR, bool DEC = false, int RBF = 0, class F = WinUnit64>
 __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     __shared__ WinLds<SBR> S;
-    constexpr int RW = 64 / SBR, RMAX = SBR / 8, NB = RMAX == 4 ? 2 : 3, DEPTH = RMAX == 4 ? 1 : 2;   // rows a unit; units a wave and trip at most; trips' buffers
+    constexpr int RW = 64 / SBR, RMAX = SBR / 8, RPASS = RMAX < F::MAXR ? RMAX : F::MAXR;   // rows a unit; units a wave at most, and of them a trip
+    constexpr int NB = RPASS == 4 ? 2 : F::NBUF, DEPTH = NB - 1;                                // trips' buffers, trips ahead
     const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63;
     // the codebook's 512 unsigned entries: the launch's first load; the blocks read different signed forms of the table in
     // memory (2 KiB apart) and negate them back, so that not every wave of the grid asks the same sixteen cache lines at once
     const int form = (2 * (int) blockIdx.x + (tid >> 9)) & 15;
-    const uint32_t tab0 = signed_entry(g_sgrid.v[(form << 9) + (tid & 511)], form);
+    const uint32_t tab0 = F::TAB ? signed_entry(g_sgrid.v[(form << 9) + (tid & 511)], form) : 0u;
     const int T = a.T, topk = a.topk, nexp = a.nexp, LS = nexp + 1, P = T * topk;
     const int Tl = a.live ? uniform(max(0, min(*a.live, T))) : T;
     if (Tl <= 0) return;
@@ -292,7 +296,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     const int r0 = g * pl.rpb, r1 = min(nexp, r0 + pl.rpb);
     auto load_router_row = [&](int row, float4(&w)[8]) {
         row = min(row, max(r1, 1) - 1);
-        if constexpr (RBF) {
+        if (RBF == 2 ? a.router_bf16 != 0 : RBF != 0) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const uint2 u = reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.router) + (size_t) row * FL_N)[c * 64 + lane];
@@ -351,7 +355,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         S.fin = -1;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) S.tab[tid + i * WN_THREADS] = signed_entry(tab0, (tid >> 9) + 2 * i);
+    for (int i = 0; i < (F::TAB ? 8 : 0); ++i) S.tab[tid + i * WN_THREADS] = signed_entry(tab0, (tid >> 9) + 2 * i);
     if (tid < FL_N / 4) S.xf[tid] = xmine;
 #pragma unroll
     for (int r = 0; r < 2; ++r) {   // kernels.cu:131-145 (quantize_q8_1), a half-wave a block
@@ -397,17 +401,10 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
 
     // ---------------------------------------------------------------- phase G
     // the lane's sub-block of the row's activations
-    int xs[8];
-    float dx;
-    {
-        const uint32_t* xb = S.xq[lane];
-        dx = half_bits_to_float(xb[0] & 0xFFFFu);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) xs[j] = (int) xb[1 + j];
-    }
+    const typename F::Act xa = F::act_x(S.xq, lane);
     const int I0 = g * pl.ipb, I1 = min(pl.per_row, I0 + pl.ipb), nsweep = max(I1 - I0, 0);   // this block's items of its row
-    const PackedVOffs o = packed_voffs(lane);
-    const int uo_g = wave * 2 * UNIT_BYTES, uo_u = uo_g + a.ff * UNIT_BYTES;   // the wave's gate units and up units from an item's first gate unit
+    const typename F::Offs o = F::offs(lane);
+    const int uo_g = wave * 2 * F::UNIT, uo_u = uo_g + a.ff * F::UNIT;   // the wave's gate units and up units from an item's first gate unit
     struct Item {
         int j, k;   // block of 32 h values, matrix (0: the shared expert's, k: pick k - 1's)
     };
@@ -423,14 +420,14 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
             ++m.j;
         }
     };
-    PackedSub A[4];
+    typename F::Raw A[4];
     auto issue_from = [&](const uint8_t* e, int j) {   // e: wave-uniform
-        const __amdgpu_buffer_rsrc_t mtx = matrix_rsrc(e);
-        const int ub = uniform(j) * 32 * UNIT_BYTES;
-        A[0] = load_packed_buf(mtx, ub + uo_g, o);
-        A[1] = load_packed_buf(mtx, ub + uo_g + UNIT_BYTES, o);
-        A[2] = load_packed_buf(mtx, ub + uo_u, o);
-        A[3] = load_packed_buf(mtx, ub + uo_u + UNIT_BYTES, o);
+        const typename F::Mat mtx = F::matrix(e);
+        const int ub = uniform(j) * 32 * F::UNIT;
+        A[0] = F::load(mtx, ub + uo_g, o);
+        A[1] = F::load(mtx, ub + uo_g + F::UNIT, o);
+        A[2] = F::load(mtx, ub + uo_u, o);
+        A[3] = F::load(mtx, ub + uo_u + F::UNIT, o);
     };
     // a wait on a word of this block's LDS; false: gave up (or another wave did)
     auto lds_wait = [&](auto cond) {
@@ -458,18 +455,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         const int slot = sw & (WN_SLOTS - 1);
         float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            int w4[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) w4[j] = *reinterpret_cast<const int*>(reinterpret_cast<const uint8_t*>(S.tab) + packed_addr(A[r].idx, j));
-            const int sc = 1 + 2 * (int) ((A[r].sc >> sc_shift) & 0xFu);
-            const float dw = half_bits_to_float(A[r].d);
-            int sum = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) sum = __builtin_amdgcn_sdot4(w4[j], xs[j], sum, false);
-            // one sub-block's term as the reference forms it: (d_w * d_x) * (float) (sumi * (1 + 2 s))
-            v[r] = (dw * dx) * (float) __mul24(sum, sc);
-        }
+        for (int r = 0; r < 4; ++r) v[r] = F::term(A[r], S.tab, xa, sc_shift);
         const float z = reduce4_units(v[0], v[1], v[2], v[3]);   // units: gate 2 i, gate 2 i + 1, up 2 i, up 2 i + 1
         // the slot's last block (of sweep sw - WN_SLOTS) must have been made: nearly always long ago
         if (sw >= WN_SLOTS &&
@@ -499,6 +485,17 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
             uint32_t* dst = a.hq + ((size_t) pair * qpp + m.j) * HQ_WORDS;
             if ((lane & 3) == 0) __hip_atomic_store(&dst[lane >> 2], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (lane == 0) __hip_atomic_store(&dst[8], __float_as_uint(half_bits_to_float(float_to_half_bits(d))), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if constexpr (F::SUM != WIN_SUM_NONE) {   // word 9: the block's sum as the type wants it
+                uint32_t sum;
+                if constexpr (F::SUM == WIN_SUM_FIELD) sum = __float_as_uint(half_bits_to_float(float_to_half_bits(group_sum<32>(h))));
+                else {
+                    int s = (int) (int8_t) qv;
+#pragma unroll
+                    for (int o_ = 16; o_; o_ >>= 1) s += __shfl_xor(s, o_, 64);
+                    sum = (uint32_t) s;
+                }
+                if (lane == 0) __hip_atomic_store(&dst[9], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
         if (lane == 0) __hip_atomic_store(&S.made[slot], q + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         return true;
@@ -706,18 +703,18 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     // load of a trip is issued on every path, the compiler knows how many loads lie behind the one it waits for, and a decode
     // waits for its own trip's weights only - not, as with loads under "if (r < R)", for everything in flight.
     auto down_phase = [&](auto RC) -> bool {
-    constexpr int RR = decltype(RC)::value;
+    constexpr int RALL = decltype(RC)::value, RR = RALL < F::MAXR ? RALL : F::MAXR;   // the wave's units, and of them a pass over the row's trips
     int TG = 1;
-    if constexpr (RR == 1) TG = pl.dwaves <= WN_WAVES / 2 && WN_WAVES % pl.dwaves == 0 ? WN_WAVES / pl.dwaves : 1;
+    if constexpr (RALL == 1) TG = pl.dwaves <= WN_WAVES / 2 && WN_WAVES % pl.dwaves == 0 ? WN_WAVES / pl.dwaves : 1;
     const bool dwave = TG > 1 || wave < pl.dwaves;
     const int tgrp = TG > 1 ? wave / pl.dwaves : 0, uw = TG > 1 ? wave - tgrp * pl.dwaves : wave;
-    const int u0 = g * pl.upb + uw * RR;   // this wave's units of every matrix
+    int u0 = g * pl.upb + uw * RALL;   // this wave's units of every matrix
     auto trip_of = [&](int i) { return first + tgrp + i * TG; };   // the wave's i-th trip
-    PackedSub B[NB][RR];
-    auto issue_trip = [&](PackedSub(&buf)[RR], int trip) {
-        const __amdgpu_buffer_rsrc_t mtx = matrix_rsrc(down_matrix(trip));
+    typename F::Raw B[NB][RR];
+    auto issue_trip = [&](typename F::Raw(&buf)[RR], int trip) {
+        const typename F::Mat mtx = F::matrix(down_matrix(trip));
 #pragma unroll
-        for (int r = 0; r < RR; ++r) buf[r] = load_packed_buf(mtx, (u0 + r) * UNIT_BYTES, o);
+        for (int r = 0; r < RR; ++r) buf[r] = F::load(mtx, (u0 + r) * F::UNIT, o);
     };
     // The picks are known (this block ranked its row), so the first trips' weights are asked for before the wait for h.
     // (The hand-over of the last pick's matrix has been seen by every wave that swept; a block without items waits here.)
@@ -755,7 +752,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         asm volatile("" : "+v"(l2));   // the addresses are worked out here, not kept in registers since phase R
 #pragma unroll
         for (int c = 0; c < 8; ++c) xr[c] = S.xf[c * 64 + l2];
-        if constexpr (RBF) {
+        if (RBF == 2 ? a.router_bf16 != 0 : RBF != 0) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const uint2 u = reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.router) + (size_t) nexp * FL_N)[c * 64 + l2];
@@ -813,27 +810,14 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         for (int r = 0; r < RR; ++r) acc[r] = zs[r] = 0.f;
         const float gate = S.gate;
         // a trip's sums of this wave's units' rows (every lane of a row's group holds the row's)
-        auto trip_rows = [&](const PackedSub(&buf)[RR], int trip, auto after_h, auto sink) {
+        auto trip_rows = [&](const typename F::Raw(&buf)[RR], int trip, auto after_h, auto sink) {
             const int k = pick_of(trip);
-            const uint32_t* hb = S.hq[k][kb];
-            const uint4 lo = *reinterpret_cast<const uint4*>(hb), hi = *reinterpret_cast<const uint4*>(hb + 4);
-            const int hx[8] = {(int) lo.x, (int) lo.y, (int) lo.z, (int) lo.w, (int) hi.x, (int) hi.y, (int) hi.z, (int) hi.w};
-            const float dh = __uint_as_float(hb[8]);
+            const typename F::Act ha = F::act_h(S.hq[k], kb, lane);
             after_h();
 #pragma unroll
-            for (int r = 0; r < RR; ++r) {
-                int w4[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) w4[j] = *reinterpret_cast<const int*>(reinterpret_cast<const uint8_t*>(S.tab) + packed_addr(buf[r].idx, j));
-                const int sc = 1 + 2 * (int) ((buf[r].sc >> sc_shift) & 0xFu);
-                const float dw = half_bits_to_float(buf[r].d);
-                int sum = 0;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) sum = __builtin_amdgcn_sdot4(w4[j], hx[j], sum, false);
-                sink(r, butterfly_sum<SBR>((dw * dh) * (float) __mul24(sum, sc)));
-            }
+            for (int r = 0; r < RR; ++r) sink(r, butterfly_sum<SBR>(F::term(buf[r], S.tab, ha, sc_shift)));
         };
-        auto decode_trip = [&](const PackedSub(&buf)[RR], int trip) {
+        auto decode_trip = [&](const typename F::Raw(&buf)[RR], int trip) {
             switch ((wave >> 2) + trip & 3) {   // every wave takes each of the four priorities in turn (see the sweeps)
                 case 0: __builtin_amdgcn_s_setprio(0); break;
                 case 1: __builtin_amdgcn_s_setprio(1); break;
@@ -848,7 +832,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
                     else acc[r] = fmaf(gk, z, acc[r]);
                 });
         };
-        if constexpr (RR == 1) {
+        if constexpr (RALL == 1) {
             if (TG > 1) {   // (the same for the whole block)
                 constexpr int MAXI = (FL_MAXK + 2) / 2;   // trips a wave at most (TG >= 2)
 #pragma unroll
@@ -877,6 +861,15 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
                 }
                 return true;
             }
+        }
+        // (a type whose lanes hold more of a unit makes a wave's units RR at a time, a pass over the row's trips each)
+#pragma unroll
+        for (int pass = 0; pass < RALL / RR; ++pass) {
+        if (pass > 0) {
+            u0 += RR;
+#pragma unroll
+            for (int r = 0; r < RR; ++r) acc[r] = zs[r] = 0.f;
+            first_trips();
         }
         // A trip's loads go to the buffer that held trip nx - NB, decoded before this one. The rounds in which every trip exists
         // and so does the one it asks for come first, without a condition on a load (see above); the last trips follow with them.
@@ -914,6 +907,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
                     // (at the device's level: the row's last block may read the row back below, from another XCD)
                     __hip_atomic_store(reinterpret_cast<unsigned*>(orow + r * RW), __float_as_uint(acc[r] + shared), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
+        }
         }
     }
     return true;

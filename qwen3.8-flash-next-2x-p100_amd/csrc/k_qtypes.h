@@ -13,6 +13,9 @@
 namespace fnx {
 
 constexpr uint32_t QT_Q4_0 = 2, QT_Q5_1 = 7, QT_Q8_0 = 8, QT_Q4_K = 12, QT_Q5_K = 13, QT_IQ4_NL = 20, QT_IQ4_XS = 23;
+inline bool qt_type(uint32_t t) {
+    return t == QT_Q4_0 || t == QT_Q5_1 || t == QT_Q8_0 || t == QT_IQ4_NL || t == QT_IQ4_XS || t == QT_Q4_K || t == QT_Q5_K;
+}
 // kvalues_iq4nl (tensor_convert.hpp): {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113}, four to a word.
 // Four 4-bit indexes (one a byte) -> their four table bytes: a byte permute over each half of the table (selector bytes
 // 0..3 take from the second operand, 4..7 from the first), the index's top bit choosing between the halves.
@@ -130,40 +133,6 @@ __device__ __forceinline__ float qt_term(const QtSub& s, const uint8_t* yb) {
     else if constexpr (TYPE == QT_Q4_K || TYPE == QT_Q5_K) return s.d * (dx * (float) (dot * s.sc)) - s.dmin * (dx * (float) (qsum * s.m));
     else if constexpr (TYPE == QT_IQ4_XS) return (s.d * dx) * (float) (dot * s.sc);
     else return (s.d * dx) * (float) dot;
-}
-
-struct QtArgs {
-    const uint8_t* wbase;
-    size_t w_stride;
-    const uint8_t* const* ep;
-    size_t row_bytes;
-    int nrows, ncols;
-    const fnx_job* jobs;
-    const int* njobs;
-    int njobs_max;
-    const uint8_t* y;
-    float* out;
-    int out_stride;
-};
-template <uint32_t TYPE>
-__global__ void __launch_bounds__(256) k_qt_jobs(const QtArgs a) {
-    const int ji = blockIdx.y;
-    if (ji >= (a.njobs ? min(*a.njobs, a.njobs_max) : a.njobs_max)) return;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= a.nrows) return;
-    const fnx_job* jb = a.jobs + ji;
-    const uint8_t* we = (a.ep ? a.ep[jb->w] : a.wbase + (size_t) jb->w * a.w_stride) + (size_t) row * a.row_bytes;
-    const int sbr = a.ncols / 32, n = min(max(jb->n, 0), FNX_MAXT);
-    const uint8_t* y = a.y ? a.y : g_moe_hq;   // moe_down: the pairs' q8_1 rows in the library's buffer
-    for (int t = 0; t < n; ++t) {
-        float acc = 0.f;
-        for (int kb = lane; kb < sbr; kb += 64) {
-            const QtSub s = qt_decode<TYPE>(we, kb);
-            acc += qt_term<TYPE>(s, y + ((size_t) jb->y[t] * sbr + kb) * FNX_Q8_1_BLOCK);
-        }
-        acc = group_sum<64>(acc);
-        if (lane == 0) a.out[(size_t) jb->out[t] * a.out_stride + row] = acc;
-    }
 }
 
 }  // namespace fnx

@@ -100,3 +100,55 @@ def test_gate_up_and_down_with_q4_k_experts(dev, oracle):
     dev.sync()
     assert rel_l2(gu.cpu().numpy(), want_gu) <= 1e-6
     assert rel_l2(part.cpu().numpy(), want_part) <= 1e-3   # SwiGLU's expf moves an int8 code by one step now and then
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("ff,T,nexp,topk", [(256, 1, 5, 2), (512, 16, 6, 3), (1024, 16, 3, 2), (1024, 2, 3, 1)])
+def test_window_over_other_types(dev, oracle, qtype, ff, T, nexp, topk):
+    """fnx_moe_verify_layer with all four matrices of one type (one launch, hidden 2048) against the oracle's operators in the
+    reference's order (engine.cu:1569-1757): the smallest and the largest window, every expert width (two wave passes a
+    trip at 1024), a window of few rows whose trips are dealt over a block's waves. The operators' bar: the same terms in
+    the same order of sums, so 1e-6."""
+    print(f"case window type={qtype} ff={ff} T={T} nexp={nexp} topk={topk}", flush=True)
+    rng = np.random.default_rng(100 * qtype + ff + T)
+    n, P, t, pkg = 2048, T * topk, dev.torch, dev.pkg
+    values, nbytes = qb.SHAPE[qtype]
+    rb = lambda cols: cols // values * nbytes
+    gu_w, dn_w, sgu, sdn = (qb.random_blocks(rng, qtype, m * r * c // values) for m, r, c in ((nexp, 2 * ff, n), (nexp, n, ff), (1, 2 * ff, n), (1, n, ff)))
+    W = (rng.standard_normal((nexp + 1, n)) * 0.02).astype(np.float32)
+    bf16 = T == 2   # a window's router may be bf16 bits: the same values, kept in the upper halves
+    if bf16:
+        W = (W.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    up = dev.up
+    d = [up(a) for a in (gu_w, dn_w, sgu, sdn)]
+    dW = up((W.view(np.uint32) >> 16).astype(np.uint16)) if bf16 else up(W)
+    mat = lambda i, cols, rows: pkg.DW(d[i].data_ptr(), qtype, cols, rows, rb(cols), None)
+    L = pkg.MoeLayer(n, ff, nexp, topk, dW.data_ptr(), int(bf16), mat(0, n, 2 * ff), 2 * ff * rb(n), mat(1, ff, n), n * rb(ff), mat(2, n, 2 * ff), mat(3, ff, n))
+    w = dict(xq=dev.zeros(T * (n // 32) * 36, t.uint8), logits=dev.zeros((T, nexp + 1), t.float32), topi=dev.zeros((T, topk), t.int32),
+             topw=dev.zeros((T, topk), t.float32), jobs_gu=dev.zeros((P + 1) * 136, t.uint8), jobs_dn=dev.zeros((P + 1) * 136, t.uint8),
+             njobs=dev.zeros(2, t.int32), gu=dev.zeros((P + T, 2 * ff), t.float32), part=dev.zeros((P + T, n), t.float32),
+             sync=dev.zeros(pkg.MOE_SYNC_WORDS, t.int32))
+    ws = pkg.MoeWs(*(w[k].data_ptr() for k in ("xq", "logits", "topi", "topw", "jobs_gu", "jobs_dn", "njobs", "gu", "part", "sync")))
+    dx, out = up(x), dev.zeros((T, n), t.float32)
+    dev.ok(dev.lib.fnx_moe_verify_layer(C.byref(L), dx.data_ptr(), T, out.data_ptr(), C.byref(ws), dev.st()))
+    dev.sync()
+    assert not w["sync"].cpu().numpy().any(), "every wait ended and the counters are back at zero"
+    logits = oracle.gemv_f32(W, x)
+    topi, topw = oracle.topk_logits(logits, nexp, topk)
+    jg, jd = (np.ascontiguousarray(j) for j in oracle.jobs(topi))
+    xq, mm, ptr = oracle.quantize_q8_1(x), oracle.lib.fnx_o_mmvq_type, ol.ptr
+    gu, part = np.zeros((P + T, 2 * ff), np.float32), np.zeros((P + T, n), np.float32)
+    sh = np.zeros(1, dtype=JOB_DTYPE)
+    sh["n"][0] = T
+    sh["y"][0, :T], sh["out"][0, :T] = np.arange(T), P + np.arange(T)
+    mm(qtype, ptr(gu_w), 2 * ff * rb(n), 2 * ff, n, ptr(jg), len(jg), ptr(xq), ptr(gu), 2 * ff, 8)
+    mm(qtype, ptr(sgu), 0, 2 * ff, n, ptr(sh), 1, ptr(xq), ptr(gu), 2 * ff, 8)
+    hq = oracle.swiglu_stacked_q8_1(gu, ff)
+    sh["y"][0, :T] = P + np.arange(T)
+    mm(qtype, ptr(dn_w), n * rb(ff), n, ff, ptr(jd), len(jd), ptr(hq), ptr(part), n, 8)
+    mm(qtype, ptr(sdn), 0, n, ff, ptr(sh), 1, ptr(hq), ptr(part), n, 8)
+    want = oracle.moe_combine(part[:P], topw, part[P:], logits[:, nexp])
+    assert np.array_equal(w["logits"].cpu().numpy().view(np.uint32), logits.view(np.uint32)) and np.array_equal(w["topi"].cpu().numpy(), topi)
+    assert int(w["njobs"][0].item()) == len(jg)
+    assert rel_l2(out.cpu().numpy(), want) <= 1e-6
