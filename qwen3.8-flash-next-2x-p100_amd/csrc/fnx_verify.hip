@@ -1413,8 +1413,14 @@ static int pf_route(const float* logits, int logits_stride, int C, int nexp, int
     const int cvt_blocks = cvt_n ? (int) std::min<size_t>((cvt_n + 4095) / 4096, 2048) : 0;   // 16 values a thread or more
     k_pf_topk<<<(C + PF_TOPK_WAVES - 1) / PF_TOPK_WAVES + cvt_blocks, PF_TOPK_WAVES * 64, 0, s>>>(logits, logits_stride, C, nexp, topk, topi, topw,
                                                                                                   cvt_x, cvt_n, cvt_y);
-    const int shb = sh_gu ? (C + PF_FILL_THREADS - 1) / PF_FILL_THREADS : 0;
-    k_pf_fill<<<nexp + shb, PF_FILL_THREADS, 0, s>>>(topi, P, topk, nexp, cnt, jbase, njobs, jobs_gu, jobs_dn, njobs_cap, C, sh_gu, sh_dn, nsh);
+    auto fill = [&](auto nw, auto epb) {
+        constexpr int NW = decltype(nw)::value, EPB = decltype(epb)::value;
+        const int shb = sh_gu ? (C + NW * 64 - 1) / (NW * 64) : 0;
+        k_pf_fill<NW, EPB><<<(nexp + EPB - 1) / EPB + shb, NW * 64, 0, s>>>(topi, P, topk, nexp, cnt, jbase, njobs, jobs_gu, jobs_dn, njobs_cap, C,
+                                                                           sh_gu, sh_dn, nsh);
+    };
+    if (P <= PF_FEW) fill(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+    else fill(std::integral_constant<int, 16>{}, std::integral_constant<int, 2>{});
     return launch_status("pf_route");
 }
 int fnx_pf_route(const float* logits, int logits_stride, int C, int nexp, int topk, int* topi, float* topw, int* cnt, int* jbase,

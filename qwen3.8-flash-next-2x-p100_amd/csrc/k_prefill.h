@@ -48,23 +48,30 @@ __global__ void __launch_bounds__(PF_TOPK_WAVES * 64) k_pf_topk(const float* __r
     if (nexp <= 512) wave_topk<8>(logits + (size_t) t * ls, nexp, topk, lane, ex[wave], topi + (size_t) t * topk, topw + (size_t) t * topk);
     else wave_topk<16>(logits + (size_t) t * ls, nexp, topk, lane, ex[wave], topi + (size_t) t * topk, topw + (size_t) t * topk);
 }
-// a block per expert: its pairs in ascending order into the slots of its jobs (a pair always lands in the same job and
-// slot, prefill.cu:340-343). A thread looks at PF_ROUNDS pairs a pass (p = p0 + 256 r + tid), all loaded together; the
-// slots come from the waves' ballot counts, one barrier a pass. Blocks past the experts write the shared expert's
-// jobs (every row: gate|up reads row t, writes row P + t; down reads and writes row P + t) and their count.
-// Where its jobs start an expert's block works out for itself - every expert's pair count (the picks are a few KB, which each
-// block reads anyway), ceil(count / FNX_PF_JOB) jobs each, the jobs of the experts before it - instead of waiting for a
-// launch of one block that does it for all; it leaves its expert's count and first job (cnt, jbase), the last expert's
-// block the job count.
-constexpr int PF_FILL_THREADS = 256, PF_ROUNDS = 8, PF_MAXE = 1024;   // (PF_MAXE: the most experts)
-__global__ void __launch_bounds__(PF_FILL_THREADS) k_pf_fill(const int* __restrict__ topi, int P, int topk, int nexp, int* __restrict__ cnt,
-                                                            int* __restrict__ jbase, int* __restrict__ njobs, fnx_bigjob* __restrict__ gu,
-                                                            fnx_bigjob* __restrict__ dn, int cap, int C, fnx_bigjob* __restrict__ sh_gu,
-                                                            fnx_bigjob* __restrict__ sh_dn, int* __restrict__ nsh) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if ((int) blockIdx.x >= nexp) {
+// A block of NW waves takes EPB experts and puts their pairs in ascending order into the slots of their jobs (a pair always lands
+// in the same job and slot, prefill.cu:340-343). Each of its waves goes through an NWth of all picks twice, PF_ROUNDS loads in
+// flight: first every expert's pairs are counted (in LDS, by all waves) and how many of the block's experts' the wave has
+// (ballots), then, with the waves' counts added up, the slots follow from the ballots; an expert's picks of 64 PF_ROUNDS are
+// packed in LDS on the way, so that a busy expert's jobs are written 64 slots a store. So a block meets three times, however many
+// pairs there are. Blocks past the experts write the shared expert's jobs (every row: gate|up reads row t, writes row P + t; down
+// reads and writes row P + t) and their count. Where its jobs start a block works out for itself - every expert's pair count,
+// ceil(count / FNX_PF_JOB) jobs each, the jobs of the experts before it - instead of waiting for a launch of one block that does
+// it for all; it leaves its experts' counts and first jobs (cnt, jbase), the last expert's block the job count.
+// Bound by the passes over the picks (LDS atomics and round trips to L2), which is why a block has the most waves there are and
+// two experts, unless four waves have all picks in one batch each (PF_FEW): then four waves' meetings are shorter (77 rows:
+// 5.3 us against 5.6, a launch's own latency). 512 experts, ten picks a row, some experts in most rows: 4096 rows 18 us,
+// 512 rows 6.2; blocks of four waves that met every 2048 picks took 81 and 12.8, and without the packing 4096 rows take 28.
+constexpr int PF_ROUNDS = 8, PF_MAXE = 1024, PF_FEW = 4 * 64 * PF_ROUNDS;   // (PF_MAXE: the most experts)
+template <int NW, int EPB>
+__global__ void __launch_bounds__(NW * 64) k_pf_fill(const int* __restrict__ topi, int P, int topk, int nexp, int* __restrict__ cnt,
+                                                     int* __restrict__ jbase, int* __restrict__ njobs, fnx_bigjob* __restrict__ gu,
+                                                     fnx_bigjob* __restrict__ dn, int cap, int C, fnx_bigjob* __restrict__ sh_gu,
+                                                     fnx_bigjob* __restrict__ sh_dn, int* __restrict__ nsh) {
+    constexpr int THREADS = NW * 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, eblocks = (nexp + EPB - 1) / EPB;
+    if ((int) blockIdx.x >= eblocks) {
         if (!sh_gu) return;
-        const int t = ((int) blockIdx.x - nexp) * PF_FILL_THREADS + tid;
+        const int t = ((int) blockIdx.x - eblocks) * THREADS + tid;
         if (t == 0) *nsh = (C + FNX_PF_JOB - 1) / FNX_PF_JOB;
         if (t >= C) return;
         const int j = t / FNX_PF_JOB, k = t % FNX_PF_JOB;
@@ -78,71 +85,89 @@ __global__ void __launch_bounds__(PF_FILL_THREADS) k_pf_fill(const int* __restri
         }
         return;
     }
-    const int e = blockIdx.x;
-    constexpr int NW = PF_FILL_THREADS / 64;
-    __shared__ int hist[PF_MAXE], wjobs[NW];
-    __shared__ int wsum[PF_ROUNDS][NW];
-    for (int i = tid; i < nexp; i += PF_FILL_THREADS) hist[i] = 0;
+    const int e0 = blockIdx.x * EPB;
+    __shared__ int hist[PF_MAXE], wjobs[NW], wcnt[EPB][NW], found[NW][64 * PF_ROUNDS];
+    for (int i = tid; i < nexp; i += THREADS) hist[i] = 0;
     __syncthreads();
-    for (int p = tid; p < P; p += PF_FILL_THREADS) atomicAdd(&hist[topi[p]], 1);
+    const int span = (P + THREADS - 1) / THREADS * 64;   // a wave's picks: whole ballots
+    const int p_lo = wave * span, p_hi = min(P, p_lo + span);
+    int mine[EPB];
+#pragma unroll
+    for (int x = 0; x < EPB; ++x) mine[x] = 0;
+    for (int p0 = p_lo; p0 < p_hi; p0 += 64 * PF_ROUNDS) {
+        int pick[PF_ROUNDS];
+#pragma unroll
+        for (int r = 0; r < PF_ROUNDS; ++r) {
+            const int p = p0 + 64 * r + lane;
+            pick[r] = p < p_hi ? topi[p] : -1;
+        }
+#pragma unroll
+        for (int r = 0; r < PF_ROUNDS; ++r) {
+            if (pick[r] >= 0) atomicAdd(&hist[pick[r]], 1);
+#pragma unroll
+            for (int x = 0; x < EPB; ++x) mine[x] += __popcll(__ballot(pick[r] == e0 + x));
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int x = 0; x < EPB; ++x) wcnt[x][wave] = mine[x];
+    }
     __syncthreads();
-    int before_me = 0;   // jobs of the experts before this one
-    for (int i = tid; i < e; i += PF_FILL_THREADS) before_me += (hist[i] + FNX_PF_JOB - 1) / FNX_PF_JOB;
+    int before_me = 0;   // jobs of the experts before this block's
+    for (int i = tid; i < e0; i += THREADS) before_me += (hist[i] + FNX_PF_JOB - 1) / FNX_PF_JOB;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) before_me += __shfl_xor(before_me, o, 64);
     if (lane == 0) wjobs[wave] = before_me;
     __syncthreads();
-    int jb = 0;
+    int jb[EPB], ce[EPB], at[EPB], some = 0;   // an expert's first job, its pairs, those before this wave's picks
+    jb[0] = 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) jb += wjobs[w];
-    const int ce = hist[e];
-    if (tid == 0) {
-        cnt[e] = ce;
-        jbase[e] = jb;
-        if (e == nexp - 1) njobs[0] = jb + (ce + FNX_PF_JOB - 1) / FNX_PF_JOB;
+    for (int w = 0; w < NW; ++w) jb[0] += wjobs[w];
+#pragma unroll
+    for (int x = 0; x < EPB; ++x) {
+        ce[x] = e0 + x < nexp ? hist[e0 + x] : 0;
+        if (x) jb[x] = jb[x - 1] + (ce[x - 1] + FNX_PF_JOB - 1) / FNX_PF_JOB;
+        at[x] = 0;
+        for (int w = 0; w < wave; ++w) at[x] += wcnt[x][w];
+        some += mine[x];
+        if (tid == 0 && e0 + x < nexp) {
+            cnt[e0 + x] = ce[x];
+            jbase[e0 + x] = jb[x];
+            if (e0 + x == nexp - 1) njobs[0] = jb[x] + (ce[x] + FNX_PF_JOB - 1) / FNX_PF_JOB;
+        }
     }
-    if (ce == 0) return;
-    int base = 0;
-    for (int p0 = 0; p0 < P; p0 += PF_FILL_THREADS * PF_ROUNDS) {
+    if (some == 0) return;
+    for (int p0 = p_lo; p0 < p_hi; p0 += 64 * PF_ROUNDS) {
         int pick[PF_ROUNDS];
 #pragma unroll
         for (int r = 0; r < PF_ROUNDS; ++r) {
-            const int p = p0 + r * PF_FILL_THREADS + tid;
-            pick[r] = p < P ? topi[p] : -1;
+            const int p = p0 + 64 * r + lane;
+            pick[r] = p < p_hi ? topi[p] : -1;
         }
-        unsigned long long m[PF_ROUNDS];
 #pragma unroll
-        for (int r = 0; r < PF_ROUNDS; ++r) {
-            m[r] = __ballot(pick[r] == e);
-            if (lane == 0) wsum[r][wave] = __popcll(m[r]);
-        }
-        __syncthreads();
-        int before = base;   // pairs of this expert before round r's wave `wave`
+        for (int x = 0; x < EPB; ++x) {   // an expert's picks among these, packed in LDS first: a busy expert's go out 64 a store
+            int n = 0;
 #pragma unroll
-        for (int r = 0; r < PF_ROUNDS; ++r) {
-            int mine_before = before;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                mine_before += w < wave ? wsum[r][w] : 0;
-                before += wsum[r][w];
+            for (int r = 0; r < PF_ROUNDS; ++r) {
+                const unsigned long long m = __ballot(pick[r] == e0 + x);
+                if (pick[r] == e0 + x) found[wave][n + __popcll(m & ((1ull << lane) - 1ull))] = p0 + 64 * r + lane;
+                n += __popcll(m);
             }
-            if (pick[r] == e) {
-                const int p = p0 + r * PF_FILL_THREADS + tid;
-                const int s = mine_before + __popcll(m[r] & ((1ull << lane) - 1ull)), j = jb + s / FNX_PF_JOB, k = s % FNX_PF_JOB;
+            for (int i = lane; i < n; i += 64) {
+                const int p = found[wave][i], s = at[x] + i, j = jb[x] + s / FNX_PF_JOB, k = s % FNX_PF_JOB;
                 if (j < cap) {
                     gu[j].y[k] = p / topk;
                     gu[j].out[k] = p;
                     dn[j].y[k] = p;
                     dn[j].out[k] = p;
                     if (k == 0) {
-                        gu[j].w = dn[j].w = e;
-                        gu[j].n = dn[j].n = min(FNX_PF_JOB, ce - (s / FNX_PF_JOB) * FNX_PF_JOB);
+                        gu[j].w = dn[j].w = e0 + x;
+                        gu[j].n = dn[j].n = min(FNX_PF_JOB, ce[x] - (s / FNX_PF_JOB) * FNX_PF_JOB);
                     }
                 }
             }
+            at[x] += n;
         }
-        base = before;
-        __syncthreads();
     }
 }
 

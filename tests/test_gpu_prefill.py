@@ -60,6 +60,26 @@ def test_pf_route_bit_exact(dev, oracle, Cn, nexp, topk, zipf):
             assert np.array_equal(g[2:2 + n], w[2:2 + n]) and np.array_equal(g[2 + PF:2 + PF + n], w[2 + PF:2 + PF + n])
 
 
+@pytest.mark.parametrize("Cn,nexp,topk", [(1, 1, 1), (63, 2, 1), (1025, 3, 1), (2731, 33, 3), (4100, 512, 10)])
+def test_pf_jobs_of_busy_experts(dev, oracle, Cn, nexp, topk):
+    """every row picks expert 0: one expert's pairs over many jobs and through every wave's list, wave spans of whole and of
+    broken sixty-fours, an odd last expert"""
+    print(f"case pf_jobs C={Cn} nexp={nexp} topk={topk}", flush=True)
+    logits = np.random.default_rng(730 + Cn).standard_normal((Cn, nexp + 1)).astype(np.float32)
+    logits[:, 0] = 9.0
+    r = dev.pf_route(logits, nexp, topk)
+    topi, _ = oracle.topk_logits(logits, nexp, topk)
+    assert np.array_equal(r["topi"], topi)
+    gu, dn, cnt = oracle.pf_jobs(topi, nexp, PF)
+    assert np.array_equal(r["cnt"], cnt) and r["njobs"] == len(gu)
+    assert np.array_equal(r["jbase"], np.concatenate([[0], np.cumsum((cnt + PF - 1) // PF)[:-1]]))
+    for got, want in ((r["gu"], gu), (r["dn"], dn)):
+        assert np.array_equal(got[:, :2], want[:, :2])
+        for g, w in zip(got, want):
+            n = w[1]
+            assert np.array_equal(g[2:2 + n], w[2:2 + n]) and np.array_equal(g[2 + PF:2 + PF + n], w[2 + PF:2 + PF + n])
+
+
 def test_pf_route_with_fewer_finite_logits_than_picks(dev, oracle):
     from test_oracle_routing import scarce_logits
     Cn, nexp, topk = 70, 512, 10
