@@ -538,26 +538,29 @@ __device__ __forceinline__ unsigned fkey(float v) {
 __device__ __forceinline__ float fkey_inv(unsigned k) { return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k); }
 constexpr int AM_THREADS = 1024, AM_PER_BLOCK = 16384;
 // keys[t] = max over the row of (fkey(value) << 32 | ~index): the greatest value, the lower index on a tie. A block
-// folds its 16,384 values to one key (four independent 16-byte loads a thread, wave butterflies, LDS) and issues one
-// atomic: atomics on one address serialise, and a row's address would otherwise take one per wave. The row's last block
-// to arrive (a count beside the keys, keys[FNX_MAXT + t]) decodes the key into (value, index + v0) and leaves both words
-// at zero for the next argmax.
+// folds its 16,384 values to one key (four independent 16-byte loads a thread, then a maximum of the keys and a minimum of the
+// indexes that hold it, both with DPP moves) and issues one atomic: atomics on one address serialise, and a row's address
+// would otherwise take one per wave. The row's last block to arrive (a count beside the keys, keys[FNX_MAXT + t]) decodes
+// the key into (value, index + v0) and leaves both words at zero for the next argmax.
+// Bound by the chain of trips to memory: launch, values, maximum, count, key. 16 rows of 151,936
+// logits: 7.8 -> 6.0 us (64-bit keys exchanged lane by lane, the sixteen waves' keys folded by one thread, a count that
+// released and acquired the caches).
+__device__ __forceinline__ unsigned wave_umin(unsigned v) { return ~wave_umax(~v); }
 __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__ logits, int rows, unsigned long long* __restrict__ keys,
                                                       unsigned* __restrict__ err, int v0, float* __restrict__ bv, int* __restrict__ bi,
                                                       const int* __restrict__ live) {
-    __shared__ unsigned long long wbest[AM_THREADS / 64];
-    __shared__ int wbad;
+    __shared__ uint2 wbest[AM_THREADS / 64];
+    __shared__ int wbad[AM_THREADS / 64];
     // live (may be null): a device word; rows from *live on do not count: they are not scanned and their picks stay what they were
     if (live && (int) blockIdx.y >= max(1, *live)) return;
-    const int t = blockIdx.y, i0 = blockIdx.x * AM_PER_BLOCK, i1 = min(rows, i0 + AM_PER_BLOCK), tid = threadIdx.x;
+    const int t = blockIdx.y, i0 = blockIdx.x * AM_PER_BLOCK, i1 = min(rows, i0 + AM_PER_BLOCK), tid = threadIdx.x, lane = tid & 63;
     const float* r = logits + (size_t) t * rows;
-    if (tid == 0) wbad = 0;
-    unsigned long long best = 0;
+    unsigned best = 0, at = 0xffffffffu;   // the thread's greatest key and the first index that holds it (it goes through its values in order)
     bool bad = false;
     auto take = [&](float v, int i) {
         bad = bad || !isfinite(v);
-        const unsigned long long k = (unsigned long long) fkey(v) << 32 | (unsigned) ~i;
-        best = k > best ? k : best;
+        const unsigned k = fkey(v);
+        if (k > best || at == 0xffffffffu) best = k, at = (unsigned) i;
     };
     if ((((uintptr_t) r) & 15) == 0 && (i0 & 3) == 0) {
         float4 v[4];
@@ -581,23 +584,24 @@ __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__
     } else {
         for (int i = i0 + tid; i < i1; i += AM_THREADS) take(r[i], i);
     }
-#pragma unroll
-    for (int o = 32; o; o >>= 1) {
-        const unsigned long long ok = __shfl_xor(best, o, 64);
-        best = ok > best ? ok : best;
+    {   // (an index fits 31 bits: a thread without values loses to every other by its index)
+        const unsigned m = wave_umax(best), w = wave_umin(best == m ? at : 0xffffffffu);
+        const bool any_bad = __any(bad);
+        if (lane == 0) wbest[tid >> 6] = make_uint2(m, w), wbad[tid >> 6] = any_bad;
     }
     __syncthreads();
-    if (bad) wbad = 1;
-    if ((tid & 63) == 0) wbest[tid >> 6] = best;
-    __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < AM_THREADS / 64; ++w) best = wbest[w] > best ? wbest[w] : best;
-        if (wbad) atomicOr(err, FNX_ERR_NONFINITE);
-        // the maximum has been taken at the device's level (its old value is back) before this block counts as arrived
-        const unsigned long long old = __hip_atomic_fetch_max(&keys[t], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long mine = old > best ? old : best;
-        asm volatile("" ::"v"(mine));
-        const unsigned long long arrived = __hip_atomic_fetch_add(&keys[FNX_MAXT + t], 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid >= 64) return;
+    const uint2 o = lane < AM_THREADS / 64 ? wbest[lane] : make_uint2(0u, 0xffffffffu);
+    const unsigned m = wave_umax(o.x), w = wave_umin(o.x == m ? o.y : 0xffffffffu);
+    const bool any_bad = __any(lane < AM_THREADS / 64 && wbad[lane] != 0);
+    if (lane == 0) {
+        if (any_bad) atomicOr(err, FNX_ERR_NONFINITE);
+        // the maximum has been taken at the device's level (its old value is back) before this block counts as arrived;
+        // nothing else passes between the blocks, so the count needs no release of the caches
+        const unsigned long long key = (unsigned long long) m << 32 | (unsigned) ~w;
+        const unsigned long long old = __hip_atomic_fetch_max(&keys[t], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::"v"(old) : "memory");
+        const unsigned long long arrived = __hip_atomic_fetch_add(&keys[FNX_MAXT + t], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (arrived == gridDim.x - 1) {
             const unsigned long long k = __hip_atomic_load(&keys[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             bv[t] = fkey_inv((unsigned) (k >> 32));

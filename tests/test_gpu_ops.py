@@ -266,6 +266,19 @@ def test_argmax_full_vocabulary(dev, oracle):
     assert bi[3] == 107 and bi[5] == 151942
 
 
+@pytest.mark.parametrize("rows", [1, 3, 63, 16383, 16384, 16385, 20000, 32771])   # ends of waves and of blocks; rows off 16-byte alignment
+def test_argmax_edges(dev, oracle, rows):
+    rng = np.random.default_rng(510 + rows)
+    logits = rng.standard_normal((5, rows)).astype(np.float32)
+    logits[1] = 0.25                                                  # every index ties
+    logits[2, rows - 1] = 9.0                                         # the last one
+    logits[3, rng.integers(0, rows, size=6)] = 9.0                    # a few tie
+    logits[4].view(np.uint32)[:] = 0xFFFFFFFF                         # the least key there is: all of them
+    bv, bi, err = dev.argmax(logits)
+    wv, wi, werr = oracle.argmax(logits)
+    assert np.array_equal(bi, wi) and np.array_equal(bv.view(np.uint32), wv.view(np.uint32)) and err == werr
+
+
 def test_argmax_flags_non_finite(dev, oracle):
     logits = np.zeros((2, 5000), dtype=np.float32)
     logits[1, 4321] = np.nan
