@@ -131,31 +131,93 @@ __device__ __forceinline__ void jm_narrow(const uint32_t* tab, const uint8_t* we
     packed_units<64, 1>(tab, we, ua, ub, cur, JobPrep<64, 1>{jb, 0, y, out, out_stride});
 }
 
+// The same for a block's first run where it leaves a wave U rows or fewer (a matrix of up to 1024 U rows a CU's block has
+// alone: the lone mat-vec). There is nothing to stream: the time is the launch and the trips to memory one after the other, so the rows
+// and the activations are asked for before the codebook is written to LDS (between() does that, and meets), and only the U rows are
+// decoded - the loop above decodes four, asks for four more, and with sixteen waves a CU that was a third of the launch.
+template <int U, class Between>
+__device__ __forceinline__ void jm_few(const uint32_t* tab, const uint8_t* we, int u0, int u1, int yi, int oi, const uint8_t* y, float* out, int out_stride,
+                                       Between between) {
+    const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6)), ua = u0 + wave * U;
+    const PackedOffs o = packed_offs(lane);
+    PackedSub cur[U];
+#pragma unroll
+    for (int r = 0; r < U; ++r) cur[r] = load_packed(as_global(uniform_ptr(we + (size_t) min(ua + r, u1 - 1) * UNIT_BYTES)), o);
+    const uint8_t* yb = y + ((size_t) yi * 64 + lane) * FNX_Q8_1_BLOCK;
+    int xs[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) xs[j] = reinterpret_cast<const int*>(yb + 4)[j];
+    const float dx = half_bits_to_float(*reinterpret_cast<const unsigned short*>(yb));
+    between();
+    float v[U];
+#pragma unroll
+    for (int r = 0; r < U; ++r) {
+        int sum = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            sum = __builtin_amdgcn_sdot4(*reinterpret_cast<const int*>(reinterpret_cast<const uint8_t*>(tab) + packed_addr(cur[r].idx, j)), xs[j], sum, false);
+        v[r] = (half_bits_to_float(cur[r].d) * dx) * (float) __mul24(sum, 1 + 2 * (int) ((cur[r].sc >> (4 * (lane & 1))) & 0xFu));
+    }
+    float* orow = out + (size_t) oi * out_stride;
+    if constexpr (U == 4) {   // (packed_units' sums)
+        const int ur = reduce4_unit_of_row(lane >> 4);
+        const float z = reduce4_units(v[0], v[1], v[2], v[3]);
+        if ((lane & 15) == 0 && ua + ur < u1) orow[ua + ur] = z;
+    } else {
+#pragma unroll
+        for (int r = 0; r < U; ++r) {
+            const float z = butterfly_sum<64>(v[r]);
+            if (lane == 63 && ua + r < u1) orow[ua + r] = z;
+        }
+    }
+}
+
 // rows of 2048 columns, a multiple of 16 of them; unit64. The blocks split the (job, 16 rows) items of all jobs evenly and
-// walk them in order, so a block streams a contiguous range of memory and changes job a few times at most.
+// walk them in order, so a block streams a contiguous range of memory and changes job a few times at most. The first run's job
+// is looked up while the codebook's entries are on their way.
+// 4,096 rows, one job of one row: 6.3 -> 4.2 us.
 __global__ void __launch_bounds__(JM_THREADS) k_iq3s_jobs_mma(const RowsArgs a) {
     __shared__ JmLds L;
-    for (int g = threadIdx.x; g < 512; g += JM_THREADS) {   // a code's sixteen signed entries from its unsigned one
-        const uint32_t g0 = g_sgrid.v[g];
-#pragma unroll
-        for (int sg = 0; sg < 16; ++sg) L.tab[sg * 512 + g] = signed_entry(g0, sg);
-    }
+    const uint32_t code = g_sgrid.v[threadIdx.x & 511];   // a code's sixteen signed entries from its unsigned one, by two threads
     const int nj = a.njobs ? min(uniform(*a.njobs), a.njobs_max) : a.njobs_max;
-    __syncthreads();
     const uint32_t gpj = (uint32_t) a.nrows / JM_ROWS;   // items per job
     const unsigned long long total = (unsigned long long) nj * gpj;
     uint32_t i = (uint32_t) (total * blockIdx.x / gridDim.x);
     const uint32_t i1 = (uint32_t) (total * (blockIdx.x + 1) / gridDim.x);
+    if (i >= i1) return;   // the same for the whole block
     const uint8_t* y = a.y ? a.y : g_moe_hq;
-    while (i < i1) {
-        const uint32_t ji = i / gpj;
-        const int g0 = (int) (i - ji * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
-        const fnx_job* jb = a.jobs + ji;
-        const int n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
-        const uint8_t* we = a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride;
-        if (n >= JM_MIN) jm_segment(L, we, g0, g1, jb, n, y, a.out, a.out_stride);
-        else if (n >= 1) jm_narrow(L.tab, we, JM_ROWS * g0, JM_ROWS * g1, jb, y, a.out, a.out_stride);
+    uint32_t ji = i / gpj;
+    int g0 = (int) (i - ji * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
+    const fnx_job* jb = a.jobs + ji;
+    int n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
+    const int y0 = uniform(jb->y[0]), out0 = uniform(jb->out[0]);
+    auto codebook = [&] {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int sg = 2 * k + (int) (threadIdx.x >> 9);
+            L.tab[sg * 512 + (threadIdx.x & 511)] = signed_entry(code, sg);
+        }
+        __syncthreads();
+    };
+    auto matrix = [&] { return a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride; };
+    bool done = true;
+    if (n == 1 && g1 - g0 == 1) jm_few<1>(L.tab, matrix(), JM_ROWS * g0, JM_ROWS * g1, y0, out0, y, a.out, a.out_stride, codebook);
+    else if (n == 1 && g1 - g0 == 2) jm_few<2>(L.tab, matrix(), JM_ROWS * g0, JM_ROWS * g1, y0, out0, y, a.out, a.out_stride, codebook);
+    else if (n == 1 && g1 - g0 <= 4) jm_few<4>(L.tab, matrix(), JM_ROWS * g0, JM_ROWS * g1, y0, out0, y, a.out, a.out_stride, codebook);
+    else codebook(), done = false;
+    while (true) {
+        if (!done) {
+            const uint8_t* we = matrix();
+            if (n >= JM_MIN) jm_segment(L, we, g0, g1, jb, n, y, a.out, a.out_stride);
+            else if (n >= 1) jm_narrow(L.tab, we, JM_ROWS * g0, JM_ROWS * g1, jb, y, a.out, a.out_stride);
+        }
+        done = false;
         i += (uint32_t) (g1 - g0);
+        if (i >= i1) break;
+        ji = i / gpj;
+        g0 = (int) (i - ji * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
+        jb = a.jobs + ji;
+        n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
     }
 }
 

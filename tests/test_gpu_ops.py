@@ -205,6 +205,16 @@ def test_gemv_iq3s_encoded_gaussian_weights(dev, oracle, packed):
         assert rel_l2(got, oracle.gemv_exact(w, nrows, ncols, x)) < 3e-2
 
 
+@pytest.mark.parametrize("nrows", [16, 4080, 4096, 4112, 8192, 8208, 16384, 16400])   # a block's run: 1, 2, 4 rows a wave, and more
+def test_gemv_iq3s_lone_row_over_unit64(dev, oracle, nrows):
+    print(f"case lone row nrows={nrows}", flush=True)
+    rng = np.random.default_rng(440 + nrows)
+    w = random_iq3s(rng, nrows * 8)
+    x = rng.standard_normal((1, 2048)).astype(np.float32)
+    got = dev.gemv_iq3s(w, nrows, 2048, x, packed=True)
+    assert rel_l2(got, oracle.gemv_iq3s(w, nrows, 2048, x)) <= 1e-6, "64 terms a row, their 32-bit sums in another order"
+
+
 # the prompt path's layout under the mat-vec operators: jobs decoded straight into the matrix cores' operands
 @pytest.mark.parametrize("nrows,ncols,T", [(4096, 2048, 16), (4096, 2048, 1), (2048, 512, 16), (1024, 2048, 3), (32, 512, 2), (64, 1024, 7),
                                            (48, 1536, 16), (16, 512, 35)])
