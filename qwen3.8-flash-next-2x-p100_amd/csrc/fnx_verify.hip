@@ -1032,8 +1032,21 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
     if (rows <= 0 || n <= 0 || n % 256) return fail(std::string(who) + ": n must be a positive multiple of 256");
     if (T < 1 || T > 65535 * FNX_MAXT) return fail(std::string(who) + ": T out of range");
     hipStream_t s = (hipStream_t) st;
-    if (!bf && T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (uint64_t) T * n * 4 < (1ull << 32) && (uint64_t) rows * n * 4 < (1ull << 32) &&
-        (((uintptr_t) W | (uintptr_t) x) & 15) == 0) {
+    // f32 weights against more rows than a window's. Tiles of 16 x 16 (k_gemv_rows_mfma16) where the larger tiles would leave CUs
+    // idle, or cannot be had; the larger ones read each row from the L2 half as often, and that is the time of a long chunk.
+    // 513 weight rows of 2048, us (small tiles / large): 77 rows 5.5 / 13.8, 200 9.7 / 14.3, 300 14.0 / 15.4, 400 18.6 / 14.9. Where
+    // the large ones cannot be had (small / k_gemv_rows_many): rows of 2048, 17 x 5.4 / 12.7, 63 x 5.5 / 12.8; of 1024, 200 x 7.5 / 8.6,
+    // 700 x 19.4 / 22.2.
+    const bool large = !bf && T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (uint64_t) T * n * 4 < (1ull << 32) &&
+                       (uint64_t) rows * n * 4 < (1ull << 32) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
+    const long small_tiles = (long) ((T + RS_TILE - 1) / RS_TILE) * ((rows + RS_TILE - 1) / RS_TILE);
+    if (!bf && T > FNX_MAXT && n % (2 * RS_COLS) == 0 && small_tiles < (1l << 24) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0 &&
+        (!large || small_tiles <= 5l * cu_count() / 2)) {
+        const int ntt = (T + RS_TILE - 1) / RS_TILE, net = (rows + RS_TILE - 1) / RS_TILE;
+        k_gemv_rows_mfma16<<<(unsigned) ((small_tiles + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
+        return launch_status(who);
+    }
+    if (large) {
         // a chunk's worth of rows against f32 weights: tiles of 32 x 32 sums on the matrix cores. The weight rows past the
         // last full 32 ride with the tiles' blocks, an item a block (a row x four rows of x); if there are more items
         // than blocks in a row of tiles, those rows go to the kernel below.

@@ -269,6 +269,111 @@ __global__ void __launch_bounds__(GM_WAVES * 64) k_gemv_rows_many(const void* __
     gemv_rows_many_wave<BF>(Wv, x, y, rows, n, T, row_begin + (blockIdx.x * GM_WAVES + wave) * GR_ROWS, blockIdx.y, lane);
 }
 
+// ---------------------------------------------------------------- the same sums in tiles of 16 x 16, for a short chunk
+// A chunk of a few hundred rows leaves the kernel below (tiles of 32 x 32: 48 blocks for 77 rows against 513 weight rows) with
+// CUs that have no tile or one, and a tile's chain of 512 MFMAs of 64 cycles a wave is its time. Here a tile is 16 x 16
+// and the instruction v_mfma_f32_16x16x1_4b_f32: its four blocks take lanes l, l + 16, l + 32 and l + 48 of the fixed order
+// (the butterfly's levels 32 and 16 are adds within the accumulator), wave w of four takes l = 4 w + j, four independent chains
+// of n / 64 MFMAs of 32 cycles that it goes through together - a quarter of the tile's work in a quarter of the time, on
+// four times the blocks. Levels 8 and 4 add the waves' sums, levels 2 and 1 the chains', through LDS at the end.
+// Operands: a stage is 256 columns of the tile's 16 + 16 rows, a row 1 KiB and a wave instruction (two loader waves, straight
+// into LDS, two stages ahead, one of three buffers); rows lie 1,040 bytes apart, so that the 16 rows an operand read
+// touches fall on 16 different bank groups. The waves multiply a stage while the next one's operands are read.
+// Bound by what the XCDs' L2s hand over (256 KB a tile; some 10 TB/s in all) once every CU has a tile: 77 rows x 513 of 2048,
+// 13.8 -> 5.5 us.
+typedef float rs_v16f __attribute__((ext_vector_type(16)));
+constexpr int RS_TILE = 16, RS_WAVES = 4, RS_LOADERS = 2, RS_THREADS = (RS_WAVES + RS_LOADERS) * 64, RS_COLS = 256, RS_ROWLD = RS_COLS * 4 + 16,
+              RS_STAGE = 2 * RS_TILE * RS_ROWLD, RS_BUFS = 3;
+__global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __restrict__ W, const float* __restrict__ x, float* __restrict__ y, int rows,
+                                                                int n, int T, int ntt, int net) {
+    __shared__ __align__(16) uint8_t lds[RS_BUFS * RS_STAGE];
+    __shared__ __align__(16) float red[RS_WAVES][4][64][4];   // [wave][chain][lane][row of the lane's four]
+    const int wave = uniform((int) (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    // an XCD's blocks (every eighth) take neighbouring tiles, a tile of W against all of x's: its L2 then holds what they share
+    const int lin = ((int) blockIdx.x % 8) * ((int) gridDim.x / 8) + (int) blockIdx.x / 8, et = lin / ntt, tt = lin - et * ntt;
+    if (et >= net) return;
+    const int t0 = tt * RS_TILE, e0 = et * RS_TILE, S = n / RS_COLS;   // stages: an even number, two at least
+    const uint32_t lds_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
+    auto meet = [&](bool newest_in_flight) {   // (see k_gemv_rows_mfma's)
+        __builtin_amdgcn_sched_barrier(0);
+        if (newest_in_flight) __builtin_amdgcn_s_waitcnt(0x4070);   // vmcnt(16) lgkmcnt(0)
+        else __builtin_amdgcn_s_waitcnt(0x0070);                    // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (wave >= RS_WAVES) {   // a loader: the first takes the stages' rows of W, the second those of x
+        const int lw = wave - RS_WAVES;
+        const uint8_t* from[RS_TILE];
+#pragma unroll
+        for (int j = 0; j < RS_TILE; ++j)   // (past the last row: that one again)
+            from[j] = reinterpret_cast<const uint8_t*>(lw == 0 ? W + (size_t) min(e0 + j, rows - 1) * n : x + (size_t) min(t0 + j, T - 1) * n);
+        auto fetch = [&](int k, int buf) {
+#pragma unroll
+            for (int j = 0; j < RS_TILE; ++j)
+                lds_load16(from[j] + (size_t) k * (RS_COLS * 4), 16u * lane, lds_at + buf * RS_STAGE + (lw * RS_TILE + j) * RS_ROWLD);
+        };
+        fetch(0, 0);
+        fetch(1, 1);
+        int buf = 2;
+        for (int k = 0; k < S; ++k) {
+            meet(k + 1 < S);   // stage k has landed; stage k - 1 has been read
+            if (k + 2 < S) fetch(k + 2, buf);
+            buf = buf == RS_BUFS - 1 ? 0 : buf + 1;
+        }
+        return;   // (a wave that has ended counts as arrived at the last meeting)
+    }
+    const int i = lane & 15, b = lane >> 4;
+    const uint8_t* row = lds + i * RS_ROWLD + 16 * (16 * b + 4 * wave);   // row i of W (of x: 16 rows on), chains 4 wave .. + 3 of block b
+    float4 A[2][4], B[2][4];
+    rs_v16f acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+    int at = 0;   // the buffer that is read next
+    auto read = [&](float4(&a)[4], float4(&bb)[4]) {
+        meet(false);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            a[j] = *reinterpret_cast<const float4*>(row + at + 16 * j);
+            bb[j] = *reinterpret_cast<const float4*>(row + at + RS_TILE * RS_ROWLD + 16 * j);
+        }
+        at = at == (RS_BUFS - 1) * RS_STAGE ? 0 : at + RS_STAGE;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const float4(&a)[4], const float4(&bb)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[j].x, bb[j].x, acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[j].y, bb[j].y, acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[j].z, bb[j].z, acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[j].w, bb[j].w, acc[j], 0, 0, 0);
+    };
+    read(A[0], B[0]);
+    for (int k = 0; k < S; k += 2) {
+        read(A[1], B[1]);
+        multiply(A[0], B[0]);
+        if (k + 2 < S) read(A[0], B[0]);
+        multiply(A[1], B[1]);
+    }
+    // block q's sums lie in registers 4 q .. 4 q + 3: weight rows 4 b .. 4 b + 3 of the tile against row i of x
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float f[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f[r] = (acc[j][r] + acc[j][8 + r]) + (acc[j][4 + r] + acc[j][12 + r]);
+        *reinterpret_cast<float4*>(red[wave][j][lane]) = make_float4(f[0], f[1], f[2], f[3]);
+    }
+    meet(false);
+    const int e = e0 + 4 * b + wave, t = t0 + i;   // this wave's row of each lane's four
+    float s[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = (red[0][j][lane][wave] + red[2][j][lane][wave]) + (red[1][j][lane][wave] + red[3][j][lane][wave]);
+    if (e < rows && t < T) y[(size_t) t * rows + e] = (s[0] + s[2]) + (s[1] + s[3]);
+}
+
 // ---------------------------------------------------------------- the same sums on the matrix cores
 // v_mfma_f32_32x32x1_2b_f32 is D = fma(a, b, D) element by element with one rounding - the fmaf of the chains above
 // (checked bit for bit on this GPU, products in the denormal range included). A chain of them over the chunks

@@ -60,6 +60,16 @@ def test_gemv_f32_many_rows_bit_exact(dev, oracle, rows, n, T):
     assert np.array_equal(dev.gemv(W, x).view(np.uint32), oracle.gemv_f32(W, x).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,n,T", [(513, 2048, 17), (513, 2048, 77), (1, 512, 18), (15, 1024, 33), (48, 4096, 31), (130, 512, 250)])
+def test_gemv_f32_short_chunks_bit_exact(dev, oracle, rows, n, T):
+    print(f"case short chunk rows={rows} n={n} T={T}", flush=True)
+    rng = np.random.default_rng(33 + rows + T)
+    w, x = rng.standard_normal((rows, n)).astype(np.float32), rng.standard_normal((T, n)).astype(np.float32)
+    w[:, ::7] *= np.float32(1e-22)   # products in the denormal range among them
+    x[:, ::7] *= np.float32(1e-20)
+    assert np.array_equal(dev.gemv(w, x).view(np.uint32), oracle.gemv_f32(w, x).view(np.uint32))
+
+
 def test_gemv_f32_sum_does_not_depend_on_T(dev):
     """A size-independent property at a size the oracle takes long for: a sum's bits do not depend on how many rows of x a
     call brings, so 4,099 rows in one call (the matrix cores' tiles, several patches of them, a ragged last tile, the 513th
