@@ -1591,7 +1591,7 @@ int fnx_embed_rows(const uint16_t* emb, const int* tokens, int T, int vocab, int
 }
 // (the forms of the kernel for a launch with a device-side row count: defined at the end of this file)
 static bool q8s_live_lds(int bytes);
-static void q8s_live_launch(bool tiled, int grid, size_t lds, hipStream_t st, const Q8sArgs& a);
+static void q8s_live_launch(bool tiled, int one, int grid, size_t lds, hipStream_t st, const Q8sArgs& a);
 // yq2 (may be null): two matrices, the second one over rows of its own - as long as every block has one tile, which is then of
 // one matrix (else refused: the caller launches twice)
 // live (may be null): a device word, the rows that count; the others are not read and their products are zeros
@@ -1623,6 +1623,8 @@ static int q8s_launch(const fnx_q8s* const* W, float* const* out, const int* out
     if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !attr_set[dev]) {
         if (hipFuncSetAttribute((const void*) k_q8s_gemv<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess ||
             hipFuncSetAttribute((const void*) k_q8s_gemv<1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess ||
+            hipFuncSetAttribute((const void*) k_q8s_gemv<1, true, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess ||
+            hipFuncSetAttribute((const void*) k_q8s_gemv<1, true, false, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess ||
             !q8s_live_lds(150 * 1024))
             return fail(std::string(who) + ": cannot raise the dynamic LDS limit");
         attr_set[dev] = true;
@@ -1635,7 +1637,12 @@ static int q8s_launch(const fnx_q8s* const* W, float* const* out, const int* out
         if (n != 2 || grid < tiles) return fail(std::string(who) + ": two sets of rows want two matrices and a block a tile");
         a.yq2 = (const uint8_t*) yq2;
     }
-    if (live) q8s_live_launch(W[0]->tiled != 0, grid, lds, (hipStream_t) st, a);
+    // a block a tile, of rows of 2048 or 4096 columns: the form that asks for a tile's weights at once (the other sizes have one
+    // batch a wave, or more than the registers hold)
+    const int one = W[0]->tiled && grid >= tiles && (a.cols == 2048 || a.cols == 4096) ? a.cols / 1024 : 0;
+    if (live) q8s_live_launch(W[0]->tiled != 0, one, grid, lds, (hipStream_t) st, a);
+    else if (one == 2) k_q8s_gemv<1, true, false, 2><<<grid, Q8S_WAVES * 64, lds, (hipStream_t) st>>>(a);
+    else if (one == 4) k_q8s_gemv<1, true, false, 4><<<grid, Q8S_WAVES * 64, lds, (hipStream_t) st>>>(a);
     else if (W[0]->tiled) k_q8s_gemv<1, true><<<grid, Q8S_WAVES * 64, lds, (hipStream_t) st>>>(a);
     else k_q8s_gemv<1><<<grid, Q8S_WAVES * 64, lds, (hipStream_t) st>>>(a);
     return launch_status(who);
@@ -2287,10 +2294,15 @@ int fnx_gguf_load_moe_layer(const fnx_gguf* g, int layer, int ff0, int ff1, int 
 // The dense mat-vec's forms for a launch with a device-side row count (k_q8s_gemv<.., LIVE = true>), asked for here, after
 // everything else, so that the kernels before them lie in the code object where they lay without them.
 static bool q8s_live_lds(int bytes) {
-    return hipFuncSetAttribute((const void*) fnx::k_q8s_gemv<1, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*) fnx::k_q8s_gemv<1, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    const void* const forms[4] = {(const void*) fnx::k_q8s_gemv<1, false, true>, (const void*) fnx::k_q8s_gemv<1, true, true>,
+                                  (const void*) fnx::k_q8s_gemv<1, true, true, 2>, (const void*) fnx::k_q8s_gemv<1, true, true, 4>};
+    for (const void* f : forms)
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
+    return true;
 }
-static void q8s_live_launch(bool tiled, int grid, size_t lds, hipStream_t st, const fnx::Q8sArgs& a) {
-    if (tiled) fnx::k_q8s_gemv<1, true, true><<<grid, fnx::Q8S_WAVES * 64, lds, st>>>(a);
+static void q8s_live_launch(bool tiled, int one, int grid, size_t lds, hipStream_t st, const fnx::Q8sArgs& a) {
+    if (one == 2) fnx::k_q8s_gemv<1, true, true, 2><<<grid, fnx::Q8S_WAVES * 64, lds, st>>>(a);
+    else if (one == 4) fnx::k_q8s_gemv<1, true, true, 4><<<grid, fnx::Q8S_WAVES * 64, lds, st>>>(a);
+    else if (tiled) fnx::k_q8s_gemv<1, true, true><<<grid, fnx::Q8S_WAVES * 64, lds, st>>>(a);
     else fnx::k_q8s_gemv<1, false, true><<<grid, fnx::Q8S_WAVES * 64, lds, st>>>(a);
 }

@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
                                                                   float eps) {
     __shared__ float sh[4];
     __shared__ float vrow[WIDE ? 256 * NQ_MAXJ : 1];
-    if (c.gate && uniform(*c.gate) == 0) return;
+    const int gate_v = c.gate ? *c.gate : 1;   // (looked at when the row is on its way: a trip to memory of its own otherwise)
     size_t row = blockIdx.x;
     const uint16_t* emb = c.emb;
     if (!WIDE && c.rows2 > 0 && (int) blockIdx.x >= c.rows1) {   // the launch's second pass
@@ -69,9 +69,10 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
         x = c.x2, w = c.w2, xq = c.xq2, emb = c.emb2;
         xn = nullptr, add = nullptr;
     }
-    float v[NQ_MAXJ];
+    float v[NQ_MAXJ], wv[NQ_MAXJ];
     float s = 0.f;
     if constexpr (WIDE) {
+        if (uniform(gate_v) == 0) return;
         // the combine's chains (k_combine's order: the picks ascending), NQ_KB experts' partial sums of this thread's
         // columns in flight at a time (one by one, each load would be a trip to the cache of its own)
         constexpr int NQ_KB = 5, NQ_WJ = NQ_MAXJ / 4;
@@ -122,6 +123,11 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
         if (threadIdx.x >= 256) return;
 #pragma unroll
         for (int j = 0; j < NQ_MAXJ; ++j) v[j] = vrow[threadIdx.x + 256 * j];
+#pragma unroll
+        for (int j = 0; j < NQ_MAXJ; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            wv[j] = i < n ? w[i] : 0.f;
+        }
     } else {
         // all loads first: a store to x between them would keep the next load waiting for it
         float av[NQ_MAXJ];
@@ -133,16 +139,16 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
             else v[j] = i < n ? x[row * n + i] : 0.f;
             av[j] = add && i < n ? add[row * n + i] : 0.f;
         }
+#pragma unroll
+        for (int j = 0; j < NQ_MAXJ; ++j) {   // the norm's weights too
+            const int i = threadIdx.x + 256 * j;
+            wv[j] = i < n ? w[i] : 0.f;
+        }
+        if (uniform(gate_v) == 0) return;
         if (add && (!c.live || (int) row < *c.live)) {
 #pragma unroll
             for (int j = 0; j < NQ_MAXJ; ++j) v[j] += av[j];
         }
-    }
-    float wv[NQ_MAXJ];   // the norm's weights too, before any store
-#pragma unroll
-    for (int j = 0; j < NQ_MAXJ; ++j) {
-        const int i = threadIdx.x + 256 * j;
-        wv[j] = i < n ? w[i] : 0.f;
     }
     if (!WIDE && (add || emb)) {
 #pragma unroll
@@ -237,20 +243,26 @@ typedef int q8s_v4i __attribute__((ext_vector_type(4)));
 // (read once). 4.7 against 4.1 TB/s for the output head; with the policy alone, over rows, 3.9.
 // LIVE: a.live is set (a launch of its own: the word is then read on every path, through the scalar unit, and waiting for it
 // does not wait for the weights on their way).
-template <int DEPTH, bool TILED = false, bool LIVE = false>
+// ONE: a block a tile, of rows of 1024 ONE columns (the projections of a layer: a few hundred tiles). Such a launch is its chain
+// of trips to memory - 1.8 us each for weights nobody has read lately: all ONE batches of a wave's quarter go out at once,
+// before the gate's word is looked at and before the activations are staged. 2,048 rows of 4,096 columns, one row:
+// 9.2 -> 6.4 us; 9,216 of 2,048: 9.0 -> 7.2.
+template <int DEPTH, bool TILED = false, bool LIVE = false, int ONE = 0>
 __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
     typedef __attribute__((address_space(1))) const at_v4u_t g128;
     extern __shared__ __align__(16) uint8_t q8s_lds[];   // [16][cols + pad] int8, [16][nb + 2] f32 scales, [3][64][4] partial sums
-    if (a.gate && uniform(*a.gate) == 0) return;
-    const int nb = a.cols >> 5, T = a.T, xld = a.cols + Q8S_XPAD, dld = nb + 2;
+    const int gate_v = a.gate ? *a.gate : 1, live_v = LIVE ? *a.live : a.T;   // (asked for together, looked at when the first weights are on their way)
+    const int nb = ONE ? 32 * ONE : a.cols >> 5, T = a.T, xld = a.cols + Q8S_XPAD, dld = nb + 2;
     int8_t* xs = reinterpret_cast<int8_t*>(q8s_lds);
     float* xd = reinterpret_cast<float*>(q8s_lds + (size_t) FNX_MAXT * xld);
     float* part = xd + FNX_MAXT * dld;
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
     const int t0 = (a.seg[0].rows + 15) / 16, t1 = t0 + (a.nseg > 1 ? (a.seg[1].rows + 15) / 16 : 0),
               tiles = t1 + (a.nseg > 2 ? (a.seg[2].rows + 15) / 16 : 0);
-    const int nq4 = a.cols >> 8;   // double steps per wave: a quarter of cols / 64
+    const int nq4 = ONE ? Q8S_BATCH * ONE : a.cols >> 8;   // double steps per wave: a quarter of cols / 64
     const bool lo_groups = g < 2;
+    const int Tl = LIVE ? max(1, min(uniform(live_v), T)) : T;   // (a window of a decode round: most of its sixteen rows do not count)
+    const int xr = min(r16, Tl - 1);   // a lane of a row that does not count works on the last one's values, and its sums are thrown away
     const int j0 = wave * nq4;     // this wave's first double step
     struct Tile {
         gbytes wrow, drow[4];
@@ -304,8 +316,8 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
         for (int u = 0; u < Q8S_BATCH; ++u)
             if (u < nstep) {
                 const int j = j0 + jb + u;
-                const at_v4u_t x = *reinterpret_cast<const at_v4u_t*>(xs + (size_t) r16 * xld + 64 * j + 16 * g);
-                const float2 dx = *reinterpret_cast<const float2*>(xd + r16 * dld + 2 * j);
+                const at_v4u_t x = *reinterpret_cast<const at_v4u_t*>(xs + (size_t) xr * xld + 64 * j + 16 * g);
+                const float2 dx = *reinterpret_cast<const float2*>(xd + xr * dld + 2 * j);
                 const long wl = (long) in.w[u].x | (long) in.w[u].y << 32, wh = (long) in.w[u].z | (long) in.w[u].w << 32;
                 const long xl = (long) x.x | (long) x.y << 32, xh = (long) x.z | (long) x.w << 32;
                 const long xl0 = lo_groups ? xl : 0, xh0 = lo_groups ? xh : 0, xl1 = lo_groups ? 0 : xl, xh1 = lo_groups ? 0 : xh;
@@ -331,7 +343,7 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
                                 (p0.w + p1.w) + (p2.w + p3.w)};
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (c.row0 + 4 * g + r < c.rows) c.out[r] = v[r];
+                if (c.row0 + 4 * g + r < c.rows) c.out[r] = !LIVE || r16 < Tl ? v[r] : 0.f;   // rows from *live on: zeros
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = 0.f;
@@ -354,34 +366,38 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
         }
     };
     Cursor lc{(int) blockIdx.x, 0, true, tile_of(blockIdx.x)}, cc = lc;   // the loads' place and the arithmetic's
-    Batch ring[DEPTH + 1];
+    Batch ring[ONE ? ONE : DEPTH + 1];
+    if constexpr (ONE) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d)
-        if (lc.valid) {
-            load(lc.t, lc.jb, ring[d]);
-            advance(lc);
-        }
+        for (int d = 0; d < ONE; ++d) load(lc.t, Q8S_BATCH * d, ring[d]);
+    } else {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+            if (lc.valid) {
+                load(lc.t, lc.jb, ring[d]);
+                advance(lc);
+            }
+    }
+    if (uniform(gate_v) == 0) return;
     // the window's q8_1 rows into LDS (the first weights are on their way meanwhile). The copy takes 3 us (6-7 us in a
     // launch of 1,024 blocks, beside their weight loads) whatever the width of its loads - nine 16-byte loads for four
     // blocks of a row were no faster than 4-byte ones - and wherever in the rows a block starts.
-    int Tl = T;   // (a window of a decode round: most of its sixteen rows do not count)
-    if constexpr (LIVE) Tl = max(1, min(*a.live, T));
-    for (int i = threadIdx.x; i < FNX_MAXT * nb; i += blockDim.x) {
+    for (int i = threadIdx.x; i < Tl * nb; i += blockDim.x) {
         const int t = i / nb, b = i - t * nb;
         uint32_t* dst = reinterpret_cast<uint32_t*>(xs + (size_t) t * xld + 32 * b);
-        if (t < Tl) {
-            const uint8_t* blk = (a.yq2 && (int) blockIdx.x >= t0 ? a.yq2 : a.yq) + (size_t) i * 36;
-            xd[t * dld + b] = half_bits_to_float(load_u16(blk));
-            const uint32_t* src = reinterpret_cast<const uint32_t*>(blk + 4);
+        const uint8_t* blk = (a.yq2 && (int) blockIdx.x >= t0 ? a.yq2 : a.yq) + (size_t) i * 36;
+        xd[t * dld + b] = half_bits_to_float(load_u16(blk));
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(blk + 4);
 #pragma unroll
-            for (int k = 0; k < 8; ++k) dst[k] = src[k];
-        } else {   // rows past the window: zeros, so their lanes' products stay finite
-            xd[t * dld + b] = 0.f;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) dst[k] = 0u;
-        }
+        for (int k = 0; k < 8; ++k) dst[k] = src[k];
     }
     __syncthreads();
+    if constexpr (ONE) {
+#pragma unroll
+        for (int d = 0; d < ONE; ++d) compute(Q8S_BATCH * d, ring[d]);
+        finish(cc.t);
+        return;
+    }
     while (cc.valid) {
 #pragma unroll
         for (int slot = 0; slot <= DEPTH; ++slot) {
