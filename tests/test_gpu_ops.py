@@ -344,6 +344,21 @@ def test_lookup_device_matches_oracle(dev, oracle, key_n):
         assert list(got) == list(want) and match == wmatch, c
 
 
+@pytest.mark.parametrize("key_n", [1, 2, 3, 4])
+def test_lookup_finds_a_key_across_the_seams_of_its_loads(dev, oracle, key_n):
+    """the key's only earlier place at every offset around a lane's 4 positions, a wave's 252, a block's 16 x 252 and a round's 64,512"""
+    rng = np.random.default_rng(640 + key_n)
+    for n, seams in [(300, (4, 252, 296)), (9000, (252, 504, 4032, 8990)), (70001, (60480, 64512, 69990))]:
+        base = rng.integers(1000, 100000, size=n).astype(np.int32)
+        base[-key_n:] = np.arange(key_n) + 1
+        for at in sorted({s + d for s in seams for d in range(-5, 5) if 0 <= s + d < n - 2 * key_n}):
+            c = base.copy()
+            c[at:at + key_n] = c[-key_n:]
+            got, match = dev.lookup(c, 15, -1, key_n)
+            want, wmatch = oracle.lookup_drafts(c, 15, -1, key_n)
+            assert list(got) == list(want) and match == wmatch == at, (n, at)
+
+
 def test_accept_device_matches_oracle(dev, oracle):
     rng = np.random.default_rng(700)
     for _ in range(64):
