@@ -94,6 +94,19 @@ def test_pf_route_with_fewer_finite_logits_than_picks(dev, oracle):
     assert np.array_equal(r["cnt"], cnt) and r["njobs"] == len(gu)
 
 
+@pytest.mark.parametrize("nexp,topk", [(3, 3), (64, 64), (65, 10), (513, 10), (1024, 64)])
+def test_pf_route_ties_and_signed_zeros(dev, oracle, nexp, topk):
+    """values from a handful (both zeros, both infinities' neighbours among them): ties within a lane's entries and across lanes"""
+    print(f"case pf_route ties nexp={nexp} topk={topk}", flush=True)
+    rng = np.random.default_rng(706 + nexp)
+    values = np.array([0.0, -0.0, 1.0, -1.0, 0.5, 1e-40, -1e-40, -88.0, np.finfo(np.float32).min], dtype=np.float32)
+    logits = values[rng.integers(0, len(values), (37, nexp + 1))]
+    r = dev.pf_route(logits, nexp, topk)
+    topi, topw = oracle.topk_logits(logits, nexp, topk)
+    assert np.array_equal(r["topi"], topi)
+    assert np.allclose(r["topw"], topw, rtol=2e-6, atol=0)
+
+
 def test_f32_f16_bit_exact(dev, oracle):
     rng = np.random.default_rng(710)
     x = (rng.standard_normal((33, 257)) * 10.0 ** rng.integers(-8, 4, (33, 257))).astype(np.float32)
