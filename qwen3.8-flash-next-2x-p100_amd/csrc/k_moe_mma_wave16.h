@@ -28,53 +28,89 @@ struct Wave16Lds {
     int first_job, first_tile, last_job, last_tile;   // the block's run: from (first_job, first_tile) up to but not including (last_job, last_tile)
     uint8_t jn[2][W16_HELD];                          // the token counts of the two lists' jobs, as far as they fit
     int jw[W16_HELD];                                 // the first list's matrices
+    int orow[FNX_PF_JOB];                             // the job's tokens' rows of the output
 };
 
-// A tile's super-step: the lane's four sub-blocks of its row (fields f) as f16 operands, against the nt token tiles of
+// f16(a0 b0) | f16(a1 b1) << 16, each product rounded once and a product that vanishes a positive zero: what the compiler makes
+// of k_swiglu_h16's expression. Left to itself it takes a multiplication and a conversion in one place and this in the next,
+// and a row's h would depend on the size of the job it falls in.
+__device__ __forceinline__ uint32_t h16_pair(float a0, float b0, float a1, float b1) {
+    uint32_t v;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0" : "=&v"(v) : "v"(a0), "v"(b0), "v"(a1), "v"(b1));
+    return v;
+}
+// A lane's half of a sub-block (fields s) as two f16 operands: weights 16 h .. 16 h + 15
+__device__ __forceinline__ void w16_half(const uint2* tab, const SubFields& s, int h, v8h (&A)[2]) {
+    const _Float16 c = (_Float16) (int) (1 + 2 * s.sc), d = __builtin_bit_cast(_Float16, (unsigned short) s.d);
+    const v2h s2 = {c, c}, d2 = {d, d};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint2 en = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(tab) + sub_entry<true>(s, 4 * h + k));
+        const v2h lo = (as_v2h(en.x) * s2) * d2, hi = (as_v2h(en.y) * s2) * d2;
+        A[k >> 1][4 * (k & 1) + 0] = lo.x;
+        A[k >> 1][4 * (k & 1) + 1] = lo.y;
+        A[k >> 1][4 * (k & 1) + 2] = hi.x;
+        A[k >> 1][4 * (k & 1) + 3] = hi.y;
+    }
+}
+// A tile's super-step: the lane's four sub-blocks of its row (fields f) as f16 operands, against the NT token tiles of
 // the activation tile in LDS (xlane: token r's row at this lane group's sub-blocks), added to acc
-__device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* xlane, const SuperFields& f, int nt, v4f (&acc)[MB_TP]) {
-    // the token tiles two at a time against the sub-block's operands
-    auto pair = [&](const v8h (&A)[4], int p, auto t0_tag, auto cnt_tag) {
-        constexpr int T0 = decltype(t0_tag)::value, CNT = decltype(cnt_tag)::value;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {   // two of the four operands at a time: the registers of a block of 1024 threads
-            v4u B[2][2];
-#pragma unroll
-            for (int tt = 0; tt < CNT; ++tt)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) B[tt][i] = *reinterpret_cast<const v4u*>(xlane + (T0 + tt) * 16 * W16_XROW + 64 * p + 32 * h + 16 * i);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int tt = 0; tt < CNT; ++tt)
-                    acc[T0 + tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[2 * h + i], __builtin_bit_cast(v8h, B[tt][i]), acc[T0 + tt], 0, 0, 0);
-        }
-    };
+template <int NT>
+__device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* xlane, const SuperFields& f, v4f (&acc)[NT]) {
     auto step = [&](auto p_c) {
         constexpr int p = decltype(p_c)::value;
         const SubFields s = super_sub<p>(f);
-        const _Float16 sc = (_Float16) (int) (1 + 2 * s.sc), d = __builtin_bit_cast(_Float16, (unsigned short) s.d);
-        const v2h s2 = {sc, sc}, d2 = {d, d};
-        v8h A[4];   // the lane's sub-block (row r, 4 grp + p) as 32 f16 weights
+        v8h A[2][2];
+        w16_half(tab, s, 0, A[0]);
+        w16_half(tab, s, 1, A[1]);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint2 en = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(tab) + sub_entry<true>(s, k));
-            const v2h lo = (as_v2h(en.x) * s2) * d2, hi = (as_v2h(en.y) * s2) * d2;
-            A[k >> 1][4 * (k & 1) + 0] = lo.x;
-            A[k >> 1][4 * (k & 1) + 1] = lo.y;
-            A[k >> 1][4 * (k & 1) + 2] = hi.x;
-            A[k >> 1][4 * (k & 1) + 3] = hi.y;
-        }
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        using I2 = std::integral_constant<int, 2>;
-        if (nt >= 2) pair(A, p, I0{}, I2{});
-        else pair(A, p, I0{}, I1{});
-        if (nt == 3) pair(A, p, I2{}, I1{});
-        else if (nt == 4) pair(A, p, I2{}, I2{});
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[h][i], *reinterpret_cast<const v8h*>(xlane + tt * 16 * W16_XROW + 64 * p + 32 * h + 16 * i),
+                                                                     acc[tt], 0, 0, 0);
     };
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
+}
+
+// Two tiles' super-steps against the same NT token tiles (fields f0 and f1, sums acc0 and acc1): an operand of the activation
+// tile read from LDS once for both. Half a sub-block of either tile is decoded at a time, so that the decoded operands take
+// the registers that one tile's whole sub-block takes above. between: run between the second and the third of the four
+// steps, where the first half of the fields is dead (loads of what comes next find registers there). Every sum is
+// accumulated as w16_super_step does it.
+template <int NT, class Between>
+__device__ __forceinline__ void w16_super_pair(const uint2* tab, const uint8_t* xlane, const SuperFields& f0, const SuperFields& f1, v4f (&acc0)[NT],
+                                               v4f (&acc1)[NT], Between between) {
+    auto step = [&](auto p_c) {
+        constexpr int p = decltype(p_c)::value;
+        const SubFields sa = super_sub<p>(f0), sb = super_sub<p>(f1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v8h A0[2], A1[2];
+            w16_half(tab, sa, h, A0);
+            w16_half(tab, sb, h, A1);
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) {
+                v4u B[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) B[i] = *reinterpret_cast<const v4u*>(xlane + tt * 16 * W16_XROW + 64 * p + 32 * h + 16 * i);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    acc0[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0[i], __builtin_bit_cast(v8h, B[i]), acc0[tt], 0, 0, 0);
+                    acc1[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1[i], __builtin_bit_cast(v8h, B[i]), acc1[tt], 0, 0, 0);
+                }
+            }
+        }
+    };
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+    __builtin_amdgcn_sched_barrier(0);
+    between();
     step(std::integral_constant<int, 2>{});
     step(std::integral_constant<int, 3>{});
 }
@@ -190,7 +226,9 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
         int y[MB_TP];
 #pragma unroll
         for (int i = 0; i < MB_TP; ++i) y[i] = ahead == j ? yahead[i] : uniform(jb->y[min(wave + 16 * i, n - 1)]);
+        const int oput = tid < n ? jb->out[tid] : -1;   // (up to 64 tokens: the first wave)
         __syncthreads();   // the job before has been read
+        if (tid < FNX_PF_JOB) L.orow[tid] = oput;
 #pragma unroll
         for (int i = 0; i < MB_TP; ++i)   // a token's row a wave instruction, 16 bytes a lane
             if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
@@ -201,34 +239,50 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
             for (int i = 0; i < MB_TP; ++i) yahead[i] = uniform(jn->y[max(0, min(wave + 16 * i, nn - 1))]);
             ahead = j + 1;
         }
-        int orow[MB_TP];
+        auto run = [&](auto nt_tag) {
+            constexpr int NT = decltype(nt_tag)::value;
+            auto put = [&](const v4f (&acc)[NT], int g) {   // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
 #pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) orow[tt] = tt * 16 + r < n ? jb->out[tt * 16 + r] : -1;
-        int g = g0 + wave;
-        SuperFields f = tile16_load(we, 16 * min(g, g1 - 1) + r, 0, 1);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        for (; g < g1; g += W16_WAVES) {
-            // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
-            // for the last: every wave takes every priority in turn, a tile each
-            switch (((wave >> 2) + ((g - g0) >> 4)) & 3) {
-                case 0: __builtin_amdgcn_s_setprio(0); break;
-                case 1: __builtin_amdgcn_s_setprio(1); break;
-                case 2: __builtin_amdgcn_s_setprio(2); break;
-                default: __builtin_amdgcn_s_setprio(3); break;
+                for (int tt = 0; tt < NT; ++tt) {
+                    const int orow = L.orow[tt * 16 + r];
+                    if (orow >= 0) *reinterpret_cast<float4*>(a.out + (size_t) orow * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
+                }
+            };
+            // the wave's tiles g, g + 16, .. two at a time, the next two's fields asked for in the middle of the two before (past
+            // the run's last tile: that one again)
+            int g = g0 + wave;
+            auto fields = [&](int t) { return tile16_load_buf(tile16_rsrc(we, min(t, g1 - 1), 1), 0); };
+            SuperFields f0 = fields(g), f1 = fields(g + W16_WAVES);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            for (; g < g1; g += 2 * W16_WAVES) {
+                // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
+                // for the last: every wave takes every priority in turn, two tiles each
+                switch (((wave >> 2) + ((g - g0) >> 5)) & 3) {
+                    case 0: __builtin_amdgcn_s_setprio(0); break;
+                    case 1: __builtin_amdgcn_s_setprio(1); break;
+                    case 2: __builtin_amdgcn_s_setprio(2); break;
+                    default: __builtin_amdgcn_s_setprio(3); break;
+                }
+                v4f acc0[NT], acc1[NT];
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) acc0[tt] = acc1[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+                if (g + W16_WAVES < g1) {
+                    SuperFields n0, n1;
+                    w16_super_pair<NT>(L.tab, xlane, f0, f1, acc0, acc1, [&] { n0 = fields(g + 2 * W16_WAVES), n1 = fields(g + 3 * W16_WAVES); });
+                    put(acc0, g);
+                    put(acc1, g + W16_WAVES);
+                    f0 = n0, f1 = n1;
+                } else {   // the run's last round, where it has an odd number of them
+                    w16_super_step<NT>(L.tab, xlane, f0, acc0);
+                    put(acc0, g);
+                }
             }
-            const SuperFields nf = tile16_load(we, 16 * (g + W16_WAVES < g1 ? g + W16_WAVES : g) + r, 0, 1);
-            v4f acc[MB_TP];
-#pragma unroll
-            for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-            w16_super_step(L.tab, xlane, f, nt, acc);
-            // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
-#pragma unroll
-            for (int tt = 0; tt < MB_TP; ++tt)
-                if (orow[tt] >= 0)
-                    *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
-            f = nf;
-        }
+        };
+        if (nt == 4) run(std::integral_constant<int, 4>{});
+        else if (nt == 3) run(std::integral_constant<int, 3>{});
+        else if (nt == 2) run(std::integral_constant<int, 2>{});
+        else run(std::integral_constant<int, 1>{});
     }
 }
 
@@ -244,15 +298,24 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
 // that every block comes near the mean load. The weights of the next tile's super-step are asked for a tile ahead. Every
 // tile is accumulated in one order (S, then the four steps, then a step's four operands) whatever a job's size or the
 // unit it falls in: a row's h does not depend on what else is in the chunk.
+// Costs, in 1/16 us at S = 4 (measured): a heavy unit of so many token tiles; a light pair, of which a block works on sixteen at a time.
+__device__ __forceinline__ int w16_heavy_cost(int nt) { return 320 + 88 * nt; }
+constexpr int W16_PAIR_COST = 18;
+__device__ __forceinline__ int w16_mean(int heavy, int np, int G) { return (int) (((long) heavy + (long) np * W16_PAIR_COST + G - 1) / G); }
+// where the stretch of np pairs begins whose share starts at c of all (monotone in c, 0 at 0 and np at all)
+__device__ __forceinline__ int w16_part(int np, int c, int all) { return all > 0 ? (int) ((double) np * (double) c / (double) all) : 0; }
 constexpr int W16_SORTJ = 1024, W16_GU_HELD = 1024, W16_PLAN = 4;   // (W16_PLAN: blocks a lane of the planning wave looks after)
 struct Wave16GuLds {
     uint2 tab[SGRID_WORDS];
     __attribute__((aligned(16))) uint8_t xt[MB_TOK64 * W16_XROW];
-    __attribute__((aligned(16))) uint8_t xs[8 * 64 * 16];      // the up tiles' sums of a light unit on their way to the gate tiles' waves
     uint8_t jn[2][W16_GU_HELD];
     int jw[W16_GU_HELD];
     unsigned short jorder[W16_SORTJ];   // the jobs, most token tiles first (the lower index first among equals)
-    int p_total[MB_TP + 1], p_sumk, p_s0, p_k;   // the jobs by token tiles; the plan where one wave made it: this block's share of the light units
+    int orow[FNX_PF_JOB];   // a heavy unit's tokens' places in the output
+    int p_total[MB_TP + 1], p_first, p_last;   // the jobs by token tiles; the plan where one wave made it: this block's stretch of the light pairs
+    int ph_jobs, ph_tokens, ph_next;                      // a phase of light pairs: its jobs, their tokens, the next pair to take
+    unsigned short ph_job[16];
+    unsigned char ph_first[16];                           // a job's first place in LDS
 };
 __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs a) {
     // the block's place in the plan: blocks with neighbouring places run on one XCD (workgroups go to the eight XCDs in turn), so
@@ -292,7 +355,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     }
     const int nj = min(a.cap, uniform(nj_raw)), nj2 = a.jobs2 ? min(a.cap2, uniform(nj2_raw)) : 0, njall = nj + nj2;
     const int ffh = a.ffh, nsuper = a.ncols >> 9, ppj = ffh >> 4;                      // pairs of tiles a job
-    const int upj = (ppj + W16_WAVES - 1) / W16_WAVES, upj_s = (ppj + 7) / 8;   // units a job: of sixteen pairs, of eight
+    const int upj = (ppj + W16_WAVES - 1) / W16_WAVES;                                  // heavy units a job
     auto job_at = [&](int j) { return j < nj ? a.jobs + j : a.jobs2 + (j - nj); };
     auto n_of = [&](int j) {
         const int l = j < nj ? 0 : 1, k = j < nj ? j : j - nj;
@@ -323,66 +386,61 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
             }
         }
         // The plan. Jobs of two token tiles and more go as units of sixteen pairs (a wave a pair), dealt heaviest first, to
-        // and fro over the blocks. Jobs of up to 16 tokens (where a row's S <= 4 activation tiles of 16 tokens fit LDS
-        // together) go as units of eight pairs, a wave a single tile, and fill the blocks up to the mean load: block b
-        // takes k_b = (mean - its heavy units' cost) / (a light unit's cost) of them, rounded, in the order of the blocks
-        // from the last one down (the lightest first); what the rounding leaves over goes one a block in that order.
+        // and fro over the blocks. The pairs of the jobs of up to 16 tokens (where a row's S <= 4 activation tiles of 16 tokens
+        // fit LDS together) fill the blocks up to the mean load: in the order of the blocks from the last one down (the lightest
+        // first) each takes the stretch of the list of those pairs that its share, the mean less its heavy units, is of all shares.
         const int G = gridDim.x, ome = G - 1 - (int) vb;
         const bool split = nsuper <= 4;
-        const int nbj = total[4] + total[3] + total[2] + (split ? 0 : total[1]), nb = nbj * upj, ns = split ? total[1] * upj_s : 0;
-        // costs as measured for S = 4 (us: 20 + 5.5 a token tile the heavy unit, 13.5 the light one), in halves of a us
+        const int nbj = total[4] + total[3] + total[2] + (split ? 0 : total[1]), nb = nbj * upj, np = split ? total[1] * ppj : 0;
         if (lane == 0) {
 #pragma unroll
             for (int c = 0; c <= MB_TP; ++c) L.p_total[c] = total[c];
         }
-        const int cs = 27 * nsuper;
         if (nb > G) {   // (heavy units on one block or none: the same plan in closed form, below, by every wave)
-        auto big_cost = [&](int u) {
-            const int jo = u / upj, nt_ = jo < total[4] ? 4 : jo < total[4] + total[3] ? 3 : jo < total[4] + total[3] + total[2] ? 2 : 1;
-            return (40 + 11 * nt_) * nsuper;
-        };
-        auto load_of = [&](int bb) {   // block bb's heavy units
-            int l = 0;
-            for (int k = 0; k * G < nb; ++k) {
-                const int u = k * G + ((k & 1) ? G - 1 - bb : bb);
-                if (u < nb) l += big_cost(u);
-            }
-            return l;
-        };
-        // a lane looks after W16_PLAN blocks (a grid of up to 64 W16_PLAN), in the order from the last block down
-        const int o0 = lane * W16_PLAN;
-        int ld[W16_PLAN], mine_sum = 0;
-#pragma unroll
-        for (int i = 0; i < W16_PLAN; ++i) {
-            ld[i] = o0 + i < G ? load_of(G - 1 - (o0 + i)) : 0;
-            mine_sum += ld[i];
-        }
-#pragma unroll
-        for (int sh = 32; sh >= 1; sh >>= 1) mine_sum += __shfl_xor(mine_sum, sh);
-        const int mean = (int) (((long) mine_sum + (long) ns * cs + G - 1) / G);
-        int kk[W16_PLAN], kl = 0;
-#pragma unroll
-        for (int i = 0; i < W16_PLAN; ++i) {
-            kk[i] = o0 + i < G ? max(0, (mean - ld[i] + cs / 2) / cs) : 0;
-            kl += kk[i];
-        }
-        int incl = kl;
-#pragma unroll
-        for (int sh = 1; sh < 64; sh <<= 1) {
-            const int up = __shfl_up(incl, sh);
-            if (lane >= sh) incl += up;
-        }
-        const int sumk = __shfl(incl, 63);
-        if (o0 <= ome && ome < o0 + W16_PLAN) {
-            int s0 = incl - kl;
+            auto load_of = [&](int bb) {   // block bb's heavy units
+                int l = 0;
+                for (int k = 0; k * G < nb; ++k) {
+                    const int u = k * G + ((k & 1) ? G - 1 - bb : bb);
+                    if (u < nb) {
+                        const int jo = u / upj;
+                        l += w16_heavy_cost(jo < total[4] ? 4 : jo < total[4] + total[3] ? 3 : jo < total[4] + total[3] + total[2] ? 2 : 1);
+                    }
+                }
+                return l;
+            };
+            // a lane looks after W16_PLAN blocks (a grid of up to 64 W16_PLAN), in the order from the last block down
+            const int o0 = lane * W16_PLAN;
+            int ld[W16_PLAN], mine_sum = 0;
 #pragma unroll
             for (int i = 0; i < W16_PLAN; ++i) {
-                if (o0 + i < ome) s0 += kk[i];
-                if (o0 + i == ome) L.p_k = kk[i];
+                ld[i] = o0 + i < G ? load_of(G - 1 - (o0 + i)) : 0;
+                mine_sum += ld[i];
             }
-            L.p_s0 = s0;
-        }
-        if (lane == 0) L.p_sumk = sumk;
+#pragma unroll
+            for (int sh = 32; sh >= 1; sh >>= 1) mine_sum += __shfl_xor(mine_sum, sh);
+            const int mean = w16_mean(mine_sum, np, G);
+            int kl = 0;
+#pragma unroll
+            for (int i = 0; i < W16_PLAN; ++i) {
+                ld[i] = o0 + i < G ? max(0, mean - ld[i]) : 0;   // from here on: the block's share
+                kl += ld[i];
+            }
+            int incl = kl;
+#pragma unroll
+            for (int sh = 1; sh < 64; sh <<= 1) {
+                const int up = __shfl_up(incl, sh);
+                if (lane >= sh) incl += up;
+            }
+            const int all = __shfl(incl, 63);
+            if (o0 <= ome && ome < o0 + W16_PLAN) {
+                int c = incl - kl, mine = 0;
+#pragma unroll
+                for (int i = 0; i < W16_PLAN; ++i) {
+                    if (o0 + i < ome) c += ld[i];
+                    if (o0 + i == ome) mine = ld[i];
+                }
+                L.p_first = w16_part(np, c, all), L.p_last = w16_part(np, c + mine, all);
+            }
         }
     }
     __syncthreads();   // the codebook, the order and the plan
@@ -395,23 +453,22 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         for (int c = 0; c <= MB_TP; ++c) tot[c] = uniform(L.p_total[c]);
     }
     const bool split = nsuper <= 4;
-    const int nbj = sorted ? tot[4] + tot[3] + tot[2] + (split ? 0 : tot[1]) : njall, nb = nbj * upj, ns = sorted && split ? tot[1] * upj_s : 0;
-    int sumk, s0, kme;
+    const int nbj = sorted ? tot[4] + tot[3] + tot[2] + (split ? 0 : tot[1]) : njall, nb = nbj * upj, np = sorted && split ? tot[1] * ppj : 0;
+    int p_first = 0, p_last = 0;   // the block's stretch of the light pairs
     if (nb <= G) {
         // every heavy unit on a block of its own, block b's of the class its place in the order says: the blocks of a class
-        // take the same number of light units, and the blocks after b (they come first) are counted class by class
-        const int cs = 27 * nsuper, b1 = (int) vb + 1;
+        // have the same share, and the blocks after b (they come first) are counted class by class
+        const int b1 = (int) vb + 1;
         const int hi4 = tot[4] * upj, hi3 = hi4 + tot[3] * upj, hi2 = hi3 + tot[2] * upj;   // where the classes end (class 1: nb)
-        const int c4 = 84 * nsuper, c3 = 73 * nsuper, c2 = 62 * nsuper, c1 = 51 * nsuper;      // (40 + 11 token tiles) S
-        const int mean = (hi4 * c4 + (hi3 - hi4) * c3 + (hi2 - hi3) * c2 + (nb - hi2) * c1 + ns * cs + G - 1) / G;
-        auto k_for = [&](int load) { return max(0, (mean - load + cs / 2) / cs); };
-        const int k4 = k_for(c4), k3 = k_for(c3), k2 = k_for(c2), k1 = k_for(c1), k0 = k_for(0);
-        auto after = [&](int lo, int hi) { return max(0, hi - max(lo, b1)); };   // blocks of [lo, hi) past this one
-        s0 = after(nb, G) * k0 + after(hi2, nb) * k1 + after(hi3, hi2) * k2 + after(hi4, hi3) * k3 + after(0, hi4) * k4;
-        kme = b1 > nb ? k0 : b1 > hi2 ? k1 : b1 > hi3 ? k2 : b1 > hi4 ? k3 : k4;
-        sumk = (G - nb) * k0 + (nb - hi2) * k1 + (hi2 - hi3) * k2 + (hi3 - hi4) * k3 + hi4 * k4;
-    } else {
-        sumk = sorted ? uniform(L.p_sumk) : 0, s0 = sorted ? uniform(L.p_s0) : 0, kme = sorted ? uniform(L.p_k) : 0;
+        const int c4 = w16_heavy_cost(4), c3 = w16_heavy_cost(3), c2 = w16_heavy_cost(2), c1 = w16_heavy_cost(1);
+        const int mean = w16_mean(hi4 * c4 + (hi3 - hi4) * c3 + (hi2 - hi3) * c2 + (nb - hi2) * c1, np, G);
+        const int s4 = max(0, mean - c4), s3 = max(0, mean - c3), s2 = max(0, mean - c2), s1 = max(0, mean - c1), s0 = mean;
+        auto after = [&](int lo, int hi, int b) { return max(0, hi - max(lo, b)); };   // blocks of [lo, hi) from b on
+        auto shares = [&](int b) { return after(nb, G, b) * s0 + after(hi2, nb, b) * s1 + after(hi3, hi2, b) * s2 + after(hi4, hi3, b) * s3 + after(0, hi4, b) * s4; };
+        const int all = shares(0);
+        p_first = uniform(w16_part(np, shares(b1), all)), p_last = uniform(w16_part(np, shares(b1 - 1), all));
+    } else if (sorted) {
+        p_first = uniform(L.p_first), p_last = uniform(L.p_last);
     }
     // The oldest wave of a SIMD goes first and the block's waves drift apart between two barriers: every wave takes each
     // priority in turn, a super-step each
@@ -428,6 +485,44 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         return j >= nj ? a.w2 : a.ep ? uniform_ptr((const uint8_t*) a.ep[e]) : a.w + (size_t) e * a.stride;
     };
     // ---- the heavy units: sixteen pairs of tiles, a pair a wave
+    auto heavy = [&](auto nt_tag, const fnx_bigjob* jb, int n, const uint8_t* we, int pr) {
+        constexpr int NT = decltype(nt_tag)::value;
+        const bool mine = pr < ppj;   // the wave's pair: gate rows 16 pr .., up rows ffh + 16 pr ..
+        const __amdgpu_buffer_rsrc_t mg = tile16_rsrc(we, min(pr, ppj - 1), nsuper), mu = tile16_rsrc(we, ppj + min(pr, ppj - 1), nsuper);
+        const int oput = tid < n ? jb->out[tid] : -1;   // (up to 64 tokens: the first wave)
+        int y[NT];   // the wave's tokens' rows: tokens wave, wave + 16, .. (past the job's last: that one again)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) y[i] = uniform(jb->y[min(wave + 16 * i, n - 1)]);
+        v4f accg[NT], accu[NT];
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) accg[tt] = accu[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+        SuperFields f = tile16_load_buf(mg, 0), fu = tile16_load_buf(mu, 0);
+        for (int S = 0; S < nsuper; ++S) {
+            __syncthreads();   // the tile before has been read
+            if (S == 0 && tid < FNX_PF_JOB) L.orow[tid] = oput;
+#pragma unroll
+            for (int i = 0; i < NT; ++i)   // a token's 512 columns a wave instruction, 16 bytes a lane
+                lds_load16(a.x + (size_t) y[i] * a.ldx + 512 * S, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            turn(S);
+            const int Sn = min(S + 1, nsuper - 1);
+            SuperFields nf, nfu;
+            w16_super_pair<NT>(L.tab, xlane, f, fu, accg, accu, [&] { nf = tile16_load_buf(mg, Sn), nfu = tile16_load_buf(mu, Sn); });
+            f = nf, fu = nfu;
+        }
+        // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the pair's tiles
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+            const int orow = mine ? L.orow[tt * 16 + r] : -1;
+            if (orow >= 0) {
+                const v4f gt = accg[tt], up = accu[tt];
+                uint2 hv;
+                hv.x = h16_pair(silu_f(gt.x), up.x, silu_f(gt.y), up.y), hv.y = h16_pair(silu_f(gt.z), up.z, silu_f(gt.w), up.w);
+                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
+            }
+        }
+    };
     for (int round = 0; round * G < nb; ++round) {
         const int u = round * G + ((round & 1) ? G - 1 - (int) vb : (int) vb);
         if (u >= nb) continue;   // the same for the whole block
@@ -435,92 +530,83 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         const fnx_bigjob* jb = job_at(j);
         const int n = uniform(n_of(j));
         if (n < 1) continue;
-        const int nt = (n + 15) >> 4;
         const uint8_t* we = matrix_of(j, jb);
-        const int pr = q * W16_WAVES + wave;   // the wave's pair: gate rows 16 pr .., up rows ffh + 16 pr ..
-        const bool mine = pr < ppj;
-        const int grow = 16 * min(pr, ppj - 1) + r;
-        int y[MB_TP];   // the wave's tokens' rows: tokens wave, wave + 16, .. (past the job's last: that one again)
-#pragma unroll
-        for (int i = 0; i < MB_TP; ++i) y[i] = uniform(jb->y[min(wave + 16 * i, n - 1)]);
-        int orow[MB_TP];
-#pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) orow[tt] = mine && tt * 16 + r < n ? jb->out[tt * 16 + r] : -1;
-        v4f accg[MB_TP], accu[MB_TP];
-#pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) accg[tt] = accu[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-        SuperFields f = tile16_load(we, grow, 0, nsuper);
-        for (int S = 0; S < nsuper; ++S) {
-            __syncthreads();   // the tile before has been read
-#pragma unroll
-            for (int i = 0; i < MB_TP; ++i)   // a token's 512 columns a wave instruction, 16 bytes a lane
-                if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx + 512 * S, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            turn(S);
-            const SuperFields fu = tile16_load(we, ffh + grow, S, nsuper);
-            if (mine) w16_super_step(L.tab, xlane, f, nt, accg);
-            f = tile16_load(we, grow, min(S + 1, nsuper - 1), nsuper);
-            if (mine) w16_super_step(L.tab, xlane, fu, nt, accu);
-        }
-        // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the pair's tiles
-#pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt)
-            if (orow[tt] >= 0) {
-                const v4f gt = accg[tt], up = accu[tt];
-                uint2 hv;
-                hv.x = (uint32_t) float_to_half_bits(silu_f(gt.x) * up.x) | (uint32_t) float_to_half_bits(silu_f(gt.y) * up.y) << 16;
-                hv.y = (uint32_t) float_to_half_bits(silu_f(gt.z) * up.z) | (uint32_t) float_to_half_bits(silu_f(gt.w) * up.w) << 16;
-                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow[tt] * ffh + 16 * pr + 4 * grp) = hv;
-            }
+        const int pr = q * W16_WAVES + wave;
+        if (n > 48) heavy(std::integral_constant<int, 4>{}, jb, n, we, pr);
+        else if (n > 32) heavy(std::integral_constant<int, 3>{}, jb, n, we, pr);
+        else if (n > 16) heavy(std::integral_constant<int, 2>{}, jb, n, we, pr);
+        else heavy(std::integral_constant<int, 1>{}, jb, n, we, pr);
     }
-    if (!sorted) return;
-    // ---- the light units: eight pairs of tiles, waves 0 .. 7 the gate tiles, 8 .. 15 the up tiles; the job's up to 16 tokens'
-    // S tiles all in LDS ([S][token]), so the waves do not meet until the up tiles' sums go over to the gate tiles' waves
-    const int ome = G - 1 - (int) vb;
-    float4* ex = reinterpret_cast<float4*>(L.xs);
-    for (int t = 0;; ++t) {
-        const int idx = t < kme ? s0 + t : sumk + (t - kme) * G + ome;
-        if (t < kme ? idx >= min(ns, sumk) : idx >= ns) {
-            if (t < kme) {   // (this block's share was cut short: on to what is left over, if anything)
-                t = kme - 1;
-                continue;
+    // ---- the light pairs, in phases: the jobs of the block's stretch as long as their tokens fit the sixteen places that LDS has for
+    // a row's S tiles ([S][place]), all staged at once; the waves then take the phase's pairs one by one as they come free and
+    // meet only where a phase ends
+    for (int p0 = p_first; p0 < p_last;) {   // the same for the whole block
+        __syncthreads();   // the units before have been read
+        if (wave == 0) {   // the phase: lane k its k-th job
+            const int jo = p0 / ppj + lane;
+            const bool in = jo * ppj < p_last && lane < 16;
+            const int j = in ? (int) L.jorder[nbj + jo] : 0, n = in ? n_of(j) : 16;   // 1 .. 16
+            int incl = n;
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) {
+                const int up = __shfl_up(incl, o, 16);
+                if ((lane & 15) >= o) incl += up;
             }
-            break;
+            const int jobs = __popcll(__ballot(in && incl <= 16));   // (at least one)
+            if (lane < jobs) {
+                L.ph_job[lane] = (unsigned short) j;
+                L.ph_first[lane] = (unsigned char) (incl - n);
+            }
+            if (lane == 0) L.ph_jobs = jobs, L.ph_next = p0 + W16_WAVES;
+            if (lane == jobs - 1) L.ph_tokens = incl;
         }
-        const int jo = idx / upj_s, q = idx - jo * upj_s, j = (int) uniform(L.jorder[nbj + jo]);
-        const fnx_bigjob* jb = job_at(j);
-        const int n = uniform(n_of(j));   // 1 .. 16
-        const uint8_t* we = matrix_of(j, jb);
-        const int pr = q * 8 + (wave & 7), up_wave = wave >> 3;
-        const bool mine = pr < ppj;
-        const int row = up_wave * ffh + 16 * min(pr, ppj - 1) + r;
-        const int y = uniform(jb->y[min(wave, n - 1)]);
-        const int orow = mine && !up_wave && r < n ? jb->out[r] : -1;
-        SuperFields f = tile16_load(we, row, 0, nsuper);
-        __syncthreads();   // the unit before has been read, its sums handed over
-        for (int S = 0; S < nsuper; ++S) lds_load16(a.x + (size_t) y * a.ldx + 512 * S, 16u * lane, xt_at + (16 * S + wave) * W16_XROW);
+        __syncthreads();
+        const int jobs = uniform(L.ph_jobs), jo0 = p0 / ppj, pe = min(p_last, (jo0 + jobs) * ppj), tokens = uniform(L.ph_tokens);
+        if (wave < tokens) {   // a place a wave: the job it belongs to is the last one that begins at or before it
+            const int k = __popcll(__ballot(lane < jobs && (int) L.ph_first[lane & 15] <= wave)) - 1;
+            const int y = uniform(job_at((int) L.ph_job[k])->y[wave - (int) L.ph_first[k]]);
+            for (int S = 0; S < nsuper; ++S) lds_load16(a.x + (size_t) y * a.ldx + 512 * S, 16u * lane, xt_at + (16 * S + wave) * W16_XROW);
+        }
+        // a wave's pair p: its job's place in the phase, its matrix's two rows of tiles
+        int p = p0 + wave;
+        __amdgpu_buffer_rsrc_t mg, mu;
+        auto tiles_of = [&](int q) {
+            const int jo = q / ppj, pr = q - jo * ppj, j = uniform((int) L.ph_job[jo - jo0]);
+            const uint8_t* we = matrix_of(j, job_at(j));
+            mg = tile16_rsrc(we, pr, nsuper), mu = tile16_rsrc(we, ppj + pr, nsuper);
+        };
+        tiles_of(min(p, pe - 1));
+        SuperFields f = tile16_load_buf(mg, 0), fu = tile16_load_buf(mu, 0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        v4f acc[MB_TP];
-#pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-        for (int S = 0; S < nsuper; ++S) {
-            turn(S);
-            const SuperFields nf = tile16_load(we, row, min(S + 1, nsuper - 1), nsuper);
-            if (mine) w16_super_step(L.tab, xlane + S * 16 * W16_XROW, f, 1, acc);
-            f = nf;
+        while (p < pe) {
+            int pn = 0;
+            if (lane == 0) pn = atomicAdd(&L.ph_next, 1);
+            pn = uniform(pn);
+            const int jo = p / ppj, pr = p - jo * ppj, k = jo - jo0, j = uniform((int) L.ph_job[k]), at = uniform((int) L.ph_first[k]);
+            const fnx_bigjob* jb = job_at(j);
+            const int orow = r < n_of(j) ? jb->out[r] : -1;
+            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 256 * grp;   // (a lane without a token: some place's values, its sums not kept)
+            v4f accg[1] = {v4f{0.f, 0.f, 0.f, 0.f}}, accu[1] = {v4f{0.f, 0.f, 0.f, 0.f}};
+            for (int S = 0; S < nsuper; ++S) {
+                turn(S);
+                SuperFields nf, nfu;
+                w16_super_pair<1>(L.tab, xk + S * 16 * W16_XROW, f, fu, accg, accu, [&] {
+                    if (S + 1 == nsuper) tiles_of(min(pn, pe - 1));
+                    const int Sn = S + 1 < nsuper ? S + 1 : 0;
+                    nf = tile16_load_buf(mg, Sn), nfu = tile16_load_buf(mu, Sn);
+                });
+                f = nf, fu = nfu;
+            }
+            if (orow >= 0) {
+                const v4f gt = accg[0], up = accu[0];
+                uint2 hv;
+                hv.x = h16_pair(silu_f(gt.x), up.x, silu_f(gt.y), up.y), hv.y = h16_pair(silu_f(gt.z), up.z, silu_f(gt.w), up.w);
+                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
+            }
+            p = pn;
         }
-        if (up_wave) ex[(wave & 7) * 64 + lane] = make_float4(acc[0].x, acc[0].y, acc[0].z, acc[0].w);
-        __syncthreads();
-        if (orow >= 0) {
-            const float4 up = ex[wave * 64 + lane];
-            const v4f gt = acc[0];
-            uint2 hv;
-            hv.x = (uint32_t) float_to_half_bits(silu_f(gt.x) * up.x) | (uint32_t) float_to_half_bits(silu_f(gt.y) * up.y) << 16;
-            hv.y = (uint32_t) float_to_half_bits(silu_f(gt.z) * up.z) | (uint32_t) float_to_half_bits(silu_f(gt.w) * up.w) << 16;
-            *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
-        }
+        p0 = pe;
     }
 }
 

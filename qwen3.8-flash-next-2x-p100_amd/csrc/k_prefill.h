@@ -862,6 +862,23 @@ __device__ __forceinline__ SuperFields tile16_load(const uint8_t* __restrict__ w
     r.d = *(g16*) (u + TILE16_D_AT + 2 * lane);
     return r;
 }
+// The same through a buffer descriptor over a row of tiles (rows 16 t .. 16 t + 15: wave-uniform), tile S of it by a scalar
+// offset: the lane's offsets are 32-bit and the planes' places ride in the instructions, where tile16_load keeps a 64-bit
+// address a plane in vector registers.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile16_rsrc(const uint8_t* __restrict__ we, int t, int nsuper) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*) uniform_ptr(we + (size_t) t * nsuper * TILE16_BYTES), 0, -1, 0x00020000);
+}
+__device__ __forceinline__ SuperFields tile16_load_buf(__amdgpu_buffer_rsrc_t m, int S) {
+    const int lane = threadIdx.x & 63, at = S * TILE16_BYTES;
+    SuperFields r;
+    r.a0 = __builtin_amdgcn_raw_buffer_load_b128(m, 32 * lane, at, 0);
+    r.a1 = __builtin_amdgcn_raw_buffer_load_b128(m, 32 * lane + 16, at, 0);
+    r.b = __builtin_amdgcn_raw_buffer_load_b128(m, 16 * lane + TILE16_B_AT, at, 0);
+    r.c = __builtin_amdgcn_raw_buffer_load_b32(m, 4 * lane + TILE16_C_AT, at, 0);
+    r.sc = __builtin_amdgcn_raw_buffer_load_b16(m, 2 * lane + TILE16_SC_AT, at, 0);
+    r.d = __builtin_amdgcn_raw_buffer_load_b16(m, 2 * lane + TILE16_D_AT, at, 0);
+    return r;
+}
 // unit64 -> tile16 (once, at load; out of place): a wave a tile, every lane reads its four sub-blocks of its row
 __global__ void __launch_bounds__(256) k_iq3s_tile16(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int nrows, int ncols, long tiles) {
     const long t = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
