@@ -28,7 +28,6 @@ struct Wave16Lds {
     int first_job, first_tile, last_job, last_tile;   // the block's run: from (first_job, first_tile) up to but not including (last_job, last_tile)
     uint8_t jn[2][W16_HELD];                          // the token counts of the two lists' jobs, as far as they fit
     int jw[W16_HELD];                                 // the first list's matrices
-    int orow[FNX_PF_JOB];                             // the job's tokens' rows of the output
 };
 
 // f16(a0 b0) | f16(a1 b1) << 16, each product rounded once and a product that vanishes a positive zero: what the compiler makes
@@ -36,7 +35,8 @@ struct Wave16Lds {
 // and a row's h would depend on the size of the job it falls in.
 __device__ __forceinline__ uint32_t h16_pair(float a0, float b0, float a1, float b1) {
     uint32_t v;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0" : "=&v"(v) : "v"(a0), "v"(b0), "v"(a1), "v"(b1));
+    // (a half register's write is not forwarded: a wait state before the next instruction that uses the register)
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\ts_nop 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0\n\ts_nop 0" : "=&v"(v) : "v"(a0), "v"(b0), "v"(a1), "v"(b1));
     return v;
 }
 // A lane's half of a sub-block (fields s) as two f16 operands: weights 16 h .. 16 h + 15
@@ -53,24 +53,48 @@ __device__ __forceinline__ void w16_half(const uint2* tab, const SubFields& s, i
         A[k >> 1][4 * (k & 1) + 3] = hi.y;
     }
 }
-// A tile's super-step: the lane's four sub-blocks of its row (fields f) as f16 operands, against the NT token tiles of
+// A tile's super-step: the lane's four sub-blocks of its row (fields f) as f16 operands, against the nt token tiles of
 // the activation tile in LDS (xlane: token r's row at this lane group's sub-blocks), added to acc
-template <int NT>
-__device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* xlane, const SuperFields& f, v4f (&acc)[NT]) {
+__device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* xlane, const SuperFields& f, int nt, v4f (&acc)[MB_TP]) {
+    // the token tiles two at a time against the sub-block's operands
+    auto pair = [&](const v8h (&A)[4], int p, auto t0_tag, auto cnt_tag) {
+        constexpr int T0 = decltype(t0_tag)::value, CNT = decltype(cnt_tag)::value;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {   // two of the four operands at a time: the registers of a block of 1024 threads
+            v4u B[2][2];
+#pragma unroll
+            for (int tt = 0; tt < CNT; ++tt)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) B[tt][i] = *reinterpret_cast<const v4u*>(xlane + (T0 + tt) * 16 * W16_XROW + 64 * p + 32 * h + 16 * i);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int tt = 0; tt < CNT; ++tt)
+                    acc[T0 + tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[2 * h + i], __builtin_bit_cast(v8h, B[tt][i]), acc[T0 + tt], 0, 0, 0);
+        }
+    };
     auto step = [&](auto p_c) {
         constexpr int p = decltype(p_c)::value;
         const SubFields s = super_sub<p>(f);
-        v8h A[2][2];
-        w16_half(tab, s, 0, A[0]);
-        w16_half(tab, s, 1, A[1]);
+        const _Float16 sc = (_Float16) (int) (1 + 2 * s.sc), d = __builtin_bit_cast(_Float16, (unsigned short) s.d);
+        const v2h s2 = {sc, sc}, d2 = {d, d};
+        v8h A[4];   // the lane's sub-block (row r, 4 grp + p) as 32 f16 weights
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[h][i], *reinterpret_cast<const v8h*>(xlane + tt * 16 * W16_XROW + 64 * p + 32 * h + 16 * i),
-                                                                     acc[tt], 0, 0, 0);
+        for (int k = 0; k < 8; ++k) {
+            const uint2 en = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(tab) + sub_entry<true>(s, k));
+            const v2h lo = (as_v2h(en.x) * s2) * d2, hi = (as_v2h(en.y) * s2) * d2;
+            A[k >> 1][4 * (k & 1) + 0] = lo.x;
+            A[k >> 1][4 * (k & 1) + 1] = lo.y;
+            A[k >> 1][4 * (k & 1) + 2] = hi.x;
+            A[k >> 1][4 * (k & 1) + 3] = hi.y;
+        }
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        if (nt >= 2) pair(A, p, I0{}, I2{});
+        else pair(A, p, I0{}, I1{});
+        if (nt == 3) pair(A, p, I2{}, I1{});
+        else if (nt == 4) pair(A, p, I2{}, I2{});
     };
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
@@ -226,9 +250,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
         int y[MB_TP];
 #pragma unroll
         for (int i = 0; i < MB_TP; ++i) y[i] = ahead == j ? yahead[i] : uniform(jb->y[min(wave + 16 * i, n - 1)]);
-        const int oput = tid < n ? jb->out[tid] : -1;   // (up to 64 tokens: the first wave)
         __syncthreads();   // the job before has been read
-        if (tid < FNX_PF_JOB) L.orow[tid] = oput;
 #pragma unroll
         for (int i = 0; i < MB_TP; ++i)   // a token's row a wave instruction, 16 bytes a lane
             if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
@@ -239,63 +261,50 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
             for (int i = 0; i < MB_TP; ++i) yahead[i] = uniform(jn->y[max(0, min(wave + 16 * i, nn - 1))]);
             ahead = j + 1;
         }
-        auto run = [&](auto nt_tag) {
-            constexpr int NT = decltype(nt_tag)::value;
-            auto put = [&](const v4f (&acc)[NT], int g) {   // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
+        int orow[MB_TP];
 #pragma unroll
-                for (int tt = 0; tt < NT; ++tt) {
-                    const int orow = L.orow[tt * 16 + r];
-                    if (orow >= 0) *reinterpret_cast<float4*>(a.out + (size_t) orow * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
-                }
-            };
-            // the wave's tiles g, g + 16, .. two at a time, the next two's fields asked for in the middle of the two before (past
-            // the run's last tile: that one again)
-            int g = g0 + wave;
-            auto fields = [&](int t) { return tile16_load_buf(tile16_rsrc(we, min(t, g1 - 1), 1), 0); };
-            SuperFields f0 = fields(g), f1 = fields(g + W16_WAVES);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            for (; g < g1; g += 2 * W16_WAVES) {
-                // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
-                // for the last: every wave takes every priority in turn, two tiles each
-                switch (((wave >> 2) + ((g - g0) >> 5)) & 3) {
-                    case 0: __builtin_amdgcn_s_setprio(0); break;
-                    case 1: __builtin_amdgcn_s_setprio(1); break;
-                    case 2: __builtin_amdgcn_s_setprio(2); break;
-                    default: __builtin_amdgcn_s_setprio(3); break;
-                }
-                v4f acc0[NT], acc1[NT];
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt) acc0[tt] = acc1[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-                if (g + W16_WAVES < g1) {
-                    SuperFields n0, n1;
-                    w16_super_pair<NT>(L.tab, xlane, f0, f1, acc0, acc1, [&] { n0 = fields(g + 2 * W16_WAVES), n1 = fields(g + 3 * W16_WAVES); });
-                    put(acc0, g);
-                    put(acc1, g + W16_WAVES);
-                    f0 = n0, f1 = n1;
-                } else {   // the run's last round, where it has an odd number of them
-                    w16_super_step<NT>(L.tab, xlane, f0, acc0);
-                    put(acc0, g);
-                }
+        for (int tt = 0; tt < MB_TP; ++tt) orow[tt] = tt * 16 + r < n ? jb->out[tt * 16 + r] : -1;
+        int g = g0 + wave;
+        SuperFields f = tile16_load(we, 16 * min(g, g1 - 1) + r, 0, 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        for (; g < g1; g += W16_WAVES) {
+            // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
+            // for the last: every wave takes every priority in turn, a tile each
+            switch (((wave >> 2) + ((g - g0) >> 4)) & 3) {
+                case 0: __builtin_amdgcn_s_setprio(0); break;
+                case 1: __builtin_amdgcn_s_setprio(1); break;
+                case 2: __builtin_amdgcn_s_setprio(2); break;
+                default: __builtin_amdgcn_s_setprio(3); break;
             }
-        };
-        if (nt == 4) run(std::integral_constant<int, 4>{});
-        else if (nt == 3) run(std::integral_constant<int, 3>{});
-        else if (nt == 2) run(std::integral_constant<int, 2>{});
-        else run(std::integral_constant<int, 1>{});
+            const SuperFields nf = tile16_load(we, 16 * (g + W16_WAVES < g1 ? g + W16_WAVES : g) + r, 0, 1);
+            v4f acc[MB_TP];
+#pragma unroll
+            for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+            w16_super_step(L.tab, xlane, f, nt, acc);
+            // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
+#pragma unroll
+            for (int tt = 0; tt < MB_TP; ++tt)
+                if (orow[tt] >= 0)
+                    *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
+            f = nf;
+        }
     }
 }
 
 // ---------------------------------------------------------------- the same form for stacked gate|up matrices (rows of 512 S columns)
 // A job's activations are S tiles of 64 tokens x 512 columns here, and LDS holds one: a block takes units of (job, sixteen
 // gate tiles and the sixteen up tiles that go with them), a wave one such pair, and walks the S super-steps with the
-// pair's accumulators in registers - activation tile S in (two barriers), the gate tile's super-step, the up tile's -
-// and leaves h = silu(gate) * up as f16 (k_swiglu_h16's values). Such a unit is eight rounds of the down kernel's kind:
-// too coarse for runs by cost, and two of even the lightest on one block made the launch half as long again as its mean
-// block. So the jobs are ranked by token tiles, the units of those with two token tiles and more dealt heaviest first,
-// to and fro over the blocks, and the jobs of up to 16 tokens cut finer - eight pairs a unit, a wave a single tile, all S
-// tiles of the 16 tokens in LDS at once, the up tiles' sums handed to the gate tiles' waves through LDS - and spread so
-// that every block comes near the mean load. The weights of the next tile's super-step are asked for a tile ahead. Every
+// pair's accumulators in registers - activation tile S in (two barriers), the gate tile's and the up tile's super-steps
+// together, so that an activation operand is read from LDS once for both (4,096 rows of a Zipf chunk: 307 -> 269 us, LDS and
+// VALU each busy a little over half the time; reading it for each tile was a third of the LDS's work) - and leaves
+// h = silu(gate) * up as f16 (k_swiglu_h16's values). Such a unit is too coarse for runs by cost, and two of even the
+// lightest on one block made the launch half as long again as its mean block. So the jobs are ranked by token tiles and the
+// units of those with two token tiles and more dealt heaviest first, to and fro over the blocks. The pairs of the jobs of up
+// to 16 tokens then fill the blocks up to the mean load: a block stages all the tokens of its stretch's jobs at once, S tiles
+// of sixteen places, and its waves take the pairs one by one as they come free (77 rows, some 400 jobs of two tokens: 84 us;
+// 114 as units of eight pairs, a wave a tile, with a job's tokens fetched and the block met twice in each of them: of such a
+// unit's 16 us the LDS needs 9). The weights of the next super-step are asked for in the middle of the one before. Every
 // tile is accumulated in one order (S, then the four steps, then a step's four operands) whatever a job's size or the
 // unit it falls in: a row's h does not depend on what else is in the chunk.
 // Costs, in 1/16 us at S = 4 (measured): a heavy unit of so many token tiles; a light pair, of which a block works on sixteen at a time.
@@ -304,7 +313,7 @@ constexpr int W16_PAIR_COST = 18;
 __device__ __forceinline__ int w16_mean(int heavy, int np, int G) { return (int) (((long) heavy + (long) np * W16_PAIR_COST + G - 1) / G); }
 // where the stretch of np pairs begins whose share starts at c of all (monotone in c, 0 at 0 and np at all)
 __device__ __forceinline__ int w16_part(int np, int c, int all) { return all > 0 ? (int) ((double) np * (double) c / (double) all) : 0; }
-constexpr int W16_SORTJ = 1024, W16_GU_HELD = 1024, W16_PLAN = 4;   // (W16_PLAN: blocks a lane of the planning wave looks after)
+constexpr int W16_SORTJ = 2048, W16_GU_HELD = 2048, W16_PLAN = 4;   // (W16_PLAN: blocks a lane of the planning wave looks after)
 struct Wave16GuLds {
     uint2 tab[SGRID_WORDS];
     __attribute__((aligned(16))) uint8_t xt[MB_TOK64 * W16_XROW];
