@@ -28,32 +28,38 @@ __device__ __forceinline__ void swap32(uint32_t& x, uint32_t& y) { asm volatile(
 __device__ __forceinline__ void swap16(uint32_t& x, uint32_t& y) { asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
 // The signed codebook twice, entry i's two copies side by side (words 2 i and 2 i + 1): even lanes read the even words,
 // odd lanes the odd ones, so the 64 random lookups of a wave instruction are two sets of 32 over 32 banks each.
+template <int TOKS>   // tokens a unit
 struct J16Lds {
     uint32_t tab[2 * SGRID_WORDS];
-    __attribute__((aligned(16))) uint8_t xq[FNX_MAXT * J16_XLD];
-    __attribute__((aligned(16))) float dx[(J16_MAXCOLS / 128) * FNX_MAXT * 4];   // [super-step][step p][token][lane group g]: the activations' block scales
-    __attribute__((aligned(16))) float sw[J16_WAVES][4][16];                     // [wave][lane group][row]: a step's weight scales d (1 + 2 s)
+    __attribute__((aligned(16))) uint8_t xq[TOKS * J16_XLD];
+    __attribute__((aligned(16))) float dx[(J16_MAXCOLS / 128) * TOKS * 4];   // [super-step][step p][token][lane group g]: the activations' block scales
+    __attribute__((aligned(16))) float sw[J16_WAVES][4][16];                 // [wave][lane group][row]: a step's weight scales d (1 + 2 s)
 };
 
-// tiles [g0, g1) of 16 rows of matrix `we` (ncols columns) against the job's tokens, staged in L: the whole block
-__device__ __forceinline__ void j16_segment(J16Lds& L, const uint8_t* __restrict__ we, int g0, int g1, int ncols, const int* __restrict__ outs, int n,
-                                            float* __restrict__ out, int out_stride) {
+// tiles [g0, g1) of 16 rows of matrix `we` (ncols columns) against the job's tokens, NT tiles of sixteen, staged in L: the whole block,
+// after a barrier. f: the fields of the wave's first super-step. A step is decoded once for all NT tiles; a token's sums are the
+// same whatever NT.
+template <int NT, int TOKS>
+__device__ __forceinline__ void j16_segment(J16Lds<TOKS>& L, const uint8_t* __restrict__ we, int g0, int g1, int ncols, const int* __restrict__ outs, int n,
+                                            float* __restrict__ out, int out_stride, SuperFields f) {
     const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6));
     const int r = lane & 15, grp = lane >> 4;   // decoding: row r of the tile, lane group grp; accumulating: token r, rows 4 grp .. 4 grp + 3
     const int nsuper = ncols / 512;
-    float* orow = out + (size_t) (r < n ? outs[r] : 0) * out_stride + 4 * grp;
+    int oi[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) oi[tt] = 16 * tt + r < n ? outs[16 * tt + r] : 0;
     const uint8_t* xrow = L.xq + r * J16_XLD + 8 * grp;   // bytes 8 grp .. of sub-block 16 S + 4 j + p of token r lie 512 S + 128 j + 32 p further
     float* myw = &L.sw[wave][grp][r];
     const uint32_t copy_at = 4u * (lane & 1);
     if (g0 + wave >= g1) return;
-    // the fields of the super-step at hand; a tile's last super-step leaves the next tile's first ones here
-    SuperFields f = tile16_load(we, 16 * (g0 + wave) + r, 0, nsuper);
     for (int g = g0 + wave; g < g1; g += J16_WAVES) {
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        float acc[NT][4];
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) acc[tt][0] = acc[tt][1] = acc[tt][2] = acc[tt][3] = 0.f;
         for (int S = 0; S < nsuper; ++S) {
             // the next super-step's fields (past the tile's last: the next tile of this wave, or this one again)
             const int gn = S + 1 < nsuper ? g : (g + J16_WAVES < g1 ? g + J16_WAVES : g);
-            const SuperFields nf = tile16_load(we, 16 * gn + r, S + 1 < nsuper ? S + 1 : 0, nsuper);
+            const SuperFields nf = tile16_load_buf(tile16_rsrc(we, gn, nsuper), S + 1 < nsuper ? S + 1 : 0);
             auto step = [&](auto p_c) {
                 constexpr int p = decltype(p_c)::value;
                 const SubFields s = super_sub<p>(f);
@@ -62,11 +68,6 @@ __device__ __forceinline__ void j16_segment(J16Lds& L, const uint8_t* __restrict
 #pragma unroll
                 for (int j = 0; j < 8; ++j) w8[j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(L.tab) + 2 * packed_addr(idx, j) + copy_at);
                 *myw = half_bits_to_float(s.d) * (float) (int) (1u + 2u * s.sc);
-                long b[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const long*>(xrow + 512 * S + 128 * j + 32 * p);
-                const float4 dxv = *reinterpret_cast<const float4*>(&L.dx[((S * 4 + p) * FNX_MAXT + r) * 4]);
-                const float dxs[4] = {dxv.x, dxv.y, dxv.z, dxv.w};
                 // pair P_k = bytes 8 k .. 8 k + 7 of the lane's sub-block; afterwards pair j holds bytes 8 grp .. of lane group j's
                 swap32(w8[0], w8[4]);
                 swap32(w8[1], w8[5]);
@@ -76,15 +77,25 @@ __device__ __forceinline__ void j16_segment(J16Lds& L, const uint8_t* __restrict
                 swap16(w8[1], w8[3]);
                 swap16(w8[4], w8[6]);
                 swap16(w8[5], w8[7]);
+                float4 fw[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {   // lane group j's sub-block, 16 S + 4 j + p
-                    const long a = (long) ((unsigned long) w8[2 * j] | (unsigned long) w8[2 * j + 1] << 32);
-                    const j16_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[j], j16_v4i{0, 0, 0, 0}, 0, 0, 0);
-                    const float4 fw = *reinterpret_cast<const float4*>(&L.sw[wave][j][4 * grp]);
-                    acc[0] = fmaf(fw.x * dxs[j], (float) d[0], acc[0]);
-                    acc[1] = fmaf(fw.y * dxs[j], (float) d[1], acc[1]);
-                    acc[2] = fmaf(fw.z * dxs[j], (float) d[2], acc[2]);
-                    acc[3] = fmaf(fw.w * dxs[j], (float) d[3], acc[3]);
+                for (int j = 0; j < 4; ++j) fw[j] = *reinterpret_cast<const float4*>(&L.sw[wave][j][4 * grp]);
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) {
+                    long b[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const long*>(xrow + 16 * tt * J16_XLD + 512 * S + 128 * j + 32 * p);
+                    const float4 dxv = *reinterpret_cast<const float4*>(&L.dx[((S * 4 + p) * TOKS + 16 * tt + r) * 4]);
+                    const float dxs[4] = {dxv.x, dxv.y, dxv.z, dxv.w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {   // lane group j's sub-block, 16 S + 4 j + p
+                        const long a = (long) ((unsigned long) w8[2 * j] | (unsigned long) w8[2 * j + 1] << 32);
+                        const j16_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[j], j16_v4i{0, 0, 0, 0}, 0, 0, 0);
+                        acc[tt][0] = fmaf(fw[j].x * dxs[j], (float) d[0], acc[tt][0]);
+                        acc[tt][1] = fmaf(fw[j].y * dxs[j], (float) d[1], acc[tt][1]);
+                        acc[tt][2] = fmaf(fw[j].z * dxs[j], (float) d[2], acc[tt][2]);
+                        acc[tt][3] = fmaf(fw[j].w * dxs[j], (float) d[3], acc[tt][3]);
+                    }
                 }
             };
             step(std::integral_constant<int, 0>{});
@@ -93,130 +104,217 @@ __device__ __forceinline__ void j16_segment(J16Lds& L, const uint8_t* __restrict
             step(std::integral_constant<int, 3>{});
             f = nf;
         }
-        if (r < n) {
-            float* op = orow + 16 * g;
-            op[0] = acc[0], op[1] = acc[1], op[2] = acc[2], op[3] = acc[3];
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+            if (16 * tt + r < n) {
+                float* op = out + (size_t) oi[tt] * out_stride + 4 * grp + 16 * g;
+                op[0] = acc[tt][0], op[1] = acc[tt][1], op[2] = acc[tt][2], op[3] = acc[tt][3];
+            }
+    }
+}
+
+// tile16 matrices of up to 2048 columns (a multiple of 512), rows in 16s.
+// MODE 0: jobs of up to FNX_MAXT rows (kernels.hpp:18-23) over q8_1 rows: the blocks split the (job, tile of 16 rows) items of all jobs
+// evenly and walk them in order; a job's activations are staged when the block comes to it.
+// MODE 1: the prompt path's jobs of up to FNX_PF_JOB rows (kernels.hpp:324, moe_gate_up_big): a job's rows in units of up to two
+// token tiles, so that a weight is decoded once for both. A unit of nt token tiles costs J16_DEC + J16_MUL nt for each of its
+// rounds, J16_ROUND tiles of 16 rows; the blocks split the costs of all rounds evenly (a prefix sum over the jobs in LDS) and each
+// takes the rounds that begin in its share. Lists of so few tiles that the blocks have no more than a tile a wave are bound by a
+// tile's chain of steps and by what comes before it: there a unit is one token tile, and a round as many tiles as leave every block
+// a round of one unit, where that can be - a second unit would be staged after the first.
+// MODE 2 (kernels.hpp:325, moe_down_big): the same with the unit's activations made on the way from the rows [gate | up] of 2 ncols floats:
+// h = silu(gate) * up quantised as k_swiglu_q8_1 does it, four threads a sub-block.
+constexpr int J16_MAXJOBS = 4096;   // big jobs a launch (their token counts and costs live in LDS)
+// us a chunk of 512 experts, Zipf (a decode for every sixteen tokens, jobs' starts looked up in memory as their turn came / this), 300
+// rows: 192 / 171, 1,024: 389 / 335, 4,096: 1,302 / 1,014; 77 rows, uniform: 234 / 210; the shared expert's launches over 300 rows 23.6 / 18.1 and
+// 30.5 / 20.5. Rounds of 8 tiles 173, 336, 1,019, 212, of 16 182, 337, 1,026, 219: a unit's last tiles and the block's run come
+// out less even than the waves' idle turns in a short round cost. Four token tiles a unit (of up to 1024 columns; sums spill) were slower: 40.9 -> 46
+// us a down launch of 300 rows.
+constexpr int J16_ROUND = 4, J16_DEC = 3, J16_MUL = 2;
+static_assert(J16_MAXJOBS * (FNX_PF_JOB / 32) * (J16_DEC + 2 * J16_MUL) < 65536, "the costs' sum in 16 bits");
+
+// a unit's activations (n tokens, toks places) to LDS
+template <int MODE, int TOKS>
+__device__ __forceinline__ void j16_stage(J16Lds<TOKS>& L, const RowsArgs& a, const uint8_t* y, const int* ys, int n, int toks) {
+    const int nsb = a.ncols / 32;
+    if constexpr (MODE == 2) {
+        for (int q = threadIdx.x; q < 4 * toks * nsb; q += J16_THREADS) {   // (token, sub-block, quarter): 8 values (the four threads of a sub-block are neighbours)
+            const int s = q >> 2, part = q & 3, t = s / nsb, sb = s - t * nsb;
+            uint32_t v[2] = {0u, 0u};
+            float d = 0.f;
+            if (t < n) {
+                const float* gp = a.gu + (size_t) ys[t] * (2 * a.ncols) + 32 * sb + 8 * part;
+                float4 gv[2], uv[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) gv[k] = reinterpret_cast<const float4*>(gp)[k], uv[k] = reinterpret_cast<const float4*>(gp + a.ncols)[k];
+                float h[8], amax = 0.f;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    h[4 * k] = silu_f(gv[k].x) * uv[k].x, h[4 * k + 1] = silu_f(gv[k].y) * uv[k].y;
+                    h[4 * k + 2] = silu_f(gv[k].z) * uv[k].z, h[4 * k + 3] = silu_f(gv[k].w) * uv[k].w;
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(h[k]));
+                amax = fmaxf(amax, __shfl_xor(amax, 1));
+                amax = fmaxf(amax, __shfl_xor(amax, 2));
+                const float dq = amax / 127.0f;   // q8_1_store's arithmetic (kernels.cu:131-145)
+                d = half_bits_to_float(float_to_half_bits(dq));
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    uint32_t word = 0;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const int8_t qv = amax == 0.0f ? (int8_t) 0 : (int8_t) roundf(h[4 * k + b] / dq);
+                        word |= (uint32_t) (uint8_t) qv << (8 * b);
+                    }
+                    v[k] = word;
+                }
+            }
+            *reinterpret_cast<uint2*>(L.xq + t * J16_XLD + 32 * sb + 8 * part) = make_uint2(v[0], v[1]);
+            if (part == 0) L.dx[(((sb >> 4) * 4 + (sb & 3)) * TOKS + t) * 4 + ((sb >> 2) & 3)] = d;
+        }
+    } else {
+        for (int q = threadIdx.x; q < toks * nsb; q += J16_THREADS) {   // (token, sub-block): its 32 int8 and its scale
+            const int t = q / nsb, sb = q - t * nsb;
+            uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+            float d = 0.f;
+            if (t < n) {
+                const uint8_t* yb = y + ((size_t) ys[t] * nsb + sb) * FNX_Q8_1_BLOCK;
+                d = half_bits_to_float(*reinterpret_cast<const unsigned short*>(yb));
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const uint32_t*>(yb + 4 + 4 * k);
+            }
+            uint32_t* dst = reinterpret_cast<uint32_t*>(L.xq + t * J16_XLD + 32 * sb);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) dst[k] = v[k];
+            L.dx[(((sb >> 4) * 4 + (sb & 3)) * TOKS + t) * 4 + ((sb >> 2) & 3)] = d;
         }
     }
 }
 
-// tile16 matrices of up to 2048 columns (a multiple of 512), rows in 16s. The blocks split the (job, tile of 16 rows) items
-// of all jobs evenly and walk them in order; a job's activations are staged when the block comes to it.
-// MODE 0: jobs of up to FNX_MAXT rows (kernels.hpp:18-23) over q8_1 rows. MODE 1: the prompt path's jobs of up to
-// FNX_PF_JOB rows (kernels.hpp:324, moe_gate_up_big): a job's rows in tiles of sixteen, each (job, token tile) a unit that
-// is staged and walked like a job of MODE 0; the units are counted first (a prefix sum over the jobs' tile counts in LDS)
-// so that the blocks split live units only. MODE 2 (kernels.hpp:325, moe_down_big): the same with the unit's activations
-// made on the way from the rows [gate | up] of 2 ncols floats: h = silu(gate) * up quantised as k_swiglu_q8_1 does it.
-constexpr int J16_MAXJOBS = 4096;   // big jobs a launch (their tile counts' prefix sums live in LDS)
 template <int MODE>
 __global__ void __launch_bounds__(J16_THREADS) k_iq3s_jobs_mma16(const RowsArgs a) {
-    __shared__ J16Lds L;
-    __shared__ uint32_t before[MODE ? J16_MAXJOBS + 1 : 1];   // units of the jobs before job j
+    __shared__ J16Lds<MODE ? 2 * FNX_MAXT : FNX_MAXT> L;
+    __shared__ uint8_t jn[MODE ? J16_MAXJOBS : 1];            // the jobs' tokens
+    __shared__ unsigned short before[MODE ? J16_MAXJOBS + 2 : 1];   // costs of the jobs before job j, a round of each of their units
+    __shared__ int tiles_sum;
+    const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6));
+    // every job's token count, whether it counts or not, asked for along with the codebook
+    int hn[MODE ? J16_MAXJOBS / J16_THREADS : 1] = {};
+    if constexpr (MODE != 0) {
+#pragma unroll
+        for (int i = 0; i < J16_MAXJOBS / J16_THREADS; ++i) {
+            const int j = (int) threadIdx.x + i * J16_THREADS;
+            if (j < a.njobs_max) hn[i] = a.big[j].n;
+        }
+    }
+    const int nj_raw = a.njobs ? *a.njobs : a.njobs_max;
     for (int g = threadIdx.x; g < 512; g += J16_THREADS) {   // a code's sixteen signed entries from its unsigned one
         const uint32_t g0 = g_sgrid.v[g];
 #pragma unroll
         for (int sg = 0; sg < 16; ++sg) L.tab[2 * (sg * 512 + g)] = L.tab[2 * (sg * 512 + g) + 1] = signed_entry(g0, sg);
     }
-    const int nj = min(a.njobs ? min(uniform(*a.njobs), a.njobs_max) : a.njobs_max, MODE ? J16_MAXJOBS : a.njobs_max);
+    const int nj = max(0, min(min(uniform(nj_raw), a.njobs_max), MODE ? J16_MAXJOBS : a.njobs_max));
     const uint32_t gpj = (uint32_t) a.nrows / 16;   // items per unit
-    uint32_t units = (uint32_t) nj;
-    if constexpr (MODE != 0) {
-        // token tiles a job, then their running sum: a wave's lanes take consecutive runs of jobs
-        for (int j = threadIdx.x; j < nj; j += J16_THREADS) before[j + 1] = (uint32_t) (min(max(a.big[j].n, 0), FNX_PF_JOB) + 15) / 16;
-        if (threadIdx.x == 0) before[0] = 0;
+    const uint8_t* y = a.y ? a.y : g_moe_hq;
+    const int nsuper = a.ncols / 512;
+    if constexpr (MODE == 0) {
+        const unsigned long long total = (unsigned long long) nj * gpj;
+        uint32_t i = (uint32_t) (total * blockIdx.x / gridDim.x);
+        const uint32_t i1 = (uint32_t) (total * (blockIdx.x + 1) / gridDim.x);
+        while (i < i1) {
+            const uint32_t ui = i / gpj;
+            const int g0 = (int) (i - ui * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
+            const fnx_job* jb = a.jobs + ui;
+            const int n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
+            const uint8_t* we = a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride;
+            const SuperFields f = tile16_load_buf(tile16_rsrc(we, min(g0 + wave, g1 - 1), nsuper), 0);
+            __syncthreads();   // the unit before has been read (and the codebook written)
+            j16_stage<0>(L, a, y, jb->y, n, FNX_MAXT);
+            __syncthreads();
+            if (n >= 1) j16_segment<1>(L, we, g0, g1, a.ncols, jb->out, n, a.out, a.out_stride, f);
+            i += (uint32_t) (g1 - g0);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < J16_MAXJOBS / J16_THREADS; ++i) {
+            const int j = (int) threadIdx.x + i * J16_THREADS;
+            if (j < nj) jn[j] = (uint8_t) min(max(hn[i], 0), FNX_PF_JOB);
+        }
         __syncthreads();
-        if (threadIdx.x < 64) {
-            const int per = (nj + 63) / 64, j0 = min(nj, (int) threadIdx.x * per), j1 = min(nj, j0 + per);
-            uint32_t mine = 0;
-            for (int j = j0; j < j1; ++j) mine += before[j + 1];
+        auto cost = [](int nt) { return nt > 0 ? (uint32_t) (J16_DEC + J16_MUL * nt) : 0u; };
+        if (wave == 0) {   // the jobs' token tiles, then their costs' running sum: a lane takes a run of jobs
+            const int per = (nj + 63) / 64, j0 = min(nj, lane * per), j1 = min(nj, j0 + per);
+            uint32_t mine = 0, tiles = 0;   // the costs as units of two token tiles
+            for (int j = j0; j < j1; ++j) {
+                const int t = (jn[j] + 15) >> 4;
+                tiles += t;
+                mine += (uint32_t) (t >> 1) * cost(2) + cost(t & 1);
+            }
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) tiles += __shfl_xor(tiles, o);
+            const bool single = (unsigned long long) tiles * gpj <= (unsigned long long) J16_WAVES * gridDim.x;
+            if (single) {   // (few jobs: a second walk)
+                mine = 0;
+                for (int j = j0; j < j1; ++j) mine += (uint32_t) ((jn[j] + 15) >> 4);
+            }
             uint32_t incl = mine;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
                 const uint32_t v = __shfl_up(incl, o, 64);
-                if ((int) threadIdx.x >= o) incl += v;
+                if (lane >= o) incl += v;
             }
             uint32_t run = incl - mine;
+            if (lane == 0) before[0] = 0, tiles_sum = (int) tiles;
             for (int j = j0; j < j1; ++j) {
-                run += before[j + 1];
-                before[j + 1] = run;
+                const int t = (jn[j] + 15) >> 4;
+                run += single ? (uint32_t) t : (uint32_t) (t >> 1) * cost(2) + cost(t & 1);
+                before[j + 1] = (unsigned short) run;
             }
         }
         __syncthreads();
-        units = before[nj];
-    }
-    const unsigned long long total = (unsigned long long) units * gpj;
-    uint32_t i = (uint32_t) (total * blockIdx.x / gridDim.x);
-    const uint32_t i1 = (uint32_t) (total * (blockIdx.x + 1) / gridDim.x);
-    const uint8_t* y = a.y ? a.y : g_moe_hq;
-    const int nsb = a.ncols / 32;
-    while (i < i1) {
-        const uint32_t ui = i / gpj;
-        const int g0 = (int) (i - ui * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
-        int n, w;
-        const int *ys, *outs;
-        if constexpr (MODE == 0) {
-            const fnx_job* jb = a.jobs + ui;
-            n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
-            ys = jb->y, outs = jb->out;
-        } else {
-            int lo = 0, hi = nj - 1;   // the job whose units hold ui: before[j] <= ui < before[j + 1]
+        const uint32_t tiles = (uint32_t) uniform(tiles_sum);
+        const bool single = (unsigned long long) tiles * gpj <= (unsigned long long) J16_WAVES * gridDim.x;
+        uint32_t round = J16_ROUND;   // tiles a round
+        if (single) {   // the smallest with a round a block at most, or a tile a wave
+            round = max(1u, (tiles * gpj + gridDim.x - 1) / gridDim.x);
+            while (round < (uint32_t) J16_WAVES && tiles * ((gpj + round - 1) / round) > gridDim.x) ++round;
+        }
+        const uint32_t rpu = (gpj + round - 1) / round;   // rounds a unit
+        const int ut = single ? 1 : 2;                    // token tiles a unit
+        auto unit_cost = [&](int nt) { return single ? 1u : cost(nt); };
+        const unsigned long long total = (unsigned long long) before[nj] * rpu;
+        unsigned long long c = total * blockIdx.x / gridDim.x;
+        const unsigned long long c1 = total * (blockIdx.x + 1) / gridDim.x;
+        while (c < c1) {   // the same for the whole block
+            int lo = 0, hi = nj - 1;   // the job that c falls in: before[j] rpu <= c < before[j + 1] rpu
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
-                if (before[mid + 1] <= ui) lo = mid + 1;
+                if ((unsigned long long) before[mid + 1] * rpu <= c) lo = mid + 1;
                 else hi = mid;
             }
-            const fnx_bigjob* jb = a.big + uniform(lo);
-            const int q = (int) (ui - before[lo]);
-            n = uniform(min(min(max(jb->n, 0), FNX_PF_JOB) - 16 * q, FNX_MAXT)), w = uniform(jb->w);
-            ys = jb->y + 16 * q, outs = jb->out + 16 * q;
+            lo = uniform(lo);
+            const fnx_bigjob* jb = a.big + lo;
+            // its unit q, which begins at `at`, and the unit's rounds from the first that begins at or after c
+            const uint32_t whole = unit_cost(ut) * rpu;
+            const unsigned long long jat = (unsigned long long) before[lo] * rpu;
+            const int q = uniform((int) ((uint32_t) (c - jat) / whole));
+            const unsigned long long at = jat + (unsigned long long) q * whole;
+            const int n = uniform(min((int) jn[lo] - 16 * ut * q, 16 * ut)), nt = (n + 15) / 16, w = uniform(jb->w);
+            const uint32_t wt = unit_cost(nt);
+            const uint32_t k0 = ((uint32_t) (c - at) + wt - 1) / wt, k1 = c1 - at >= (unsigned long long) wt * rpu ? rpu : ((uint32_t) (c1 - at) + wt - 1) / wt;
+            c = at + (unsigned long long) wt * rpu;
+            const int g0 = uniform((int) (k0 * round)), g1 = uniform((int) min(gpj, k1 * round));
+            if (g0 >= g1) continue;
+            const int *ys = jb->y + 16 * ut * q, *outs = jb->out + 16 * ut * q;
+            const uint8_t* we = a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride;
+            const SuperFields f = tile16_load_buf(tile16_rsrc(we, min(g0 + wave, g1 - 1), nsuper), 0);
+            __syncthreads();   // the unit before has been read (and the codebook written)
+            j16_stage<MODE>(L, a, y, ys, n, 16 * nt);
+            __syncthreads();
+            if (nt == 1) j16_segment<1>(L, we, g0, g1, a.ncols, outs, n, a.out, a.out_stride, f);
+            else j16_segment<2>(L, we, g0, g1, a.ncols, outs, n, a.out, a.out_stride, f);
         }
-        const uint8_t* we = a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride;
-        __syncthreads();   // the unit before has been read (and the codebook written)
-        for (int q = threadIdx.x; q < FNX_MAXT * nsb; q += J16_THREADS) {   // (token, sub-block): its 32 int8 and its scale
-            const int t = q / nsb, sb = q - t * nsb;
-            uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-            float d = 0.f;
-            if (t < n) {
-                if constexpr (MODE == 2) {
-                    const float* gp = a.gu + (size_t) ys[t] * (2 * a.ncols) + 32 * sb;
-                    float4 gv[8], uv[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) gv[k] = reinterpret_cast<const float4*>(gp)[k], uv[k] = reinterpret_cast<const float4*>(gp + a.ncols)[k];
-                    float h[32], amax = 0.f;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        h[4 * k] = silu_f(gv[k].x) * uv[k].x, h[4 * k + 1] = silu_f(gv[k].y) * uv[k].y;
-                        h[4 * k + 2] = silu_f(gv[k].z) * uv[k].z, h[4 * k + 3] = silu_f(gv[k].w) * uv[k].w;
-                    }
-#pragma unroll
-                    for (int k = 0; k < 32; ++k) amax = fmaxf(amax, fabsf(h[k]));
-                    const float dq = amax / 127.0f;   // q8_1_store's arithmetic (kernels.cu:131-145)
-                    d = half_bits_to_float(float_to_half_bits(dq));
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        uint32_t word = 0;
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) {
-                            const int8_t qv = amax == 0.0f ? (int8_t) 0 : (int8_t) roundf(h[4 * k + b] / dq);
-                            word |= (uint32_t) (uint8_t) qv << (8 * b);
-                        }
-                        v[k] = word;
-                    }
-                } else {
-                    const uint8_t* yb = y + ((size_t) ys[t] * nsb + sb) * FNX_Q8_1_BLOCK;
-                    d = half_bits_to_float(*reinterpret_cast<const unsigned short*>(yb));
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const uint32_t*>(yb + 4 + 4 * k);
-                }
-            }
-            uint32_t* dst = reinterpret_cast<uint32_t*>(L.xq + t * J16_XLD + 32 * sb);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) dst[k] = v[k];
-            L.dx[(((sb >> 4) * 4 + (sb & 3)) * FNX_MAXT + t) * 4 + ((sb >> 2) & 3)] = d;
-        }
-        __syncthreads();
-        if (n >= 1) j16_segment(L, we, g0, g1, a.ncols, outs, n, a.out, a.out_stride);
-        i += (uint32_t) (g1 - g0);
     }
 }
 

@@ -251,6 +251,30 @@ def test_moe_big_jobs_over_q8_1_match_the_oracle(dev, oracle, nrows, ncols, nexp
     assert not np.any(got[total:])
 
 
+@pytest.mark.parametrize("nrows,ncols,sizes", [(1024, 2048, [64, 1, 17, 0, 16, 33, 48, 5, 32, 31] * 5), (2048, 512, [64, 1, 17, 0, 33, 48, 16, 5, 50, 49] * 2),
+                                            (528, 1024, [64, 1, 17, 0, 33, 48, 16, 5, 50, 0] * 7), (16, 512, [64, 63, 33, 2] * 400)])
+def test_moe_big_lists_give_the_bits_of_their_jobs_alone(dev, nrows, ncols, sizes):
+    """a long list's jobs go as units of two or four token tiles (a last round of a unit's tiles may be short), a job alone as units of
+    one: a token's sums are the same bits. The last list has more jobs than a launch has rounds a block."""
+    print(f"case moe_big bits nrows={nrows} ncols={ncols} jobs={len(sizes)}", flush=True)
+    rng = np.random.default_rng(97 + nrows)
+    nexp = 3
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, nexp * nrows * ncols // 256, dmax=2e-2)
+    rows = 200
+    jobs, total = make_jobs(rng, nexp, rows, sizes)
+    gu = (rng.standard_normal((rows, 2 * ncols)) * 2).astype(np.float32)
+    xq = dev.quantize_q8_1(gu[:, :ncols])
+    for down, y in ((False, xq), (True, gu)):
+        got = dev.moe_big(w, stride, nrows, ncols, jobs, y, total + 3, down=down, cap=len(jobs) + 5)
+        assert np.any(got[:total] != 0) and not np.any(got[total:])
+        for j in range(10):
+            n = int(jobs[j][1])
+            one = dev.moe_big(w, stride, nrows, ncols, jobs[j:j + 1], y, total + 3, down=down, cap=1)
+            at = jobs[j][2 + PF:2 + PF + n]
+            assert np.array_equal(got[at].view(np.uint32), one[at].view(np.uint32)), f"job {j} of {n} rows, down={down}"
+
+
 def test_moe_mma_weights_equal_the_oracles_f16(dev, oracle):
     # x = unit vectors: the product returns single weights, so every dequantised f16 value is checked bit for bit,
     # subnormal ones included (tiny d)
