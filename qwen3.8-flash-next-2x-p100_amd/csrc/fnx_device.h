@@ -73,8 +73,7 @@ __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + fnx_
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + fnx_expf(-x)); }
 
 // q8_1 quantisation (kernels.cu:131-145), one 32-lane half-wave per block of 32 values
-__device__ __forceinline__ void q8_1_store(float xi, uint8_t* blk, int lane32) {
-    const float amax = group_max<32>(fabsf(xi)), sum = group_sum<32>(xi);
+__device__ __forceinline__ void q8_1_put(float xi, float amax, float sum, uint8_t* blk, int lane32) {   // the block's largest magnitude and sum are known
     const float d = amax / 127.0f;
     const int8_t qv = amax == 0.0f ? (int8_t) 0 : (int8_t) roundf(xi / d);
     reinterpret_cast<int8_t*>(blk + 4)[lane32] = qv;
@@ -82,6 +81,9 @@ __device__ __forceinline__ void q8_1_store(float xi, uint8_t* blk, int lane32) {
         reinterpret_cast<unsigned short*>(blk)[0] = float_to_half_bits(d);
         reinterpret_cast<unsigned short*>(blk)[1] = float_to_half_bits(sum);
     }
+}
+__device__ __forceinline__ void q8_1_store(float xi, uint8_t* blk, int lane32) {
+    q8_1_put(xi, group_max<32>(fabsf(xi)), group_sum<32>(xi), blk, lane32);
 }
 
 // Sums over a weight row's lanes in the reference's order: lane l holds the terms of sub-block l of the row (for rows of 64

@@ -1579,17 +1579,21 @@ int fnx_rms_norm_rows(const float* x, const float* w, float* y, int rows, int n,
     k_rms_norm_rows<<<rows, 256, 0, (hipStream_t) st>>>(x, w, y, n, eps);
     return launch_status("rms_norm_rows");
 }
+static void add_norm_rows(int rows, float* x, const float* add, const CombineArgs& c, const float* w, float* xn, uint8_t* xq, int n, float eps, void* st) {
+    if (n <= 256 * 8) k_add_norm_q8<false, 8><<<rows, 256, 0, (hipStream_t) st>>>(x, add, c, w, xn, xq, n, eps);
+    else k_add_norm_q8<false, NQ_MAXJ><<<rows, 256, 0, (hipStream_t) st>>>(x, add, c, w, xn, xq, n, eps);
+}
 int fnx_add_norm_q8(float* x, const float* add, const float* w, float* xn, void* xq, int rows, int n, float eps, void* st) {
     if (!x || !w) return fail("add_norm_q8: null argument");
     if (rows < 1 || n < 32 || n % 32 || n > 256 * NQ_MAXJ) return fail("add_norm_q8: rows of 32 .. 4096 values in whole 32-value blocks");
-    k_add_norm_q8<false><<<rows, 256, 0, (hipStream_t) st>>>(x, add, CombineArgs{}, w, xn, (uint8_t*) xq, n, eps);
+    add_norm_rows(rows, x, add, CombineArgs{}, w, xn, (uint8_t*) xq, n, eps, st);
     return launch_status("add_norm_q8");
 }
 int fnx_combine_add_norm_q8(const float* part, const float* topw, const float* sh, const float* sh_logit, int sh_logit_stride, int topk, float* x,
                             const float* w, float* xn, void* xq, int rows, int n, float eps, void* st) {
     if (!part || !topw || !sh || !sh_logit || !x || !w) return fail("combine_add_norm_q8: null argument");
     if (rows < 1 || n < 32 || n % 32 || n > 256 * NQ_MAXJ || topk < 1) return fail("combine_add_norm_q8: rows of 32 .. 4096 values in whole 32-value blocks");
-    k_add_norm_q8<true><<<rows, 1024, 0, (hipStream_t) st>>>(x, nullptr, CombineArgs{part, topw, sh, sh_logit, sh_logit_stride, topk, nullptr, nullptr, nullptr, 0},
+    k_add_norm_q8<true, NQ_MAXJ><<<rows, 1024, 0, (hipStream_t) st>>>(x, nullptr, CombineArgs{part, topw, sh, sh_logit, sh_logit_stride, topk, nullptr, nullptr, nullptr, 0},
                                                              w, xn, (uint8_t*) xq, n, eps);
     return launch_status("combine_add_norm_q8");
 }
@@ -1763,7 +1767,7 @@ static int dec_add_norm_q8(const fnx_decoder* D, const DecPending& pend, const f
     }
     if (D->n < 32 || D->n % 32 || D->n > 256 * NQ_MAXJ) return fail("decoder: rows of 32 .. 4096 values in whole 32-value blocks");
     // (after a window that made another pass than this one, x already holds the add)
-    k_add_norm_q8<false><<<T, 256, 0, (hipStream_t) st>>>(ws->x, pend.done_w ? nullptr : pend.rows, c, w, nullptr, (uint8_t*) ws->xq, D->n, D->eps);
+    add_norm_rows(T, ws->x, pend.done_w ? nullptr : pend.rows, c, w, nullptr, (uint8_t*) ws->xq, D->n, D->eps, st);
     return launch_status("decoder add_norm_q8");
 }
 // x (ws->x) through one layer, in place; the layer's own MoE output is left pending for whatever comes next
@@ -1804,7 +1808,7 @@ static int dec_layer(const fnx_decoder* D, const fnx_dec_layer* L, int T, const 
     {   // x += o; xn = norm(x) (fnx_add_norm_q8)
         CombineArgs c{};
         c.gate = gate;
-        k_add_norm_q8<false><<<T, 256, 0, (hipStream_t) st>>>(ws->x, ws->o, c, L->ffn_norm, ws->xn, nullptr, n, D->eps);
+        add_norm_rows(T, ws->x, ws->o, c, L->ffn_norm, ws->xn, nullptr, n, D->eps, st);
         if (launch_status("decoder add_norm")) return 1;
     }
     // the MoE half's rows (those that count) are added by the next pass over x
@@ -1873,7 +1877,7 @@ static int mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, c
         c.vocab = D->vocab;
         c.rows1 = T, c.rows2 = T;
         c.x2 = ws->xn, c.w2 = M->norm_emb, c.xq2 = xq2, c.emb2 = D->emb;
-        k_add_norm_q8<false><<<2 * T, 256, 0, (hipStream_t) st>>>(const_cast<float*>(src), nullptr, c, M->norm_hid, nullptr, (uint8_t*) ws->xq, n, D->eps);
+        add_norm_rows(2 * T, const_cast<float*>(src), nullptr, c, M->norm_hid, nullptr, (uint8_t*) ws->xq, n, D->eps, st);
         if (launch_status("mtp_draft")) return 1;
         // and the two projections one: a block a tile of one of the two matrices, over that matrix's rows
         const long fc_tiles = (M->fc_hid.n_out + 15) / 16 + (M->fc_emb.n_out + 15) / 16;
@@ -1892,7 +1896,7 @@ static int mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, c
         {   // nothing to add: src is only read (fnx_add_norm_q8)
             CombineArgs c{};
             c.gate = gate;
-            k_add_norm_q8<false><<<T, 256, 0, (hipStream_t) st>>>(const_cast<float*>(src), nullptr, c, M->norm_hid, nullptr, (uint8_t*) ws->xq, n, D->eps);
+            add_norm_rows(T, const_cast<float*>(src), nullptr, c, M->norm_hid, nullptr, (uint8_t*) ws->xq, n, D->eps, st);
             if (launch_status("mtp_draft")) return 1;
         }
         if (q8s_one(&M->fc_hid, ws->xq, ws->x, n, T, st, gate, live)) return 1;
@@ -1902,7 +1906,7 @@ static int mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, c
             c.tokens = tokens;
             c.vocab = D->vocab;
             c.gate = gate;
-            k_add_norm_q8<false><<<T, 256, 0, (hipStream_t) st>>>(ws->xn, nullptr, c, M->norm_emb, nullptr, (uint8_t*) ws->xq, n, D->eps);
+            add_norm_rows(T, ws->xn, nullptr, c, M->norm_emb, nullptr, (uint8_t*) ws->xq, n, D->eps, st);
             if (launch_status("mtp_draft")) return 1;
         }
         if (q8s_one(&M->fc_emb, ws->xq, ws->o, n, T, st, gate, live)) return 1;

@@ -56,13 +56,20 @@ struct CombineArgs {
 // WIDE (the combine's form): 1024 threads make the row after the add - a thread the columns p, p + 1024, ..., with all
 // of an expert batch's partial sums in flight (256 threads with 8 columns each took 13 us a call, against 7 us without
 // the combine) - and hand it over in LDS to the first 256, which go on as in the narrow form: the same values and orders.
-template <bool WIDE>
+// NJ: columns a thread, 8 (rows of up to 2048 values) or 16. A launch is a few blocks and their chain of trips: the device words, the
+// row and the norm's weights are asked for together, a lane past the row's end loads the last column and drops it (loads under
+// a condition of their own, the table's converted where they were made, went out one by one), and the NJ blocks of a wave are quantised side by side,
+// their maxima and sums through lane exchanges that would otherwise wait for each other. Rows of 2,048
+// values: eight decode rounds, some ten such launches each, 7,145 -> 6,931 us; a verify step of 16 rows, three launches, 790 -> 779
+template <bool WIDE, int NJ>
 __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __restrict__ x, const float* __restrict__ add, const CombineArgs c,
                                                                   const float* __restrict__ w, float* __restrict__ xn, uint8_t* __restrict__ xq, int n,
                                                                   float eps) {
     __shared__ float sh[4];
-    __shared__ float vrow[WIDE ? 256 * NQ_MAXJ : 1];
-    if (c.gate && uniform(*c.gate) == 0) return;   // (see k_q8s_gemv)
+    __shared__ float vrow[WIDE ? 256 * NJ : 1];
+    int gate_v = 1;   // (looked at when the row has been asked for, see k_q8s_gemv for launches that move more)
+    if (c.gate) gate_v = *c.gate;
+    if (WIDE && uniform(gate_v) == 0) return;
     size_t row = blockIdx.x;
     const uint16_t* emb = c.emb;
     if (!WIDE && c.rows2 > 0 && (int) blockIdx.x >= c.rows1) {   // the launch's second pass
@@ -70,12 +77,12 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
         x = c.x2, w = c.w2, xq = c.xq2, emb = c.emb2;
         xn = nullptr, add = nullptr;
     }
-    float v[NQ_MAXJ], wv[NQ_MAXJ];
+    float v[NJ], wv[NJ];
     float s = 0.f;
     if constexpr (WIDE) {
         // the combine's chains (k_combine's order: the picks ascending), NQ_KB experts' partial sums of this thread's
         // columns in flight at a time (one by one, each load would be a trip to the cache of its own)
-        constexpr int NQ_KB = 5, NQ_WJ = NQ_MAXJ / 4;
+        constexpr int NQ_KB = 5, NQ_WJ = NJ / 4;
         float m[NQ_WJ];
 #pragma unroll
         for (int j = 0; j < NQ_WJ; ++j) m[j] = 0.f;
@@ -122,60 +129,93 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
         __syncthreads();
         if (threadIdx.x >= 256) return;
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) v[j] = vrow[threadIdx.x + 256 * j];
+        for (int j = 0; j < NJ; ++j) v[j] = vrow[threadIdx.x + 256 * j];
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) {
+        for (int j = 0; j < NJ; ++j) {
             const int i = threadIdx.x + 256 * j;
             wv[j] = i < n ? w[i] : 0.f;
         }
     } else {
         // all loads first: a store to x between them would keep the next load waiting for it
-        float av[NQ_MAXJ];
-        const size_t erow = emb ? (size_t) min(max(c.tokens[row], 0), c.vocab - 1) : 0;   // k_embed_rows' clamp
+        const float* arow = add ? add + row * n : x + row * n;
+        const int live_v = c.live ? *c.live : 0x7fffffff;
+        float av[NJ];
+        int at[NJ];
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) {
-            const int i = threadIdx.x + 256 * j;
-            if (emb) v[j] = i < n ? half_bits_to_float(emb[erow * n + i]) : 0.f;
-            else v[j] = i < n ? x[row * n + i] : 0.f;
-            av[j] = add && i < n ? add[row * n + i] : 0.f;
+        for (int j = 0; j < NJ; ++j) at[j] = min((int) threadIdx.x + 256 * j, n - 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) wv[j] = w[at[j]];   // the norm's weights too
+        if (emb) {
+            const uint16_t* er = emb + (size_t) min(max(c.tokens[row], 0), c.vocab - 1) * n;   // k_embed_rows' clamp
+            uint16_t ev[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) ev[j] = er[at[j]];
+            if (add) {
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) av[j] = arow[at[j]];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) v[j] = half_bits_to_float(ev[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) v[j] = x[row * n + at[j]];
+            if (add) {
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) av[j] = arow[at[j]];
+            }
+        }
+        if (uniform(gate_v) == 0) return;
+        if (add && (int) row < live_v) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) v[j] += av[j];
         }
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) {   // the norm's weights too
-            const int i = threadIdx.x + 256 * j;
-            wv[j] = i < n ? w[i] : 0.f;
-        }
-        if (add && (!c.live || (int) row < *c.live)) {
-#pragma unroll
-            for (int j = 0; j < NQ_MAXJ; ++j) v[j] += av[j];
-        }
+        for (int j = 0; j < NJ; ++j)
+            if ((int) threadIdx.x + 256 * j >= n) v[j] = 0.f;
     }
     if (!WIDE && (add || emb)) {
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) {
+        for (int j = 0; j < NJ; ++j) {
             const int i = threadIdx.x + 256 * j;
             if (i < n) x[row * n + i] = v[j];
         }
     }
     if (!WIDE && c.xcopy) {
 #pragma unroll
-        for (int j = 0; j < NQ_MAXJ; ++j) {
+        for (int j = 0; j < NJ; ++j) {
             const int i = threadIdx.x + 256 * j;
             if (i < n) c.xcopy[row * n + i] = v[j];
         }
     }
 #pragma unroll
-    for (int j = 0; j < NQ_MAXJ; ++j) s = fmaf(v[j], v[j], s);   // columns past n hold zeros
+    for (int j = 0; j < NJ; ++j) s = fmaf(v[j], v[j], s);   // columns past n hold zeros
     s = group_sum<64>(s);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
     const float r = rsqrtf((sh[0] + sh[1] + sh[2] + sh[3]) / (float) n + eps);
+    float y[NJ];
 #pragma unroll
-    for (int j = 0; j < NQ_MAXJ; ++j) {
-        const int i = threadIdx.x + 256 * j;
-        if (i < n) {   // n is a multiple of 32: the 32 threads of a q8_1 block are live together
-            const float y = v[j] * r * wv[j];
-            if (xn) xn[row * n + i] = y;
-            if (xq) q8_1_store(y, xq + (row * (n / 32) + i / 32) * FNX_Q8_1_BLOCK, threadIdx.x & 31);
+    for (int j = 0; j < NJ; ++j) y[j] = v[j] * r * wv[j];
+    if (xn) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            if (i < n) xn[row * n + i] = y[j];
+        }
+    }
+    if (xq) {   // n is a multiple of 32: the 32 threads of a q8_1 block are live together (q8_1_store's values)
+        float amax[NJ], sum[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) amax[j] = fabsf(y[j]), sum[j] = y[j];
+#pragma unroll
+        for (int o = 16; o; o >>= 1)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) amax[j] = fmaxf(amax[j], __shfl_xor(amax[j], o, WAVE)), sum[j] += __shfl_xor(sum[j], o, WAVE);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            if (i < n) q8_1_put(y[j], amax[j], sum[j], xq + (row * (n / 32) + i / 32) * FNX_Q8_1_BLOCK, threadIdx.x & 31);
         }
     }
 }
