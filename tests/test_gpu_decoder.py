@@ -45,7 +45,7 @@ def test_rms_norm_rows(dev, oracle):
     assert err <= 3e-6 * float(np.abs(want).max()), err
 
 
-@pytest.mark.parametrize("n,with_add", [(2048, True), (2048, False), (4096, True), (96, True)])
+@pytest.mark.parametrize("n,with_add", [(2048, True), (2048, False), (4096, True), (96, True), (2080, True), (800, False)])
 def test_add_norm_q8_equals_the_three_operators(dev, n, with_add):
     rng = np.random.default_rng(805 + n)
     x, w = rng.standard_normal((5, n)).astype(np.float32) * 2, rng.standard_normal(n).astype(np.float32)
