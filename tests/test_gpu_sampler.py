@@ -67,6 +67,27 @@ def test_top_tokens_ties_zeros_and_non_finite(dev, oracle):
     assert tied.size > 32 and np.all(np.diff(tied) > 0) and tied[0] < 64
 
 
+@pytest.mark.parametrize("kind", ["close", "lowest", "outliers", "spread", "negative"])
+def test_top_tokens_where_the_threshold_is_looked_for(dev, oracle, kind):
+    """keys a few steps apart, all but a handful of the lowest value, a few far above the rest, from one end of the floats to the other"""
+    print(f"case top_tokens threshold {kind}", flush=True)
+    rng = np.random.default_rng(15)
+    n = 5120 + 66   # two whole slices and one of little more than the candidates
+    x = rng.standard_normal((3, n)).astype(np.float32)
+    if kind == "close":
+        x = (np.float32(1.0).view(np.int32) + rng.integers(-40, 40, (3, n))).astype(np.int32).view(np.float32)
+    elif kind == "lowest":
+        x[:] = -np.finfo(np.float32).max
+        x[0, 5:60], x[1, 2500:2564], x[2, 100:165] = 1.0, 2.0, rng.standard_normal(65).astype(np.float32)
+    elif kind == "outliers":
+        x[:, rng.integers(0, n, 20)] = np.finfo(np.float32).max
+    elif kind == "spread":
+        x = (x * np.exp(rng.uniform(-80, 80, (3, n)))).astype(np.float32)
+    else:
+        x = -np.abs(x) - 1
+    same(d_top_tokens(dev, x), o_top_tokens(oracle, x))
+
+
 def test_top_tokens_bias_and_penalties(dev, oracle):
     rng = np.random.default_rng(9)
     n, T, v0 = 151936, 16, 0
