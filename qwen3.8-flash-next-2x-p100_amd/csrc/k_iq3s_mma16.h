@@ -227,13 +227,14 @@ __global__ void __launch_bounds__(J16_THREADS) k_iq3s_jobs_mma16(const RowsArgs 
             const int g0 = (int) (i - ui * gpj), g1 = (int) min(gpj, g0 + (i1 - i));
             const fnx_job* jb = a.jobs + ui;
             const int n = uniform(min(jb->n, FNX_MAXT)), w = uniform(jb->w);
+            i += (uint32_t) (g1 - g0);
+            if (n < 1) continue;   // the same for the whole block; a job without rows names no matrix
             const uint8_t* we = a.ep ? uniform_ptr(a.ep[w]) : a.wbase + (size_t) w * a.w_stride;
             const SuperFields f = tile16_load_buf(tile16_rsrc(we, min(g0 + wave, g1 - 1), nsuper), 0);
             __syncthreads();   // the unit before has been read (and the codebook written)
             j16_stage<0>(L, a, y, jb->y, n, FNX_MAXT);
             __syncthreads();
-            if (n >= 1) j16_segment<1>(L, we, g0, g1, a.ncols, jb->out, n, a.out, a.out_stride, f);
-            i += (uint32_t) (g1 - g0);
+            j16_segment<1>(L, we, g0, g1, a.ncols, jb->out, n, a.out, a.out_stride, f);
         }
     } else {
 #pragma unroll

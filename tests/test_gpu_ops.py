@@ -279,6 +279,27 @@ def test_mmvq_jobs_pick_experts_and_rows(dev, oracle, packed, tile16):
     assert np.array_equal(dev.mmvq(w, stride, nrows, ncols, jobs, yq, at, njobs_dev=False, packed=packed, tile16=tile16), got)
 
 
+def test_mmvq_tile16_jobs_without_rows_name_no_matrix(dev, oracle):
+    """a job of no rows is passed by whatever its matrix number says: nothing is read through it (first, last and between others)"""
+    print("case tile16 empty jobs", flush=True)
+    rng = np.random.default_rng(422)
+    nexp, nrows, ncols = 3, 512, 1024
+    w = random_iq3s(rng, nexp * nrows * ncols // 256)
+    yq = oracle.quantize_q8_1(rng.standard_normal((16, ncols)).astype(np.float32))
+    counts = [0, 0, 5, 0, 16, 1, 0, 0] * 3
+    jobs = np.zeros(len(counts), dtype=JOB_DTYPE)
+    at = 0
+    for j, n in enumerate(counts):
+        jobs["w"][j], jobs["n"][j] = (j % nexp, n) if n else ((-1, 1 << 30, -1 << 31)[j % 3], -(j % 2))
+        jobs["y"][j, :n] = rng.permutation(16)[:n]
+        jobs["out"][j, :n] = np.arange(at, at + n)
+        at += n
+    got = dev.mmvq(w, nrows * (ncols // 256) * 110, nrows, ncols, jobs, yq, at, tile16=True)
+    live = jobs[jobs["n"] > 0]
+    assert np.array_equal(got, dev.mmvq(w, nrows * (ncols // 256) * 110, nrows, ncols, live, yq, at, tile16=True))
+    assert rel_l2(got, oracle.mmvq(w, nrows * (ncols // 256) * 110, nrows, ncols, live, yq, at)) <= 1e-5
+
+
 # a block's first run comes in every kind (no rows, one row over few and over many units, several rows) and is followed by jobs of
 # another kind: the codebook is written once, whichever comes first
 @pytest.mark.parametrize("nrows,counts", [(96, [0, 1, 2, 16, 1, 5, 0]), (16, [1, 0, 16, 3]), (1040, [1, 4]), (20480, [1]), (20480, [3, 1]),
