@@ -267,7 +267,8 @@ int fnx_f32_f16(const float* x, size_t n, uint16_t* out, void* st);
  * products of a sub-block, then d_w (1 + 2 s) d_x) for jobs of up to FNX_PF_JOB rows. gate_up: gu[jobs.out][2 ffs] from the
  * q8_1 rows xq[jobs.y] of A->n_in values; down: part[jobs.out][n] from h = silu(gate) * up of the rows gu[jobs.y] ([gate |
  * up] of 2 * A->n_in floats), quantised to q8_1 on the way (moe.cuh:597-608). tile16 matrices (rows in 16s, 512 .. 2048
- * columns in 512s), 1 .. 4096 jobs a launch; a job's rows go sixteen at a time through the int8 matrix cores. The two
+ * columns in 512s), 1 .. 4096 jobs a launch (njobs_cap bounds *njobs; no entry from *njobs on is read); a job's rows go
+ * through the int8 matrix cores in units of up to thirty-two, two tiles of sixteen to a decode. The two
  * families of prompt kernels - these and the f16 ones below - differ by the activations' q8_1 rounding: a caller's choice,
  * as the reference's. */
 int fnx_moe_gate_up_big(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const int* njobs, int njobs_cap, const void* xq, float* gu,

@@ -1149,7 +1149,7 @@ int fnx_moe_down(const fnx_dw* A, size_t sa, const fnx_job* jobs, const int* njo
     if (launch_status("moe_down")) return 1;
     return rows_launch(A, sa, jobs, njobs, njobs_max, nullptr, part, A->n_out, st, "moe_down");
 }
-// the prompt path's jobs over q8_1 activations (kernels.hpp:324-325): tile16 matrices, a job's rows sixteen at a time on the
+// the prompt path's jobs over q8_1 activations (kernels.hpp:324-325): tile16 matrices, a job's rows up to thirty-two at a time on the
 // int8 matrix cores (k_iq3s_mma16.h)
 static int big_launch(const fnx_dw* W, size_t w_stride, const fnx_bigjob* jobs, const int* njobs, int njobs_cap, const void* xq, const float* gu,
                       float* out, const char* who) {

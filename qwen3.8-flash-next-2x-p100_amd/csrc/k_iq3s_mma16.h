@@ -199,22 +199,23 @@ __global__ void __launch_bounds__(J16_THREADS) k_iq3s_jobs_mma16(const RowsArgs 
     __shared__ unsigned short before[MODE ? J16_MAXJOBS + 2 : 1];   // costs of the jobs before job j, a round of each of their units
     __shared__ int tiles_sum;
     const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6));
-    // every job's token count, whether it counts or not, asked for along with the codebook
+    const int nj_raw = a.njobs ? *a.njobs : a.njobs_max;
+    const uint32_t code0 = g_sgrid.v[threadIdx.x & 511];
+    const int nj = max(0, min(min(uniform(nj_raw), a.njobs_max), MODE ? J16_MAXJOBS : a.njobs_max));
+    // the token counts of the jobs that count, on their way while the codebook is written
     int hn[MODE ? J16_MAXJOBS / J16_THREADS : 1] = {};
     if constexpr (MODE != 0) {
 #pragma unroll
         for (int i = 0; i < J16_MAXJOBS / J16_THREADS; ++i) {
             const int j = (int) threadIdx.x + i * J16_THREADS;
-            if (j < a.njobs_max) hn[i] = a.big[j].n;
+            if (j < nj) hn[i] = a.big[j].n;
         }
     }
-    const int nj_raw = a.njobs ? *a.njobs : a.njobs_max;
-    for (int g = threadIdx.x; g < 512; g += J16_THREADS) {   // a code's sixteen signed entries from its unsigned one
-        const uint32_t g0 = g_sgrid.v[g];
+    if (threadIdx.x < 512) {   // a code's sixteen signed entries from its unsigned one
+        const int g = threadIdx.x;
 #pragma unroll
-        for (int sg = 0; sg < 16; ++sg) L.tab[2 * (sg * 512 + g)] = L.tab[2 * (sg * 512 + g) + 1] = signed_entry(g0, sg);
+        for (int sg = 0; sg < 16; ++sg) L.tab[2 * (sg * 512 + g)] = L.tab[2 * (sg * 512 + g) + 1] = signed_entry(code0, sg);
     }
-    const int nj = max(0, min(min(uniform(nj_raw), a.njobs_max), MODE ? J16_MAXJOBS : a.njobs_max));
     const uint32_t gpj = (uint32_t) a.nrows / 16;   // items per unit
     const uint8_t* y = a.y ? a.y : g_moe_hq;
     const int nsuper = a.ncols / 512;

@@ -275,6 +275,24 @@ def test_moe_big_lists_give_the_bits_of_their_jobs_alone(dev, nrows, ncols, size
             assert np.array_equal(got[at].view(np.uint32), one[at].view(np.uint32)), f"job {j} of {n} rows, down={down}"
 
 
+@pytest.mark.parametrize("sizes,cap", [([5, 64, 17], 4096), ([3] * 1100 + [40], 4096), ([], 4096)])
+def test_moe_big_reads_no_job_past_the_count(dev, sizes, cap):
+    """njobs_cap bounds the count that the device word gives: the array itself may end with the last job that counts"""
+    print(f"case moe_big short array jobs={len(sizes)} cap={cap}", flush=True)
+    rng = np.random.default_rng(98)
+    nrows, ncols, nexp, rows = 64, 512, 3, 200
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, nexp * nrows * ncols // 256, dmax=2e-2)
+    jobs, total = make_jobs(rng, nexp, rows, sizes)
+    if not sizes:   # one job that does not count
+        jobs = make_jobs(rng, nexp, rows, [7])[0]
+    gu = (rng.standard_normal((rows, 2 * ncols)) * 2).astype(np.float32)
+    for down, y in ((False, dev.quantize_q8_1(gu[:, :ncols])), (True, gu)):
+        got = dev.moe_big(w, stride, nrows, ncols, jobs, y, total + 3, down=down, cap=cap, short=True, count=len(sizes))
+        want = dev.moe_big(w, stride, nrows, ncols, jobs, y, total + 3, down=down, cap=len(jobs), count=len(sizes))
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) and bool(np.any(want[:total] != 0)) == bool(sizes)
+
+
 def test_moe_mma_weights_equal_the_oracles_f16(dev, oracle):
     # x = unit vectors: the product returns single weights, so every dequantised f16 value is checked bit for bit,
     # subnormal ones included (tiny d)
