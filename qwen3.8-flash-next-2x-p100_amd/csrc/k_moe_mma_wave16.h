@@ -332,16 +332,19 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     const unsigned vb = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     __shared__ Wave16GuLds L;
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), r = lane & 15, grp = lane >> 4;
+    const int nj_raw = *a.njobs, nj2_raw = a.jobs2 ? *a.njobs2 : 0;
+    const uint32_t tab0 = g_sgrid.v[tid & 511];
+    const int nj = min(a.cap, uniform(nj_raw)), nj2 = a.jobs2 ? min(a.cap2, uniform(nj2_raw)) : 0, njall = nj + nj2;
+    // the token counts and matrices of the jobs that count, on their way while the codebook is written
+    const int held = min(nj, W16_GU_HELD), held2 = min(nj2, W16_GU_HELD);
     int hn[2] = {0, 0}, hn2 = 0, hw[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int j = tid + i * W16_THREADS;
-        if (j < min(a.cap, W16_GU_HELD)) hn[i] = a.jobs[j].n, hw[i] = a.jobs[j].w;
+        if (j < held) hn[i] = a.jobs[j].n, hw[i] = a.jobs[j].w;
     }
-    if (a.jobs2 && tid < min(a.cap2, W16_GU_HELD)) hn2 = a.jobs2[tid].n;
-    const int nj_raw = *a.njobs, nj2_raw = a.jobs2 ? *a.njobs2 : 0;
+    if (tid < held2) hn2 = a.jobs2[tid].n;
     {
-        const uint32_t tab0 = g_sgrid.v[tid & 511];
 #pragma unroll
         for (int i = tid; i < SGRID_WORDS; i += W16_THREADS) {
             const uint32_t g = signed_entry(tab0, i >> 9);
@@ -356,13 +359,10 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int j = tid + i * W16_THREADS;
-        if (j < min(a.cap, W16_GU_HELD)) L.jn[0][j] = (uint8_t) max(0, min(FNX_PF_JOB, hn[i])), L.jw[j] = hw[i];
+        if (j < held) L.jn[0][j] = (uint8_t) max(0, min(FNX_PF_JOB, hn[i])), L.jw[j] = hw[i];
     }
-    if (a.jobs2) {
-        if (tid < min(a.cap2, W16_GU_HELD)) L.jn[1][tid] = (uint8_t) max(0, min(FNX_PF_JOB, hn2));
-        for (int j = tid + W16_THREADS; j < min(a.cap2, W16_GU_HELD); j += W16_THREADS) L.jn[1][j] = (uint8_t) max(0, min(FNX_PF_JOB, a.jobs2[j].n));
-    }
-    const int nj = min(a.cap, uniform(nj_raw)), nj2 = a.jobs2 ? min(a.cap2, uniform(nj2_raw)) : 0, njall = nj + nj2;
+    if (tid < held2) L.jn[1][tid] = (uint8_t) max(0, min(FNX_PF_JOB, hn2));
+    for (int j = tid + W16_THREADS; j < held2; j += W16_THREADS) L.jn[1][j] = (uint8_t) max(0, min(FNX_PF_JOB, a.jobs2[j].n));
     const int ffh = a.ffh, nsuper = a.ncols >> 9, ppj = ffh >> 4;                      // pairs of tiles a job
     const int upj = (ppj + W16_WAVES - 1) / W16_WAVES;                                  // heavy units a job
     auto job_at = [&](int j) { return j < nj ? a.jobs + j : a.jobs2 + (j - nj); };
