@@ -119,20 +119,36 @@ __device__ __forceinline__ void j16_segment(J16Lds<TOKS>& L, const uint8_t* __re
 // MODE 1: the prompt path's jobs of up to FNX_PF_JOB rows (kernels.hpp:324, moe_gate_up_big): a job's rows in units of up to two
 // token tiles, so that a weight is decoded once for both. A unit of nt token tiles costs J16_DEC + J16_MUL nt for each of its
 // rounds, J16_ROUND tiles of 16 rows; the blocks split the costs of all rounds evenly (a prefix sum over the jobs in LDS) and each
-// takes the rounds that begin in its share. Lists of so few tiles that the blocks have no more than a tile a wave are bound by a
-// tile's chain of steps and by what comes before it: there a unit is one token tile, and a round as many tiles as leave every block
-// a round of one unit, where that can be - a second unit would be staged after the first.
+// takes the rounds that begin in its share. Lists of so few tiles that the blocks have no more than J16_SINGLE each are bound by a
+// tile's chain of steps and by what comes before it: there a unit is one token tile, and up to a tile a wave a round is as many
+// tiles as leave every block a round of one unit, where that can be - a second unit would be staged after the first.
 // MODE 2 (kernels.hpp:325, moe_down_big): the same with the unit's activations made on the way from the rows [gate | up] of 2 ncols floats:
 // h = silu(gate) * up quantised as k_swiglu_q8_1 does it, four threads a sub-block.
 constexpr int J16_MAXJOBS = 4096;   // big jobs a launch (their token counts and costs live in LDS)
 // us a chunk of 512 experts, Zipf (a decode for every sixteen tokens, jobs' starts looked up in memory as their turn came / this), 300
 // rows: 192 / 171, 1,024: 389 / 335, 4,096: 1,302 / 1,014; 77 rows, uniform: 234 / 210; the shared expert's launches over 300 rows 23.6 / 18.1 and
-// 30.5 / 20.5. Rounds of 8 tiles 173, 336, 1,019, 212, of 16 182, 337, 1,026, 219: a unit's last tiles and the block's run come
-// out less even than the waves' idle turns in a short round cost. Four token tiles a unit (of up to 1024 columns; sums spill) were slower: 40.9 -> 46
+// 30.5 / 20.5. Rounds of 8 tiles are the same within the noise (173, 336, 1,019, 212), of 16 slower (182, 337, 1,026, 219): a unit's
+// last tiles and the block's run come out less even. Four token tiles a unit (of up to 1024 columns; sums spill) were slower: 40.9 -> 46
 // us a down launch of 300 rows.
-constexpr int J16_ROUND = 4, J16_DEC = 3, J16_MUL = 2;
+// J16_SINGLE: us a launch of gate|up (1,024 x 2,048) and down (2,048 x 512), units of one token tile up to 16 / 24 / 32 tiles a block: 17
+// jobs of 64 rows 29.5 / 26.9 / 26.8 and 27, ten 17.1 and 24.8 / 17.7 / 17.7, 24 of them 29.7 / 29.1 / 29.1 and 28, 32 26.3 / 26.6 / 33.4 and
+// 24.2. What comes before a block's first tile is a launch of its own size: a job of one row 11.5 and 8.7 us with the costs' sums
+// exchanged through LDS and a division for each rule, 10.0 and 7.3 with DPP moves and divisions only where a list needs them.
+constexpr int J16_SINGLE = 24, J16_ROUND = 4, J16_DEC = 3, J16_MUL = 2;
 static_assert(J16_MAXJOBS * (FNX_PF_JOB / 32) * (J16_DEC + 2 * J16_MUL) < 65536, "the costs' sum in 16 bits");
 
+// the sum of the wave's lanes up to and including this one (DPP moves: an exchange through LDS is a trip of its own a step)
+__device__ __forceinline__ uint32_t wave_running(uint32_t v) {
+#define FNX_DPP_ADDU(ctrl, rmask) v += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, ctrl, rmask, 0xF, false)
+    FNX_DPP_ADDU(0x111, 0xF);   // row_shr:1, 2, 4, 8
+    FNX_DPP_ADDU(0x112, 0xF);
+    FNX_DPP_ADDU(0x114, 0xF);
+    FNX_DPP_ADDU(0x118, 0xF);
+    FNX_DPP_ADDU(0x142, 0xA);   // row_bcast15 into rows 1 and 3
+    FNX_DPP_ADDU(0x143, 0xC);   // row_bcast31 into rows 2 and 3
+#undef FNX_DPP_ADDU
+    return v;
+}
 // a unit's activations (n tokens, toks places) to LDS
 template <int MODE, int TOKS>
 __device__ __forceinline__ void j16_stage(J16Lds<TOKS>& L, const RowsArgs& a, const uint8_t* y, const int* ys, int n, int toks) {
@@ -244,50 +260,45 @@ __global__ void __launch_bounds__(J16_THREADS) k_iq3s_jobs_mma16(const RowsArgs 
             if (j < nj) jn[j] = (uint8_t) min(max(hn[i], 0), FNX_PF_JOB);
         }
         __syncthreads();
-        auto cost = [](int nt) { return nt > 0 ? (uint32_t) (J16_DEC + J16_MUL * nt) : 0u; };
-        if (wave == 0) {   // the jobs' token tiles, then their costs' running sum: a lane takes a run of jobs
+        constexpr uint32_t C1 = J16_DEC + J16_MUL, C2 = J16_DEC + 2 * J16_MUL;   // a round's cost in a unit of one token tile, of two
+        if (wave == 0) {
+            // the jobs' token tiles (high half) and their costs as units of two token tiles (low half), their running sums made
+            // together: a lane takes a run of jobs
             const int per = (nj + 63) / 64, j0 = min(nj, lane * per), j1 = min(nj, j0 + per);
-            uint32_t mine = 0, tiles = 0;   // the costs as units of two token tiles
-            for (int j = j0; j < j1; ++j) {
-                const int t = (jn[j] + 15) >> 4;
-                tiles += t;
-                mine += (uint32_t) (t >> 1) * cost(2) + cost(t & 1);
-            }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) tiles += __shfl_xor(tiles, o);
-            const bool single = (unsigned long long) tiles * gpj <= (unsigned long long) J16_WAVES * gridDim.x;
-            if (single) {   // (few jobs: a second walk)
-                mine = 0;
-                for (int j = j0; j < j1; ++j) mine += (uint32_t) ((jn[j] + 15) >> 4);
-            }
-            uint32_t incl = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t v = __shfl_up(incl, o, 64);
-                if (lane >= o) incl += v;
-            }
+            auto of_job = [&](int j) {
+                const uint32_t t = (jn[j] + 15u) >> 4;
+                return t << 16 | ((t >> 1) * C2 + (t & 1) * C1);
+            };
+            uint32_t mine = 0;
+            for (int j = j0; j < j1; ++j) mine += of_job(j);
+            const uint32_t incl = wave_running(mine);
+            const uint32_t tiles = (uint32_t) __builtin_amdgcn_readlane((int) incl, 63) >> 16;
+            const int half = (unsigned long long) tiles * gpj <= (unsigned long long) J16_SINGLE * gridDim.x ? 16 : 0;   // units of one token tile count as one
             uint32_t run = incl - mine;
             if (lane == 0) before[0] = 0, tiles_sum = (int) tiles;
             for (int j = j0; j < j1; ++j) {
-                const int t = (jn[j] + 15) >> 4;
-                run += single ? (uint32_t) t : (uint32_t) (t >> 1) * cost(2) + cost(t & 1);
-                before[j + 1] = (unsigned short) run;
+                run += of_job(j);
+                before[j + 1] = (unsigned short) (run >> half);
             }
         }
         __syncthreads();
         const uint32_t tiles = (uint32_t) uniform(tiles_sum);
-        const bool single = (unsigned long long) tiles * gpj <= (unsigned long long) J16_WAVES * gridDim.x;
-        uint32_t round = J16_ROUND;   // tiles a round
-        if (single) {   // the smallest with a round a block at most, or a tile a wave
-            round = max(1u, (tiles * gpj + gridDim.x - 1) / gridDim.x);
-            while (round < (uint32_t) J16_WAVES && tiles * ((gpj + round - 1) / round) > gridDim.x) ++round;
+        const bool single = (unsigned long long) tiles * gpj <= (unsigned long long) J16_SINGLE * gridDim.x;
+        uint32_t round = J16_ROUND, rpu = (gpj + J16_ROUND - 1) / J16_ROUND;   // tiles a round, rounds a unit
+        if (single && tiles * gpj <= J16_WAVES * gridDim.x) {   // the smallest with a round a block at most, or a tile a wave
+            round = 1, rpu = gpj;
+            if (tiles * gpj > gridDim.x) {
+                round = (tiles * gpj + gridDim.x - 1) / gridDim.x, rpu = (gpj + round - 1) / round;
+                for (; round < (uint32_t) J16_WAVES && tiles * rpu > gridDim.x; rpu = (gpj + round - 1) / round) ++round;
+            }
         }
-        const uint32_t rpu = (gpj + round - 1) / round;   // rounds a unit
-        const int ut = single ? 1 : 2;                    // token tiles a unit
-        auto unit_cost = [&](int nt) { return single ? 1u : cost(nt); };
+        const int ut = single ? 1 : 2;   // token tiles a unit
+        const uint32_t whole = (single ? 1u : C2) * rpu;
+        // the block's share of the costs: the blocks' shares differ by one at most
         const unsigned long long total = (unsigned long long) before[nj] * rpu;
-        unsigned long long c = total * blockIdx.x / gridDim.x;
-        const unsigned long long c1 = total * (blockIdx.x + 1) / gridDim.x;
+        const unsigned long long each = total >> 32 ? total / gridDim.x : total < gridDim.x ? 0u : (uint32_t) total / gridDim.x, rest = total - each * gridDim.x;
+        unsigned long long c = each * blockIdx.x + min((unsigned long long) blockIdx.x, rest);
+        const unsigned long long c1 = c + each + (blockIdx.x < rest ? 1u : 0u);
         while (c < c1) {   // the same for the whole block
             int lo = 0, hi = nj - 1;   // the job that c falls in: before[j] rpu <= c < before[j + 1] rpu
             while (lo < hi) {
@@ -298,14 +309,17 @@ __global__ void __launch_bounds__(J16_THREADS) k_iq3s_jobs_mma16(const RowsArgs 
             lo = uniform(lo);
             const fnx_bigjob* jb = a.big + lo;
             // its unit q, which begins at `at`, and the unit's rounds from the first that begins at or after c
-            const uint32_t whole = unit_cost(ut) * rpu;
             const unsigned long long jat = (unsigned long long) before[lo] * rpu;
-            const int q = uniform((int) ((uint32_t) (c - jat) / whole));
+            const int nall = uniform((int) jn[lo]), q = nall > 16 * ut ? uniform((int) ((uint32_t) (c - jat) / whole)) : 0;
             const unsigned long long at = jat + (unsigned long long) q * whole;
-            const int n = uniform(min((int) jn[lo] - 16 * ut * q, 16 * ut)), nt = (n + 15) / 16, w = uniform(jb->w);
-            const uint32_t wt = unit_cost(nt);
-            const uint32_t k0 = ((uint32_t) (c - at) + wt - 1) / wt, k1 = c1 - at >= (unsigned long long) wt * rpu ? rpu : ((uint32_t) (c1 - at) + wt - 1) / wt;
-            c = at + (unsigned long long) wt * rpu;
+            const int n = min(nall - 16 * ut * q, 16 * ut), nt = (n + 15) / 16, w = uniform(jb->w);
+            const uint32_t end = (single ? 1u : nt == 1 ? C1 : C2) * rpu;   // the unit's costs
+            uint32_t k0 = (uint32_t) (c - at), k1 = c1 - at >= end ? end : (uint32_t) (c1 - at);
+            if (!single) {
+                k0 = nt == 1 ? (k0 + C1 - 1) / C1 : (k0 + C2 - 1) / C2;
+                k1 = nt == 1 ? (k1 + C1 - 1) / C1 : (k1 + C2 - 1) / C2;
+            }
+            c = at + end;
             const int g0 = uniform((int) (k0 * round)), g1 = uniform((int) min(gpj, k1 * round));
             if (g0 >= g1) continue;
             const int *ys = jb->y + 16 * ut * q, *outs = jb->out + 16 * ut * q;

@@ -252,10 +252,14 @@ def test_moe_big_jobs_over_q8_1_match_the_oracle(dev, oracle, nrows, ncols, nexp
 
 
 @pytest.mark.parametrize("nrows,ncols,sizes", [(1024, 2048, [64, 1, 17, 0, 16, 33, 48, 5, 32, 31] * 5), (2048, 512, [64, 1, 17, 0, 33, 48, 16, 5, 50, 49] * 2),
-                                            (528, 1024, [64, 1, 17, 0, 33, 48, 16, 5, 50, 0] * 7), (16, 512, [64, 63, 33, 2] * 400)])
+                                            (528, 1024, [64, 1, 17, 0, 33, 48, 16, 5, 50, 0] * 7), (16, 512, [64, 63, 33, 2] * 400),
+                                            (1024, 2048, [64] * 17), (2048, 512, [40] * 13), (1024, 2048, [1] * 5), (1024, 2048, [64, 2] * 20),
+                                            (48, 512, [64, 1, 33, 0, 17] * 819)])
 def test_moe_big_lists_give_the_bits_of_their_jobs_alone(dev, nrows, ncols, sizes):
-    """a long list's jobs go as units of two or four token tiles (a last round of a unit's tiles may be short), a job alone as units of
-    one: a token's sums are the same bits. The last list has more jobs than a launch has rounds a block."""
+    """a long list's jobs go as units of one or two token tiles, runs of their rounds dealt to the blocks (a last round of a unit's
+    tiles may be short), a short list's as units of one: a token's sums are the same bits. Every job of the list is compared
+    with the same job in a list of a few, its first and last jobs with those jobs alone. (Jobs to a block, rounds to a block, a
+    few tiles more than a wave each, 4,095 jobs: the plan's forms and their ends.)"""
     print(f"case moe_big bits nrows={nrows} ncols={ncols} jobs={len(sizes)}", flush=True)
     rng = np.random.default_rng(97 + nrows)
     nexp = 3
@@ -265,10 +269,16 @@ def test_moe_big_lists_give_the_bits_of_their_jobs_alone(dev, nrows, ncols, size
     jobs, total = make_jobs(rng, nexp, rows, sizes)
     gu = (rng.standard_normal((rows, 2 * ncols)) * 2).astype(np.float32)
     xq = dev.quantize_q8_1(gu[:, :ncols])
+    pieces = max(2, min(len(jobs) // 4, 60))
     for down, y in ((False, xq), (True, gu)):
-        got = dev.moe_big(w, stride, nrows, ncols, jobs, y, total + 3, down=down, cap=len(jobs) + 5)
-        assert np.any(got[:total] != 0) and not np.any(got[total:])
-        for j in range(10):
+        got = dev.moe_big(w, stride, nrows, ncols, jobs, y, total + 3, down=down, cap=min(len(jobs) + 5, 4096))
+        assert np.all(np.any(got[:total] != 0, axis=1)) and not np.any(got[total:])
+        few = np.zeros_like(got)
+        for part in np.array_split(np.arange(len(jobs)), pieces):
+            lo, hi = sum(sizes[:part[0]]), sum(sizes[:part[-1] + 1])
+            few[lo:hi] = dev.moe_big(w, stride, nrows, ncols, jobs[part], y, total + 3, down=down)[lo:hi]
+        assert np.array_equal(got.view(np.uint32), few.view(np.uint32)), f"rows {np.flatnonzero(np.any(got != few, axis=1))[:8]}, down={down}"
+        for j in [*range(min(10, len(jobs))), len(jobs) - 2, len(jobs) - 1]:
             n = int(jobs[j][1])
             one = dev.moe_big(w, stride, nrows, ncols, jobs[j:j + 1], y, total + 3, down=down, cap=1)
             at = jobs[j][2 + PF:2 + PF + n]
