@@ -302,17 +302,23 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
 // lightest on one block made the launch half as long again as its mean block. So the jobs are ranked by token tiles and the
 // units of those with two token tiles and more dealt heaviest first, to and fro over the blocks. The pairs of the jobs of up
 // to 16 tokens then fill the blocks up to the mean load: a block stages all the tokens of its stretch's jobs at once, S tiles
-// of sixteen places, and its waves take the pairs one by one as they come free (77 rows, some 400 jobs of two tokens: 84 us;
+// of sixteen places, and its waves take the pairs one by one as they come free (77 rows, some 400 jobs of two tokens: 87 us;
 // 114 as units of eight pairs, a wave a tile, with a job's tokens fetched and the block met twice in each of them: of such a
-// unit's 16 us the LDS needs 9). The weights of the next super-step are asked for in the middle of the one before. Every
-// tile is accumulated in one order (S, then the four steps, then a step's four operands) whatever a job's size or the
-// unit it falls in: a row's h does not depend on what else is in the chunk.
+// unit's 16 us the LDS needs 9). A stage with pairs for half of the waves or fewer goes a wave a tile, the up tiles' sums handed to
+// the gate tiles' waves (a lone job of 5 tokens 16.0 -> 15.5 us, 125 jobs of 9, some of whose stretches are two stages, 36.3 -> 33.7).
+// The weights of the next super-step are asked for in the middle of the one before. Every tile is accumulated in one order (S,
+// then the four steps, then a step's four operands) whatever a job's size or the unit it falls in: a row's h does not
+// depend on what else is in the chunk.
 // Costs, in 1/16 us at S = 4 (measured): a heavy unit of so many token tiles; a light pair, of which a block works on sixteen at a time.
 __device__ __forceinline__ int w16_heavy_cost(int nt) { return 320 + 88 * nt; }
 constexpr int W16_PAIR_COST = 18;
 __device__ __forceinline__ int w16_mean(int heavy, int np, int G) { return (int) (((long) heavy + (long) np * W16_PAIR_COST + G - 1) / G); }
-// where the stretch of np pairs begins whose share starts at c of all (monotone in c, 0 at 0 and np at all)
-__device__ __forceinline__ int w16_part(int np, int c, int all) { return all > 0 ? (int) ((double) np * (double) c / (double) all) : 0; }
+__device__ __forceinline__ double w16_inverse(int all) {   // of a positive count, to the last bits: a step on the unit's estimate
+    const double v = __builtin_amdgcn_rcp((double) all);
+    return fma(v, fma((double) -all, v, 1.0), v);
+}
+// where the stretch of n pairs begins whose share starts at c of all (monotone in c, 0 at 0 and n at all)
+__device__ __forceinline__ int w16_part(int n, int c, int all, double inv) { return c >= all ? n : min(n, (int) fma((double) n, (double) c * inv, 1e-4)); }
 constexpr int W16_SORTJ = 2048, W16_GU_HELD = 2048, W16_PLAN = 4;   // (W16_PLAN: blocks a lane of the planning wave looks after)
 struct Wave16GuLds {
     uint2 tab[SGRID_WORDS];
@@ -321,7 +327,8 @@ struct Wave16GuLds {
     int jw[W16_GU_HELD];
     unsigned short jorder[W16_SORTJ];   // the jobs, most token tiles first (the lower index first among equals)
     int orow[FNX_PF_JOB];   // a heavy unit's tokens' places in the output
-    int p_total[MB_TP + 1], p_first, p_last;   // the jobs by token tiles; the plan where one wave made it: this block's stretch of the light pairs
+    float4 xs[W16_WAVES / 2][64];   // up tiles' sums on their way to the gate tiles' waves
+    int p_total[MB_TP + 1], p_alone, p_first, p_last;   // the jobs by token tiles, those of 9 .. 16 tokens; the plan where one wave made it: this block's stretch of the light pairs
     int ph_jobs, ph_tokens, ph_next;                      // a phase of light pairs: its jobs, their tokens, the next pair to take
     unsigned short ph_job[16];
     unsigned char ph_first[16];                           // a job's first place in LDS
@@ -373,11 +380,12 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     __syncthreads();
     const bool sorted = njall <= W16_SORTJ;
     if (sorted && wave == 0) {   // a counting sort by one wave, 64 jobs a trip: class totals, then every job's place
-        int total[MB_TP + 1];
+        int total[MB_TP + 1], alone = 0;   // alone: light jobs of more than half of a phase's places
 #pragma unroll
         for (int c = 0; c <= MB_TP; ++c) total[c] = 0;
         for (int j0 = 0; j0 < njall; j0 += 64) {
-            const int kj = j0 + lane < njall ? (n_of(j0 + lane) + 15) >> 4 : -1;
+            const int n = j0 + lane < njall ? n_of(j0 + lane) : -16, kj = (n + 15) >> 4;
+            alone += __popcll(__ballot(n > 8 && n <= 16));
 #pragma unroll
             for (int c = 0; c <= MB_TP; ++c) total[c] += __popcll(__ballot(kj == c));
         }
@@ -404,6 +412,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         if (lane == 0) {
 #pragma unroll
             for (int c = 0; c <= MB_TP; ++c) L.p_total[c] = total[c];
+            L.p_alone = alone;
         }
         if (nb > G) {   // (heavy units on one block or none: the same plan in closed form, below, by every wave)
             auto load_of = [&](int bb) {   // block bb's heavy units
@@ -448,7 +457,8 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
                     if (o0 + i < ome) c += ld[i];
                     if (o0 + i == ome) mine = ld[i];
                 }
-                L.p_first = w16_part(np, c, all), L.p_last = w16_part(np, c + mine, all);
+                const double inv = w16_inverse(all);
+                L.p_first = w16_part(np, c, all, inv), L.p_last = w16_part(np, c + mine, all, inv);
             }
         }
     }
@@ -475,7 +485,17 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         auto after = [&](int lo, int hi, int b) { return max(0, hi - max(lo, b)); };   // blocks of [lo, hi) from b on
         auto shares = [&](int b) { return after(nb, G, b) * s0 + after(hi2, nb, b) * s1 + after(hi3, hi2, b) * s2 + after(hi4, hi3, b) * s3 + after(0, hi4, b) * s4; };
         const int all = shares(0);
-        p_first = uniform(w16_part(np, shares(b1), all)), p_last = uniform(w16_part(np, shares(b1 - 1), all));
+        // A stretch in which two jobs meet whose tokens do not fit the places together is two phases. Where that happens to lists of
+        // so few pairs that a block has one phase, the stretches are whole eights of one job instead (us a launch, S = 4; units of
+        // eight pairs / as their shares fall / eights): 128 jobs of some 6 tokens, 8 pairs a block, 19.5 / 27.2 / 19.8; 60 jobs of 16
+        // tokens, 15 a block, 31.9 / 34.3 / 32.1. Not where few jobs are large (64 of 5 tokens, 8 a block, 19.2 / 19.0) nor at 9 to 13
+        // pairs a block (80 jobs of 16 tokens, 10 a block, 31.2 / 26.1 / 31.1; 100, 12.5 a block, 31.4 / 29.6 / 31.0).
+        const int most = nb < G ? s0 : hi2 < nb ? s1 : hi3 < hi2 ? s2 : hi4 < hi3 ? s3 : s4, alone = uniform(L.p_alone);
+        const long load = (long) np * most;   // the longest stretch is load / all
+        const bool eights = ppj % 8 == 0 && (load <= 8l * all ? 16 * alone > tot[1] : load > 13l * all && load <= 16l * all && 2 * alone > tot[1]);
+        const int by = eights ? 3 : 0;
+        const double inv = w16_inverse(all);
+        p_first = uniform(w16_part(np >> by, shares(b1), all, inv) << by), p_last = uniform(w16_part(np >> by, shares(b1 - 1), all, inv) << by);
     } else if (sorted) {
         p_first = uniform(L.p_first), p_last = uniform(L.p_last);
     }
@@ -575,6 +595,36 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
             const int k = __popcll(__ballot(lane < jobs && (int) L.ph_first[lane & 15] <= wave)) - 1;
             const int y = uniform(job_at((int) L.ph_job[k])->y[wave - (int) L.ph_first[k]]);
             for (int S = 0; S < nsuper; ++S) lds_load16(a.x + (size_t) y * a.ldx + 512 * S, 16u * lane, xt_at + (16 * S + wave) * W16_XROW);
+        }
+        if (pe - p0 <= W16_WAVES / 2) {   // pairs for half of the waves: a wave a tile, the up tiles' sums go over to the gate tiles' waves
+            constexpr int HALF = W16_WAVES / 2;
+            const int q = p0 + wave % HALF, up = wave / HALF, jo = min(q, pe - 1) / ppj, pr = min(q, pe - 1) - jo * ppj;
+            const int k = jo - jo0, j = uniform((int) L.ph_job[k]), at = uniform((int) L.ph_first[k]);
+            const fnx_bigjob* jb = job_at(j);
+            const int orow = q < pe && !up && r < n_of(j) ? jb->out[r] : -1;
+            const __amdgpu_buffer_rsrc_t m = tile16_rsrc(matrix_of(j, jb), up * ppj + pr, nsuper);
+            SuperFields f = tile16_load_buf(m, 0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            v4f acc[MB_TP] = {};
+            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 256 * grp;
+            for (int S = 0; S < nsuper && q < pe; ++S) {
+                turn(S);
+                const SuperFields nf = tile16_load_buf(m, min(S + 1, nsuper - 1));
+                w16_super_step(L.tab, xk + S * 16 * W16_XROW, f, 1, acc);
+                f = nf;
+            }
+            if (up) L.xs[wave % HALF][lane] = make_float4(acc[0].x, acc[0].y, acc[0].z, acc[0].w);
+            __syncthreads();
+            if (orow >= 0) {
+                const float4 ut = L.xs[wave % HALF][lane];
+                const v4f gt = acc[0];
+                uint2 hv;
+                hv.x = h16_pair(silu_f(gt.x), ut.x, silu_f(gt.y), ut.y), hv.y = h16_pair(silu_f(gt.z), ut.z, silu_f(gt.w), ut.w);
+                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
+            }
+            p0 = pe;
+            continue;
         }
         // a wave's pair p: its job's place in the phase, its matrix's two rows of tiles
         int p = p0 + wave;

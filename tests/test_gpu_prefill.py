@@ -208,6 +208,41 @@ def test_moe_gate_up_h16_one_launch_equals_two(dev, oracle, ffs, ncols, nexp, si
         assert rel_l2(one.astype(np.float32), want.astype(np.float32)) <= 1e-3
 
 
+@pytest.mark.parametrize("ffs,ncols,sizes", [
+    (512, 2048, [1, 2, 3] * 140),                                              # some 400 jobs of two tokens: phases of many jobs
+    (32, 512, [16, 8, 8, 15, 2, 16, 0, 1, 1, 14, 9, 7, 0, 16] * 20),           # two pairs a job: phases that end at sixteen tokens and just past them
+    (16, 512, [1] * 600 + [16, 1]),                                            # a pair a job: phases of sixteen jobs
+    (256, 2048, [9, 3, 12, 7] * 32), (1024, 2048, [16] * 60), (512, 2048, [9] * 125),   # stretches of whole eights
+    (512, 2048, [16] * 80), (512, 1536, [5] * 40), (80, 1024, [16, 3] * 50),   # ten pairs a block, five, ten pairs a job
+    (512, 2048, [20] * 3 + [9] * 50), (512, 2048, [64] * 40 + [12] * 60), (256, 1024, [64] * 300 + [10, 2] * 40),   # beside heavy units: some blocks, several a block
+    (32, 512, [3, 16, 1, 40, 0, 17, 64, 33] * 270)])                           # more jobs than are ranked
+def test_moe_gate_up_h16_lists_give_the_bits_of_their_jobs_alone(dev, ffs, ncols, sizes):
+    """however a list's work is dealt to the blocks (a wave a tile or a pair of tiles, jobs staged together, ranked or in the
+    list's order), a row's h is the same bits: every job of the list is compared with the same job in a list of a few, some of them with the job alone"""
+    print(f"case moe_gate_up_h16 bits ffs={ffs} ncols={ncols} jobs={len(sizes)}", flush=True)
+    assert len(sizes) <= 2048 or ffs == 32, "the kernel ranks up to 2,048 jobs"
+    rng = np.random.default_rng(743 + ffs + len(sizes))
+    nexp, nrows, rows = 3, 2 * ffs, 200
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, nexp * nrows * ncols // 256, dmax=2e-2)
+    x16 = rng.standard_normal((rows, ncols)).astype(np.float16)
+    jobs, total = make_jobs(rng, nexp, rows, sizes)
+
+    def h_of(some):
+        return dev.moe_mma(w, stride, nrows, ncols, some, x16, total + 3, packed=True, tile16=True, h16=True)[0]
+
+    got = h_of(jobs)
+    assert np.all(np.any(got[:total] != 0, axis=1)) and not np.any(got[total:])
+    few = np.zeros_like(got)
+    for part in np.array_split(np.arange(len(jobs)), max(2, min(len(jobs) // 4, 60))):
+        lo, hi = sum(sizes[:part[0]]), sum(sizes[:part[-1] + 1])
+        few[lo:hi] = h_of(jobs[part])[lo:hi]
+    assert np.array_equal(got.view(np.uint16), few.view(np.uint16)), f"rows {np.flatnonzero(np.any(got != few, axis=1))[:8]}"
+    for j in [0, 1, 2, len(jobs) // 2, len(jobs) - 2, len(jobs) - 1]:
+        at = jobs[j][2 + PF:2 + PF + int(jobs[j][1])]
+        assert np.array_equal(got[at].view(np.uint16), h_of(jobs[j:j + 1])[at].view(np.uint16)), f"job {j} of {jobs[j][1]} rows"
+
+
 def split_in_16s(jobs):
     """jobs of up to 64 rows as the jobs of up to 16 rows they consist of (the oracle's mmvq takes those)"""
     out = []
@@ -367,12 +402,13 @@ def test_prefill_layer_tile16_equals_unit64(dev, oracle, n, ff, nexp, topk, Cn):
     assert rel_l2(b["out"], want["out"]) <= REL_L2
 
 
-@pytest.mark.parametrize("tile16,Cn", [(False, 8192), (True, 8192), (True, 2048)])
+@pytest.mark.parametrize("tile16,Cn", [(False, 8192), (True, 8192), (True, 2048), (True, 16384)])
 def test_prefill_layer_large_chunk_equals_small_chunks(dev, tile16, Cn):
     """A size-independent property at a size the oracle does not reach: a row's result does not depend on what else is in
     its chunk, so 8,192 rows in one call (more tasks than one pass of a block's task list holds, every kernel form's loop
     over list passes, a thousand jobs and more split over the wave form's blocks) must equal the same rows in 16 calls of
-    512, bit for bit, in either layout. (2,048 rows: a few hundred jobs, ranked, their heavy units several to a block.)"""
+    512, bit for bit, in either layout. (2,048 rows: a few hundred jobs, ranked, their heavy units several to a block; 16,384:
+    more jobs than the wave form ranks, the shared expert's in a list of their own.)"""
     n, ff, nexp, topk, small = 2048, 512, 64, 10, 512
     print(f"case prefill_layer large n={n} ff={ff} nexp={nexp} topk={topk} C={Cn} tile16={tile16}", flush=True)
     rng = np.random.default_rng(777)
@@ -382,7 +418,10 @@ def test_prefill_layer_large_chunk_equals_small_chunks(dev, tile16, Cn):
     sh_gu, sh_down = random_iq3s(rng, nb(2 * ff, n), dmax=1e-3), random_iq3s(rng, nb(n, ff), dmax=1e-3)
     router = (rng.standard_normal((nexp + 1, n)) * 0.05).astype(np.float32)
     x = rng.standard_normal((Cn, n)).astype(np.float32)
-    big = fnx_gpu.PfLayerDev(dev, n, ff, nexp, topk, router, gu, down, sh_gu, sh_down, Cn, packed=True, tile16=tile16).run(x)["out"]
+    r = fnx_gpu.PfLayerDev(dev, n, ff, nexp, topk, router, gu, down, sh_gu, sh_down, Cn, packed=True, tile16=tile16).run(x)
+    big = r["out"]
+    assert Cn != 16384 or int(r["njobs"].sum()) > 2048, "more jobs than are ranked"
+    del r
     L = fnx_gpu.PfLayerDev(dev, n, ff, nexp, topk, router, gu, down, sh_gu, sh_down, small, packed=True, tile16=tile16)
     assert np.all(np.isfinite(big))
     for c0 in range(0, Cn, small):
