@@ -1510,7 +1510,11 @@ static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const 
         a.h16 = h16;
         a.ffh = A->n_out / 2;
         if (h16_done) *h16_done = true;
-        const long upj = (a.ffh / 16 + 7) / 8;   // the finer of its two kinds of units
+        // eight pairs a block at least, what its waves take a tile each. A grid of a pair a block is better where every job is of a few
+        // tokens (one job of 5: 15.8 -> 11.1 us), worse where a short list has large jobs too, whose units then come to lie on fewer
+        // of the eight XCDs (four jobs of 64 tokens and four of 3: 37.3 -> 39.0 us, 37.8 -> 40.8 at a feed-forward width of
+        // 1,024); the jobs' sizes are not known here
+        const long upj = (a.ffh / 16 + 7) / 8;
         const int grid = (int) std::max(1l, std::min<long>(std::min(cu_count(), 64 * W16_PLAN), caps * upj));
         k_moe_mma_wave16_gu<<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
         return launch_status(who);
