@@ -118,6 +118,23 @@ __device__ __forceinline__ float butterfly_sum(float v) {
 #undef FNX_DPP_ADD
     return v;
 }
+// the same exchanges for the greatest value (width >= 16)
+template <int width>
+__device__ __forceinline__ float butterfly_max(float v) {
+    static_assert(width == 16 || width == 32, "of one or two 16-lane rows");
+#define FNX_DPP_MAX(ctrl) v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false)))
+    if constexpr (width == 32) {
+        float x = v, y = v;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+        v = fmaxf(x, y);
+    }
+    FNX_DPP_MAX(0x128);
+    FNX_DPP_MAX(0x124);
+    FNX_DPP_MAX(0x4E);
+    FNX_DPP_MAX(0xB1);
+#undef FNX_DPP_MAX
+    return v;
+}
 
 // A value every lane of the wave holds alike, moved to a scalar register: what is computed from it (addresses, loop
 // bounds) then runs on the scalar unit. Loads from memory the kernel may also write are vector loads even at a uniform

@@ -56,11 +56,14 @@ struct CombineArgs {
 // WIDE (the combine's form): 1024 threads make the row after the add - a thread the columns p, p + 1024, ..., with all
 // of an expert batch's partial sums in flight (256 threads with 8 columns each took 13 us a call, against 7 us without
 // the combine) - and hand it over in LDS to the first 256, which go on as in the narrow form: the same values and orders.
-// NJ: columns a thread, 8 (rows of up to 2048 values) or 16. A launch is a few blocks and their chain of trips: the device words, the
+// NJ: columns a thread. A launch over a window is a few blocks and their chain of trips: the device words, the
 // row and the norm's weights are asked for together, a lane past the row's end loads the last column and drops it (loads under
-// a condition of their own, the table's converted where they were made, went out one by one), and the NJ blocks of a wave are quantised side by side,
-// their maxima and sums through lane exchanges that would otherwise wait for each other. Rows of 2,048
-// values: eight decode rounds, some ten such launches each, 7,145 -> 6,931 us; a verify step of 16 rows, three launches, 790 -> 779
+// a condition of their own, the table's converted where they were made, went out one by one), and a wave's blocks are quantised
+// four side by side, their maxima and sums through the vector unit's own exchanges, the columns past the row's end left out. Rows of
+// 2,048 values: eight decode rounds, some ten such launches each, 7,145 -> 6,931 us; a verify step of 16 rows, three
+// launches, 790 -> 779; a launch of 16 rows 7.2 -> 4.6 us. A launch over 4,096 rows is bound by the exchanges and by what lies past the
+// row's end: 2,048 values (with add / without) 29.7 / 20.1 -> 22.4 / 18.5 us, 1,024 17.1 / 13.6 -> 12.9 / 10.8, 32 10.8 / 9.6 -> 4.9 / 4.7
+// (exchanges through LDS, all of 8 or 16 columns a thread whatever the row: 23.6 / 19.5, 19.7 / 17.8, 17.4 / 16.9)
 template <bool WIDE, int NJ>
 __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __restrict__ x, const float* __restrict__ add, const CombineArgs c,
                                                                   const float* __restrict__ w, float* __restrict__ xn, uint8_t* __restrict__ xq, int n,
@@ -205,17 +208,18 @@ __global__ void __launch_bounds__(WIDE ? 1024 : 256) k_add_norm_q8(float* __rest
         }
     }
     if (xq) {   // n is a multiple of 32: the 32 threads of a q8_1 block are live together (q8_1_store's values)
-        float amax[NJ], sum[NJ];
+        constexpr int CH = NJ < 4 ? NJ : 4;   // columns side by side; a wave leaves out those past the row's end
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) amax[j] = fabsf(y[j]), sum[j] = y[j];
+        for (int j0 = 0; j0 < NJ; j0 += CH) {
+            if (uniform((int) threadIdx.x & ~63) + 256 * j0 >= n) break;
+            float amax[CH], sum[CH];
 #pragma unroll
-        for (int o = 16; o; o >>= 1)
+            for (int j = 0; j < CH; ++j) amax[j] = butterfly_max<32>(fabsf(y[j0 + j])), sum[j] = butterfly_sum<32>(y[j0 + j]);
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) amax[j] = fmaxf(amax[j], __shfl_xor(amax[j], o, WAVE)), sum[j] += __shfl_xor(sum[j], o, WAVE);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int i = threadIdx.x + 256 * j;
-            if (i < n) q8_1_put(y[j], amax[j], sum[j], xq + (row * (n / 32) + i / 32) * FNX_Q8_1_BLOCK, threadIdx.x & 31);
+            for (int j = 0; j < CH; ++j) {
+                const int i = threadIdx.x + 256 * (j0 + j);
+                if (i < n) q8_1_put(y[j0 + j], amax[j], sum[j], xq + (row * (n / 32) + i / 32) * FNX_Q8_1_BLOCK, threadIdx.x & 31);
+            }
         }
     }
 }

@@ -45,7 +45,8 @@ def test_rms_norm_rows(dev, oracle):
     assert err <= 3e-6 * float(np.abs(want).max()), err
 
 
-@pytest.mark.parametrize("n,with_add", [(2048, True), (2048, False), (4096, True), (96, True), (2080, True), (800, False)])
+@pytest.mark.parametrize("n,with_add", [(2048, True), (2048, False), (4096, True), (96, True), (2080, True), (800, False),
+                                        (32, True), (256, False), (288, True), (1024, True), (1056, False), (3072, True), (3104, False)])   # where a thread's columns change
 def test_add_norm_q8_equals_the_three_operators(dev, n, with_add):
     rng = np.random.default_rng(805 + n)
     x, w = rng.standard_normal((5, n)).astype(np.float32) * 2, rng.standard_normal(n).astype(np.float32)
@@ -58,7 +59,20 @@ def test_add_norm_q8_equals_the_three_operators(dev, n, with_add):
     assert np.array_equal(xq, dev.quantize_q8_1(want_n))
 
 
-@pytest.mark.parametrize("T,n,topk", [(16, 2048, 10), (3, 2048, 10), (5, 96, 2)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_add_norm_q8_of_rows_that_are_not_finite(dev, bad):
+    """the scale and codes of a block with a value that is no number are those of the quantisation by itself; other rows do not see it"""
+    rng = np.random.default_rng(807)
+    x, w = rng.standard_normal((3, 800)).astype(np.float32), rng.standard_normal(800).astype(np.float32)
+    x[1, 40] = bad
+    _, xn, xq = dev.add_norm_q8(x, None, w, 1e-6)
+    got, want = xq.reshape(3, -1, 36), dev.quantize_q8_1(xn).reshape(3, -1, 36)
+    keep = np.r_[0:2, 4:36]   # (a sum that is no number may hold any payload)
+    assert np.array_equal(got[..., keep], want[..., keep]) and np.array_equal(got[[0, 2]], want[[0, 2]])
+    assert np.all(np.isfinite(xn[[0, 2]])) and not np.all(np.isfinite(xn[1]))
+
+
+@pytest.mark.parametrize("T,n,topk", [(16, 2048, 10), (3, 2048, 10), (5, 96, 2), (2, 1024, 10), (2, 1056, 3), (2, 4096, 10)])
 def test_combine_add_norm_q8_equals_combine_then_add_norm(dev, oracle, T, n, topk):
     """the hand-over between two decoder layers in one launch: the values of fnx_moe_combine followed by fnx_add_norm_q8"""
     rng = np.random.default_rng(806 + T)
