@@ -67,6 +67,19 @@ def test_top_tokens_ties_zeros_and_non_finite(dev, oracle):
     assert tied.size > 32 and np.all(np.diff(tied) > 0) and tied[0] < 64
 
 
+@pytest.mark.parametrize("n", [64, 65, 66, 100, 127, 128, 129, 2560, 2561, 2563, 2600, 2624, 2688, 5121])
+def test_top_tokens_of_little_more_than_the_candidates(dev, oracle, n):
+    """a row, or a row's last slice, that brings the wave's real pairs to the candidates' number or just past it: the one too many at
+    either end of the row, in the last slice's only place, and tied with the last that is kept"""
+    print(f"case top_tokens n={n}", flush=True)
+    rng = np.random.default_rng(16 + n)
+    x = rng.standard_normal((5, n)).astype(np.float32)
+    x[1, -1], x[2, 0] = -100.0, -100.0
+    x[3, -1] = np.sort(x[3])[-64]
+    x[4] = (np.float32(1.0).view(np.int32) + rng.permutation(n)).astype(np.int32).view(np.float32)   # a key apart each
+    same(d_top_tokens(dev, x), o_top_tokens(oracle, x))
+
+
 @pytest.mark.parametrize("kind", ["close", "lowest", "outliers", "spread", "negative"])
 def test_top_tokens_where_the_threshold_is_looked_for(dev, oracle, kind):
     """keys a few steps apart, all but a handful of the lowest value, a few far above the rest, from one end of the floats to the other"""
