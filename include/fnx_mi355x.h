@@ -276,7 +276,8 @@ int fnx_moe_gate_up_big(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, cons
 int fnx_moe_down_big(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const int* njobs, int njobs_cap, const float* gu, float* part,
                      void* st);
 /* kernels.hpp:328  moe_gate_up_mma: gu[jobs.out][2 ffs] = W_e[2 ffs][n] . xh[jobs.y] with f16 weights (each the f32
- * value rounded once), f16 activations, fp32 accumulation, on the matrix cores. xh rows of A->n_in halves. Raw blocks and
+ * value rounded once), f16 activations, fp32 accumulation, on the matrix cores. xh rows of A->n_in halves; njobs_cap =
+ * capacity of the job array, in these operators and the next (entries from *njobs on may be read, and are not used). Raw blocks and
  * unit64 (tile16 gate|up matrices go through fnx_moe_gate_up_h16_mma, which leaves h). */
 int fnx_moe_gate_up_mma(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const int* njobs, int njobs_cap, const uint16_t* xh, float* gu,
                         void* st);
