@@ -243,6 +243,28 @@ def test_moe_gate_up_h16_lists_give_the_bits_of_their_jobs_alone(dev, ffs, ncols
         assert np.array_equal(got[at].view(np.uint16), h_of(jobs[j:j + 1])[at].view(np.uint16)), f"job {j} of {jobs[j][1]} rows"
 
 
+@pytest.mark.parametrize("sizes", [[5, 64, 17], [3] * 1100 + [40]])
+def test_moe_gate_up_h16_reads_no_job_past_the_count(dev, sizes):
+    """the capacity bounds the count that the device word gives: the job array may end with the last job that counts"""
+    import ctypes as C
+    print(f"case moe_gate_up_h16 short array jobs={len(sizes)}", flush=True)
+    rng = np.random.default_rng(744)
+    ffs, ncols, nexp, rows, t = 32, 512, 3, 200, dev.torch
+    w = random_iq3s(rng, nexp * 2 * ffs * ncols // 256, dmax=2e-2)
+    x16 = rng.standard_normal((rows, ncols)).astype(np.float16)
+    jobs, total = make_jobs(rng, nexp, rows, sizes)
+    want = dev.moe_mma(w, 2 * ffs * ncols // 256 * 110, 2 * ffs, ncols, jobs, x16, total, packed=True, tile16=True, h16=True)[0]
+    u64, tiles = dev.up(w), dev.zeros(dev.lib.fnx_iq3s_tile16_bytes(2 * ffs, ncols, nexp), t.uint8)
+    dev.ok(dev.lib.fnx_iq3s_repack(u64.data_ptr(), u64.data_ptr(), w.size // 110 * 256, dev.st()))
+    dev.ok(dev.lib.fnx_iq3s_tile16(u64.data_ptr(), tiles.data_ptr(), 2 * ffs, ncols, nexp, dev.st()))
+    W, dj, dx, got = dev.pkg.dw(tiles, ncols, 2 * ffs, tile16=True), dev.up(jobs), dev.up(x16), dev.zeros((total, ffs), t.float16)
+    count = dev.up(np.array([len(sizes)], dtype=np.int32))
+    dev.ok(dev.lib.fnx_moe_gate_up_h16_mma(C.byref(W), dev.lib.fnx_iq3s_tile16_bytes(2 * ffs, ncols, 1), dj.data_ptr(), count.data_ptr(), 4096, dx.data_ptr(),
+                                           got.data_ptr(), dev.st()))
+    dev.sync()
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16)) and np.all(np.any(want != 0, axis=1))
+
+
 def split_in_16s(jobs):
     """jobs of up to 64 rows as the jobs of up to 16 rows they consist of (the oracle's mmvq takes those)"""
     out = []
