@@ -268,27 +268,52 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
         SuperFields f = tile16_load(we, 16 * min(g, g1 - 1) + r, 0, 1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        for (; g < g1; g += W16_WAVES) {
-            // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
-            // for the last: every wave takes every priority in turn, a tile each
-            switch (((wave >> 2) + ((g - g0) >> 4)) & 3) {
-                case 0: __builtin_amdgcn_s_setprio(0); break;
-                case 1: __builtin_amdgcn_s_setprio(1); break;
-                case 2: __builtin_amdgcn_s_setprio(2); break;
-                default: __builtin_amdgcn_s_setprio(3); break;
+        // A tile's results go out as buffer stores that every path issues (a lane without a token: past the buffer's end, where
+        // a store is dropped): stores under a condition of their own cannot be counted, and the wait for the next tile's weights,
+        // asked for before them, was a wait for the stores too (77 rows, some 400 jobs of two tokens: 59.1 -> 56.7 us a launch, 512 rows
+        // 36.0 -> 35.2, 4,096 rows the same 186). A job with a row past what 32-bit offsets reach stores under the condition.
+        const uint32_t rowb = (uint32_t) a.nrows * 4u, end = 0xE0000000u, none = 0xF0000000u;   // (none and a row's bytes: no wrap)
+        const int reach = (int) (end / rowb);
+        uint32_t at[MB_TP];
+        bool near = true;
+#pragma unroll
+        for (int tt = 0; tt < MB_TP; ++tt) near = near && orow[tt] < reach, at[tt] = orow[tt] >= 0 ? (uint32_t) orow[tt] * rowb + 16u * grp : none;
+        const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*) a.out, 0, (int) end, 0x00020000);
+        auto rounds = [&](auto nt_tag, auto near_tag) {
+            constexpr int NT = decltype(nt_tag)::value;
+            for (; g < g1; g += W16_WAVES) {
+                // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
+                // for the last: every wave takes every priority in turn, a tile each
+                switch (((wave >> 2) + ((g - g0) >> 4)) & 3) {
+                    case 0: __builtin_amdgcn_s_setprio(0); break;
+                    case 1: __builtin_amdgcn_s_setprio(1); break;
+                    case 2: __builtin_amdgcn_s_setprio(2); break;
+                    default: __builtin_amdgcn_s_setprio(3); break;
+                }
+                const SuperFields nf = tile16_load(we, 16 * (g + W16_WAVES < g1 ? g + W16_WAVES : g) + r, 0, 1);
+                __builtin_amdgcn_sched_barrier(0);   // (left to itself the compiler asks for them behind the products)
+                v4f acc[MB_TP];
+#pragma unroll
+                for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+                w16_super_step(L.tab, xlane, f, NT, acc);
+                // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) {
+                    if constexpr (decltype(near_tag)::value) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[tt]), to, at[tt], 64u * g, 0);
+                    else if (orow[tt] >= 0)
+                        *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
+                }
+                f = nf;
             }
-            const SuperFields nf = tile16_load(we, 16 * (g + W16_WAVES < g1 ? g + W16_WAVES : g) + r, 0, 1);
-            v4f acc[MB_TP];
-#pragma unroll
-            for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-            w16_super_step(L.tab, xlane, f, nt, acc);
-            // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
-#pragma unroll
-            for (int tt = 0; tt < MB_TP; ++tt)
-                if (orow[tt] >= 0)
-                    *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
-            f = nf;
-        }
+        };
+        auto any_nt = [&](auto near_tag) {
+            if (nt == 4) rounds(std::integral_constant<int, 4>{}, near_tag);
+            else if (nt == 3) rounds(std::integral_constant<int, 3>{}, near_tag);
+            else if (nt == 2) rounds(std::integral_constant<int, 2>{}, near_tag);
+            else rounds(std::integral_constant<int, 1>{}, near_tag);
+        };
+        if (__all(near)) any_nt(std::true_type{});
+        else any_nt(std::false_type{});
     }
 }
 

@@ -181,6 +181,38 @@ def test_moe_mma_wave_form_tile16_rows_of_512(dev, oracle, nrows, nexp, sizes):
         assert rel_l2(got, want) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
 
 
+@pytest.mark.parametrize("n", [1, 17, 64])
+def test_moe_mma_wave_form_output_rows_past_32_bit_offsets(dev, n):
+    # a job with an output row past 3.5 GiB stores by whole addresses: the same bits as by buffer offsets, in both orders of rows
+    print(f"case moe_mma wave form far rows n={n}", flush=True)
+    import ctypes as C
+    t, nrows, ncols = dev.torch, 2048, 512
+    far = 0xE0000000 // (nrows * 4)
+    rng = np.random.default_rng(760 + n)
+    w = dev.up(random_iq3s(rng, nrows * ncols // 256, dmax=2e-2))
+    dev.ok(dev.lib.fnx_iq3s_repack(w.data_ptr(), w.data_ptr(), nrows * ncols, dev.st()))
+    d16 = dev.zeros(dev.lib.fnx_iq3s_tile16_bytes(nrows, ncols, 1), t.uint8)
+    dev.ok(dev.lib.fnx_iq3s_tile16(w.data_ptr(), d16.data_ptr(), nrows, ncols, 1, dev.st()))
+    W = dev.pkg.dw(d16, ncols, nrows, tile16=True)
+    x = dev.up(rng.standard_normal((n, ncols)).astype(np.float16).view(np.int16))
+    out = t.empty((far + 80, nrows), dtype=t.float32, device="cuda:0")
+    nj, got = dev.up(np.array([1], dtype=np.int32)), []
+    for last in (n - 1, far - 1, far, far + 79):   # the last token's row
+        job = np.zeros((1, 2 + 2 * PF), dtype=np.int32)
+        job[0, 1], job[0, 2:2 + n] = n, np.arange(n)
+        job[0, 2 + PF:2 + PF + n] = np.arange(n)
+        job[0, 2 + PF + n - 1] = last
+        rows = t.from_numpy(job[0, 2 + PF:2 + PF + n].astype(np.int64)).to(out.device)
+        out[rows] = float("nan")
+        dj = dev.up(job)
+        dev.ok(dev.lib.fnx_moe_down_mma(C.byref(W), 0, dj.data_ptr(), nj.data_ptr(), 1, x.data_ptr(), out.data_ptr(), dev.st()))
+        dev.sync()
+        got.append(out[rows].cpu().numpy())
+    assert np.isfinite(got[0]).all()
+    for g in got[1:]:
+        assert np.array_equal(g, got[0])
+
+
 @pytest.mark.parametrize("ffs,ncols,nexp,sizes", [(512, 2048, 24, [64, 1, 17, 0, 16, 33, 48, 5, 64, 64, 2, 0, 31, 64, 49, 15] * 3), (128, 512, 3, [64, 1, 17, 16, 33, 48, 5]),
                                                   (256, 1024, 2, [3]), (640, 2048, 2, [64, 9]), (128, 2560, 2, [5, 64, 20, 16])])
 def test_moe_gate_up_h16_one_launch_equals_two(dev, oracle, ffs, ncols, nexp, sizes):
