@@ -569,15 +569,23 @@ constexpr int AM_THREADS = 1024, AM_PER_BLOCK = 16384;
 // logits, behind one another: 8.2 -> 6.8 us, with the lookup between 6.3 (64-bit keys exchanged lane by lane, the sixteen waves' keys folded by one thread, a count that
 // released and acquired the caches).
 __device__ __forceinline__ unsigned wave_umin(unsigned v) { return ~wave_umax(~v); }
+// KEEP: a chain step's head (one row): the row's last block keeps the pick, and makes the next window after the last step (k_round.h).
+template <bool KEEP>
 __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__ logits, int rows, unsigned long long* __restrict__ keys,
-                                                      unsigned* __restrict__ err, int v0, float* __restrict__ bv, int* __restrict__ bi,
-                                                      const int* __restrict__ live) {
+                                                      unsigned* __restrict__ err, int v0, float* __restrict__ bv, int* bi,
+                                                      const int* __restrict__ live, const ChainKeep keep) {
     __shared__ uint2 wbest[AM_THREADS / 64];
     __shared__ int wbad[AM_THREADS / 64];
     // live (may be null): a device word; rows from *live on do not count: they are not scanned and their picks stay what they were
     if (live && (int) blockIdx.y >= max(1, *live)) return;
     const int t = blockIdx.y, i0 = blockIdx.x * AM_PER_BLOCK, i1 = min(rows, i0 + AM_PER_BLOCK), tid = threadIdx.x, lane = tid & 63;
     const float* r = logits + (size_t) t * rows;
+    // the chain's words, asked for now and used at the end: a lane a word of the drafts
+    int chain = 0, stop = 0, n_ctx = 1, kept = 1, draft = 0;
+    if constexpr (KEEP) {
+        chain = keep.state[FNX_RS_CHAIN], stop = keep.state[FNX_RS_STOP], n_ctx = keep.state[FNX_RS_NCTX], kept = keep.state[FNX_RS_ACCEPTED];
+        if (lane < FNX_MAXT) draft = keep.scratch[lane];   // lane 0: how many the lookup found
+    }
     unsigned best = 0, at = 0xffffffffu;   // the thread's greatest key and the first index that holds it (it goes through its values in order)
     bool bad = false;
     auto take = [&](float v, int i) {
@@ -617,6 +625,7 @@ __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__
     const uint2 o = lane < AM_THREADS / 64 ? wbest[lane] : make_uint2(0u, 0xffffffffu);
     const unsigned m = wave_umax(o.x), w = wave_umin(o.x == m ? o.y : 0xffffffffu);
     const bool any_bad = __any(lane < AM_THREADS / 64 && wbad[lane] != 0);
+    int pick = -1;   // the row's, in its last block
     if (lane == 0) {
         if (any_bad) atomicOr(err, FNX_ERR_NONFINITE);
         // the maximum has been taken at the device's level (its old value is back) before this block counts as arrived;
@@ -628,10 +637,33 @@ __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__
         if (arrived == gridDim.x - 1) {
             const unsigned long long k = __hip_atomic_load(&keys[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             bv[t] = fkey_inv((unsigned) (k >> 32));
-            bi[t] = (int) ~(unsigned) k + v0;
+            bi[t] = pick = (int) ~(unsigned) k + v0;
             __hip_atomic_store(&keys[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&keys[FNX_MAXT + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+    }
+    if constexpr (KEEP) {
+        pick = uniform(pick);
+        if (pick < 0) return;   // (not the last block)
+        const bool on = uniform(chain) != 0, last = keep.j == keep.K - 1;
+        if (lane == 0 && on) {
+            keep.scratch[1 + keep.j] = pick;
+            if (last) keep.scratch[0] = keep.K;
+        }
+        if (!last || uniform(stop) != 0) return;
+        // the next window's rows and count
+        const int nd = on ? keep.K : min(max(uniform(draft), 0), FNX_MAXT - 1), first = uniform(n_ctx) - 1;
+        int tok = 0, R = 2;
+        if (nd > 0) {
+            R = 1 + nd;
+            if (lane <= nd) tok = on && lane == keep.K ? pick : draft;
+        } else if (lane == 1) {
+            const int n = min(max(uniform(kept), 1), FNX_MAXT);
+            tok = n == 1 ? pick : keep.best[n - 1];
+        }
+        if (lane == 0) tok = keep.ctx[first];
+        if (lane < FNX_MAXT) keep.rows[lane] = tok;
+        if (lane == 0) keep.state[FNX_RS_ROWS] = R;
     }
 }
 
@@ -648,16 +680,28 @@ constexpr int LK_THREADS = 1024, LK_STEPS = 16, LK_SPAN = 4 * 63, LOOKUP_MIN = 3
 __device__ __forceinline__ int lane_above(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xF, 0xF, false); }   // wave_shl:1; lane 63: its own
 // n_ctx_p (may be null): the context's length is that device word instead of n_ctx; d1_at (may be null): d1 is
 // d1p[*d1_at - 1] instead of d1p[0] (the pick of the last row kept). rs, rs_rows (may be null; only with n_ctx_p and d1_at
-// the round's own words): a decode round's state and window - the round's next window (k_round_window's rows and count,
+// the round's own words): a decode round's state and window - the round's next window (its rows and count,
 // k_round.h) is made here as well, from the drafts this launch finds: a launch less a round.
+// CHAIN: the round's MTP chain begins here (k_round.h).
+template <bool CHAIN>
 __global__ void __launch_bounds__(LK_THREADS) k_lookup(const int* __restrict__ ctx, int n_ctx, int key_n, int lk, const int* __restrict__ d1p,
                                                       int* __restrict__ out, int* __restrict__ n_out, int* __restrict__ match,
                                                       const int* __restrict__ n_ctx_p, const int* __restrict__ d1_at,
-                                                      int* __restrict__ rs = nullptr, int* __restrict__ rs_rows = nullptr) {
-    __shared__ int best;
+                                                      int* __restrict__ rs = nullptr, int* __restrict__ rs_rows = nullptr, const ChainBegin chain = {}) {
+    __shared__ int best, found;   // (found: how many drafts, for the chain)
     if (threadIdx.x == 0) best = -1;
     if (n_ctx_p) n_ctx = *n_ctx_p;
-    const int d1 = d1p[d1_at ? min(max(*d1_at, 1), FNX_MAXT) - 1 : 0];   // asked for now, used at the end
+    const int kept = d1_at ? min(max(*d1_at, 1), FNX_MAXT) : 1, d1 = d1p[kept - 1];   // asked for now, used at the end
+    float row[4] = {0.f, 0.f, 0.f, 0.f};
+    int chain_stop = 1, chain_pos = 0;
+    if constexpr (CHAIN) {
+        chain_stop = chain.state[FNX_RS_STOP], chain_pos = chain.state[FNX_RS_POS];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = threadIdx.x + LK_THREADS * j;
+            if (i < chain.n) row[j] = chain.hidden[(size_t) (kept - 1) * chain.n + i];
+        }
+    }
     // (what the next window needs beside the drafts, asked for now as well)
     const int rs_stop = rs ? rs[FNX_RS_STOP] : 1, last_tok = rs && n_ctx > 0 ? ctx[n_ctx - 1] : 0;
     __syncthreads();
@@ -704,7 +748,18 @@ __global__ void __launch_bounds__(LK_THREADS) k_lookup(const int* __restrict__ c
         if ((threadIdx.x & 63) == 0 && mine >= 0) atomicMax(&best, mine);
     }
     __syncthreads();
-    if (threadIdx.x >= 64) return;
+    if (threadIdx.x >= 64) {
+        if (!CHAIN) return;
+        __syncthreads();   // (the first wave's, below)
+        if (!chain_stop && found <= 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = threadIdx.x + LK_THREADS * j;
+                if (i < chain.n) chain.src[i] = row[j];
+            }
+        }
+        return;
+    }
     const int lane = threadIdx.x;
     int nr = 0, m_at = -1, dtok = 0;   // (dtok: this lane's draft)
     const int s = best;
@@ -739,6 +794,23 @@ done:
         else if (lane == 1) tok = d1;
         if (lane < FNX_MAXT) rs_rows[lane] = tok;
         if (lane == 0) rs[FNX_RS_ROWS] = nd > 0 ? 1 + nd : 2;
+    }
+    if constexpr (CHAIN) {   // (the whole block)
+        if (lane == 0) found = nr;
+        __syncthreads();
+        const bool run = !chain_stop && uniform(nr) <= 0;
+        if (lane < FNX_MAXT) chain.state[FNX_RS_CHAIN_POS + lane] = chain_pos + lane;
+        if (lane == 0) {
+            chain.state[FNX_RS_CHAIN] = run ? 1 : 0;
+            if (run) chain.scratch[1] = d1;
+        }
+        if (run) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = lane + LK_THREADS * j;
+                if (i < chain.n) chain.src[i] = row[j];
+            }
+        }
     }
 }
 __global__ void k_accept(const int* __restrict__ rows, const int* __restrict__ o, int R, int* __restrict__ n_accept) {
@@ -1216,10 +1288,12 @@ int fnx_moe_combine(const float* part, const float* topw, const float* sh, const
 }
 
 static int argmax_launch(const float* logits, int rows, int T, int v0, float* best_v, int* best_i, unsigned long long* keys, unsigned* err, void* st,
-                         const int* live) {
+                         const int* live, const ChainKeep* keep = nullptr) {
     if (!logits || !best_v || !best_i || !keys || !err) return fail("argmax: null argument");
     if (rows < 1 || T < 1 || T > FNX_MAXT) return fail("argmax: bad shape");
-    k_argmax<<<dim3((rows + AM_PER_BLOCK - 1) / AM_PER_BLOCK, T), AM_THREADS, 0, (hipStream_t) st>>>(logits, rows, keys, err, v0, best_v, best_i, live);
+    const dim3 grid((rows + AM_PER_BLOCK - 1) / AM_PER_BLOCK, T);
+    if (keep) k_argmax<true><<<grid, AM_THREADS, 0, (hipStream_t) st>>>(logits, rows, keys, err, v0, best_v, best_i, live, *keep);
+    else k_argmax<false><<<grid, AM_THREADS, 0, (hipStream_t) st>>>(logits, rows, keys, err, v0, best_v, best_i, live, ChainKeep{});
     return launch_status("argmax");
 }
 int fnx_argmax(const float* logits, int rows, int T, int v0, float* best_v, int* best_i, unsigned long long* keys, unsigned* err, void* st) {
@@ -1252,7 +1326,7 @@ int fnx_lookup_drafts(const int* ctx, int n_ctx, int key_n, int lk, int d1, int*
 int fnx_lookup_drafts_dev(const int* ctx, int n_ctx, int key_n, int lk, const int* d1, int* out, int* n_out, int* match, void* st) {
     if (!ctx || !d1 || !out || !n_out) return fail("lookup_drafts_dev: null argument");
     if (n_ctx < 0 || lk < 0 || lk > 64 || key_n < 1 || key_n > 4) return fail("lookup_drafts_dev: bad argument (keys of 1..4 tokens, up to 64 drafts)");
-    k_lookup<<<1, LK_THREADS, 0, (hipStream_t) st>>>(ctx, n_ctx, key_n, lk, d1, out, n_out, match, nullptr, nullptr);
+    k_lookup<false><<<1, LK_THREADS, 0, (hipStream_t) st>>>(ctx, n_ctx, key_n, lk, d1, out, n_out, match, nullptr, nullptr);
     return launch_status("lookup_drafts_dev");
 }
 
@@ -1863,12 +1937,12 @@ static int dec_shape_check(const fnx_decoder* D, int T, const char* who) {
 // nv head rows for the tokens from v0; pen (may be null): the last row's penalty list, applied before the picks (engine.cu:2130-2131)
 static int dec_head(const fnx_decoder* D, const float* norm, const fnx_q8s* head, int T, const fnx_dec_ws* ws, const DecPending& pend, void* st,
                     const int* gate = nullptr, int nv = 0, int v0 = 0, const int* pen = nullptr, const float* pen_par = nullptr,
-                    const int* live = nullptr) {
+                    const int* live = nullptr, const ChainKeep* keep = nullptr) {
     if (nv == 0) nv = D->vocab;
     if (dec_add_norm_q8(D, pend, norm, T, ws, st, ws->hidden, gate)) return 1;   // hidden = x, written by the same pass
     if (q8s_one(head, ws->xq, ws->logits, nv, T, st, gate, live)) return 1;
     if (pen && fnx_penalize_row(ws->logits + (size_t) (T - 1) * nv, nv, pen, pen_par, st)) return 1;
-    return argmax_launch(ws->logits, nv, T, v0, ws->best_v, ws->best_i, ws->keys, ws->err, st, live);
+    return argmax_launch(ws->logits, nv, T, v0, ws->best_v, ws->best_i, ws->keys, ws->err, st, live, keep);
 }
 static int decoder_verify(const fnx_decoder* D, const int* tokens, int T, const int* pos0, const fnx_dec_ws* ws, void* st, const int* live) {
     if (!D || !tokens || !pos0 || !ws || !D->layers || !D->out_norm || !D->emb) return fail("decoder_verify: null argument");
@@ -1893,7 +1967,7 @@ int fnx_decoder_layer(const fnx_decoder* D, const fnx_dec_layer* L, const float*
     return dec_layer(D, L, T, pos0, ws, pend, st);
 }
 static int mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, const int* tokens, int T, const int* pos0, const fnx_dec_ws* ws,
-                     void* st, const int* live, const int* gate = nullptr) {
+                     void* st, const int* live, const int* gate = nullptr, const ChainKeep* keep = nullptr) {
     if (!D || !M || !src || !tokens || !pos0 || !ws || !M->norm_emb || !M->norm_hid || !M->out_norm || !D->emb) return fail("mtp_draft: null argument");
     if (dec_shape_check(D, T, "mtp_draft") || dec_ws_check(ws, "mtp_draft")) return 1;
     const bool whole = M->dv0 == 0 && M->dv1 == 0;
@@ -1950,7 +2024,7 @@ static int mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, c
     }
     DecPending pend{ws->o, nullptr, nullptr};
     if (dec_layer(D, &M->layer, T, pos0, ws, pend, st, live, gate, M->out_norm, ws->hidden)) return 1;
-    return dec_head(D, M->out_norm, &M->head, T, ws, pend, st, gate, nv, M->dv0, M->pen, M->pen_par, live);
+    return dec_head(D, M->out_norm, &M->head, T, ws, pend, st, gate, nv, M->dv0, M->pen, M->pen_par, live, keep);
 }
 int fnx_mtp_draft(const fnx_decoder* D, const fnx_mtp* M, const float* src, const int* tokens, int T, const int* pos0, const fnx_dec_ws* ws,
                   void* st) {
@@ -1972,21 +2046,23 @@ int fnx_decode_round(const fnx_decoder* D, const fnx_mtp* M, const fnx_round* R,
     if (R->speculate) {
         // the rows kept and their picks are where the verify left them; the draft layer overwrites both only at its end
         if (mtp_draft(D, M, ws->hidden, ws->best_i, FNX_MAXT, S + FNX_RS_POS_PREV, ws, st, S + FNX_RS_ACCEPTED)) return 1;
-        // (with a single draft a round the lookup's launch makes the next window too)
-        k_lookup<<<1, LK_THREADS, 0, s>>>(R->ctx, 0, R->key_n, R->lk, ws->best_i, R->scratch + 1, R->scratch, nullptr, S + FNX_RS_NCTX,
-                                          S + FNX_RS_ACCEPTED, K == 1 ? S : nullptr, K == 1 ? R->rows : nullptr);
-        if (K > 1) {
-            // the chain (session.cpp:666-678): step j reads the draft before it at the position after it, from the draft
-            // layer's own row; one row, which counts (is routed, runs the big kernels) only while state[CHAIN] is set
-            const int* on = S + FNX_RS_CHAIN;
-            k_chain_begin<<<1, 256, 0, s>>>(S, R->scratch, ws->best_i, ws->hidden, D->n, R->chain_src, K);
-            for (int j = 1; j < K; ++j) {
-                if (mtp_draft(D, M, j == 1 ? R->chain_src : ws->hidden, R->scratch + j, 1, S + FNX_RS_CHAIN_POS + (j - 1), ws, st, on, on)) return 1;
-                k_chain_keep<<<1, 64, 0, s>>>(S, R->scratch, ws->best_i, j, K);
-            }
+        // (with a single draft a round the lookup's launch makes the next window too, with a chain it begins the chain)
+        if (K == 1)
+            k_lookup<false><<<1, LK_THREADS, 0, s>>>(R->ctx, 0, R->key_n, R->lk, ws->best_i, R->scratch + 1, R->scratch, nullptr, S + FNX_RS_NCTX,
+                                                     S + FNX_RS_ACCEPTED, S, R->rows);
+        else
+            k_lookup<true><<<1, LK_THREADS, 0, s>>>(R->ctx, 0, R->key_n, R->lk, ws->best_i, R->scratch + 1, R->scratch, nullptr, S + FNX_RS_NCTX,
+                                                    S + FNX_RS_ACCEPTED, nullptr, nullptr, ChainBegin{S, R->scratch, ws->hidden, R->chain_src, D->n});
+        // the chain (session.cpp:666-678): step j reads the draft before it at the position after it, from the draft
+        // layer's own row; one row, which counts (is routed, runs the big kernels) only while state[CHAIN] is set
+        const int* on = S + FNX_RS_CHAIN;
+        for (int j = 1; j < K; ++j) {
+            const ChainKeep keep{S, R->scratch, R->ctx, ws->best_i, R->rows, j, K};
+            if (mtp_draft(D, M, j == 1 ? R->chain_src : ws->hidden, R->scratch + j, 1, S + FNX_RS_CHAIN_POS + (j - 1), ws, st, on, on, &keep)) return 1;
         }
+    } else {
+        k_round_window<<<1, 64, 0, s>>>(R->ctx, S, R->rows);
     }
-    if (!R->speculate || K > 1) k_round_window<<<1, 64, 0, s>>>(R->ctx, S, R->scratch + 1, R->scratch, ws->best_i, R->speculate, R->rows);
     return launch_status("decode_round");
 }
 

@@ -45,51 +45,36 @@ __global__ void k_round_commit(const int* __restrict__ rows, const int* __restri
     }
 }
 
-// the MTP chain (session.cpp:666-678) starts when the lookup found nothing: its first draft is the draft layer's pick for
-// the last row kept, its source that row of the draft layer's output. The steps' positions are written in any case (a
-// step that does not count still appends its row to the draft layer's cache, in cells that the next round's pass over the
-// rows kept writes again before anything reads them). One block.
-__global__ void k_chain_begin(int* __restrict__ state, int* __restrict__ scratch, const int* __restrict__ draft_best,
-                              const float* __restrict__ hidden, int n, float* __restrict__ chain_src, int K) {
-    const int kept = min(max(state[FNX_RS_ACCEPTED], 1), FNX_MAXT), pos = state[FNX_RS_POS];
-    const bool run = !state[FNX_RS_STOP] && scratch[0] <= 0;
-    __syncthreads();   // every thread has read the words that thread 0 is about to write
-    if (threadIdx.x < FNX_MAXT) state[FNX_RS_CHAIN_POS + threadIdx.x] = pos + threadIdx.x;
-    if (threadIdx.x == 0) {
-        state[FNX_RS_CHAIN] = run ? 1 : 0;
-        if (run) scratch[1] = draft_best[kept - 1];
-    }
-    if (run)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) chain_src[i] = hidden[(size_t) (kept - 1) * n + i];
-}
-// after step j (1 .. K - 1) of the chain: its pick is draft j + 1; the last step hands the K drafts to the next window
-__global__ void k_chain_keep(const int* __restrict__ state, int* __restrict__ scratch, const int* __restrict__ best, int j, int K) {
-    if (threadIdx.x != 0 || !state[FNX_RS_CHAIN]) return;
-    scratch[1 + j] = best[0];
-    if (j == K - 1) scratch[0] = K;
-}
+// The MTP chain (session.cpp:666-678) has no launches of its own but its steps': it begins in the lookup's, and a step's pick is
+// kept by the step's argmax, the last one's making the next window too. A launch that does no more than move a word takes 4.5 us
+// between others (eight rounds with a chain of three drafts: 6,929 -> 6,860 us for the four launches less a round).
+//
+// It starts when the lookup found nothing: its first draft is the draft layer's pick for the last row kept, its source that
+// row of the draft layer's output. The steps' positions are written in any case (a step that does not count still appends
+// its row to the draft layer's cache, in cells that the next round's pass over the rows kept writes again before
+// anything reads them).
+struct ChainBegin {
+    int *state, *scratch;
+    const float* hidden;             // the draft layer's output rows
+    float* src;                      // the row kept last goes here
+    int n;                           // values a row, 4,096 at most
+};
+// after step j (1 .. K - 1): its pick is draft j + 1; the last step hands the K drafts to the next window
+struct ChainKeep {
+    int *state, *scratch;
+    const int *ctx, *best;           // best: the draft layer's picks
+    int* rows;                       // the next window, made after the last step
+    int j, K;
+};
 
-// the next window (session.cpp:530-560): the last token of the context, then the lookup's drafts, or else the draft
-// layer's pick for the last row kept; without speculation the token alone. One wave.
-__global__ void k_round_window(const int* __restrict__ ctx, int* __restrict__ state, const int* __restrict__ drafts,
-                               const int* __restrict__ n_drafts, const int* __restrict__ draft_best, int speculate, int* __restrict__ rows) {
+// the next window without speculation (session.cpp:530-560): the last token of the context alone. One wave. (With it the
+// lookup's launch or the chain's last step makes the window: that token, then the drafts, or else the draft layer's pick for the
+// last row kept.)
+__global__ void k_round_window(const int* __restrict__ ctx, int* __restrict__ state, int* __restrict__ rows) {
     const int i = threadIdx.x;
     if (state[FNX_RS_STOP]) return;
-    const int n_ctx = state[FNX_RS_NCTX], n = min(max(state[FNX_RS_ACCEPTED], 1), FNX_MAXT);
-    int R = 1, tok = 0;
-    if (speculate) {
-        const int nd = min(max(*n_drafts, 0), FNX_MAXT - 1);
-        if (nd > 0) {
-            R = 1 + nd;
-            if (i >= 1 && i <= nd) tok = drafts[i - 1];
-        } else {
-            R = 2;
-            if (i == 1) tok = draft_best[n - 1];
-        }
-    }
-    if (i == 0) tok = ctx[n_ctx - 1];
-    if (i < FNX_MAXT) rows[i] = tok;
-    if (i == 0) state[FNX_RS_ROWS] = R;
+    if (i < FNX_MAXT) rows[i] = i == 0 ? ctx[state[FNX_RS_NCTX] - 1] : 0;
+    if (i == 0) state[FNX_RS_ROWS] = 1;
 }
 
 }  // namespace fnx
