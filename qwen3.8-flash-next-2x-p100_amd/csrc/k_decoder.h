@@ -276,6 +276,8 @@ struct Q8sArgs {
     const int* gate;     // may be null; else a device word: at zero the launch leaves at once (a chain step that does not count)
     const uint8_t* yq2;  // may be null; else the second matrix's rows are these (two matrices, a block a tile: the host sees to that)
     const int* live;     // may be null; else a device word: rows from *live on do not count - they are not read and their products are zeros
+    int pieces;          // a lane's four results of a tile are one aligned 16-byte piece, all of it inside the rows or none: one store
+                         // instead of four (the head over 16 rows: 70.6 -> 67.5 us)
 };
 typedef int q8s_v4i __attribute__((ext_vector_type(4)));
 // DEPTH: the (tile, batch) items whose loads are in flight ahead of the one being worked on, where a block goes through more
@@ -390,9 +392,14 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
                          p2 = *reinterpret_cast<const float4*>(part + (64 + lane) * 4), p3 = *reinterpret_cast<const float4*>(part + (128 + lane) * 4);
             const float v[4] = {(p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y), (p0.z + p1.z) + (p2.z + p3.z),
                                 (p0.w + p1.w) + (p2.w + p3.w)};
+            const bool counts = !LIVE || r16 < Tl;   // (rows from *live on: zeros)
+            if (a.pieces) {
+                if (c.row0 + 4 * g < c.rows) *reinterpret_cast<float4*>(c.out) = counts ? make_float4(v[0], v[1], v[2], v[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (c.row0 + 4 * g + r < c.rows) c.out[r] = !LIVE || r16 < Tl ? v[r] : 0.f;   // rows from *live on: zeros
+                for (int r = 0; r < 4; ++r)
+                    if (c.row0 + 4 * g + r < c.rows) c.out[r] = counts ? v[r] : 0.f;
+            }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = 0.f;
@@ -459,6 +466,126 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
             advance(cc);
         }
     }
+}
+
+// The same for a matrix of many tiles a block in the tile-major layout, quarters of an even number of whole batches (columns in
+// 2,048s; the output heads). What a wave waits for is counted exactly: no load and no store stands under a condition (the last tile
+// is peeled off), every wave stores a quarter of a tile's results, and the block meets once a tile, the quarters' sums in two
+// places in turn. A wave then has two batches in flight until the one it needs is there, and two blocks a CU (half as many copies of
+// the activations, half the uneven end) read faster than three or four: 151,936 rows over matrices in turn, us, k_q8s_gemv with four
+// blocks / this with 1, 2, 3, 4: one row of x 55.7 / 64.7, 51.6, 52.2, 55.0; five 58.4 / 66.9, 54.1, 56.7, 58.7; sixteen
+// 66.9 / 71.4, 60.4, 62.6, 65.0. Both of a tile's batches asked for ahead of the activations: 61.3. Bound by the matrix's one read.
+constexpr int Q8S_PART_G = 80;   // floats between two lane groups' sums: the sixteen (row, token) places a read touches in different banks
+constexpr uint32_t Q8S_STREAM_OUT = 0xE0000000u;   // the results' bytes that its stores' offsets reach
+inline size_t q8s_stream_lds(int cols) {
+    return (size_t) FNX_MAXT * (cols + Q8S_XPAD) + (size_t) FNX_MAXT * (cols / 32 + 2) * 4 + 2 * Q8S_WAVES * 4 * Q8S_PART_G * 4;
+}
+template <bool LIVE>
+__global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_stream(const Q8sArgs a) {
+    typedef __attribute__((address_space(1))) const at_v4u_t g128;
+    extern __shared__ __align__(16) uint8_t q8s_lds[];   // [16][cols + pad] int8, [16][nb + 2] f32 scales, [2][4][4 * Q8S_PART_G] partial sums
+    const int live_v = LIVE ? *a.live : a.T;
+    if (a.gate && uniform(*a.gate) == 0) return;
+    const int nb = a.cols >> 5, T = a.T, xld = a.cols + Q8S_XPAD, dld = nb + 2, nq4 = q8s_quarter(a.cols);
+    int8_t* xs = reinterpret_cast<int8_t*>(q8s_lds);
+    float* xd = reinterpret_cast<float*>(q8s_lds + (size_t) FNX_MAXT * xld);
+    float* part = xd + FNX_MAXT * dld;
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+    const int rows = a.seg[0].rows, tiles = (rows + 15) / 16;
+    const bool lo_groups = g < 2;
+    const int Tl = LIVE ? max(1, min(uniform(live_v), T)) : T, xr = min(r16, Tl - 1), j0 = wave * nq4;
+    if ((int) blockIdx.x >= tiles) return;   // the same for every thread of the block
+    struct Batch {
+        at_v4u_t w[Q8S_BATCH], dd[4];
+    };
+    auto load = [&](int tile, int jb, Batch& o) {
+        const gbytes w = as_global(reinterpret_cast<const uint8_t*>(a.seg[0].q) + (size_t) tile * 16 * a.cols + Q8S_TILE_STEP * (j0 + jb)) + 16 * lane;
+#pragma unroll
+        for (int u = 0; u < Q8S_BATCH; ++u) o.w[u] = __builtin_nontemporal_load((g128*) (w + Q8S_TILE_STEP * u));
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            o.dd[r] = *(g128*) as_global(reinterpret_cast<const uint8_t*>(a.seg[0].d + (size_t) min(tile * 16 + 4 * g + r, rows - 1) * nb + 2 * (j0 + jb)));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](int jb, const Batch& in) {
+#pragma unroll
+        for (int u = 0; u < Q8S_BATCH; ++u) {
+            const int j = j0 + jb + u;
+            const at_v4u_t x = *reinterpret_cast<const at_v4u_t*>(xs + (size_t) xr * xld + 64 * j + 16 * g);
+            const float2 dx = *reinterpret_cast<const float2*>(xd + xr * dld + 2 * j);
+            const long wl = (long) in.w[u].x | (long) in.w[u].y << 32, wh = (long) in.w[u].z | (long) in.w[u].w << 32;
+            const long xl = (long) x.x | (long) x.y << 32, xh = (long) x.z | (long) x.w << 32;
+            const long xl0 = lo_groups ? xl : 0, xh0 = lo_groups ? xh : 0, xl1 = lo_groups ? 0 : xl, xh1 = lo_groups ? 0 : xh;
+            q8s_v4i s0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(wl, xl0, q8s_v4i{0, 0, 0, 0}, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(wh, xh0, s0, 0, 0, 0);
+            q8s_v4i s1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(wl, xl1, q8s_v4i{0, 0, 0, 0}, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(wh, xh1, s1, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[r] = fmaf(half_bits_to_float(in.dd[r][u] & 0xFFFFu) * dx.x, (float) s0[r], acc[r]);
+                acc[r] = fmaf(half_bits_to_float(in.dd[r][u] >> 16) * dx.y, (float) s1[r], acc[r]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // wave w finishes the tokens 4 w .. 4 w + 3: lane (token lane / 16, row lane % 16)
+    const int tok = 4 * wave + (lane >> 4), row = lane & 15;
+    const uint32_t none = 0xF0000000u;   // past the buffer's end: a store there is dropped
+    const uint32_t oat = tok < T ? ((uint32_t) tok * (uint32_t) a.seg[0].out_stride + row) * 4u : none;
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*) a.seg[0].out, 0, (int) Q8S_STREAM_OUT, 0x00020000);
+    int turn = 0;
+    auto finish = [&](int tile) {   // the four quarters through LDS: (s0 + s1) + (s2 + s3)
+        float* p = part + turn * (Q8S_WAVES * 4 * Q8S_PART_G);
+        turn ^= 1;
+        *reinterpret_cast<float4*>(p + (wave * 4 + g) * Q8S_PART_G + 4 * r16) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the loads on their way stay there
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        const float* q = p + (row >> 2) * Q8S_PART_G + 4 * tok + (row & 3);
+        constexpr int W = 4 * Q8S_PART_G;
+        const float v = (q[0] + q[W]) + (q[2 * W] + q[3 * W]);
+        const float out = !LIVE || tok < Tl ? v : 0.f;   // rows from *live on: zeros
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out), to, tile * 16 + row < rows ? oat : none, 64u * (uint32_t) tile, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = 0.f;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Batch A, B;
+    int tile = blockIdx.x;
+    load(tile, 0, A);
+    for (int i = threadIdx.x; i < Tl * nb; i += blockDim.x) {   // the window's q8_1 rows into LDS
+        const int t = i / nb, b = i - t * nb;
+        uint32_t* dst = reinterpret_cast<uint32_t*>(xs + (size_t) t * xld + 32 * b);
+        const uint8_t* blk = a.yq + (size_t) i * 36;
+        xd[t * dld + b] = half_bits_to_float(load_u16(blk));
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(blk + 4);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) dst[k] = src[k];
+    }
+    __syncthreads();
+    for (; tile + (int) gridDim.x < tiles; tile += gridDim.x) {
+        for (int jb = 0; jb < nq4; jb += 2 * Q8S_BATCH) {
+            const bool end = jb + 2 * Q8S_BATCH >= nq4;
+            load(tile, jb + Q8S_BATCH, B);
+            compute(jb, A);
+            load(end ? tile + gridDim.x : tile, end ? 0 : jb + 2 * Q8S_BATCH, A);
+            compute(jb + Q8S_BATCH, B);
+        }
+        finish(tile);
+    }
+    int jb = 0;
+    for (; jb + 2 * Q8S_BATCH < nq4; jb += 2 * Q8S_BATCH) {
+        load(tile, jb + Q8S_BATCH, B);
+        compute(jb, A);
+        load(tile, jb + 2 * Q8S_BATCH, A);
+        compute(jb + Q8S_BATCH, B);
+    }
+    load(tile, jb + Q8S_BATCH, B);
+    compute(jb, A);
+    compute(jb + Q8S_BATCH, B);
+    finish(tile);
 }
 
 // ---------------------------------------------------------------- attention: prepare and append (kernels.cu:513-537, 1878-1910)

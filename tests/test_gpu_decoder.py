@@ -115,6 +115,12 @@ def test_q8s_gemv_short_last_batch(dev, oracle, rows, cols, T):
     test_q8s_gemv_bit_exact(dev, oracle, rows, cols, T)
 
 
+@pytest.mark.parametrize("rows,T", [(24576, 1), (24579, 16), (24577, 5), (32772, 4), (40015, 3)])
+def test_q8s_gemv_many_tiles_a_block(dev, oracle, rows, T):
+    """2,048 columns, three tiles of 16 rows a block and more (the last of them short, results that are no whole 16-byte pieces), bit for bit"""
+    test_q8s_gemv_bit_exact(dev, oracle, rows, 2048, T)
+
+
 @pytest.mark.parametrize("rope", [ROPE, YARN])
 @pytest.mark.parametrize("nq,nkv,T,pos0", [(4, 2, 3, 5), (16, 2, 16, 32000), (8, 1, 1, 0)])
 def test_attn_prep_append(dev, oracle, nq, nkv, T, pos0, rope):

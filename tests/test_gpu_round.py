@@ -136,6 +136,19 @@ def test_rounds_without_the_host_equal_the_host_driven_rounds(dev, oracle, model
         assert all(entry == (0, 1) for entry in log)
 
 
+def test_rounds_over_a_head_of_many_tiles_equal_the_host_driven_rounds(dev, oracle):
+    """an output head of three tiles a block and more, with and without the device-side row count"""
+    model = td.TinyDecoder(oracle, seed=61, n=2048, nq=4, nkv=2, nlayers=1, vocab=24603, max_ctx=192, nexp=16, topk=4, ff=256)
+    prompt = repeating_prompt(13)
+    r = RoundDev(dev, model, prompt, chain=2)
+    print("case decode_round vocab=24603", flush=True)
+    for _ in range(5):
+        r.launch()
+    out, log, st = r.result()
+    assert st[dev.pkg.RS_ROUNDS] == 5 and int(r.d.b["err"].item()) == 0
+    assert (out, log) == host_loop(dev, model, prompt, len(out), K=2)
+
+
 @pytest.mark.parametrize("nq", [6, 10, 12, 14])
 def test_rounds_over_other_projection_widths_equal_the_host_driven_rounds(dev, oracle, nq):
     """the output projection's 256 nq columns: two to four load batches a wave, whole and short last ones, with and without the
