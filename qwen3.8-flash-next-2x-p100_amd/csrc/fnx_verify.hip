@@ -1141,7 +1141,8 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
     hipStream_t s = (hipStream_t) st;
     // f32 weights against more rows than a window's. Tiles of 16 x 16 (k_gemv_rows_mfma16) where the larger tiles would leave CUs
     // idle, or cannot be had; the larger ones read each row from the L2 half as often, and that is the time of a long chunk.
-    // 513 weight rows of 2048, over one set of weights, us (small tiles / large): 77 rows 5.5 / 13.8, 200 9.7 / 14.3, 300 14.0 / 15.4, 400 18.6 / 14.9.
+    // 513 weight rows of 2048, weights in turn, us (small tiles / large): 64 rows 5.7 / 13.2, 128 10.0 / 13.4, 240 10.2 / 13.4, 280 14.3 / 13.7, 320 15.1 / 13.5:
+    // a CU takes its small tiles one after the other, 4.5 us each, and three take longer than its one large one.
     // Where the large ones cannot be had, k_gemv_rows_many is the other kernel: it reads a row of x once for four weight rows a
     // wave, and fills the chip only with many rows. The narrower the rows, the more of a small tile's time is its start and its
     // end, so it is the better one up to 5/2, 8 and 12 tiles a CU at widths of 512, 1024 and 1536, and always from 2048 on.
@@ -1152,18 +1153,18 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
                        (uint64_t) rows * n * 4 < (1ull << 32) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
     const long small_tiles = (long) ((T + RS_TILE - 1) / RS_TILE) * ((rows + RS_TILE - 1) / RS_TILE);
     if (!bf && T > FNX_MAXT && n % (2 * RS_COLS) == 0 && small_tiles < (1l << 24) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0 &&
-        small_tiles <= (large || n == 512 ? 5l * cu_count() / 2 : n == 1024 ? 8l * cu_count() : n == 1536 ? 12l * cu_count() : 1l << 24)) {
+        small_tiles <= (large ? 2l * cu_count() : n == 512 ? 5l * cu_count() / 2 : n == 1024 ? 8l * cu_count() : n == 1536 ? 12l * cu_count() : 1l << 24)) {
         const int ntt = (T + RS_TILE - 1) / RS_TILE, net = (rows + RS_TILE - 1) / RS_TILE;
         k_gemv_rows_mfma16<<<(unsigned) ((small_tiles + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
         return launch_status(who);
     }
     if (large) {
         // a chunk's worth of rows against f32 weights: tiles of 32 x 32 sums on the matrix cores. The weight rows past the
-        // last full 32 ride with the tiles' blocks, an item a block (a row x four rows of x); if there are more items
-        // than blocks in a row of tiles, those rows go to the kernel below.
+        // last full 32 ride with the tiles' blocks, an item a wave (a row x a row of x); if there are more items
+        // than waves in a row of tiles, those rows go to the kernel below.
         const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE;
         const int tile_blocks = ((ntt + 3) / 4) * ((net + 7) / 8) * 32;
-        const bool along = 8 * left <= net;   // a row and four rows of x a block, within the block's own rows of x
+        const bool along = 8 * left <= net;   // (32 left items, 4 net waves)
         k_gemv_rows_mfma<<<tile_blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, tile_blocks, along ? 1 : 0);
         if (left == 0 || along) return launch_status(who);
         const dim3 gm((left + GM_WAVES * GR_ROWS - 1) / (GM_WAVES * GR_ROWS), (T + FNX_MAXT - 1) / FNX_MAXT);

@@ -378,248 +378,179 @@ __global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __
 // v_mfma_f32_32x32x1_2b_f32 is D = fma(a, b, D) element by element with one rounding - the fmaf of the chains above
 // (checked bit for bit on this GPU, products in the denormal range included). A chain of them over the chunks
 // l, l + 64, ... therefore leaves lane l's partial sum of 32 activation rows x 32 weight rows at once; the instruction's
-// two blocks take l and l + 32, the pair that the butterfly adds first. A block owns such a tile of 32 x 32 sums. Wave
-// w of its RM_WAVES multiplying waves walks the lanes l = w mod 4 in eight phases - l = 8 a + 4 h + w and l + 32, (h; a)
-// in the order (0; 0, 2, 1, 3), (1; 0, 2, 1, 3) - so that the butterfly's levels 16, 8 and 4 are adds of whole
-// accumulator tiles as the phases end (done while the next phase multiplies into a second accumulator); levels 2 and 1
-// add the four waves' tiles through LDS. The operands (f32 weights only) come through LDS: a stage is 64 rows (32 of x,
-// 32 of W) x 512 bytes - four chunks of the four lanes l and of l + 32 - sent there by global_load_lds_dwordx4 from two
-// waves of their own (an instruction issued between MFMAs holds its wave up for about 40 cycles), two stages ahead, into
-// one of three buffers; an instruction carries two rows, and row r's piece p lies at place p ^ (r % 16) (within its
-// half of 16), so that the 16 rows an operand read touches fall on 16 different bank groups. The waves read a stage's
-// operands right after the meeting that says it has landed and multiply the stage before it meanwhile.
-// The weight rows past the last full 32 (the router's 513th) are left to the first loading wave, idle half of the
-// time: an item is one such row against four rows of x, its loads go out in pieces after the first stages' and are
-// back, the loads completing in order, where a stage asked for after them is waited for.
+// two blocks take l and l + 32, the pair that the butterfly adds first. A block owns such a tile of 32 x 32 sums; wave w of four
+// takes the lanes l = 16 h + 4 w + j: for h = 0 and then h = 1 the four chains of j side by side, so that an MFMA never waits for
+// the one before it. Level 16 of the butterfly adds the two halves' accumulators, levels 8 and 4 the waves', levels 2 and 1 the four
+// chains', through LDS at the end.
+// Operands (f32 weights only): a step is a chunk of each of the wave's chains of 32 + 32 rows, a row's four chunks (and those of
+// l + 32) 64 bytes in a row: eight kilobytes that the wave sends to a ring of its own in LDS (global_load_lds_dwordx4, sixteen
+// such runs an instruction), RM_RING - 1 steps ahead, and nobody else reads: no wave meets another before the end, and a
+// wait is for its own loads, counted. A step's sixteen MFMAs (64 cycles each) hide the eight reads of the next step's operands and
+// the eight loads of the ring's next step, one behind each MFMA. Run r of eight rows' runs lies at place p = 4 r + (j ^ f), f of the row,
+// so that the 16 rows an operand read touches fall on 16 different bank groups.
+// Bound by the MFMAs and the loads behind them: 513 rows of 2,048 columns, 512 rows of x 16.6 -> 14.6 us, 4,096 114 -> 101 over weights in turn (134 -> 111-117 in
+// a layer, whose x comes from memory): 9.1 us a tile's steps where the MFMAs alone take 6.8, with the operands' reads 7.5. Before, four waves
+// took a chain each, met after every 64 columns' step and had two loading waves beside them: 11.7 us a tile's steps.
+// The weight rows past the last full 32 (the router's 513th) are items of such a row against one row of x, one a wave at most,
+// added up while the first steps are on their way.
 typedef float v32f __attribute__((ext_vector_type(32)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr int RM_TILE = 32, RM_WAVES = 4, RM_LOADERS = 2, RM_THREADS = (RM_WAVES + RM_LOADERS) * 64, RM_ROWB = 512, RM_STAGE = 2 * RM_TILE * RM_ROWB, RM_BUFS = 3;
-constexpr int RM_PIECE = 10 * 1024, RM_PIECES = 4;   // an item's loads of two steps (a weight row's and four x rows' chunks), pieces in LDS at a time
-constexpr int RM_ITEM_AT = 4;                        // the stage after whose loads an item's first piece goes out
-__global__ void __launch_bounds__(RM_THREADS) k_gemv_rows_mfma(const float* __restrict__ W, const float* __restrict__ x, float* __restrict__ y,
-                                                              int rows, int n, int T, int ntt, int net, int tile_blocks, int along) {
-    __shared__ __align__(16) uint8_t lds[RM_BUFS * RM_STAGE + RM_PIECES * RM_PIECE];
+constexpr int RM_TILE = 32, RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4;
+__global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) k_gemv_rows_mfma(const float* __restrict__ W, const float* __restrict__ x,
+                                                                                                         float* __restrict__ y, int rows, int n, int T, int ntt,
+                                                                                                         int net, int tile_blocks, int along) {
+    __shared__ __align__(16) uint8_t lds[RM_WAVES * RM_RING * RM_STEP];
     const int wave = uniform((int) (threadIdx.x >> 6)), lane = threadIdx.x & 63;
     // Which tile: block ids go round the eight XCDs, each with an L2 of its own, so an XCD's blocks are given one patch of
-    // 4 x 8 tiles after another (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them, every block re-reads both
-    // eight times over the phases). The grid covers whole patches; a block whose tile lies outside leaves.
+    // 4 x 8 tiles after another (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them).
+    // The grid covers whole patches; a block whose tile lies outside leaves.
     const int lin = ((int) blockIdx.x % 8) * (tile_blocks / 8) + (int) blockIdx.x / 8, patches_e = (net + 7) / 8;
     const int tt = 4 * ((lin / 32) / patches_e) + (lin % 32) / 8, et = 8 * ((lin / 32) % patches_e) + lin % 8;
     if (tt >= ntt || et >= net) return;
     const int t0 = tt * RM_TILE, e0 = et * RM_TILE;
-    const int nh = n / 1024, S = 8 * nh;   // stages: phase-major, a row's quarters of 1024 values within a phase (nh is even)
-    const uint32_t lds_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
-    // All waves meet where a stage must have landed. A loader's loads complete in order: it waits until only the newest
-    // stage's (and an item's pieces after them) may be on their way; the others wait for their own LDS reads. (A plain barrier instruction: __syncthreads() would wait for every load.)
-    auto meet = [&](int in_flight) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (in_flight == 36) __builtin_amdgcn_s_waitcnt(0x8074);        // vmcnt(36) lgkmcnt(0)
-        else if (in_flight == 26) __builtin_amdgcn_s_waitcnt(0x407A);   // vmcnt(26) lgkmcnt(0)
-        else if (in_flight == 16) __builtin_amdgcn_s_waitcnt(0x4070);   // vmcnt(16) lgkmcnt(0)
-        else __builtin_amdgcn_s_waitcnt(0x0070);                        // vmcnt(0) lgkmcnt(0)
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+    const int half = n / 256, S = 2 * half;   // steps: a multiple of 16
+    uint8_t* ring = lds + wave * (RM_RING * RM_STEP);
+    const uint32_t ring_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) ring;
+    uint32_t xoff[4], woff[4];   // instruction g: rows 8 g .. 8 g + 7, this lane's piece
+    {
+        const int r7 = (lane >> 2) & 7, b = lane >> 5;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t piece = 512u * b + 16u * ((lane & 3) ^ ((r7 >> 2) | ((g & 1) << 1)));
+            xoff[g] = (uint32_t) min(t0 + 8 * g + r7, T - 1) * (uint32_t) n * 4u + piece;
+            woff[g] = (uint32_t) (e0 + 8 * g + r7) * (uint32_t) n * 4u + piece;
+        }
+    }
+    auto from_of = [&](int s) { return 64 * wave + (s >= half ? 256 + 1024 * (s - half) : 1024 * s); };
+    auto fetch = [&](int op, int from, int slot) {   // one of a step's eight instructions
+        const int g = op & 3;
+        if (op < 4) lds_load16(reinterpret_cast<const uint8_t*>(x) + from, xoff[g], ring_at + slot * RM_STEP + g * 1024);
+        else lds_load16(reinterpret_cast<const uint8_t*>(W) + from, woff[g], ring_at + slot * RM_STEP + 4096 + g * 1024);
     };
-    if (wave >= RM_WAVES) {   // a loader: the first takes the stages' rows of x, the second those of W
-        const int lw = wave - RM_WAVES;
-        uint32_t off[16];   // instruction j: rows 2 j and 2 j + 1 of this loader's half of the stage, this lane's piece
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int row = 2 * j + (lane >> 5), q = lane & 31, p = (q & 16) | ((q & 15) ^ (row & 15));
-            const int r = lw == 0 ? min(t0 + row, T - 1) : e0 + row;
-            off[j] = (uint32_t) r * (uint32_t) n * 4u + 1024u * (p >> 3) + 512u * ((p >> 2) & 1) + 16u * (p & 3);
-        }
-        const uint8_t* src = reinterpret_cast<const uint8_t*>(lw == 0 ? x : W);
-        int ph = 0, hf = 0;   // the next stage to fetch
-        auto fetch = [&](int buf) {
-            const int q = ph & 3, l0 = 8 * (((q & 1) << 1) | (q >> 1)) + 4 * (ph >> 2);
-            const uint8_t* from = src + 16 * l0 + 4096 * hf;
+    for (int s = 0; s < RM_RING; ++s)   // (S >= 16)
 #pragma unroll
-            for (int j = 0; j < 16; ++j) lds_load16(from, off[j], lds_at + buf * RM_STAGE + lw * (RM_TILE * RM_ROWB) + j * 1024);
-            if (++hf == nh) hf = 0, ++ph;
-        };
-        // This loader's item of the rows past the tiles: weight row irow against the rows it0 .. it0 + 3 of x, lane l the
-        // chunks l, l + 64, ... A piece - two steps' chunks, ten instructions - goes out after each of the first stages'
-        // loads, into LDS like them (so that every load in flight is one that the meetings count), and is added up three
-        // meetings later: the stage waited for there was asked for after it.
-        // (Block (tt, et) takes the row et / 8 past the tiles against the et % 8-th four of its own 32 rows of x: rows that its
-        // XCD's L2 holds anyway.)
-        const int steps = n / 256, pieces = steps / 2;
-        const bool has_item = lw == 0 && along && et < 8 * (rows - net * RM_TILE);
-        const int irow = has_item ? net * RM_TILE + et / 8 : 0, it0 = has_item ? t0 + 4 * (et % 8) : 0;
-        const uint8_t* irows[5] = {reinterpret_cast<const uint8_t*>(W + (size_t) irow * n), nullptr, nullptr, nullptr, nullptr};
+        for (int op = 0; op < 8; ++op) fetch(op, from_of(s), s);
+    if (along && 4 * et + wave < RM_TILE * (rows - net * RM_TILE)) {
+        const int item = 4 * et + wave, irow = net * RM_TILE + item / RM_TILE, it = t0 + item % RM_TILE;
+        const float4 *wp = reinterpret_cast<const float4*>(W + (size_t) irow * n) + lane, *xp = reinterpret_cast<const float4*>(x + (size_t) min(it, T - 1) * n) + lane;
+        float v = 0.f;
+        for (int c0 = 0; c0 < n / 4; c0 += 8 * 64) {
+            float4 wv[8], xv[8];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) irows[1 + t] = reinterpret_cast<const uint8_t*>(x + (size_t) min(it0 + t, T - 1) * n);
-        const uint8_t* ilds = lds + RM_BUFS * RM_STAGE;
-        float iacc[4] = {0.f, 0.f, 0.f, 0.f};
-        fetch(0);
-        fetch(1);   // (S >= 16)
-        int buf = 2;
-        for (int k = 0; k <= S; ++k) {   // (the others meet once more than there are stages: they read one ahead)
-            const int kp = k - RM_ITEM_AT;   // the piece that goes out in this round
-            const int younger = (has_item && kp >= 2 && kp - 2 < pieces ? 10 : 0) + (has_item && kp >= 1 && kp - 1 < pieces ? 10 : 0);
-            meet(k + 1 >= S ? 0 : 16 + younger);
-            if (k + 2 < S) fetch(buf);
-            buf = buf == RM_BUFS - 1 ? 0 : buf + 1;
-            if (has_item && kp >= 0 && kp < pieces) {
-                const uint32_t at = lds_at + RM_BUFS * RM_STAGE + (kp & (RM_PIECES - 1)) * RM_PIECE;
+            for (int k = 0; k < 8; ++k) wv[k] = wp[c0 + 64 * k], xv[k] = xp[c0 + 64 * k];
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int r = 0; r < 5; ++r) lds_load16(irows[r] + (2 * kp + s) * 1024, 16u * lane, at + (5 * s + r) * 1024);
-            }
-            if (has_item && kp >= 3 && kp - 3 < pieces) {
-                const uint8_t* p = ilds + ((kp - 3) & (RM_PIECES - 1)) * RM_PIECE + 16 * lane;
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const float4 w = *reinterpret_cast<const float4*>(p + 5 * s * 1024);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const float4 bv = *reinterpret_cast<const float4*>(p + (5 * s + 1 + t) * 1024);
-                        float a = iacc[t];
-                        a = fmaf(w.x, bv.x, a);
-                        a = fmaf(w.y, bv.y, a);
-                        a = fmaf(w.z, bv.z, a);
-                        a = fmaf(w.w, bv.w, a);
-                        iacc[t] = a;
-                    }
-                }
+            for (int k = 0; k < 8; ++k) {
+                v = fmaf(wv[k].x, xv[k].x, v);
+                v = fmaf(wv[k].y, xv[k].y, v);
+                v = fmaf(wv[k].z, xv[k].z, v);
+                v = fmaf(wv[k].w, xv[k].w, v);
             }
         }
-        meet(0);   // the tiles' meeting below
-        if (has_item) {   // the butterfly over the item's four sums (when nobody waits for this wave any more): levels 32 and 16
-                          // for all four at once, a 16-lane row then holds one sum's values for levels 8 .. 1
-            float v = swap16_add(swap32_add(iacc[0], iacc[1]), swap32_add(iacc[2], iacc[3]));   // rows: sums 0, 2, 1, 3
-#pragma unroll
-            for (int o = 8; o; o >>= 1) v += __shfl_xor(v, o, WAVE);
-            const int row = lane >> 4, ti = it0 + (((row & 1) << 1) | (row >> 1));
-            if ((lane & 15) == 0 && ti < T) y[(size_t) ti * rows + irow] = v;
-        }
-        return;
+        v = group_sum<64>(v);
+        if (lane == 0 && it < T) y[(size_t) it * rows + irow] = v;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the counts below are of the steps' loads alone)
     }
     const int i = lane & 31, b = lane >> 5;
-    // this lane's operands of a stage: row i of x and row i of W, chunks 0 .. 3 of lane l (block b: l + 32)
-    const uint8_t* r0 = lds + i * RM_ROWB + 16 * ((4 * b + wave) ^ (i & 15));       // chunks 0 and 2 (256 bytes on)
-    const uint8_t* r1 = lds + i * RM_ROWB + 16 * ((8 + 4 * b + wave) ^ (i & 15));   // chunks 1 and 3
+    const int rd = (i >> 3) * 1024 + 64 * ((i & 7) + 8 * b), f = ((i & 7) >> 2) | (((i >> 3) & 1) << 1);
+    const uint8_t* at[4];   // this lane's pieces of a step: row i of x (of W: 4 KiB on), chunk j of its block
+#pragma unroll
+    for (int j = 0; j < 4; ++j) at[j] = ring + rd + 16 * (j ^ f);
     float4 A[2][4], B[2][4];
-    int buf = 0;   // the buffer whose operands are read next
-    auto next_stage = [&](float4 (&a)[4], float4 (&bb)[4]) {
-        meet(0);
-        const int o = buf * RM_STAGE;   // (past the last stage: a buffer's old contents, not used)
-        a[0] = *reinterpret_cast<const float4*>(r0 + o);
-        a[1] = *reinterpret_cast<const float4*>(r1 + o);
-        a[2] = *reinterpret_cast<const float4*>(r0 + o + 256);
-        a[3] = *reinterpret_cast<const float4*>(r1 + o + 256);
-        bb[0] = *reinterpret_cast<const float4*>(r0 + o + RM_TILE * RM_ROWB);
-        bb[1] = *reinterpret_cast<const float4*>(r1 + o + RM_TILE * RM_ROWB);
-        bb[2] = *reinterpret_cast<const float4*>(r0 + o + RM_TILE * RM_ROWB + 256);
-        bb[3] = *reinterpret_cast<const float4*>(r1 + o + RM_TILE * RM_ROWB + 256);
-        buf = buf == RM_BUFS - 1 ? 0 : buf + 1;
+    v32f acc[4];
+    float held[4][16];
+    auto wait = [&](int steps) {   // until only the newest so many steps' loads may be on their way
+        __builtin_amdgcn_sched_barrier(0);
+        if (steps == 2) __builtin_amdgcn_s_waitcnt(0x4F70);        // vmcnt(16)
+        else if (steps == 1) __builtin_amdgcn_s_waitcnt(0x0F78);   // vmcnt(8)
+        else __builtin_amdgcn_s_waitcnt(0x0F70);                   // vmcnt(0)
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    v32f acc[2];
-    float held[16], u0[16], sum[16];   // (plain arrays: no need for runs of 16 registers)
-    // The fold of a phase, whose accumulator is cf: the butterfly's levels 32 (the instruction's two blocks; the sums
-    // take the place of the first block), 16, 8 and 4, in three pieces that go between the next phase's first MFMAs on
-    // the vector unit. The phases of a = 0 and a = 1 (kind 0) leave held; that of a = 2 (odd) adds level 16 with a = 0
-    // into u0; that of a = 3 adds level 16 with a = 1 and level 8 into sum, and at the very end (last) level 4. Which of
-    // the latter two it is, is a select on a scalar, not a branch: the stretch of MFMAs stays one block of code.
-    auto fold_a = [&](v32f& cf) {
+    // A step: its sixteen MFMAs over the operands a, bb, and behind one of them each the reads of the next step's (READ, from slot
+    // rs) and the loads of the step RM_RING on (FETCH, into the slot this step was read from). FIRST: a half's first step,
+    // whose chains start from zero; the half before is folded (the instruction's two blocks, level 32) into held ahead of its chain.
+    auto step = [&](const float4 (&a)[4], const float4 (&bb)[4], float4 (&na)[4], float4 (&nb)[4], int rs, int from, auto first_c, auto fold_c, auto read_c, auto fetch_c) {
+        constexpr bool FIRST = decltype(first_c)::value, FOLD = decltype(fold_c)::value, READ = decltype(read_c)::value, FETCH = decltype(fetch_c)::value;
+        const int ro = rs * RM_STEP, fs = (rs + RM_RING - 1) % RM_RING;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) cf[v] = cf[v] + cf[16 + v];
-    };
-    auto fold_b = [&](bool first_of_pair, bool odd, v32f& cf) {
+        for (int m = 0; m < 16; ++m) {
+            const int j = m & 3, c = m >> 2;
+            if (FOLD && c == 0) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            if (first_of_pair) {
-                held[v] = cf[v];
-            } else {
-                cf[v] = held[v] + cf[v];
-                u0[v] = odd ? cf[v] : u0[v];
+                for (int v = 0; v < 16; ++v) held[j][v] = acc[j][v] + acc[j][16 + v];
             }
-        }
-    };
-    auto fold_c = [&](bool first_of_pair, bool odd, bool last, const v32f& cf) {
-        if (first_of_pair) return;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            if (last) sum[v] = sum[v] + (u0[v] + cf[v]);
-            else sum[v] = odd ? sum[v] : u0[v] + cf[v];
-        }
-    };
-    // a stage's 16 steps into accumulator c (first: the phase's first stage, which starts from zero, with the fold of the
-    // phase before, unless it is a later stage)
-    auto multiply = [&](const float4 (&a)[4], const float4 (&bb)[4], v32f& c, auto first_c, bool first_of_pair, bool odd, v32f& cf) {
-        constexpr bool first = decltype(first_c)::value;
-        if constexpr (first) asm volatile("" : "+v"(cf));   // (keeps the fold's adds on this side of the meeting)
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-            if (first && cc == 0) {
+            const float av = c == 0 ? a[j].x : c == 1 ? a[j].y : c == 2 ? a[j].z : a[j].w, bv = c == 0 ? bb[j].x : c == 1 ? bb[j].y : c == 2 ? bb[j].z : bb[j].w;
+            if (FIRST && c == 0) {
                 v32f z;
 #pragma unroll
                 for (int v = 0; v < 32; ++v) z[v] = 0.f;
-                c = __builtin_amdgcn_mfma_f32_32x32x1f32(a[cc].x, bb[cc].x, z, 0, 0, 0);
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(av, bv, z, 0, 0, 0);
             } else {
-                c = __builtin_amdgcn_mfma_f32_32x32x1f32(a[cc].x, bb[cc].x, c, 0, 0, 0);
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(av, bv, acc[j], 0, 0, 0);
             }
-            if constexpr (first) {
-                if (cc < 3) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (cc == 0) fold_a(cf);
-                    else if (cc == 1) fold_b(first_of_pair, odd, cf);
-                    else fold_c(first_of_pair, odd, false, cf);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+            __builtin_amdgcn_sched_barrier(0);
+            if (READ && m < 8) {
+                if (m < 4) na[m] = *reinterpret_cast<const float4*>(at[m] + ro);
+                else nb[m & 3] = *reinterpret_cast<const float4*>(at[m & 3] + ro + 4096);
             }
-            c = __builtin_amdgcn_mfma_f32_32x32x1f32(a[cc].y, bb[cc].y, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x1f32(a[cc].z, bb[cc].z, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x1f32(a[cc].w, bb[cc].w, c, 0, 0, 0);
+            if (FETCH && m >= 8) fetch(m - 8, from, fs);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
     };
     using std::integral_constant;
     constexpr integral_constant<bool, true> yes{};
     constexpr integral_constant<bool, false> no{};
-    // a phase into accumulator c, the phase before's fold (accumulator cf) along with its first stage
-    auto phase = [&](v32f& c, bool first_of_pair, bool odd, v32f& cf) {
-        next_stage(A[1], B[1]);
-        multiply(A[0], B[0], c, yes, first_of_pair, odd, cf);
-        next_stage(A[0], B[0]);
-        multiply(A[1], B[1], c, no, false, false, c);
-        for (int h2 = 2; h2 < nh; h2 += 2) {
-            next_stage(A[1], B[1]);
-            multiply(A[0], B[0], c, no, false, false, c);
-            next_stage(A[0], B[0]);
-            multiply(A[1], B[1], c, no, false, false, c);
-        }
-    };
+    wait(2);   // (the first two steps have landed)
 #pragma unroll
-    for (int v = 0; v < 32; ++v) acc[1][v] = 0.f;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) held[v] = u0[v] = sum[v] = 0.f;
-    next_stage(A[0], B[0]);
-    // pairs of phases: (a = 0, a = 2), (a = 1, a = 3), and again for h = 1. The first of a pair folds the second of the pair
-    // before (the very first: nothing, and what that leaves is overwritten), the second the first.
-#pragma unroll 1
-    for (int pp = 0; pp < 4; ++pp) {
-        phase(acc[0], false, (pp & 1) != 0, acc[1]);
-        phase(acc[1], true, false, acc[0]);
+    for (int j = 0; j < 4; ++j) {
+        A[0][j] = *reinterpret_cast<const float4*>(at[j]);
+        B[0][j] = *reinterpret_cast<const float4*>(at[j] + 4096);
     }
-    fold_a(acc[1]);
-    fold_b(false, false, acc[1]);
-    fold_c(false, false, true, acc[1]);
-    // levels 2 and 1 over the waves' tiles, in the buffer that the stage before the last left (all have read it; the
-    // last one's successor may still be being read, for nothing, by another wave)
-    float* red = reinterpret_cast<float*>(lds + ((S - 2) % RM_BUFS) * RM_STAGE);
+    // step k reads step k + 1's operands and fetches step k + RM_RING; RM_RING steps a trip, so that the ring's places are constants
+    auto trip = [&](int k, auto first_c, auto fold_c, auto fetch_c, auto last_c) {
+        constexpr bool LAST = decltype(last_c)::value;
+        wait(2);
+        step(A[0], B[0], A[1], B[1], 1, from_of(k + 4), first_c, fold_c, yes, fetch_c);
+        wait(LAST ? 1 : 2);
+        step(A[1], B[1], A[0], B[0], 2, from_of(k + 5), no, no, yes, fetch_c);
+        wait(LAST ? 0 : 2);
+        step(A[0], B[0], A[1], B[1], 3, from_of(k + 6), no, no, yes, fetch_c);
+        if constexpr (!LAST) wait(2);
+        step(A[1], B[1], A[0], B[0], 0, from_of(k + 7), no, no, integral_constant<bool, !LAST>{}, fetch_c);
+    };
+    trip(0, yes, no, yes, no);
+    for (int k = RM_RING; k < half; k += RM_RING) trip(k, no, no, yes, no);
+    trip(half, yes, yes, yes, no);
+    for (int k = half + RM_RING; k + RM_RING < S; k += RM_RING) trip(k, no, no, yes, no);
+    trip(S - RM_RING, no, no, no, yes);
+    // levels 32 and 16 here, 8 and 4 over the waves, 2 and 1 over the chains: wave w the accumulator's registers 4 w .. 4 w + 3, the
+    // sums through the waves' own rings (each has been read by its wave)
+    static_assert(4 * 4 * 64 * 16 <= RM_RING * RM_STEP, "a wave's sums fit its ring");
 #pragma unroll
-    for (int v = 0; v < 16; ++v) red[(wave * 16 + v) * 64 + lane] = sum[v];
-    meet(0);
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int v = 4 * wave + q;
-        const float s = (red[v * 64 + lane] + red[(32 + v) * 64 + lane]) + (red[(16 + v) * 64 + lane] + red[(48 + v) * 64 + lane]);
-        const int tk = t0 + 8 * (v >> 2) + 4 * b + (v & 3);
-        if (tk < T) y[(size_t) tk * rows + e0 + i] = s;
+        for (int q = 0; q < 4; ++q) {
+            float u[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) u[v] = held[j][4 * q + v] + (acc[j][4 * q + v] + acc[j][16 + 4 * q + v]);
+            *reinterpret_cast<float4*>(ring + ((j * 4 + q) * 64 + lane) * 16) = make_float4(u[0], u[1], u[2], u[3]);
+        }
+    __syncthreads();
+    float s[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float4 u[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) u[w] = *reinterpret_cast<const float4*>(lds + w * (RM_RING * RM_STEP) + ((j * 4 + wave) * 64 + lane) * 16);
+        s[j][0] = (u[0].x + u[2].x) + (u[1].x + u[3].x);
+        s[j][1] = (u[0].y + u[2].y) + (u[1].y + u[3].y);
+        s[j][2] = (u[0].z + u[2].z) + (u[1].z + u[3].z);
+        s[j][3] = (u[0].w + u[2].w) + (u[1].w + u[3].w);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int t = t0 + 8 * wave + 4 * b + v;
+        if (t < T) y[(size_t) t * rows + e0 + i] = (s[0][v] + s[2][v]) + (s[1][v] + s[3][v]);
     }
 }
 

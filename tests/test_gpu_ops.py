@@ -47,6 +47,12 @@ def test_gemv_f32_bit_exact(dev, oracle, rows, n, T):
     assert np.array_equal(dev.gemv(W, x).view(np.uint32), oracle.gemv_f32(W, x).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,n,T", [(513, 2048, 300), (514, 2048, 321), (256, 2048, 520), (600, 4096, 333), (545, 6144, 257)])
+def test_gemv_f32_large_tiles_bit_exact(dev, oracle, rows, n, T):
+    """tiles of 32 x 32: no, one, two and many weight rows past the last full tile, a last tile of few rows of x, wider rows"""
+    test_gemv_f32_bit_exact(dev, oracle, rows, n, T)
+
+
 # 64 rows of x and more against f32 weights with rows of a multiple of 2048: the tiles on the matrix cores (ragged last
 # tiles of both kinds, weight rows past the last full 32, more than one patch of tiles, rows of 4096), with values over
 # many binades so that a sum's bits depend on the order of its adds
