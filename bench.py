@@ -785,7 +785,7 @@ def decoder_main(args):
                                         "tokens_kept_per_round": kept_graph / (NR + 3),
                                         "ms_eager_with_chain_of_3": round_chain_ms,
                                         "ms_two_chain_steps_switched_off": stopped_chain_ms - stopped_ms}},
-            "roofline": {"bound": "hbm", "kernel": "k_q8s_gemv (output head 151,936 x 2048)", "achieved": head_bytes / (head_ms * 1e-3) / 1e9,
+            "roofline": {"bound": "hbm", "kernel": "k_q8s_stream (output head 151,936 x 2048)", "achieved": head_bytes / (head_ms * 1e-3) / 1e9,
                          "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": head_bytes / (head_ms * 1e-3) / HBM_PEAK, "traffic": None, "kernel_ms": head_ms,
                          "algorithmic_bytes": head_bytes},
             "cpu_baseline": cpu}

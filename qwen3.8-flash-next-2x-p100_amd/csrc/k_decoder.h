@@ -474,7 +474,8 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
 // places in turn. A wave then has two batches in flight until the one it needs is there, and two blocks a CU (half as many copies of
 // the activations, half the uneven end) read faster than three or four: 151,936 rows over matrices in turn, us, k_q8s_gemv with four
 // blocks / this with 1, 2, 3, 4: one row of x 55.7 / 64.7, 51.6, 52.2, 55.0; five 58.4 / 66.9, 54.1, 56.7, 58.7; sixteen
-// 66.9 / 71.4, 60.4, 62.6, 65.0. Both of a tile's batches asked for ahead of the activations: 61.3. Bound by the matrix's one read.
+// 66.9 / 71.4, 60.4, 62.6, 65.0. Both of a tile's batches asked for ahead of the activations: 61.3; neighbouring tiles to one block, one
+// after the other: 63.4; the streaming policy on the stores: 61.6. Bound by the matrix's one read and, over many rows of x, by the stores.
 constexpr int Q8S_PART_G = 80;   // floats between two lane groups' sums: the sixteen (row, token) places a read touches in different banks
 constexpr uint32_t Q8S_STREAM_OUT = 0xE0000000u;   // the results' bytes that its stores' offsets reach
 inline size_t q8s_stream_lds(int cols) {

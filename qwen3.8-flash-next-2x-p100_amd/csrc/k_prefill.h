@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(GM_WAVES * 64) k_gemv_rows_many(const void* __
 
 // ---------------------------------------------------------------- the same sums in tiles of 16 x 16, for a short chunk
 // A chunk of a few hundred rows leaves the kernel below (tiles of 32 x 32: 48 blocks for 77 rows against 513 weight rows) with
-// CUs that have no tile or one, and a tile's chain of 512 MFMAs of 64 cycles a wave is its time. Here a tile is 16 x 16
+// CUs that have no tile or one, and a tile's chain of 256 MFMAs of 64 cycles a wave is its time. Here a tile is 16 x 16
 // and the instruction v_mfma_f32_16x16x1_4b_f32: its four blocks take lanes l, l + 16, l + 32 and l + 48 of the fixed order
 // (the butterfly's levels 32 and 16 are adds within the accumulator), wave w of four takes l = 4 w + j, four independent chains
 // of n / 64 MFMAs of 32 cycles that it goes through together - a quarter of the tile's work in a quarter of the time, on
