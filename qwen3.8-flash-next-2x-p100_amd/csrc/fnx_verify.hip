@@ -2096,7 +2096,10 @@ int fnx_top_tokens(float* logits, int n, int T, int v0, const int* pen_tok, cons
     BufferScope candidates(g_cand_order, st);
     k_top_slices<<<dim3(nslice, T), SM_THREADS, 0, s>>>(
         TopArgs{logits, n, v0, nslice, pen_tok, pen_cnt, pen_n, pen_stride, pen_par, bias_tok, bias_val, bias_off, bias_n, err});
-    k_top_merge<<<T, SM_MERGE_THREADS, 0, s>>>(logits, n, v0, nslice, out_v, out_i);
+    const int lanes = SM_MERGE_THREADS / SM_N;   // slices to one candidate a lane
+    if (nslice <= 2 * lanes) k_top_merge<2><<<T, SM_MERGE_THREADS, 0, s>>>(logits, n, v0, nslice, out_v, out_i);
+    else if (nslice <= 4 * lanes) k_top_merge<4><<<T, SM_MERGE_THREADS, 0, s>>>(logits, n, v0, nslice, out_v, out_i);
+    else k_top_merge<SM_MERGE_V><<<T, SM_MERGE_THREADS, 0, s>>>(logits, n, v0, nslice, out_v, out_i);
     return launch_status("top_tokens");
 }
 int fnx_penalize_row(float* row, int n, const int* pen, const float* par, void* st) {

@@ -234,7 +234,10 @@ __global__ void __launch_bounds__(SM_THREADS) k_top_slices(const TopArgs a) {
     wave_emit64<W>(k2, f2, wave_select64<W>(k2, f2), g_topk_cand + ((size_t) row * a.nslice + s) * SM_N);
 }
 // launch 2: a block per row: the 64 best of its slices' candidates, sorted. The same rows: 12.7 -> 9.5 us with the
-// search between two ends and places counted instead of a sorting network.
+// search between two ends and places counted instead of a sorting network. V: candidates a lane, no more than the row's slices
+// make, since the search goes through all of them at every step (both launches over 5 rows, us, always eight / as many as needed: 32,000
+// logits 17.1 / 16.7, 81,920 19.9 / 19.2, 151,936 20.7 / 19.9, 163,840 21.3 / 20.1).
+template <int V>
 __global__ void __launch_bounds__(SM_MERGE_THREADS) k_top_merge(const float* __restrict__ logits, int n, int v0, int nslice, float* __restrict__ out_v,
                                                                int* __restrict__ out_i) {
     __shared__ unsigned long long cand[SM_MERGE_THREADS / 64][SM_N];
@@ -242,15 +245,15 @@ __global__ void __launch_bounds__(SM_MERGE_THREADS) k_top_merge(const float* __r
     const unsigned long long* C = g_topk_cand + (size_t) row * nslice * SM_N;
     const int total = nslice * SM_N;
     {
-        unsigned key[SM_MERGE_V], idf[SM_MERGE_V];
+        unsigned key[V], idf[V];
 #pragma unroll
-        for (int v = 0; v < SM_MERGE_V; ++v) {
+        for (int v = 0; v < V; ++v) {
             const int i = v * SM_MERGE_THREADS + tid;
             const unsigned long long c = i < total ? C[i] : 0ull;
             key[v] = (unsigned) (c >> 32);
             idf[v] = (unsigned) c;
         }
-        wave_emit64<SM_MERGE_V>(key, idf, wave_select64<SM_MERGE_V>(key, idf), cand[wave]);
+        wave_emit64<V>(key, idf, wave_select64<V>(key, idf), cand[wave]);
     }
     __syncthreads();
     if (wave != 0) return;

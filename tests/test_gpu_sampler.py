@@ -67,6 +67,12 @@ def test_top_tokens_ties_zeros_and_non_finite(dev, oracle):
     assert tied.size > 32 and np.all(np.diff(tied) > 0) and tied[0] < 64
 
 
+@pytest.mark.parametrize("n,T", [(81920, 2), (81921, 3), (163840, 2), (163841, 1)])
+def test_top_tokens_where_the_merge_takes_more_candidates_a_lane(dev, oracle, n, T):
+    """32 and 64 whole slices a row, and one logit more"""
+    test_top_tokens_shapes(dev, oracle, n, T)
+
+
 @pytest.mark.parametrize("n", [64, 65, 66, 100, 127, 128, 129, 2560, 2561, 2563, 2600, 2624, 2688, 5121])
 def test_top_tokens_of_little_more_than_the_candidates(dev, oracle, n):
     """a row, or a row's last slice, that brings the wave's real pairs to the candidates' number or just past it: the one too many at
