@@ -271,7 +271,9 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
         // A tile's results go out as buffer stores that every path issues (a lane without a token: past the buffer's end, where
         // a store is dropped): stores under a condition of their own cannot be counted, and the wait for the next tile's weights,
         // asked for before them, was a wait for the stores too (77 rows, some 400 jobs of two tokens: 59.1 -> 56.7 us a launch, 512 rows
-        // 36.0 -> 35.2, 4,096 rows the same 186). A job with a row past what 32-bit offsets reach stores under the condition.
+        // 36.0 -> 35.2, 4,096 rows the same 186). The loop stands once for each number of token tiles, so that their stores are counted too.
+        // A job with a row past what 32-bit offsets reach stores under the condition, in one loop for all numbers: with four of
+        // them the kernel was 32.7 KB of code instead of 24.9, at the same speed (8 picks of 512 experts, 29 rows 29.7 / 29.1 us a launch).
         const uint32_t rowb = (uint32_t) a.nrows * 4u, end = 0xE0000000u, none = 0xF0000000u;   // (none and a row's bytes: no wrap)
         const int reach = (int) (end / rowb);
         uint32_t at[MB_TP];
@@ -279,8 +281,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
 #pragma unroll
         for (int tt = 0; tt < MB_TP; ++tt) near = near && orow[tt] < reach, at[tt] = orow[tt] >= 0 ? (uint32_t) orow[tt] * rowb + 16u * grp : none;
         const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*) a.out, 0, (int) end, 0x00020000);
-        auto rounds = [&](auto nt_tag, auto near_tag) {
-            constexpr int NT = decltype(nt_tag)::value;
+        auto rounds = [&](auto ntiles, auto near_tag) {   // (ntiles: a constant, or nt)
             for (; g < g1; g += W16_WAVES) {
                 // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
                 // for the last: every wave takes every priority in turn, a tile each
@@ -295,25 +296,23 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
                 v4f acc[MB_TP];
 #pragma unroll
                 for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-                w16_super_step(L.tab, xlane, f, NT, acc);
+                w16_super_step(L.tab, xlane, f, ntiles, acc);
                 // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
 #pragma unroll
-                for (int tt = 0; tt < NT; ++tt) {
-                    if constexpr (decltype(near_tag)::value) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[tt]), to, at[tt], 64u * g, 0);
-                    else if (orow[tt] >= 0)
+                for (int tt = 0; tt < MB_TP; ++tt) {
+                    if constexpr (decltype(near_tag)::value) {
+                        if (tt < ntiles) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[tt]), to, at[tt], 64u * g, 0);
+                    } else if (orow[tt] >= 0)
                         *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
                 }
                 f = nf;
             }
         };
-        auto any_nt = [&](auto near_tag) {
-            if (nt == 4) rounds(std::integral_constant<int, 4>{}, near_tag);
-            else if (nt == 3) rounds(std::integral_constant<int, 3>{}, near_tag);
-            else if (nt == 2) rounds(std::integral_constant<int, 2>{}, near_tag);
-            else rounds(std::integral_constant<int, 1>{}, near_tag);
-        };
-        if (__all(near)) any_nt(std::true_type{});
-        else any_nt(std::false_type{});
+        if (!__all(near)) rounds(nt, std::false_type{});
+        else if (nt == 4) rounds(std::integral_constant<int, 4>{}, std::true_type{});
+        else if (nt == 3) rounds(std::integral_constant<int, 3>{}, std::true_type{});
+        else if (nt == 2) rounds(std::integral_constant<int, 2>{}, std::true_type{});
+        else rounds(std::integral_constant<int, 1>{}, std::true_type{});
     }
 }
 

@@ -181,7 +181,7 @@ def test_moe_mma_wave_form_tile16_rows_of_512(dev, oracle, nrows, nexp, sizes):
         assert rel_l2(got, want) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
 
 
-@pytest.mark.parametrize("n", [1, 17, 64])
+@pytest.mark.parametrize("n", [1, 17, 33, 64])
 def test_moe_mma_wave_form_output_rows_past_32_bit_offsets(dev, n):
     # a job with an output row past 3.5 GiB stores by whole addresses: the same bits as by buffer offsets, in both orders of rows
     print(f"case moe_mma wave form far rows n={n}", flush=True)
