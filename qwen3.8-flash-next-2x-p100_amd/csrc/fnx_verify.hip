@@ -1139,34 +1139,20 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
     if (rows <= 0 || n <= 0 || n % 256) return fail(std::string(who) + ": n must be a positive multiple of 256");
     if (T < 1 || T > 65535 * FNX_MAXT) return fail(std::string(who) + ": T out of range");
     hipStream_t s = (hipStream_t) st;
-    // f32 weights against more rows than a window's. Tiles of 16 x 16 (k_gemv_rows_mfma16) where the larger tiles would leave CUs
-    // idle, or cannot be had; the larger ones read each row from the L2 half as often, and that is the time of a long chunk.
-    // 513 weight rows of 2048, weights in turn, us (small tiles / large): 64 rows 5.7 / 13.2, 128 10.0 / 13.4, 240 10.2 / 13.4, 280 14.3 / 13.7, 320 15.1 / 13.5:
-    // a CU takes its small tiles one after the other, 4.5 us each, and three take longer than its one large one.
-    // Where the large ones cannot be had, k_gemv_rows_many is the other kernel: it reads a row of x once for four weight rows a
-    // wave, and fills the chip only with many rows. The narrower the rows, the more of a small tile's time is its start and its
-    // end, so it is the better one up to 5/2, 8 and 12 tiles a CU at widths of 512, 1024 and 1536, and always from 2048 on.
-    // 513 weight rows, us (small / many): 512 wide, 64 rows 4.5 / 6.9, 300 9.6 / 10.2, 450 11.9 / 10.7, 3000 66.6 / 44.1; 1024 wide, 64
-    // 5.1 / 9.7, 1000 30.4 / 31.8, 1500 48.6 / 41.6; 1536 wide, 64 5.7 / 12.4, 1000 42.8 / 43.5, 1500 60.9 / 57.5; 2560 wide, 64 7.3 / 17.8,
-    // 3000 163 / 185; 2048 weight rows of 1024, 300 32.5 / 32.6, 450 47.0 / 46.2; of 3072, 3000 647 / 750.
-    const bool large = !bf && T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (uint64_t) T * n * 4 < (1ull << 32) &&
-                       (uint64_t) rows * n * 4 < (1ull << 32) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
-    const long small_tiles = (long) ((T + RS_TILE - 1) / RS_TILE) * ((rows + RS_TILE - 1) / RS_TILE);
-    if (!bf && T > FNX_MAXT && n % (2 * RS_COLS) == 0 && small_tiles < (1l << 24) && (((uintptr_t) W | (uintptr_t) x) & 15) == 0 &&
-        small_tiles <= (large ? 2l * cu_count() : n == 512 ? 5l * cu_count() / 2 : n == 1024 ? 8l * cu_count() : n == 1536 ? 12l * cu_count() : 1l << 24)) {
+    // f32 weights against more rows than a window's: tiles on the matrix cores, or none (gemv_rows_plan.h)
+    const bool tiles = !bf && T > FNX_MAXT && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
+    const GemvRows form = tiles ? gemv_rows_form(rows, n, T, cu_count()) : GemvRows::many;
+    if (form == GemvRows::small_tiles) {
         const int ntt = (T + RS_TILE - 1) / RS_TILE, net = (rows + RS_TILE - 1) / RS_TILE;
-        k_gemv_rows_mfma16<<<(unsigned) ((small_tiles + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
+        k_gemv_rows_mfma16<<<(unsigned) ((gemv_small_tiles(rows, T) + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
         return launch_status(who);
     }
-    if (large) {
-        // a chunk's worth of rows against f32 weights: tiles of 32 x 32 sums on the matrix cores. The weight rows past the
-        // last full 32 ride with the tiles' blocks, an item a wave (a row x a row of x); if there are more items
-        // than waves in a row of tiles, those rows go to the kernel below.
+    if (form != GemvRows::many) {
         const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE;
         const int tile_blocks = ((ntt + 3) / 4) * ((net + 7) / 8) * 32;
-        const bool along = 8 * left <= net;   // (32 left items, 4 net waves)
+        const bool along = form == GemvRows::large_tiles;
         k_gemv_rows_mfma<<<tile_blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, tile_blocks, along ? 1 : 0);
-        if (left == 0 || along) return launch_status(who);
+        if (along) return launch_status(who);
         const dim3 gm((left + GM_WAVES * GR_ROWS - 1) / (GM_WAVES * GR_ROWS), (T + FNX_MAXT - 1) / FNX_MAXT);
         k_gemv_rows_many<false><<<gm, GM_WAVES * 64, 0, s>>>(W, x, y, rows, n, T, net * RM_TILE);
         return launch_status(who);

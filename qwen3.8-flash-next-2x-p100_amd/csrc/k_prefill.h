@@ -11,6 +11,7 @@
 // second rounds once - the same value as the reference's f32 product rounded to f16 (moe_mma_iq.cuh:136-149).
 #pragma once
 
+#include "gemv_rows_plan.h"
 #include "k_moe_layer.h"
 
 namespace fnx {
@@ -282,7 +283,7 @@ __global__ void __launch_bounds__(GM_WAVES * 64) k_gemv_rows_many(const void* __
 // Bound by what the XCDs' L2s hand over (256 KB a tile; some 10 TB/s in all) once every CU has a tile: 77 rows x 513 of 2048,
 // 13.8 -> 5.5 us over one set of weights; 7.5 inside a layer, whose other launches have the caches in between.
 typedef float rs_v16f __attribute__((ext_vector_type(16)));
-constexpr int RS_TILE = 16, RS_WAVES = 4, RS_LOADERS = 2, RS_THREADS = (RS_WAVES + RS_LOADERS) * 64, RS_COLS = 256, RS_ROWLD = RS_COLS * 4 + 16,
+constexpr int RS_WAVES = 4, RS_LOADERS = 2, RS_THREADS = (RS_WAVES + RS_LOADERS) * 64, RS_ROWLD = RS_COLS * 4 + 16,
               RS_STAGE = 2 * RS_TILE * RS_ROWLD, RS_BUFS = 3;
 __global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __restrict__ W, const float* __restrict__ x, float* __restrict__ y, int rows,
                                                                 int n, int T, int ntt, int net) {
@@ -394,7 +395,7 @@ __global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __
 // The weight rows past the last full 32 (the router's 513th) are items of such a row against one row of x, one a wave at most,
 // added up while the first steps are on their way.
 typedef float v32f __attribute__((ext_vector_type(32)));
-constexpr int RM_TILE = 32, RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4;
+constexpr int RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4;
 __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) k_gemv_rows_mfma(const float* __restrict__ W, const float* __restrict__ x,
                                                                                                          float* __restrict__ y, int rows, int n, int T, int ntt,
                                                                                                          int net, int tile_blocks, int along) {

@@ -47,9 +47,11 @@ def test_gemv_f32_bit_exact(dev, oracle, rows, n, T):
     assert np.array_equal(dev.gemv(W, x).view(np.uint32), oracle.gemv_f32(W, x).view(np.uint32))
 
 
-@pytest.mark.parametrize("rows,n,T", [(513, 2048, 300), (514, 2048, 321), (256, 2048, 520), (600, 4096, 333), (545, 6144, 257)])
+@pytest.mark.parametrize("rows,n,T", [(513, 2048, 300), (514, 2048, 321), (256, 2048, 520), (600, 4096, 333), (545, 6144, 257), (600, 2048, 430), (129, 2048, 900),
+                                      (129, 2048, 1809), (65, 2048, 1640), (65, 2048, 3265)])
 def test_gemv_f32_large_tiles_bit_exact(dev, oracle, rows, n, T):
-    """tiles of 32 x 32: no, one, two and many weight rows past the last full tile, a last tile of few rows of x, wider rows"""
+    """tiles of 32 x 32: no, one, two and many weight rows past the last full tile, a last tile of few rows of x, wider rows; left
+    weight rows with a launch of their own (600, 129 and 65) and, below four small tiles a CU, without one"""
     test_gemv_f32_bit_exact(dev, oracle, rows, n, T)
 
 
@@ -85,7 +87,7 @@ def test_gemv_f32_narrow_rows_bit_exact(dev, oracle, rows, n, T):
 def test_gemv_f32_sum_does_not_depend_on_T(dev):
     """A size-independent property at a size the oracle takes long for: a sum's bits do not depend on how many rows of x a
     call brings, so 4,099 rows in one call (the matrix cores' tiles, several patches of them, a ragged last tile, the 513th
-    weight row with the loading waves) must equal the same rows in calls of 16 and fewer (the vector units' kernel)."""
+    weight row as items beside the tiles) must equal the same rows in calls of 16 and fewer (the vector units' kernel)."""
     rows, n, T = 513, 2048, 4099
     print(f"case gemv_f32 T-independence rows={rows} n={n} T={T}", flush=True)
     rng = np.random.default_rng(240)

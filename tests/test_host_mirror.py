@@ -58,3 +58,13 @@ def test_q8s_split(tmp_path):
                     os.path.join(HERE, "q8s_split_check.cpp")], check=True, capture_output=True, text=True)
     r = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120)
     assert r.stdout.startswith("ok "), r.stdout
+
+
+def test_gemv_rows_plan(tmp_path):
+    """which kernel takes a router's product over a chunk, compiled for the host: no launch more and no larger tiles than
+    the measured lines say, at every number of weight rows up to 600"""
+    exe = str(tmp_path / "gemv_rows_plan_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I", os.path.join(fnx_gpu.PKG_DIR, "csrc"), "-o", exe,
+                    os.path.join(HERE, "gemv_rows_plan_check.cpp")], check=True, capture_output=True, text=True)
+    r = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120)
+    assert r.stdout.startswith("ok "), r.stdout
