@@ -572,7 +572,7 @@ __device__ __forceinline__ unsigned wave_umin(unsigned v) { return ~wave_umax(~v
 // KEEP: a chain step's head (one row): the row's last block keeps the pick, and makes the next window after the last step (k_round.h).
 template <bool KEEP>
 __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__ logits, int rows, unsigned long long* __restrict__ keys,
-                                                      unsigned* __restrict__ err, int v0, float* __restrict__ bv, int* bi,
+                                                      unsigned* __restrict__ err, int v0, float* __restrict__ bv, int* __restrict__ bi,
                                                       const int* __restrict__ live, const ChainKeep keep) {
     __shared__ uint2 wbest[AM_THREADS / 64];
     __shared__ int wbad[AM_THREADS / 64];
@@ -581,9 +581,9 @@ __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__
     const int t = blockIdx.y, i0 = blockIdx.x * AM_PER_BLOCK, i1 = min(rows, i0 + AM_PER_BLOCK), tid = threadIdx.x, lane = tid & 63;
     const float* r = logits + (size_t) t * rows;
     // the chain's words, asked for now and used at the end: a lane a word of the drafts
-    int chain = 0, stop = 0, n_ctx = 1, kept = 1, draft = 0;
+    int chain = 0, stop = 0, n_ctx = 1, draft = 0;
     if constexpr (KEEP) {
-        chain = keep.state[FNX_RS_CHAIN], stop = keep.state[FNX_RS_STOP], n_ctx = keep.state[FNX_RS_NCTX], kept = keep.state[FNX_RS_ACCEPTED];
+        chain = keep.state[FNX_RS_CHAIN], stop = keep.state[FNX_RS_STOP], n_ctx = keep.state[FNX_RS_NCTX];
         if (lane < FNX_MAXT) draft = keep.scratch[lane];   // lane 0: how many the lookup found
     }
     unsigned best = 0, at = 0xffffffffu;   // the thread's greatest key and the first index that holds it (it goes through its values in order)
@@ -651,19 +651,13 @@ __global__ void __launch_bounds__(AM_THREADS) k_argmax(const float* __restrict__
             if (last) keep.scratch[0] = keep.K;
         }
         if (!last || uniform(stop) != 0) return;
-        // the next window's rows and count
-        const int nd = on ? keep.K : min(max(uniform(draft), 0), FNX_MAXT - 1), first = uniform(n_ctx) - 1;
-        int tok = 0, R = 2;
-        if (nd > 0) {
-            R = 1 + nd;
-            if (lane <= nd) tok = on && lane == keep.K ? pick : draft;
-        } else if (lane == 1) {
-            const int n = min(max(uniform(kept), 1), FNX_MAXT);
-            tok = n == 1 ? pick : keep.best[n - 1];
-        }
+        // the next window: the context's last token, then the drafts - the chain's, or the lookup's: with the chain off in a session
+        // that goes on, the lookup has left one at least
+        const int nd = on ? keep.K : min(max(uniform(draft), 1), FNX_MAXT - 1), first = uniform(n_ctx) - 1;
+        int tok = lane > nd ? 0 : on && lane == keep.K ? pick : draft;
         if (lane == 0) tok = keep.ctx[first];
         if (lane < FNX_MAXT) keep.rows[lane] = tok;
-        if (lane == 0) keep.state[FNX_RS_ROWS] = R;
+        if (lane == 0) keep.state[FNX_RS_ROWS] = 1 + nd;
     }
 }
 
@@ -2058,7 +2052,7 @@ int fnx_decode_round(const fnx_decoder* D, const fnx_mtp* M, const fnx_round* R,
         // layer's own row; one row, which counts (is routed, runs the big kernels) only while state[CHAIN] is set
         const int* on = S + FNX_RS_CHAIN;
         for (int j = 1; j < K; ++j) {
-            const ChainKeep keep{S, R->scratch, R->ctx, ws->best_i, R->rows, j, K};
+            const ChainKeep keep{S, R->scratch, R->ctx, R->rows, j, K};
             if (mtp_draft(D, M, j == 1 ? R->chain_src : ws->hidden, R->scratch + j, 1, S + FNX_RS_CHAIN_POS + (j - 1), ws, st, on, on, &keep)) return 1;
         }
     } else {

@@ -62,14 +62,14 @@ struct ChainBegin {
 // after step j (1 .. K - 1): its pick is draft j + 1; the last step hands the K drafts to the next window
 struct ChainKeep {
     int *state, *scratch;
-    const int *ctx, *best;           // best: the draft layer's picks
+    const int* ctx;
     int* rows;                       // the next window, made after the last step
     int j, K;
 };
 
-// the next window without speculation (session.cpp:530-560): the last token of the context alone. One wave. (With it the
-// lookup's launch or the chain's last step makes the window: that token, then the drafts, or else the draft layer's pick for the
-// last row kept.)
+// the next window without speculation (session.cpp:530-560): the last token of the context alone. One wave. (With it
+// the window is that token, then the drafts: with a single draft a round the lookup's launch makes it, of what it found or else the
+// draft layer's pick for the last row kept; with a chain the chain's last step, of what the lookup found or else the chain's drafts.)
 __global__ void k_round_window(const int* __restrict__ ctx, int* __restrict__ state, int* __restrict__ rows) {
     const int i = threadIdx.x;
     if (state[FNX_RS_STOP]) return;

@@ -227,21 +227,35 @@ def test_rounds_replayed_from_one_graph(dev, oracle, cyclic_model, chain, lk):
     assert out_g == out_e and log_g == log_e, "a round has no argument that changes: one captured round replays as every round"
 
 
-def test_rounds_stop_before_the_cache_is_full(dev, oracle, cyclic_model):
+@pytest.mark.parametrize("chain,lk", [(0, 15), (3, 15), (3, 0)])
+def test_rounds_stop_before_the_cache_is_full(dev, oracle, cyclic_model, chain, lk):
+    """with a chain the stop is looked at in the lookup's launch (the chain does not begin) and in the last step's argmax (the
+    window stays), whether the lookup's drafts (lk = 15) or the chain's (lk = 0) made the windows before"""
     model = cyclic_model
     prompt = [t % model.cfg["vocab"] for t in repeating_prompt(12)]
-    r = RoundDev(dev, model, prompt)
+    r = RoundDev(dev, model, prompt, chain=chain, lk=lk)
     cap = model.cfg["max_ctx"]
-    print("case decode_round until the cache is full", flush=True)
+    print(f"case decode_round until the cache is full chain={chain} lk={lk}", flush=True)
     for _ in range(cap):   # more rounds than the cache has room for
         r.launch()
     out, log, st = r.result()
     pkg = dev.pkg
     assert st[pkg.RS_STOP] == 1 and st[pkg.RS_POS] + 16 <= cap and st[pkg.RS_NCTX] == st[pkg.RS_POS] + 1
     assert st[pkg.RS_POS] + 16 + 16 > cap, "it stopped no earlier than it had to"
+    assert chain == 0 or st[pkg.RS_CHAIN] == 0, "no chain begins in a stopped session"
     for _ in range(3):
         r.launch()
     out2, log2, st2 = r.result()
     assert out2 == out and np.array_equal(st2, st), "a stopped session stays as it is"
-    out_h, _ = host_loop(dev, model, prompt, len(out))
+    # and so does a window that is not the one its rounds would make, and its count
+    r.rows[1:] = 7
+    r.chain_src[:] = 3.0
+    r.state[pkg.RS_ROWS] = 6
+    words = lambda: {k: getattr(r, k).cpu().numpy() for k in ("rows", "ctx", "log", "chain_src", "state")}
+    before = words()
+    for _ in range(2):
+        r.launch()
+    dev.sync()
+    assert all(np.array_equal(v, before[k]) for k, v in words().items())
+    out_h, _ = host_loop(dev, model, prompt, len(out), K=max(1, chain), lk=lk)
     assert out == out_h
