@@ -1753,15 +1753,13 @@ static int q8s_launch(const fnx_q8s* const* W, float* const* out, const int* out
         if (n != 2 || grid < tiles) return fail(std::string(who) + ": two sets of rows want two matrices and a block a tile");
         a.yq2 = (const uint8_t*) yq2;
     }
-    // three tiles a block and more, of quarters of whole pairs of batches, where two blocks' activations fit a CU (2,048 columns): the
-    // form that counts what it waits for. At two tiles a block (16,384 rows) one row of x 8.7 / 9.4 us, sixteen 12.1 / 10.7 (this
+    // three tiles a block and more of 2,048 columns: the form that counts what it waits for. At two tiles a block (16,384 rows) one row of x 8.7 / 9.4 us, sixteen 12.1 / 10.7 (this
     // form second); at three (24,576) 12.2 / 12.1 and 14.7 / 13.2.
-    const size_t slds = q8s_stream_lds(a.cols);
-    if (n == 1 && W[0]->tiled && a.cols % 2048 == 0 && 2 * slds <= 160 * 1024 && tiles >= 6l * cu_count() &&
+    if (n == 1 && W[0]->tiled && a.cols == Q8S_STREAM_COLS && tiles >= 6l * cu_count() &&
         (unsigned long long) out_stride[0] * FNX_MAXT * 4 < Q8S_STREAM_OUT) {
         const int blocks = 2 * cu_count();
-        if (live) k_q8s_stream<true><<<blocks, Q8S_WAVES * 64, slds, (hipStream_t) st>>>(a);
-        else k_q8s_stream<false><<<blocks, Q8S_WAVES * 64, slds, (hipStream_t) st>>>(a);
+        if (live) k_q8s_stream<true><<<blocks, Q8S_WAVES * 64, Q8S_STREAM_LDS, (hipStream_t) st>>>(a);
+        else k_q8s_stream<false><<<blocks, Q8S_WAVES * 64, Q8S_STREAM_LDS, (hipStream_t) st>>>(a);
         return launch_status(who);
     }
     // a block a tile, of rows of two to four batches a wave: the form that asks for a tile's weights at once (measured at the kernel)

@@ -468,8 +468,8 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
     }
 }
 
-// The same for a matrix of many tiles a block in the tile-major layout, quarters of an even number of whole batches (columns in
-// 2,048s; the output heads). What a wave waits for is counted exactly: no load and no store stands under a condition (the last tile
+// The same for a matrix of many tiles a block in the tile-major layout and of 2,048 columns (the output heads): a quarter is two
+// batches, and the activations of two blocks fit a CU's LDS (of 4,096 columns one block's). What a wave waits for is counted exactly: no load and no store stands under a condition (the last tile
 // is peeled off), every wave stores a quarter of a tile's results, and the block meets once a tile, the quarters' sums in two
 // places in turn. A wave then has two batches in flight until the one it needs is there, and two blocks a CU (half as many copies of
 // the activations, half the uneven end) read faster than three or four: 151,936 rows over matrices in turn, us, k_q8s_gemv with four
@@ -478,16 +478,17 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
 // after the other: 63.4; the streaming policy on the stores: 61.6. Bound by the matrix's one read and, over many rows of x, by the stores.
 constexpr int Q8S_PART_G = 80;   // floats between two lane groups' sums: the sixteen (row, token) places a read touches in different banks
 constexpr uint32_t Q8S_STREAM_OUT = 0xE0000000u;   // the results' bytes that its stores' offsets reach
-inline size_t q8s_stream_lds(int cols) {
-    return (size_t) FNX_MAXT * (cols + Q8S_XPAD) + (size_t) FNX_MAXT * (cols / 32 + 2) * 4 + 2 * Q8S_WAVES * 4 * Q8S_PART_G * 4;
-}
+constexpr int Q8S_STREAM_COLS = 2048, Q8S_STREAM_LDS = FNX_MAXT * (Q8S_STREAM_COLS + Q8S_XPAD) + FNX_MAXT * (Q8S_STREAM_COLS / 32 + 2) * 4 + 2 * Q8S_WAVES * 4 * Q8S_PART_G * 4;
+static_assert(2 * Q8S_STREAM_LDS <= 160 * 1024, "two blocks a CU");
 template <bool LIVE>
 __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_stream(const Q8sArgs a) {
     typedef __attribute__((address_space(1))) const at_v4u_t g128;
     extern __shared__ __align__(16) uint8_t q8s_lds[];   // [16][cols + pad] int8, [16][nb + 2] f32 scales, [2][4][4 * Q8S_PART_G] partial sums
     const int live_v = LIVE ? *a.live : a.T;
     if (a.gate && uniform(*a.gate) == 0) return;
-    const int nb = a.cols >> 5, T = a.T, xld = a.cols + Q8S_XPAD, dld = nb + 2, nq4 = q8s_quarter(a.cols);
+    constexpr int cols = Q8S_STREAM_COLS, nb = cols >> 5, xld = cols + Q8S_XPAD, dld = nb + 2, nq4 = 2 * Q8S_BATCH;
+    static_assert(nq4 * 256 == cols, "a quarter is two batches");
+    const int T = a.T;
     int8_t* xs = reinterpret_cast<int8_t*>(q8s_lds);
     float* xd = reinterpret_cast<float*>(q8s_lds + (size_t) FNX_MAXT * xld);
     float* part = xd + FNX_MAXT * dld;
@@ -500,7 +501,7 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_stream(const Q8sArgs a) 
         at_v4u_t w[Q8S_BATCH], dd[4];
     };
     auto load = [&](int tile, int jb, Batch& o) {
-        const gbytes w = as_global(reinterpret_cast<const uint8_t*>(a.seg[0].q) + (size_t) tile * 16 * a.cols + Q8S_TILE_STEP * (j0 + jb)) + 16 * lane;
+        const gbytes w = as_global(reinterpret_cast<const uint8_t*>(a.seg[0].q) + (size_t) tile * 16 * cols + Q8S_TILE_STEP * (j0 + jb)) + 16 * lane;
 #pragma unroll
         for (int u = 0; u < Q8S_BATCH; ++u) o.w[u] = __builtin_nontemporal_load((g128*) (w + Q8S_TILE_STEP * u));
 #pragma unroll
@@ -567,25 +568,15 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_stream(const Q8sArgs a) 
     }
     __syncthreads();
     for (; tile + (int) gridDim.x < tiles; tile += gridDim.x) {
-        for (int jb = 0; jb < nq4; jb += 2 * Q8S_BATCH) {
-            const bool end = jb + 2 * Q8S_BATCH >= nq4;
-            load(tile, jb + Q8S_BATCH, B);
-            compute(jb, A);
-            load(end ? tile + gridDim.x : tile, end ? 0 : jb + 2 * Q8S_BATCH, A);
-            compute(jb + Q8S_BATCH, B);
-        }
+        load(tile, Q8S_BATCH, B);
+        compute(0, A);
+        load(tile + gridDim.x, 0, A);
+        compute(Q8S_BATCH, B);
         finish(tile);
     }
-    int jb = 0;
-    for (; jb + 2 * Q8S_BATCH < nq4; jb += 2 * Q8S_BATCH) {
-        load(tile, jb + Q8S_BATCH, B);
-        compute(jb, A);
-        load(tile, jb + 2 * Q8S_BATCH, A);
-        compute(jb + Q8S_BATCH, B);
-    }
-    load(tile, jb + Q8S_BATCH, B);
-    compute(jb, A);
-    compute(jb + Q8S_BATCH, B);
+    load(tile, Q8S_BATCH, B);
+    compute(0, A);
+    compute(Q8S_BATCH, B);
     finish(tile);
 }
 
