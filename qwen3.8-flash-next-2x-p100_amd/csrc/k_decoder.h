@@ -277,7 +277,8 @@ struct Q8sArgs {
     const uint8_t* yq2;  // may be null; else the second matrix's rows are these (two matrices, a block a tile: the host sees to that)
     const int* live;     // may be null; else a device word: rows from *live on do not count - they are not read and their products are zeros
     int pieces;          // a lane's four results of a tile are one aligned 16-byte piece, all of it inside the rows or none: one store
-                         // instead of four (the head over 16 rows: 70.6 -> 67.5 us)
+                         // instead of four, in the forms of one tile a block (2,048 rows of 2,048 columns 4.44 -> 4.36 us, 16,384 over
+                         // sixteen rows of x 12.05 -> 11.80; 32,000 of 4,096, many tiles a block, 29.1 -> 29.6: not there)
 };
 typedef int q8s_v4i __attribute__((ext_vector_type(4)));
 // DEPTH: the (tile, batch) items whose loads are in flight ahead of the one being worked on, where a block goes through more
@@ -393,7 +394,7 @@ __global__ void __launch_bounds__(Q8S_WAVES * 64) k_q8s_gemv(const Q8sArgs a) {
             const float v[4] = {(p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y), (p0.z + p1.z) + (p2.z + p3.z),
                                 (p0.w + p1.w) + (p2.w + p3.w)};
             const bool counts = !LIVE || r16 < Tl;   // (rows from *live on: zeros)
-            if (a.pieces) {
+            if (ONE && a.pieces) {
                 if (c.row0 + 4 * g < c.rows) *reinterpret_cast<float4*>(c.out) = counts ? make_float4(v[0], v[1], v[2], v[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
             } else {
 #pragma unroll

@@ -121,6 +121,11 @@ def test_q8s_gemv_many_tiles_a_block(dev, oracle, rows, T):
     test_q8s_gemv_bit_exact(dev, oracle, rows, 2048, T)
 
 
+@pytest.mark.parametrize("rows,cols,T", [(16404, 512, 7), (24600, 1024, 16), (20003, 768, 2)])
+def test_q8s_gemv_many_tiles_a_block_of_other_widths(dev, oracle, rows, cols, T):
+    test_q8s_gemv_bit_exact(dev, oracle, rows, cols, T)
+
+
 @pytest.mark.parametrize("rope", [ROPE, YARN])
 @pytest.mark.parametrize("nq,nkv,T,pos0", [(4, 2, 3, 5), (16, 2, 16, 32000), (8, 1, 1, 0)])
 def test_attn_prep_append(dev, oracle, nq, nkv, T, pos0, rope):
