@@ -1757,7 +1757,8 @@ static int q8s_launch(const fnx_q8s* const* W, float* const* out, const int* out
     // form second); at three (24,576) 12.2 / 12.1 and 14.7 / 13.2.
     if (n == 1 && W[0]->tiled && a.cols == Q8S_STREAM_COLS && tiles >= 6l * cu_count() &&
         (unsigned long long) out_stride[0] * FNX_MAXT * 4 < Q8S_STREAM_OUT) {
-        const int blocks = 2 * cu_count();
+        static const int stream_per_cu = env_int("FNX_Q8S_BLOCKS_PER_CU", 2, 1, 16);   // (measured at the kernel)
+        const int blocks = (int) std::min<long>((long) stream_per_cu * cu_count(), tiles);
         if (live) k_q8s_stream<true><<<blocks, Q8S_WAVES * 64, Q8S_STREAM_LDS, (hipStream_t) st>>>(a);
         else k_q8s_stream<false><<<blocks, Q8S_WAVES * 64, Q8S_STREAM_LDS, (hipStream_t) st>>>(a);
         return launch_status(who);
