@@ -497,9 +497,12 @@ __global__ void __launch_bounds__(256) k_iq3s_jobs_any(const RowsArgs a) {
 
 // ================================================================ combine (kernels.cu:412-419)
 // Bound by the partial sums' one read. A thread takes four columns (V4) in 16-byte loads of the streaming policy, or one; the
-// operations on a column are the same. Ten picks, rows of 2,048, us (one column / four): 4,096 rows 67.3 / 65.9, 512 rows 11.0 / 9.3,
-// 300 rows 7.9 / 6.8; 150 rows 5.3 / 5.5 and 77 rows 4.8 / 5.6, where four columns a thread leave the chip too few waves.
-constexpr size_t COMBINE_V4 = 1u << 19;   // columns of all rows from which a thread takes four: eight waves a CU
+// operations on a column are the same. Four where they still make more than eight waves a CU. Behind the down launch of a layer, its sums
+// just written, us (one column / four): rows of 2,048 and ten picks, 256 rows (eight waves) 5.4 / 5.7, 272 6.2 / 5.7, 300 6.6 / 6.1, 512 9.4 /
+// 9.2, 4,096 76 / 60; eight picks, 256 5.0 / 5.0, 300 5.4 / 5.1; seven, 4,096 48.4 / 45.7; rows of 4,096, eight picks, 144 5.3 / 5.2, ten, 160 7.0 / 6.3; of
+// 512, eight, 1,200 5.5 / 5.3. Over sums that lie in the caches (calls of this alone, over 160 MB in turn) one column is ahead for longer: ten
+// picks, 300 rows 6.6 / 6.8, 400 8.4 / 8.1, 512 10.5 / 9.2; one pick, 300 4.3 / 4.2, 512 5.4 / 4.3.
+constexpr int COMBINE_V4_WAVES = 8;   // waves a CU
 template <bool V4>
 __global__ void __launch_bounds__(256) k_combine(const float* __restrict__ part, const float* __restrict__ topw, const float* __restrict__ sh,
                                                 const float* __restrict__ sh_logit, int sh_logit_stride, float* __restrict__ out, int n,
@@ -1263,7 +1266,7 @@ int fnx_moe_combine(const float* part, const float* topw, const float* sh, const
     if (!part || !topw || !sh || !sh_logit || !out) return fail("moe_combine: null argument");
     if (T < 1 || n < 1 || topk < 1) return fail("moe_combine: bad shape");
     const bool aligned = n % 4 == 0 && (((uintptr_t) part | (uintptr_t) sh | (uintptr_t) out) & 15) == 0;
-    if (aligned && (size_t) T * n >= COMBINE_V4) k_combine<true><<<dim3((n / 4 + 255) / 256, T), 256, 0, (hipStream_t) st>>>(part, topw, sh, sh_logit, sh_logit_stride, out, n, topk);
+    if (aligned && (size_t) T * n > (size_t) COMBINE_V4_WAVES * 4 * 64 * cu_count()) k_combine<true><<<dim3((n / 4 + 255) / 256, T), 256, 0, (hipStream_t) st>>>(part, topw, sh, sh_logit, sh_logit_stride, out, n, topk);
     else k_combine<false><<<dim3((n + 255) / 256, T), 256, 0, (hipStream_t) st>>>(part, topw, sh, sh_logit, sh_logit_stride, out, n, topk);
     return launch_status("moe_combine");
 }

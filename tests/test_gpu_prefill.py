@@ -181,6 +181,34 @@ def test_moe_mma_wave_form_tile16_rows_of_512(dev, oracle, nrows, nexp, sizes):
         assert rel_l2(got, want) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
 
 
+# More than 524,288 columns of all rows (on 256 CUs): a thread of the combine takes four columns, unless the rows are no whole
+# 16-byte pieces or a buffer is not aligned to them (`off`: by how many floats part, sh and out are shifted).
+@pytest.mark.parametrize("T,n,topk,off", [(257, 2048, 10, (0, 0, 0)), (300, 2048, 1, (0, 0, 0)), (410, 1300, 3, (0, 0, 0)), (140, 3844, 16, (0, 0, 0)), (1100, 512, 8, (0, 0, 0)),
+                                          (300, 2050, 10, (0, 0, 0)), (300, 2047, 9, (0, 0, 0)), (257, 2048, 8, (1, 0, 0)), (257, 2048, 7, (0, 2, 0)), (257, 2048, 10, (0, 0, 1)),
+                                          (256, 2048, 10, (0, 0, 0))])
+def test_combine_of_many_rows_equals_few(dev, oracle, T, n, topk, off):
+    """a row's bits do not depend on how many rows a call brings: against the same rows 64 a call (one column a thread), and the oracle"""
+    print(f"case combine T={T} n={n} topk={topk} off={off}", flush=True)
+    rng = np.random.default_rng(790 + T + n + topk)
+    part, sh = rng.standard_normal((T * topk, n)).astype(np.float32), rng.standard_normal((T, n)).astype(np.float32)
+    topw, logit = rng.random((T, topk)).astype(np.float32), rng.standard_normal((T, 1)).astype(np.float32)
+    t = dev.torch
+    flat = lambda a, o: t.cat((t.zeros(o, device="cuda:0"), dev.up(a).flatten()))
+    dp, ds, dt, dl = flat(part, off[0]), flat(sh, off[1]), dev.up(topw), dev.up(logit)
+    out, few = t.full((off[2] + T * n + 4,), float("nan"), device="cuda:0"), t.zeros((T, n), device="cuda:0")
+    dev.ok(dev.lib.fnx_moe_combine(dp.data_ptr() + 4 * off[0], dt.data_ptr(), ds.data_ptr() + 4 * off[1], dl.data_ptr(), 1, out.data_ptr() + 4 * off[2], T, n, topk, dev.st()))
+    for t0 in range(0, T, 64):
+        k = min(64, T - t0)
+        dev.ok(dev.lib.fnx_moe_combine(dp.data_ptr() + 4 * (off[0] + t0 * topk * n), dt.data_ptr() + 4 * t0 * topk, ds.data_ptr() + 4 * (off[1] + t0 * n), dl.data_ptr() + 4 * t0, 1,
+                                       few.data_ptr() + 4 * t0 * n, k, n, topk, dev.st()))
+    dev.sync()
+    got = out.cpu().numpy()
+    assert np.isnan(got[:off[2]]).all() and np.isnan(got[off[2] + T * n:]).all(), "nothing beside the rows"
+    got = got[off[2]:off[2] + T * n].reshape(T, n)
+    assert np.array_equal(got.view(np.uint32), few.cpu().numpy().view(np.uint32))
+    assert rel_l2(got, oracle.moe_combine(part, topw, sh, logit[:, 0])) <= 1e-6   # the sigmoid's expf is the device's
+
+
 @pytest.mark.parametrize("n", [1, 17, 33, 64])
 def test_moe_mma_wave_form_output_rows_past_32_bit_offsets(dev, n):
     # a job with an output row past 3.5 GiB stores by whole addresses: the same bits as by buffer offsets, in both orders of rows
