@@ -55,10 +55,11 @@ def test_gemv_f32_large_tiles_bit_exact(dev, oracle, rows, n, T):
     test_gemv_f32_bit_exact(dev, oracle, rows, n, T)
 
 
-# 64 rows of x and more against f32 weights with rows of a multiple of 2048: the tiles on the matrix cores (ragged last
-# tiles of both kinds, weight rows past the last full 32, more than one patch of tiles, rows of 4096), with values over
+# 64 rows of x and more against f32 weights with rows of a multiple of 2048: the tiles on the matrix cores (those of 32 x 32: 513 weight
+# rows x 512, whose last one rides along, 600 x 430, whose last 24 have a launch of their own; else those of 16 x 16; ragged last
+# tiles of both kinds, more than one patch of tiles, rows of 4096), with values over
 # many binades so that a sum's bits depend on the order of its adds
-@pytest.mark.parametrize("rows,n,T", [(513, 2048, 512), (96, 2048, 70), (290, 2048, 200), (64, 4096, 64), (35, 2048, 129), (33, 4096, 66), (65, 3072, 96)])
+@pytest.mark.parametrize("rows,n,T", [(513, 2048, 512), (600, 2048, 430), (96, 2048, 70), (290, 2048, 200), (64, 4096, 64), (35, 2048, 129), (33, 4096, 66), (65, 3072, 96)])
 def test_gemv_f32_many_rows_bit_exact(dev, oracle, rows, n, T):
     print(f"case gemv_f32 (tiles) rows={rows} n={n} T={T}", flush=True)
     rng = np.random.default_rng(230 + rows + T)
@@ -99,10 +100,11 @@ def test_gemv_f32_sum_does_not_depend_on_T(dev):
         assert np.array_equal(big[t0:t0 + len(small)], small), f"rows {t0}.."
 
 
-def test_gemv_f32_many_rows_non_finite(dev, oracle):
+@pytest.mark.parametrize("rows,T", [(65, 64), (513, 260)])   # tiles of 16 x 16, of 32 x 32
+def test_gemv_f32_many_rows_non_finite(dev, oracle, rows, T):
     """Infinities and NaNs in x and W go through the matrix cores' chains as through fmaf: the same sums are NaN, the same
     +-inf, the finite ones keep their bits (a NaN's payload is not compared)."""
-    rows, n, T = 65, 2048, 64
+    n = 2048
     rng = np.random.default_rng(241)
     W = (rng.standard_normal((rows, n)) * 0.02).astype(np.float32)
     x = rng.standard_normal((T, n)).astype(np.float32)
@@ -111,7 +113,7 @@ def test_gemv_f32_many_rows_non_finite(dev, oracle):
     x[9, 2000] = np.nan
     W[10, 100] = 0.0        # inf * 0 = NaN in row 3 x weight row 10
     W[20, 50] = np.inf
-    W[64, 1] = np.nan       # the weight row past the tiles
+    W[rows - 1, 1] = np.nan   # the weight row past the whole tiles
     got, want = dev.gemv(W, x), oracle.gemv_f32(W, x)
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
