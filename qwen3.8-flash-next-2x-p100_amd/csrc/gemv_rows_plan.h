@@ -25,8 +25,11 @@ inline bool gemv_rest_along(int rows) { return 8 * (rows % RM_TILE) <= rows / RM
 // 13.2, 128 10.0 / 13.4, 240 10.2 / 13.4, 280 14.3 / 13.7, 320 15.1 / 13.5; 257 weight rows, 482 rows of x 15.9 / 13.3.
 // Where the left weight rows want a second launch (11 us and more, whatever it computes), four a CU. 2,048 columns (small / large and
 // rest): 33 weight rows, 2,900 rows of x 18.1 / 34.9, 5,000 24.5 / 47.1, 6,000 29.8 / 48.1; 65, 1,633 17.4 / 24.2, 3,200 25.3 / 35.4; 129, 897
-// 17.0 / 23.9, 1,300 19.1 / 24.4, 1,400 23.6 / 24.3, 1,820 (five a CU) 29.2 / 25.1; 300, 512 16.7 / 25.0, 800 24.8 / 35.3; 1,000, 140 14.2 / 24.7,
-// 240 19.5 / 25.6; of 4,096, 129, 1,500 39.3 / 40.9, 1,820 49.4 / 42.1.
+// 17.0 / 23.9, 1,300 19.1 / 24.4; 300, 512 16.7 / 25.0; 1,000, 140 14.2 / 24.7, 240 19.5 / 25.6. Between 7/2 and four a CU most shapes still gain, their
+// large tiles being more than a round of the CUs: 97, 2,330 25.4 / 35.0; 161, 1,480 25.8 / 34.6; 193, 1,240 25.9 / 34.5; 300, 780 24.4 / 35.3; those whose large
+// tiles are one round are a little behind: 129, 1,600 24.3 / 24.5, 1,728 25.0 / 24.6, 1,808 25.3 / 25.0, 225, 1,020 24.8 / 24.4, and at five 129, 1,820 29.2 / 25.1. Wider
+// rows the same: of 4,096, 129, 1,500 39.4 / 40.9, 1,808 44.5 / 41.6, 161, 1,480 43.8 / 58.8; of 8,192, 129, 1,500 71.9 / 73.8, 1,808 81.0 / 75.4, 300, 800 76.7 / 109, 65,
+// 3,200 79.4 / 108.
 // Where the large ones cannot be had, k_gemv_rows_many is the other kernel: it reads a row of x once for four weight rows a
 // wave, and fills the chip only with many rows. The narrower the rows, the more of a small tile's time is its start and its
 // end, so it is the better one up to 5/2, 8 and 12 tiles a CU at widths of 512, 1024 and 1536, and always from 2048 on.
