@@ -56,7 +56,7 @@ WINDOW_TRAFFIC = {"bytes": 209.47e6, "algorithmic_bytes": 192.96e6, "distinct_ex
                              "this run's algorithmic bytes; not measured in this run)"}
 # the same for the prompt path's gate|up launch (profiles/prefill_chunk_counters.md: FETCH_SIZE x 2 + WRITE_SIZE)
 PF_WINDOW_TRAFFIC = {"bytes": 127.8e6, "algorithmic_bytes": 98.6e6,
-                      "source": "profiles/prefill_chunk_counters.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE of this file's prefill workload, k_moe_mma_wave16_gu; "
+                      "source": "profiles/prefill_chunk_counters.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE of this file's prefill workload, k_moe_mma_wave16_pairs; "
                                 "scaled to this run's algorithmic bytes; not measured in this run)"}
 IQ3S_BLOCK = 110
 GU_BYTES = 2 * FF * (N // 256) * IQ3S_BLOCK      # 901,120 per expert
@@ -201,7 +201,7 @@ def main():
                     help="the shared expert as dense split Q8_0 (the reference's own form, three more launches a window) instead of IQ3_S")
     ap.add_argument("--no-extras", action="store_true", help="skip the legs beside the metric (verify: streaming calibration, config 1, the other weight kind; prefill: two chunks in flight)")
     ap.add_argument("--raw-layout", action="store_true", help="verify: leave the weights as raw ggml blocks (skip the load-time re-laying); prefill: unit64 only, no tile16 copies")
-    ap.add_argument("--down-unit64", action="store_true", help="prefill: leave the down matrices in the unit64 layout (k_moe_mma) instead of tile16 (k_moe_mma_wave16)")
+    ap.add_argument("--down-unit64", action="store_true", help="prefill: leave the down matrices in the unit64 layout instead of tile16 (k_moe_mma_wave16 either way)")
     ap.add_argument("--workload", choices=["verify", "prefill", "decoder", "head", "gemv"], default="verify",
                     help="verify: benchmark config 2 (the headline metric, the default); prefill: config 5, one MoE layer over prompt chunks of 512 "
                          "rows; decoder: config 4, a verify step of the reduced decoder plus the draft layer; head: config 3, argmax + prompt "
@@ -976,8 +976,8 @@ def prefill_main(args):
         cpu = {"value": CS / cdt, "unit": "tokens/s per layer", "cores": threads, "kind": "port",
                "sample": f"one pass of the oracle's prefill layer over the first {CS} rows of chunk 0 (f16 operands, f64 accumulation)",
                "parity_rel_l2": err}
-    gu_kernel = ("k_moe_mma (routed gate|up over unit64, a wave a task of 32 rows x 32 tokens; h by fnx_swiglu_h16)" if args.raw_layout else
-                 "k_moe_mma_wave16_gu (routed gate|up over tile16, leaves h = silu(gate) * up; a wave a pair of gate and up tiles, a job's up to 64 tokens a decode)")
+    gu_kernel = ("k_moe_mma_wave16_pairs (routed gate|up over unit64, leaves the products; h by fnx_swiglu_h16)" if args.raw_layout else
+                 "k_moe_mma_wave16_pairs (routed gate|up over tile16, leaves h = silu(gate) * up; a wave a pair of gate and up tiles, a job's up to 64 tokens a decode)")
     line = {
         "metric": "prefill MoE tokens/sec per layer (chunks of 512 rows) + grouped IQ3_S expert GEMM achieved GB/s and MFMA utilisation",
         "value": CH * steps / dt, "unit": "tokens/s per layer", "n_gpus": 1, "steps": steps, "warmup": warmup,
@@ -991,8 +991,8 @@ def prefill_main(args):
                      "traffic": PF_WINDOW_TRAFFIC["bytes"] * gu_bytes / PF_WINDOW_TRAFFIC["algorithmic_bytes"] if nsets == 4 and not args.raw_layout else None,
                      "traffic_source": PF_WINDOW_TRAFFIC["source"] if nsets == 4 and not args.raw_layout else None, "kernel_ms": gu_ms, "algorithmic_bytes": gu_bytes,
                      "mfma_tflops": gu_flops / (gu_ms * 1e-3) / 1e12, "mfma_frac": gu_flops / (gu_ms * 1e-3) / MFMA_F16,
-                     "down": {"kernel": "k_moe_mma (unit64)" if args.down_unit64 or args.raw_layout else "k_moe_mma_wave16 (tile16)", "kernel_ms": dn_ms, "achieved": dn_bytes / (dn_ms * 1e-3) / 1e9, "mfma_tflops": dn_flops / (dn_ms * 1e-3) / 1e12},
-                     "two_launches": {"gate_up_ms": gu2_ms, "swiglu_ms": sw_ms, "note": "fnx_moe_gate_up_mma (k_moe_mma over the unit64 copy, f32 products written) and fnx_swiglu_h16"},
+                     "down": {"kernel": "k_moe_mma_wave16 (unit64)" if args.down_unit64 or args.raw_layout else "k_moe_mma_wave16 (tile16)", "kernel_ms": dn_ms, "achieved": dn_bytes / (dn_ms * 1e-3) / 1e9, "mfma_tflops": dn_flops / (dn_ms * 1e-3) / 1e12},
+                     "two_launches": {"gate_up_ms": gu2_ms, "swiglu_ms": sw_ms, "note": "fnx_moe_gate_up_mma (k_moe_mma_wave16_pairs over the unit64 copy, f32 products written) and fnx_swiglu_h16"},
                      # the piecewise bound: a launch cannot be faster than its bytes at the HBM peak or its flops at the MFMA peak
                      "piecewise_bound": {"gate_up_us": max(gu_bytes / HBM_PEAK, gu_flops / MFMA_F16) * 1e6,
                                          "gate_up_frac": max(gu_bytes / HBM_PEAK, gu_flops / MFMA_F16) / (gu_ms * 1e-3),

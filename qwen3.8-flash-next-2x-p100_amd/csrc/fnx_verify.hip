@@ -1557,7 +1557,7 @@ int fnx_swiglu_h16(const float* gu, int ffs, int P, uint16_t* h16, void* st) {
     return launch_status("swiglu_h16");
 }
 // A2 (may be null): one more matrix of the same shape and layout with a job list of its own (jobs2, njobs2, cap2), run in
-// the same launch by the wave forms (tile16), else right after
+// the same launch by the wave forms, else right after
 static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const int* njobs, int njobs_cap, const uint16_t* x, float* out,
                       void* st, const char* who, const fnx_dw* A2 = nullptr, const fnx_bigjob* jobs2 = nullptr, const int* njobs2 = nullptr,
                       int cap2 = 0, uint16_t* h16 = nullptr, bool* h16_done = nullptr) {
@@ -1570,8 +1570,10 @@ static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const 
     if (njobs_cap < 1) return fail(std::string(who) + ": no jobs");
     MmaArgs a{(const uint8_t*) A->p, sa, A->ep, A->n_out, A->n_in, jobs, njobs, njobs_cap, x, A->n_in, out};
     const bool tile16 = A->type == FNX_T_IQ3S_TILE16;
-    // the wave forms (tile16) take the second list - the shared expert's matrix - in the same launch
-    const bool merged = A2 && tile16 && A2->p && A2->type == A->type && A2->n_in == A->n_in && A2->n_out == A->n_out;
+    // unit64 rows that the wave forms take: whole units a tile of 16 rows, a lane's sub-blocks of a super-step inside one unit
+    const bool unit64 = A->type == FNX_T_IQ3S_UNIT64 && (A->n_in == 256 || A->n_in == 512 || A->n_in == 1024 || A->n_in % 2048 == 0);
+    // the wave forms take the second list - the shared expert's matrix - in the same launch
+    const bool merged = A2 && (tile16 || unit64) && A2->p && A2->type == A->type && A2->n_in == A->n_in && A2->n_out == A->n_out;
     if (A2 && !merged) {   // two launches
         if (h16_done) *h16_done = false;
         if (!out) return fail(std::string(who) + ": h alone is left by the wave form only (both matrices tile16)");
@@ -1591,26 +1593,38 @@ static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const 
         // wave form for stacked gate|up matrices, which leaves h = silu(gate) * up itself: a wave a (gate tile, up tile) pair over
         // the row's super-steps, one block a CU
         a.h16 = h16;
-        a.ffh = A->n_out / 2;
         if (h16_done) *h16_done = true;
         // eight pairs a block at least, what its waves take a tile each. A grid of a pair a block is better where every job is of a few
         // tokens (one job of 5: 15.8 -> 11.1 us), worse where a short list has large jobs too, whose units then come to lie on fewer
         // of the eight XCDs (four jobs of 64 tokens and four of 3: 37.3 -> 39.0 us, 37.8 -> 40.8 at a feed-forward width of
         // 1,024); the jobs' sizes are not known here
-        const long upj = (a.ffh / 16 + 7) / 8;
+        const long upj = (A->n_out / 32 + 7) / 8;
         const int grid = (int) std::max(1l, std::min<long>(std::min(cu_count(), 64 * W16_PLAN), caps * upj));
-        k_moe_mma_wave16_gu<<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
+        k_moe_mma_wave16_pairs<true, W16Tile16><<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
         return launch_status(who);
     }
     if (!out) return fail(std::string(who) + ": h alone is left by the wave form only (tile16 gate|up, 2 ff rows in 32s)");
-    if (tile16 && A->n_in == W16_COLS) {
-        // wave form: rows of 512 columns (the down projection), a job's whole activation tile in LDS, one block a CU
+    // The forms that decode a job's weights once for all its tokens take unit64 rows too, whatever widths of rows lie whole in its units (the
+    // kernel without them: a wave a task of 32 rows x 32 tokens, each cache line of the planes fetched four times). us a launch, routed and
+    // shared experts' jobs, 2,048 rows a matrix; before (two launches) / now: 256 columns, 512 tokens on some 100 of 512 experts 65 + 11 / 29;
+    // 1,024 columns, 40 tokens on 128 experts 124 + 26 / 41, 512 on some 100 of 512 219 + 27 / 73, 4,096 1,087 + 93 / 378.
+    if ((tile16 && A->n_in == W16_COLS) || (unit64 && A->n_in <= W16_COLS)) {
+        // rows of up to 512 columns (the down projection), a job's whole activation tile in LDS, one block a CU. (As pairs of tiles, below: 64 tokens of
+        // 128 jobs 28 -> 38 us over 512 columns; 512 tokens over 256 columns 111 -> 113 us a chunk)
         const int grid = (int) std::max(1l, std::min<long>((long) cu_count(), caps * (A->n_out / 16)));
-        k_moe_mma_wave16<<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
+        if (tile16) k_moe_mma_wave16<W16Tile16><<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
+        else if (A->n_in == 256) k_moe_mma_wave16<W16Unit64<2>><<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
+        else k_moe_mma_wave16<W16Unit64<4>><<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
+        return launch_status(who);
+    }
+    if (unit64) {   // longer rows: pairs of tiles, super-step by super-step
+        const long upj = (A->n_out / 32 + 7) / 8;   // (as above)
+        const int grid = (int) std::max(1l, std::min<long>(std::min(cu_count(), 64 * W16_PLAN), caps * upj));
+        k_moe_mma_wave16_pairs<false, W16Unit64<4>><<<grid, W16_THREADS, 0, (hipStream_t) st>>>(a);
         return launch_status(who);
     }
     if (tile16) return fail(std::string(who) + ": tile16 matrices are the prompt path's two: stacked gate|up leaving h, and rows of 512 columns");
-    // raw blocks and unit64: a wave a task of 32 rows x 32 tokens
+    // raw blocks, and unit64 rows of other widths: a wave a task of 32 rows x 32 tokens
     static const int per_cu = env_int("FNX_MMA_BLOCKS_PER_CU", 2, 1, 8);
     const long tasks = (long) njobs_cap * (A->n_out / 32) * (MM_TT / MM_TP);
     const int grid = (int) std::max(1l, std::min<long>((long) per_cu * cu_count(), (tasks + MM_WAVES - 1) / MM_WAVES));

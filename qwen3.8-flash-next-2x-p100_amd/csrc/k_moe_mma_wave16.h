@@ -1,4 +1,4 @@
-// The routed experts' down projection on the matrix cores over tile16 matrices of 512 columns, a wave a tile of 16 rows.
+// The routed experts' down projection on the matrix cores over matrices of up to 512 columns (tile16, unit64), a wave a tile of 16 rows.
 //
 // A block that takes one (job, 256 rows) task at a time, its activations staged per step, meets at two barriers a stage:
 // with rows of 512 columns a task is a single stage, the eight waves of such a block meet four times per 32 rows each, and
@@ -55,6 +55,7 @@ __device__ __forceinline__ void w16_half(const uint2* tab, const SubFields& s, i
 }
 // A tile's super-step: the lane's four sub-blocks of its row (fields f) as f16 operands, against the nt token tiles of
 // the activation tile in LDS (xlane: token r's row at this lane group's sub-blocks), added to acc
+template <int PS = 4>
 __device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* xlane, const SuperFields& f, int nt, v4f (&acc)[MB_TP]) {
     // the token tiles two at a time against the sub-block's operands
     auto pair = [&](const v8h (&A)[4], int p, auto t0_tag, auto cnt_tag) {
@@ -98,8 +99,10 @@ __device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* 
     };
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
-    step(std::integral_constant<int, 2>{});
-    step(std::integral_constant<int, 3>{});
+    if constexpr (PS == 4) {
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+    }
 }
 
 // Two tiles' super-steps against the same NT token tiles (fields f0 and f1, sums acc0 and acc1): an operand of the activation
@@ -107,7 +110,7 @@ __device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* 
 // the registers that one tile's whole sub-block takes above. between: run between the second and the third of the four
 // steps, where the first half of the fields is dead (loads of what comes next find registers there). Every sum is
 // accumulated as w16_super_step does it.
-template <int NT, class Between>
+template <int NT, int PS, class Between>
 __device__ __forceinline__ void w16_super_pair(const uint2* tab, const uint8_t* xlane, const SuperFields& f0, const SuperFields& f1, v4f (&acc0)[NT],
                                                v4f (&acc1)[NT], Between between) {
     auto step = [&](auto p_c) {
@@ -132,14 +135,62 @@ __device__ __forceinline__ void w16_super_pair(const uint2* tab, const uint8_t* 
         }
     };
     step(std::integral_constant<int, 0>{});
-    step(std::integral_constant<int, 1>{});
+    if constexpr (PS == 4) step(std::integral_constant<int, 1>{});
     __builtin_amdgcn_sched_barrier(0);
     between();
-    step(std::integral_constant<int, 2>{});
-    step(std::integral_constant<int, 3>{});
+    step(std::integral_constant<int, PS == 4 ? 2 : 1>{});
+    if constexpr (PS == 4) step(std::integral_constant<int, 3>{});
 }
 
+// Where a lane finds its sub-blocks of a tile of 16 rows: PS of them a super-step of 128 PS columns, PS (lane / 16) .. of its row.
+struct W16Tile16 {
+    static constexpr int PS = 4;
+    int nsuper;
+    __device__ __forceinline__ W16Tile16(int ncols) : nsuper(ncols >> 9) {}
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t tiles(const uint8_t* we, int t) const { return tile16_rsrc(we, t, nsuper); }
+    __device__ __forceinline__ SuperFields load(__amdgpu_buffer_rsrc_t m, int S) const { return tile16_load_buf(m, S); }
+};
+// unit64: rows of 256 columns (half a super-step: two sub-blocks a lane), 512, 1,024 or whole 2,048s. A lane's loads are runs of 32 (16), 16 (8),
+// 4 (2), 2 (1) and 2 bytes of its row's planes, a tile's rows in whole units side by side: some more cache lines an instruction than tile16's
+// contiguous planes, at the same speed (512 columns, 64 tokens of 128 jobs 29.0 us against 28.1, 8 tokens of 256 jobs 29.0 against 28.2).
+template <int STEPS>
+struct W16Unit64 {
+    static constexpr int PS = STEPS;
+    int nsuper, tile_bytes, a, b, c, sc, d;
+    __device__ __forceinline__ W16Unit64(int ncols) : nsuper(ncols / (128 * STEPS)), tile_bytes((ncols >> 5) * (UNIT_BYTES / 4)) {
+        const int lane = threadIdx.x & 63, at = (lane & 15) * (ncols >> 5) + STEPS * (lane >> 4), u = (at >> 6) * UNIT_BYTES, l = at & 63;
+        a = u + 8 * l, b = u + UNIT_B_AT + 4 * l, c = u + UNIT_C_AT + l, sc = u + UNIT_SCALES_AT + (l >> 1), d = u + UNIT_D_AT + 2 * (l >> 3);
+    }
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t tiles(const uint8_t* we, int t) const {
+        return __builtin_amdgcn_make_buffer_rsrc((void*) uniform_ptr(we + (size_t) t * tile_bytes), 0, -1, 0x00020000);
+    }
+    __device__ __forceinline__ SuperFields load(__amdgpu_buffer_rsrc_t m, int S) const {
+        SuperFields r;
+        if constexpr (STEPS == 4) {
+            const int u = (S >> 2) * UNIT_BYTES, s = S & 3;   // 16 sub-blocks further in the unit's planes; a unit after four
+            r.a0 = __builtin_amdgcn_raw_buffer_load_b128(m, a, u + 128 * s, 0);
+            r.a1 = __builtin_amdgcn_raw_buffer_load_b128(m, a + 16, u + 128 * s, 0);
+            r.b = __builtin_amdgcn_raw_buffer_load_b128(m, b, u + 64 * s, 0);
+            r.c = __builtin_amdgcn_raw_buffer_load_b32(m, c, u + 16 * s, 0);
+            r.sc = __builtin_amdgcn_raw_buffer_load_b16(m, sc, u + 8 * s, 0);
+            r.d = __builtin_amdgcn_raw_buffer_load_b16(m, d, u + 4 * s, 0);
+        } else {   // (one super-step a row)
+            const v2u h = __builtin_amdgcn_raw_buffer_load_b64(m, b, 0, 0);
+            r.a0 = __builtin_amdgcn_raw_buffer_load_b128(m, a, 0, 0);
+            r.a1 = r.b = v4u{0, 0, 0, 0};
+            r.b.x = h.x, r.b.y = h.y;
+            r.c = __builtin_amdgcn_raw_buffer_load_b16(m, c, 0, 0);
+            r.sc = __builtin_amdgcn_raw_buffer_load_b8(m, sc, 0, 0);
+            r.d = __builtin_amdgcn_raw_buffer_load_b16(m, d, 0, 0);
+        }
+        return r;
+    }
+};
+
+// (rows of one super-step)
+template <class LY>
 __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a) {
+    constexpr int PS = LY::PS;
     // the block's place in the plan: blocks with neighbouring places run on one XCD (workgroups go to the eight XCDs in turn), so
     // the units of one expert, which the plan deals to neighbouring places, find the expert's weights in that XCD's L2
     const unsigned vb = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
@@ -236,7 +287,8 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
     __syncthreads();   // the codebook and the run
     const int jA = uniform(L.first_job), tA = uniform(L.first_tile), jB = uniform(L.last_job), tB = uniform(L.last_tile);
     const uint32_t xt_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) L.xt;
-    const uint8_t* xlane = L.xt + r * W16_XROW + 256 * grp;   // token r of a tile, this lane group's four sub-blocks of a super-step
+    const LY ly(a.ncols);
+    const uint8_t* xlane = L.xt + r * W16_XROW + 64 * PS * grp;   // token r of a tile, this lane group's four sub-blocks of a super-step
     int yahead[MB_TP] = {0, 0, 0, 0}, ahead = -1;
     for (int j = jA; j <= jB && j < njall; ++j) {
         const int g0 = j == jA ? tA : 0, g1 = j == jB ? min(tB, gpj) : gpj;
@@ -253,7 +305,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
         __syncthreads();   // the job before has been read
 #pragma unroll
         for (int i = 0; i < MB_TP; ++i)   // a token's row a wave instruction, 16 bytes a lane
-            if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
+            if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx, 16u * (lane & (16 * PS - 1)), xt_at + (wave + 16 * i) * W16_XROW);
         if (j + 1 <= jB && j + 1 < njall) {
             const int nn = uniform(n_of(j + 1));
             const fnx_bigjob* jn = job_at(j + 1);
@@ -265,7 +317,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
 #pragma unroll
         for (int tt = 0; tt < MB_TP; ++tt) orow[tt] = tt * 16 + r < n ? jb->out[tt * 16 + r] : -1;
         int g = g0 + wave;
-        SuperFields f = tile16_load(we, 16 * min(g, g1 - 1) + r, 0, 1);
+        SuperFields f = ly.load(ly.tiles(we, min(g, g1 - 1)), 0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         // A tile's results go out as buffer stores that every path issues (a lane without a token: past the buffer's end, where
@@ -291,12 +343,12 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
                     case 2: __builtin_amdgcn_s_setprio(2); break;
                     default: __builtin_amdgcn_s_setprio(3); break;
                 }
-                const SuperFields nf = tile16_load(we, 16 * (g + W16_WAVES < g1 ? g + W16_WAVES : g) + r, 0, 1);
+                const SuperFields nf = ly.load(ly.tiles(we, g + W16_WAVES < g1 ? g + W16_WAVES : g), 0);
                 __builtin_amdgcn_sched_barrier(0);   // (left to itself the compiler asks for them behind the products)
                 v4f acc[MB_TP];
 #pragma unroll
                 for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-                w16_super_step(L.tab, xlane, f, ntiles, acc);
+                w16_super_step<PS>(L.tab, xlane, f, ntiles, acc);
                 // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
 #pragma unroll
                 for (int tt = 0; tt < MB_TP; ++tt) {
@@ -316,7 +368,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
     }
 }
 
-// ---------------------------------------------------------------- the same form for stacked gate|up matrices (rows of 512 S columns)
+// ---------------------------------------------------------------- the same form for longer rows (512 S columns): stacked gate|up matrices, and plain ones
 // A job's activations are S tiles of 64 tokens x 512 columns here, and LDS holds one: a block takes units of (job, sixteen
 // gate tiles and the sixteen up tiles that go with them), a wave one such pair, and walks the S super-steps with the
 // pair's accumulators in registers - activation tile S in (two barriers), the gate tile's and the up tile's super-steps
@@ -357,7 +409,11 @@ struct Wave16GuLds {
     unsigned short ph_job[16];
     unsigned char ph_first[16];                           // a job's first place in LDS
 };
-__global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs a) {
+// GU: stacked gate|up matrices, a pair = 16 gate rows and the 16 up rows that go with them, h = silu(gate) * up out as f16; else any matrix, a pair = two
+// tiles side by side, the products out as f32 rows.
+template <bool GU, class LY>
+__global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_pairs(const MmaArgs a) {
+    constexpr int PS = LY::PS;
     // the block's place in the plan: blocks with neighbouring places run on one XCD (workgroups go to the eight XCDs in turn), so
     // the units of one expert, which the plan deals to neighbouring places, find the expert's weights in that XCD's L2
     const unsigned vb = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
@@ -394,7 +450,8 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     }
     if (tid < held2) L.jn[1][tid] = (uint8_t) max(0, min(FNX_PF_JOB, hn2));
     for (int j = tid + W16_THREADS; j < held2; j += W16_THREADS) L.jn[1][j] = (uint8_t) max(0, min(FNX_PF_JOB, a.jobs2[j].n));
-    const int ffh = a.ffh, nsuper = a.ncols >> 9, ppj = ffh >> 4;                      // pairs of tiles a job
+    const LY ly(a.ncols);
+    const int nsuper = ly.nsuper, ppj = a.nrows >> 5;                                   // pairs of tiles a job
     const int upj = (ppj + W16_WAVES - 1) / W16_WAVES;                                  // heavy units a job
     auto job_at = [&](int j) { return j < nj ? a.jobs + j : a.jobs2 + (j - nj); };
     auto n_of = [&](int j) {
@@ -488,7 +545,21 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     }
     __syncthreads();   // the codebook, the order and the plan
     const uint32_t xt_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) L.xt;
-    const uint8_t* xlane = L.xt + r * W16_XROW + 256 * grp;
+    const uint8_t* xlane = L.xt + r * W16_XROW + 64 * PS * grp;
+    const uint32_t xl16 = 16u * (lane & (16 * PS - 1));   // a lane's 16 bytes of a row's super-step
+    auto first_tile = [&](int pr) { return GU ? pr : 2 * pr; };   // a pair's two tiles
+    auto second_tile = [&](int pr) { return GU ? ppj + pr : 2 * pr + 1; };
+    auto put = [&](int orow, int pr, v4f gt, v4f up) {   // lane: a token's rows 4 grp .. 4 grp + 3 of the pair's tiles
+        if constexpr (GU) {
+            uint2 hv;
+            hv.x = h16_pair(silu_f(gt.x), up.x, silu_f(gt.y), up.y), hv.y = h16_pair(silu_f(gt.z), up.z, silu_f(gt.w), up.w);
+            *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * (a.nrows >> 1) + 16 * pr + 4 * grp) = hv;
+        } else {
+            float* o = a.out + (size_t) orow * a.nrows + 32 * pr + 4 * grp;
+            *reinterpret_cast<float4*>(o) = make_float4(gt.x, gt.y, gt.z, gt.w);
+            *reinterpret_cast<float4*>(o + 16) = make_float4(up.x, up.y, up.z, up.w);
+        }
+    };
     const int G = gridDim.x;
     int tot[MB_TP + 1] = {0, 0, 0, 0, 0};
     if (sorted) {
@@ -540,8 +611,8 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
     // ---- the heavy units: sixteen pairs of tiles, a pair a wave
     auto heavy = [&](auto nt_tag, const fnx_bigjob* jb, int n, const uint8_t* we, int pr) {
         constexpr int NT = decltype(nt_tag)::value;
-        const bool mine = pr < ppj;   // the wave's pair: gate rows 16 pr .., up rows ffh + 16 pr ..
-        const __amdgpu_buffer_rsrc_t mg = tile16_rsrc(we, min(pr, ppj - 1), nsuper), mu = tile16_rsrc(we, ppj + min(pr, ppj - 1), nsuper);
+        const bool mine = pr < ppj;
+        const __amdgpu_buffer_rsrc_t mg = ly.tiles(we, first_tile(min(pr, ppj - 1))), mu = ly.tiles(we, second_tile(min(pr, ppj - 1)));
         const int oput = tid < n ? jb->out[tid] : -1;   // (up to 64 tokens: the first wave)
         int y[NT];   // the wave's tokens' rows: tokens wave, wave + 16, .. (past the job's last: that one again)
 #pragma unroll
@@ -549,31 +620,26 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         v4f accg[NT], accu[NT];
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) accg[tt] = accu[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-        SuperFields f = tile16_load_buf(mg, 0), fu = tile16_load_buf(mu, 0);
+        SuperFields f = ly.load(mg, 0), fu = ly.load(mu, 0);
         for (int S = 0; S < nsuper; ++S) {
             __syncthreads();   // the tile before has been read
             if (S == 0 && tid < FNX_PF_JOB) L.orow[tid] = oput;
 #pragma unroll
-            for (int i = 0; i < NT; ++i)   // a token's 512 columns a wave instruction, 16 bytes a lane
-                lds_load16(a.x + (size_t) y[i] * a.ldx + 512 * S, 16u * lane, xt_at + (wave + 16 * i) * W16_XROW);
+            for (int i = 0; i < NT; ++i)   // a token's super-step a wave instruction, 16 bytes a lane
+                lds_load16(a.x + (size_t) y[i] * a.ldx + 128 * PS * S, xl16, xt_at + (wave + 16 * i) * W16_XROW);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             turn(S);
             const int Sn = min(S + 1, nsuper - 1);
             SuperFields nf, nfu;
-            w16_super_pair<NT>(L.tab, xlane, f, fu, accg, accu, [&] { nf = tile16_load_buf(mg, Sn), nfu = tile16_load_buf(mu, Sn); });
+            w16_super_pair<NT, PS>(L.tab, xlane, f, fu, accg, accu, [&] { nf = ly.load(mg, Sn), nfu = ly.load(mu, Sn); });
             f = nf, fu = nfu;
         }
         // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the pair's tiles
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) {
             const int orow = mine ? L.orow[tt * 16 + r] : -1;
-            if (orow >= 0) {
-                const v4f gt = accg[tt], up = accu[tt];
-                uint2 hv;
-                hv.x = h16_pair(silu_f(gt.x), up.x, silu_f(gt.y), up.y), hv.y = h16_pair(silu_f(gt.z), up.z, silu_f(gt.w), up.w);
-                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
-            }
+            if (orow >= 0) put(orow, pr, accg[tt], accu[tt]);
         }
     };
     for (int round = 0; round * G < nb; ++round) {
@@ -618,7 +684,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         if (wave < tokens) {   // a place a wave: the job it belongs to is the last one that begins at or before it
             const int k = __popcll(__ballot(lane < jobs && (int) L.ph_first[lane & 15] <= wave)) - 1;
             const int y = uniform(job_at((int) L.ph_job[k])->y[wave - (int) L.ph_first[k]]);
-            for (int S = 0; S < nsuper; ++S) lds_load16(a.x + (size_t) y * a.ldx + 512 * S, 16u * lane, xt_at + (16 * S + wave) * W16_XROW);
+            for (int S = 0; S < nsuper; ++S) lds_load16(a.x + (size_t) y * a.ldx + 128 * PS * S, xl16, xt_at + (16 * S + wave) * W16_XROW);
         }
         if (pe - p0 <= W16_WAVES / 2) {   // pairs for half of the waves: a wave a tile, the up tiles' sums go over to the gate tiles' waves
             constexpr int HALF = W16_WAVES / 2;
@@ -626,26 +692,23 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
             const int k = jo - jo0, j = uniform((int) L.ph_job[k]), at = uniform((int) L.ph_first[k]);
             const fnx_bigjob* jb = job_at(j);
             const int orow = q < pe && !up && r < n_of(j) ? jb->out[r] : -1;
-            const __amdgpu_buffer_rsrc_t m = tile16_rsrc(matrix_of(j, jb), up * ppj + pr, nsuper);
-            SuperFields f = tile16_load_buf(m, 0);
+            const __amdgpu_buffer_rsrc_t m = ly.tiles(matrix_of(j, jb), up ? second_tile(pr) : first_tile(pr));
+            SuperFields f = ly.load(m, 0);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             v4f acc[MB_TP] = {};
-            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 256 * grp;
+            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 64 * PS * grp;
             for (int S = 0; S < nsuper && q < pe; ++S) {
                 turn(S);
-                const SuperFields nf = tile16_load_buf(m, min(S + 1, nsuper - 1));
-                w16_super_step(L.tab, xk + S * 16 * W16_XROW, f, 1, acc);
+                const SuperFields nf = ly.load(m, min(S + 1, nsuper - 1));
+                w16_super_step<PS>(L.tab, xk + S * 16 * W16_XROW, f, 1, acc);
                 f = nf;
             }
             if (up) L.xs[wave % HALF][lane] = make_float4(acc[0].x, acc[0].y, acc[0].z, acc[0].w);
             __syncthreads();
             if (orow >= 0) {
                 const float4 ut = L.xs[wave % HALF][lane];
-                const v4f gt = acc[0];
-                uint2 hv;
-                hv.x = h16_pair(silu_f(gt.x), ut.x, silu_f(gt.y), ut.y), hv.y = h16_pair(silu_f(gt.z), ut.z, silu_f(gt.w), ut.w);
-                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
+                put(orow, pr, acc[0], v4f{ut.x, ut.y, ut.z, ut.w});
             }
             p0 = pe;
             continue;
@@ -656,10 +719,10 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
         auto tiles_of = [&](int q) {
             const int jo = q / ppj, pr = q - jo * ppj, j = uniform((int) L.ph_job[jo - jo0]);
             const uint8_t* we = matrix_of(j, job_at(j));
-            mg = tile16_rsrc(we, pr, nsuper), mu = tile16_rsrc(we, ppj + pr, nsuper);
+            mg = ly.tiles(we, first_tile(pr)), mu = ly.tiles(we, second_tile(pr));
         };
         tiles_of(min(p, pe - 1));
-        SuperFields f = tile16_load_buf(mg, 0), fu = tile16_load_buf(mu, 0);
+        SuperFields f = ly.load(mg, 0), fu = ly.load(mu, 0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         while (p < pe) {
@@ -669,24 +732,19 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_gu(const MmaArgs
             const int jo = p / ppj, pr = p - jo * ppj, k = jo - jo0, j = uniform((int) L.ph_job[k]), at = uniform((int) L.ph_first[k]);
             const fnx_bigjob* jb = job_at(j);
             const int orow = r < n_of(j) ? jb->out[r] : -1;
-            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 256 * grp;   // (a lane without a token: some place's values, its sums not kept)
+            const uint8_t* xk = L.xt + min(at + r, 15) * W16_XROW + 64 * PS * grp;   // (a lane without a token: some place's values, its sums not kept)
             v4f accg[1] = {v4f{0.f, 0.f, 0.f, 0.f}}, accu[1] = {v4f{0.f, 0.f, 0.f, 0.f}};
             for (int S = 0; S < nsuper; ++S) {
                 turn(S);
                 SuperFields nf, nfu;
-                w16_super_pair<1>(L.tab, xk + S * 16 * W16_XROW, f, fu, accg, accu, [&] {
+                w16_super_pair<1, PS>(L.tab, xk + S * 16 * W16_XROW, f, fu, accg, accu, [&] {
                     if (S + 1 == nsuper) tiles_of(min(pn, pe - 1));
                     const int Sn = S + 1 < nsuper ? S + 1 : 0;
-                    nf = tile16_load_buf(mg, Sn), nfu = tile16_load_buf(mu, Sn);
+                    nf = ly.load(mg, Sn), nfu = ly.load(mu, Sn);
                 });
                 f = nf, fu = nfu;
             }
-            if (orow >= 0) {
-                const v4f gt = accg[0], up = accu[0];
-                uint2 hv;
-                hv.x = h16_pair(silu_f(gt.x), up.x, silu_f(gt.y), up.y), hv.y = h16_pair(silu_f(gt.z), up.z, silu_f(gt.w), up.w);
-                *reinterpret_cast<uint2*>(a.h16 + (size_t) orow * ffh + 16 * pr + 4 * grp) = hv;
-            }
+            if (orow >= 0) put(orow, pr, accg[0], accu[0]);
             p = pn;
         }
         p0 = pe;

@@ -573,11 +573,9 @@ struct MmaArgs {
     const fnx_bigjob* jobs2 = nullptr;
     const int* njobs2 = nullptr;
     int cap2 = 0;
-    // wave form, stacked gate|up matrices (nrows = 2 ffh, ffh in 16s): a wave's two tiles are 16 gate rows and the
-    // 16 up rows that go with them, and what is written is h = silu(gate) * up as f16 rows of ffh (k_swiglu_h16's values)
-    // instead of the products themselves
+    // wave form, stacked gate|up matrices: a wave's two tiles are 16 gate rows and the 16 up rows that go with them, and
+    // what is written is h = silu(gate) * up as f16 rows of nrows / 2 (k_swiglu_h16's values) instead of the products themselves
     uint16_t* h16 = nullptr;
-    int ffh = 0;
 };
 constexpr int MM_THREADS = 512, MM_WAVES = MM_THREADS / 64, MM_TT = FNX_PF_JOB / 16;
 
@@ -736,7 +734,7 @@ __global__ void __launch_bounds__(MM_THREADS) __attribute__((amdgpu_waves_per_eu
 }
 
 // ---------------------------------------------------------------- a lane's four consecutive sub-blocks of a row
-// What limits the wave-a-task kernel above on MI355X is the vector-memory front end: every wave gathers its weights 32
+// What limits the wave-a-task kernel above (what is left to it: raw blocks, and unit64 rows of widths that are not 256, 512, 1,024 or whole 2,048s) on MI355X is the vector-memory front end: every wave gathers its weights 32
 // bytes per row at a time, so each cache line is fetched four times. A lane that owns four consecutive sub-blocks of its
 // row per super-step of 512 columns (sub-block 16 S + 4 g + p at step p) loads whole 32/16/4/2-byte runs of the planes,
 // 6 loads per row and super-step, each line of a plane touched once: the loads of the tile16 re-laying below and of the

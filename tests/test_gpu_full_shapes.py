@@ -237,8 +237,8 @@ def config5_inputs(rng, n, ff, nexp, Cn, zipf):
     return router, gu, down, sh_gu, sh_down, x
 
 
-# unit64: every matrix in the verify path's layout (k_moe_mma, a wave a task); tile16: the prompt path's own
-# copies of gate|up and down, the layout the benchmark's prefill workload times (k_moe_mma_wave16_gu, k_moe_mma_wave16)
+# unit64: every matrix in the verify path's layout (k_moe_mma_wave16_pairs leaving the products, k_moe_mma_wave16); tile16: the prompt path's own
+# copies of gate|up and down, the layout the benchmark's prefill workload times (k_moe_mma_wave16_pairs, k_moe_mma_wave16)
 @pytest.mark.parametrize("layout", ["unit64", "tile16"])
 def test_config5_chunk_of_512_rows(dev, oracle, layout):
     n, ff, nexp, topk, Cn = 2048, 512, 512, 10, 512

@@ -173,12 +173,42 @@ def test_moe_mma_wave_form_tile16_rows_of_512(dev, oracle, nrows, nexp, sizes):
     x16 = rng.standard_normal((rows, ncols)).astype(np.float16)
     jobs, total = make_jobs(rng, nexp, rows, sizes)
     got = dev.moe_mma(w, stride, nrows, ncols, jobs, x16, total, packed=True, down=True, cap=len(jobs) + 5, tile16=True)
-    other = dev.moe_mma(w, stride, nrows, ncols, jobs, x16, total, packed=True, down=True, cap=len(jobs) + 5)   # the wave-a-task kernel over unit64
+    other = dev.moe_mma(w, stride, nrows, ncols, jobs, x16, total, packed=True, down=True, cap=len(jobs) + 5)   # the same form over unit64
     assert rel_l2(got, other) <= 1e-6, "the same f16 products: only the summation order differs"
     assert np.array_equal(got == 0, other == 0)   # (rows no job writes stay as they were)
     if len(sizes) <= 8:
         want = oracle.moe_mma(w, stride, nrows, ncols, jobs, PF, x16, total)
         assert rel_l2(got, want) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
+
+
+@pytest.mark.parametrize("nrows,ncols,sizes", [
+    (2048, 256, [64, 1, 17, 0, 16, 33, 48, 5, 64, 49] * 4), (32, 256, [3]), (64, 256, [9, 64, 31]),    # half a super-step a row: a job's whole tile in LDS
+    (2048, 512, [64, 1, 17, 0, 16, 33, 48, 5, 64, 49] * 4), (96, 512, [16, 2, 64]),                    # one super-step, the same form
+    (2048, 1024, [64, 1, 17, 0, 16, 33, 48, 5, 64, 49] * 4), (32, 1024, [5]), (96, 1024, [7, 40, 64]), # two, pairs of tiles: light lists, heavy units
+    (1024, 2048, [2, 3, 1] * 100), (64, 4096, [64, 12, 20, 16]), (64, 6144, [3, 33]),                  # a unit a row, two and three
+    (64, 768, [64, 1, 17, 33]), (32, 1536, [9, 48]), (64, 1280, [5, 64])])                             # rows that no wave form takes
+def test_moe_mma_over_unit64_rows(dev, oracle, nrows, ncols, sizes):
+    """every form that unit64 rows of a width go to: against the oracle, and a row's bits do not depend on what else the list holds"""
+    print(f"case moe_mma unit64 nrows={nrows} ncols={ncols} jobs={len(sizes)}", flush=True)
+    rng = np.random.default_rng(751 + nrows + ncols + len(sizes))
+    nexp = 3
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, nexp * nrows * ncols // 256, dmax=2e-2)
+    x16 = rng.standard_normal((200, ncols)).astype(np.float16)
+    jobs, total = make_jobs(rng, nexp, 200, sizes)
+
+    def out_of(some):
+        return dev.moe_mma(w, stride, nrows, ncols, some, x16, total + 2, packed=True, down=True, cap=len(some) + 3)
+
+    got = out_of(jobs)
+    assert not np.any(got[total:]), "rows no job writes stay as they were"
+    few = jobs if len(jobs) <= 12 else jobs[:10]
+    n = sum(sizes[:len(few)])
+    want = oracle.moe_mma(w, stride, nrows, ncols, few, PF, x16, total + 2)
+    assert rel_l2(got[:n], want[:n]) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
+    for j in {0, len(jobs) // 2, len(jobs) - 1}:
+        at = jobs[j][2 + PF:2 + PF + int(jobs[j][1])]
+        assert np.array_equal(got[at].view(np.uint32), out_of(jobs[j:j + 1])[at].view(np.uint32)), f"job {j} of {jobs[j][1]} rows"
 
 
 # More than 524,288 columns of all rows (on 256 CUs): a thread of the combine takes four columns, unless the rows are no whole
@@ -465,7 +495,7 @@ def test_prefill_layer_matches_oracle(dev, oracle, n, ff, nexp, topk, Cn):
 @pytest.mark.parametrize("n,ff,nexp,topk,Cn", [(2048, 512, 48, 10, 300), (1024, 256, 8, 2, 70)])
 def test_prefill_layer_tile16_equals_unit64(dev, oracle, n, ff, nexp, topk, Cn):
     """the gate|up matrices (and the down matrices, where ff comes in 512s) in the prompt path's own layout: the same f16
-    weights and activations as the unit64 layout's kernel, whose tasks add a row's products up in another order, so h and the
+    weights and activations as the unit64 layout's kernels; h and the
     chunk's result agree to float rounding (and with the oracle's within the bar either way)"""
     print(f"case prefill_layer tile16 n={n} ff={ff} nexp={nexp} topk={topk} C={Cn}", flush=True)
     rng = np.random.default_rng(760 + nexp)
