@@ -969,8 +969,13 @@ static int rows_launch(const fnx_dw* W, size_t w_stride, const fnx_job* jobs, co
         const long items = (long) njobs_max * (W->n_out / JM_ROWS);
         const long most = blocks ? blocks : cu_count();
         // a group of 16 rows a block, or blocks that stream (where the line lies: at the first kernel)
-        if (items <= most || (njobs_max > 1 && items % most && items < 3 * most)) k_iq3s_jobs_mma_one<<<(int) items, JM_THREADS, 0, s>>>(a);
+        if (items <= most || (njobs_max > 1 && items % most && items < 3 * most)) k_iq3s_jobs_mma_one<64><<<(int) items, JM_THREADS, 0, s>>>(a);
         else k_iq3s_jobs_mma<<<(int) most, JM_THREADS, 0, s>>>(a);
+    } else if (const long items = (long) njobs_max * ((units / njobs_max + 15) / 16);   // sixteen units a block (where the line lies: at the kernel)
+               packed && jobs_mma && wide && y && !blocks && W->n_out % JM_ROWS == 0 && items <= 2 * cu_count()) {
+        if (sbr == 8) k_iq3s_jobs_mma_one<8><<<(int) items, JM_THREADS, 0, s>>>(a);
+        else if (sbr == 32) k_iq3s_jobs_mma_one<32><<<(int) items, JM_THREADS, 0, s>>>(a);
+        else k_iq3s_jobs_mma_one<16><<<(int) items, JM_THREADS, 0, s>>>(a);
     } else if (!whole_units) k_iq3s_jobs_any<<<dim3((W->n_out + 3) / 4, njobs_max), 256, 0, s>>>(a);
     else if (packed && wide) FNX_ROWS_SBR(true, true);
     else if (packed) FNX_ROWS_SBR(false, true);

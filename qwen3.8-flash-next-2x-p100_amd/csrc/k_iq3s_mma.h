@@ -33,12 +33,13 @@ struct JmLds {
     __attribute__((aligned(16))) float sw[JM_NI][64][JM_SLD];   // [sub-block][row]: d (1 + 2 s), exact in f32 (11 + 5 bits): a lane's four rows are one 16-byte read
     __attribute__((aligned(16))) float red[JM_NI][JM_WAVES][64][4];
 };
-struct JmOneLds {   // for one group of 16 rows: 71 KB, two blocks a CU
+template <int SBR>
+struct JmOneLds {   // for one group of 16 units: 71 to 74 KB, two blocks a CU
     union {
         uint32_t tab[SGRID_WORDS];
         __attribute__((aligned(16))) float red[1][JM_WAVES][64][4];   // (when every row has been decoded)
     };
-    __attribute__((aligned(16))) uint8_t tile[1][JM_ROWS * JM_ROWLD];
+    __attribute__((aligned(16))) uint8_t tile[1][JM_ROWS * (64 / SBR) * (32 * SBR + 32)];
     __attribute__((aligned(16))) float sw[1][64][JM_SLD];
 };
 
@@ -47,8 +48,9 @@ struct JmOneLds {   // for one group of 16 rows: 71 KB, two blocks a CU
 // memory each
 struct JmActs {
     uint32_t lo[4], hi[4], dh[4];
+    template <int SBR = 64>
     __device__ __forceinline__ void load(const uint8_t* __restrict__ y, int yi, bool on, int sb0, int kg) {
-        const uint8_t* yr = y + ((size_t) (on ? yi : uniform(yi)) * 64 + sb0) * FNX_Q8_1_BLOCK;
+        const uint8_t* yr = y + ((size_t) (on ? yi : uniform(yi)) * SBR + sb0) * FNX_Q8_1_BLOCK;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const uint8_t* yb = yr + s * FNX_Q8_1_BLOCK;
@@ -58,8 +60,8 @@ struct JmActs {
         }
     }
 };
-// 1. this wave's row of group i: 32 int8 weights a lane
-template <class Lds>
+// 1. this wave's unit of group i: 32 int8 weights a lane (SBR sub-blocks a row: row wave of the group, or its 64 / SBR rows from there on)
+template <int SBR = 64, class Lds>
 __device__ __forceinline__ void jm_decode(Lds& L, int i, int wave, int lane, const PackedSub& cur) {
     v4u lo, hi;
 #pragma unroll
@@ -67,21 +69,22 @@ __device__ __forceinline__ void jm_decode(Lds& L, int i, int wave, int lane, con
         lo[j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(L.tab) + packed_addr(cur.idx, j));
         hi[j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(L.tab) + packed_addr(cur.idx, 4 + j));
     }
-    uint8_t* dst = L.tile[i] + wave * JM_ROWLD + lane * 32;
+    const int row = wave * (64 / SBR) + lane / SBR, sb = lane % SBR;
+    uint8_t* dst = L.tile[i] + row * (32 * SBR + 32) + sb * 32;
     *reinterpret_cast<v4u*>(dst) = lo;
     *reinterpret_cast<v4u*>(dst + 16) = hi;
-    L.sw[i][lane][wave] = half_bits_to_float(cur.d) * (float) (int) (1u + 2u * ((cur.sc >> (4 * (lane & 1))) & 0xFu));
+    L.sw[i][row / JM_ROWS * SBR + sb][row % JM_ROWS] = half_bits_to_float(cur.d) * (float) (int) (1u + 2u * ((cur.sc >> (4 * (lane & 1))) & 0xFu));
 }
-// 2. this wave's four sub-blocks of group i's 16 rows against the tokens
-template <class Lds>
+// 2. this wave's four sub-blocks of group i's 16 rows against the tokens (shorter rows: of the 16 rows that SBR / 4 waves share)
+template <int SBR = 64, class Lds>
 __device__ __forceinline__ void jm_multiply(Lds& L, int i, int wave, int lane, const JmActs& x, const float (&dx)[4]) {
     const int col = lane & 15, kg = lane >> 4;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const int sb = 4 * wave + s;
-        const long a = *reinterpret_cast<const long*>(L.tile[i] + col * JM_ROWLD + sb * 32 + 8 * kg);
-        const float4 f = *reinterpret_cast<const float4*>(&L.sw[i][sb][4 * kg]);
+        const int rg = wave / (SBR / 4), sb = 4 * (wave % (SBR / 4)) + s;
+        const long a = *reinterpret_cast<const long*>(L.tile[i] + (JM_ROWS * rg + col) * (32 * SBR + 32) + sb * 32 + 8 * kg);
+        const float4 f = *reinterpret_cast<const float4*>(&L.sw[i][rg * SBR + sb][4 * kg]);
         const long xb = (long) ((unsigned long) x.lo[s] | (unsigned long) x.hi[s] << 32);
         const jm_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, xb, jm_v4i{0, 0, 0, 0}, 0, 0, 0);
         // a term is d_w (1 + 2 s) d_x sumi: the reference's (d_w d_x) (float) (sumi (1 + 2 s)) with the factors taken in another order
@@ -92,13 +95,13 @@ __device__ __forceinline__ void jm_multiply(Lds& L, int i, int wave, int lane, c
     }
     *reinterpret_cast<float4*>(L.red[i][wave][lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
 }
-// 3. one wave adds group i's sums of the sixteen in wave order and stores the tile
-template <class Lds>
-__device__ __forceinline__ void jm_store(const Lds& L, int i, int lane, float* op) {
-    float4 z = *reinterpret_cast<const float4*>(L.red[i][0][lane]);
+// 3. one wave adds group i's sums of the sixteen (shorter rows: of the SBR / 4 from wave w0 on) in wave order and stores the tile
+template <int SBR = 64, class Lds>
+__device__ __forceinline__ void jm_store(const Lds& L, int i, int lane, float* op, int w0 = 0) {
+    float4 z = *reinterpret_cast<const float4*>(L.red[i][w0][lane]);
 #pragma unroll
-    for (int w = 1; w < JM_WAVES; ++w) {
-        const float4 p = *reinterpret_cast<const float4*>(L.red[i][w][lane]);
+    for (int w = 1; w < SBR / 4; ++w) {
+        const float4 p = *reinterpret_cast<const float4*>(L.red[i][w0 + w][lane]);
         z.x += p.x, z.y += p.y, z.z += p.z, z.w += p.w;
     }
     op[0] = z.x, op[1] = z.y, op[2] = z.z, op[3] = z.w;
@@ -148,19 +151,20 @@ __device__ __forceinline__ void jm_segment(JmLds& L, const uint8_t* __restrict__
     }
 }
 
-// 16 rows of a matrix against the job's tokens, and nothing after them: a wave decodes one row, no ring and no second group. The sums are
+// 16 units of a matrix of nunits (16 rows, or 64 / SBR times as many shorter ones) against the job's tokens, and nothing after them: a wave
+// decodes one, no ring and no second group. Past the last unit: that one again, its rows not stored. Over rows of 2,048 columns the sums are
 // jm_segment's, bit for bit.
-template <class Between>
-__device__ __forceinline__ void jm_group(JmOneLds& L, const uint8_t* __restrict__ we, int g, const fnx_job* jb, int n, const uint8_t* __restrict__ y,
+template <int SBR, class Between>
+__device__ __forceinline__ void jm_group(JmOneLds<SBR>& L, const uint8_t* __restrict__ we, int g, int nunits, const fnx_job* jb, int n, const uint8_t* __restrict__ y,
                                          float* __restrict__ out, int out_stride, Between between) {
     const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6));
     const int col = lane & 15, kg = lane >> 4;
     const int yi = jb->y[col], oi = jb->out[col];
-    const PackedSub cur = load_packed_buf(matrix_rsrc(we), (JM_ROWS * g + wave) * UNIT_BYTES, packed_voffs(lane));
+    const PackedSub cur = load_packed_buf(matrix_rsrc(we), min(16 * g + wave, nunits - 1) * UNIT_BYTES, packed_voffs(lane));
     JmActs x;
-    x.load(y, yi, col < n, 4 * wave, kg);
+    x.load<SBR>(y, yi, col < n, 4 * (wave % (SBR / 4)), kg);
     between();
-    jm_decode(L, 0, wave, lane, cur);
+    jm_decode<SBR>(L, 0, wave, lane, cur);
     __syncthreads();   // the rows are in LDS
     float dx[4];
 #pragma unroll
@@ -168,9 +172,10 @@ __device__ __forceinline__ void jm_group(JmOneLds& L, const uint8_t* __restrict_
         asm volatile("" : "+v"(x.dh[s]));   // (converted here: before, the decode would wait for the activations)
         dx[s] = half_bits_to_float(x.dh[s]);
     }
-    jm_multiply(L, 0, wave, lane, x, dx);
+    jm_multiply<SBR>(L, 0, wave, lane, x, dx);
     __syncthreads();   // the waves' sums are in LDS
-    if (wave == 0 && col < n) jm_store(L, 0, lane, out + (size_t) oi * out_stride + 4 * kg + JM_ROWS * g);
+    const int row = JM_ROWS * (64 / SBR * g + wave / (SBR / 4)) + 4 * kg;
+    if (wave % (SBR / 4) == 0 && col < n && row < 64 / SBR * nunits) jm_store<SBR>(L, 0, lane, out + (size_t) oi * out_stride + row, wave);
 }
 
 // units [u0, u1) of matrix `we` for a job of one row: the block's waves share them, each a contiguous run. between(): as in jm_segment
@@ -190,7 +195,7 @@ __device__ __forceinline__ void jm_narrow(const uint32_t* tab, const uint8_t* we
 // alone: the lone mat-vec). There is nothing to stream: the time is the launch and the trips to memory one after the other, so the rows
 // and the activations are asked for before the codebook is written to LDS (between() does that, and meets), and only the U rows are
 // decoded - the loop above decodes four, asks for four more, and with sixteen waves a CU that was a third of the launch.
-template <int U, class Between>
+template <int U, int SBR = 64, class Between>
 __device__ __forceinline__ void jm_few(const uint32_t* tab, const uint8_t* we, int u0, int u1, int yi, int oi, const uint8_t* y, float* out, int out_stride,
                                        Between between) {
     const int lane = threadIdx.x & 63, wave = uniform((int) (threadIdx.x >> 6)), ua = u0 + wave * U;
@@ -198,7 +203,7 @@ __device__ __forceinline__ void jm_few(const uint32_t* tab, const uint8_t* we, i
     PackedSub cur[U];
 #pragma unroll
     for (int r = 0; r < U; ++r) cur[r] = load_packed(as_global(uniform_ptr(we + (size_t) min(ua + r, u1 - 1) * UNIT_BYTES)), o);
-    const uint8_t* yb = y + ((size_t) yi * 64 + lane) * FNX_Q8_1_BLOCK;
+    const uint8_t* yb = y + ((size_t) yi * SBR + lane % SBR) * FNX_Q8_1_BLOCK;
     int xs[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) xs[j] = reinterpret_cast<const int*>(yb + 4)[j];
@@ -221,9 +226,42 @@ __device__ __forceinline__ void jm_few(const uint32_t* tab, const uint8_t* we, i
     } else {
 #pragma unroll
         for (int r = 0; r < U; ++r) {
-            const float z = butterfly_sum<64>(v[r]);
-            if (lane == 63 && ua + r < u1) orow[ua + r] = z;
+            const float z = butterfly_sum<SBR>(v[r]);
+            if (lane % SBR == SBR - 1 && ua + r < u1) orow[(size_t) (ua + r) * (64 / SBR) + lane / SBR] = z;
         }
+    }
+}
+
+// A unit a wave against two rows of activations, over rows of SBR < 64 sub-blocks: no trip of the decoded weights through LDS and no second meeting
+// (9,600 rows of 1,024 columns, two rows, with their quantisation: 8.9 us by jm_group, 7.6 here, 8.5 before)
+template <int SBR, class Between>
+__device__ __forceinline__ void jm_two(const uint32_t* tab, const uint8_t* we, int u, int nunits, const fnx_job* jb, const uint8_t* y, float* out, int out_stride,
+                                       Between between) {
+    const int lane = threadIdx.x & 63, y0 = uniform(jb->y[0]), y1 = uniform(jb->y[1]), o0 = uniform(jb->out[0]), o1 = uniform(jb->out[1]);
+    const PackedSub cur = load_packed(as_global(uniform_ptr(we + (size_t) min(u, nunits - 1) * UNIT_BYTES)), packed_offs(lane));
+    int xs[2][8];
+    float dx[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const uint8_t* yb = y + ((size_t) (t ? y1 : y0) * SBR + lane % SBR) * FNX_Q8_1_BLOCK;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xs[t][j] = reinterpret_cast<const int*>(yb + 4)[j];
+        dx[t] = half_bits_to_float(*reinterpret_cast<const unsigned short*>(yb));
+    }
+    between();
+    int sum[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int w4 = *reinterpret_cast<const int*>(reinterpret_cast<const uint8_t*>(tab) + packed_addr(cur.idx, j));
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sum[t] = __builtin_amdgcn_sdot4(w4, xs[t][j], sum[t], false);
+    }
+    const float dw = half_bits_to_float(cur.d);
+    const int sc = 1 + 2 * (int) ((cur.sc >> (4 * (lane & 1))) & 0xFu);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const float z = butterfly_sum<SBR>((dw * dx[t]) * (float) __mul24(sum[t], sc));
+        if (lane % SBR == SBR - 1 && u < nunits) out[(size_t) (t ? o1 : o0) * out_stride + u * (64 / SBR) + lane / SBR] = z;
     }
 }
 
@@ -234,11 +272,17 @@ __device__ __forceinline__ void jm_few(const uint32_t* tab, const uint8_t* we, i
 // Over weights nobody has read lately, us (streaming / this), jobs of 1 row, 2, 5, 16: 4,096 rows, one job 4.4 / 3.8, 7.7 / 5.9, 8.0 / 6.4,
 // 9.5 / 7.7; 1,024 rows, five jobs 8.1 / 4.5, 11.8 / 7.5, 12.6 / 8.2, 15.6 / 11.5; ten 8.6 / 6.1, 12.3 / 10.2, 13.1 / 11.2, 16.4 / 15.7. Not for the
 // others: every block fetches its job's activations, 8,192 rows, sixteen rows of one job 9.7 / 11.7; 1,024 rows, twenty jobs 19.4 / 24.1.
+// SBR < 64: a mat-vec call of up to eight jobs over shorter rows, 16 64 / SBR of them a block. The vector-ALU kernel that took them loads and
+// decodes a weight once for every two rows of a job, or four. Us a call with its quantisation, before / now, jobs of 1 row, 5, 16: 8,192
+// rows of 512 columns 8.5 / 6.8, 11.0 / 7.4, 15.8 / 8.4, of 1,024 columns 8.3 / 7.1, 11.4 / 7.9, 17.6 / 9.4; two blocks on some CUs: 12,288
+// rows of 1,024 columns 7.9 / 7.4, 11.4 / 9.8, 18.0 / 13.6. Past two blocks a CU the streaming kernel's runs stay.
+template <int SBR>
 __global__ void __launch_bounds__(JM_THREADS) k_iq3s_jobs_mma_one(const RowsArgs a) {
-    __shared__ JmOneLds L;
+    __shared__ JmOneLds<SBR> L;
     const uint32_t code = g_sgrid.v[threadIdx.x & 511];   // a code's sixteen signed entries from its unsigned one, by two threads
     const int nj = a.njobs ? min(uniform(*a.njobs), a.njobs_max) : a.njobs_max;
-    const uint32_t gpj = (uint32_t) a.nrows / JM_ROWS, ji = blockIdx.x / gpj;
+    const int nunits = a.nrows / (64 / SBR);
+    const uint32_t gpj = (uint32_t) (nunits + 15) / 16, ji = blockIdx.x / gpj;
     if ((int) ji >= nj) return;   // the same for the whole block
     const int g = (int) (blockIdx.x - ji * gpj);
     const fnx_job* jb = a.jobs + ji;
@@ -256,8 +300,9 @@ __global__ void __launch_bounds__(JM_THREADS) k_iq3s_jobs_mma_one(const RowsArgs
         }
         __syncthreads();
     };
-    if (n == 1) jm_few<1>(L.tab, we, JM_ROWS * g, JM_ROWS * (g + 1), y0, out0, y, a.out, a.out_stride, codebook);
-    else jm_group(L, we, g, jb, n, y, a.out, a.out_stride, codebook);
+    if (n == 1) jm_few<1, SBR>(L.tab, we, 16 * g, min(16 * (g + 1), nunits), y0, out0, y, a.out, a.out_stride, codebook);
+    else if (SBR < 64 && n == 2) jm_two<SBR>(L.tab, we, 16 * g + uniform((int) (threadIdx.x >> 6)), nunits, jb, y, a.out, a.out_stride, codebook);
+    else jm_group<SBR>(L, we, g, nunits, jb, n, y, a.out, a.out_stride, codebook);
 }
 
 // rows of 2048 columns, a multiple of 16 of them; unit64. The blocks split the (job, 16 rows) items of all jobs evenly and

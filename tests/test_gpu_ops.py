@@ -333,6 +333,31 @@ def test_mmvq_first_runs_of_every_kind(dev, oracle, nrows, counts):
     assert rel_l2(got, oracle.mmvq(w, nrows * 880, nrows, 2048, jobs, yq, at)) <= 1e-6, "a row's 64 terms in another order"
 
 
+# rows of 256, 512 and 1,024 columns: a group of sixteen units (128, 64, 32 rows) a block, whole groups and ones that end early, jobs of one
+# row beside others, up to eight jobs a call, no more groups than two a CU
+@pytest.mark.parametrize("ncols", [256, 512, 1024])
+@pytest.mark.parametrize("units,counts", [(1, [16]), (4, [1]), (15, [2, 0, 9]), (16, [1, 16]), (17, [5]), (33, [3, 1, 16, 7, 1, 0, 2, 4]), (1040, [16, 1, 8])])
+def test_mmvq_lone_calls_over_shorter_rows(dev, oracle, ncols, units, counts):
+    nrows, nexp = units * (2048 // ncols), 2
+    print(f"case shorter rows nrows={nrows} ncols={ncols} counts={counts}", flush=True)
+    rng = np.random.default_rng(423 + units + ncols)
+    w = random_iq3s(rng, nexp * nrows * ncols // 256)
+    yq = oracle.quantize_q8_1(rng.standard_normal((16, ncols)).astype(np.float32))
+    jobs = np.zeros(len(counts), dtype=JOB_DTYPE)
+    at = 0
+    for j, n in enumerate(counts):
+        jobs["w"][j], jobs["n"][j] = j % nexp, n
+        jobs["y"][j, :n] = rng.permutation(16)[:n]
+        jobs["out"][j, :n] = np.arange(at, at + n)
+        at += n
+    got = dev.mmvq(w, nrows * ncols // 256 * 110, nrows, ncols, jobs, yq, at, packed=True)
+    want = oracle.mmvq(w, nrows * ncols // 256 * 110, nrows, ncols, jobs, yq, at)
+    assert rel_l2(got, want) <= 1e-6, "a row's terms in another order"
+    for j in range(0, len(counts), 3):   # a job's bits are its own
+        o = jobs["out"][j, :counts[j]]
+        assert np.array_equal(got[o], dev.mmvq(w, nrows * ncols // 256 * 110, nrows, ncols, jobs[j:j + 1], yq, at, packed=True)[o])
+
+
 # ---------------------------------------------------------------- head, drafting, acceptance
 def test_argmax_full_vocabulary(dev, oracle):
     rng = np.random.default_rng(500)
