@@ -1144,16 +1144,18 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
     // f32 weights against more rows than a window's: tiles on the matrix cores, or none (gemv_rows_plan.h)
     const bool tiles = !bf && T > FNX_MAXT && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
     const GemvRows form = tiles ? gemv_rows_form(rows, n, T, cu_count()) : GemvRows::many;
-    if (form == GemvRows::small_tiles) {
+    const bool spread = tiles && gemv_rest_spread(rows, n, T, cu_count());
+    if (form == GemvRows::small_tiles && !spread) {
         const int ntt = (T + RS_TILE - 1) / RS_TILE, net = (rows + RS_TILE - 1) / RS_TILE;
         k_gemv_rows_mfma16<<<(unsigned) ((gemv_small_tiles(rows, T) + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
         return launch_status(who);
     }
     if (form != GemvRows::many) {
-        const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE;
-        const int tile_blocks = ((ntt + 3) / 4) * ((net + 7) / 8) * 32;
-        const bool along = form == GemvRows::large_tiles;
-        k_gemv_rows_mfma<<<tile_blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, tile_blocks, along ? 1 : 0);
+        const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE, most = 8 * std::max(1, cu_count() / 8);
+        const bool along = form == GemvRows::large_tiles || spread;
+        const int blocks = spread ? most : std::min((ntt * net + 7) / 8 * 8, most), items = along ? left * T : 0;
+        if (blocks >= ntt * net) k_gemv_rows_mfma<false><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items, spread);
+        else k_gemv_rows_mfma<true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items, 1);
         if (along) return launch_status(who);
         const dim3 gm((left + GM_WAVES * GR_ROWS - 1) / (GM_WAVES * GR_ROWS), (T + FNX_MAXT - 1) / FNX_MAXT);
         k_gemv_rows_many<false><<<gm, GM_WAVES * 64, 0, s>>>(W, x, y, rows, n, T, net * RM_TILE);

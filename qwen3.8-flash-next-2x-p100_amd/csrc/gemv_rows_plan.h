@@ -46,5 +46,14 @@ inline GemvRows gemv_rows_form(int rows, int n, int T, int cus) {
     if (!large) return GemvRows::many;
     return gemv_rest_along(rows) ? GemvRows::large_tiles : GemvRows::large_rest;
 }
+// Large tiles with the left weight rows' items spread over the waves of all CUs, up to four each, instead of the small tiles or the second
+// launch that the form says: from where the small tiles are more than two a CU, the line of the rows that ride along. 2,048 columns, us (as the
+// form says / so): 33 weight rows, 2,900 rows of x 18.0 / 16.8; 65, 1,633 17.4 / 14.9, 4,000 36.3 / 18.4; 97, 2,330 25.3 / 16.2; 129, 918 17.7 / 13.7, 1,820
+// 25.0 / 15.4, 4,096 37.9 / 29.3; 161, 770 17.2 / 13.4; 258, 500 16.3 / 13.6, 1,500 35.5 / 26.1; 1,000, 500 36.9 / 27.5.
+inline bool gemv_rest_spread(int rows, int n, int T, int cus) {
+    const bool large = T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (unsigned long long) T * n * 4 < (1ull << 32) &&
+                       (unsigned long long) rows * n * 4 < (1ull << 32);
+    return large && rows % RM_TILE && !gemv_rest_along(rows) && gemv_small_tiles(rows, T) > 2l * cus && (long) (rows % RM_TILE) * T <= 16l * cus;
+}
 
 }  // namespace fnx

@@ -389,30 +389,40 @@ __global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __
 // wait is for its own loads, counted. A step's sixteen MFMAs (64 cycles each) hide the eight reads of the next step's operands and
 // the eight loads of the ring's next step, one behind each MFMA. Run r of eight rows' runs lies at place p = 4 r + (j ^ f), f of the row,
 // so that the 16 rows an operand read touches fall on 16 different bank groups.
-// Bound by the MFMAs and the loads behind them: 513 rows of 2,048 columns, 512 rows of x 16.6 -> 14.6 us, 4,096 114 -> 101 over weights in turn (134 -> 111-117 in
-// a layer, whose x comes from memory): 9.1 us a tile's steps where the MFMAs alone take 6.8, with the operands' reads 7.5. Before, four waves
-// took a chain each, met after every 64 columns' step and had two loading waves beside them: 11.7 us a tile's steps.
-// The weight rows past the last full 32 (the router's 513th) are items of such a row against one row of x, one a wave at most,
-// added up while the first steps are on their way.
+// A CU has one block (its rings fill the LDS), which takes its tiles one after another (MANY): the next tile's first steps come in
+// behind the last ones of the tile before, and its sums go through a place of their own, so that a tile's start is not waited for and
+// its end is the exchange alone. With a block a tile the CU stood still from one tile's last MFMA to the next one's first: 513 rows of 2,048
+// columns, 4,096 rows of x 95 -> 88 us over weights in turn, 1,900 50.5 -> 46.6; two tiles a block the same (700: 24.4), and where every block
+// has one tile that form is 4 % behind the plain one (its sums in the ring, nothing asked for past the end).
+// Bound by the MFMAs and the loads behind them: some 10.5 us a tile where the MFMAs alone take 6.8, the operands' reads 0.7.
+// The weight rows past the last full 32 (the router's 513th) are items of such a row against one row of x, added up while the first
+// steps are on their way: where a row of tiles has a wave for each of its items, and a block one tile, those; else dealt to all waves of the grid.
 typedef float v32f __attribute__((ext_vector_type(32)));
-constexpr int RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4;
+constexpr int RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4, RM_PART = 2 * 4 * 64 * 16;   // (RM_PART: a wave's sums of two chains)
+template <bool MANY>
 __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) k_gemv_rows_mfma(const float* __restrict__ W, const float* __restrict__ x,
                                                                                                          float* __restrict__ y, int rows, int n, int T, int ntt,
-                                                                                                         int net, int tile_blocks, int along) {
+                                                                                                         int net, int items, int spread) {
     __shared__ __align__(16) uint8_t lds[RM_WAVES * RM_RING * RM_STEP];
+    __shared__ __align__(16) uint8_t red[MANY ? RM_WAVES * RM_PART : 16];   // the waves' sums of two chains at a tile's end
     const int wave = uniform((int) (threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    // Which tile: block ids go round the eight XCDs, each with an L2 of its own, so an XCD's blocks are given one patch of
-    // 4 x 8 tiles after another (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them).
-    // The grid covers whole patches; a block whose tile lies outside leaves.
-    const int lin = ((int) blockIdx.x % 8) * (tile_blocks / 8) + (int) blockIdx.x / 8, patches_e = (net + 7) / 8;
-    const int tt = 4 * ((lin / 32) / patches_e) + (lin % 32) / 8, et = 8 * ((lin / 32) % patches_e) + lin % 8;
-    if (tt >= ntt || et >= net) return;
-    const int t0 = tt * RM_TILE, e0 = et * RM_TILE;
+    // Which tiles: block ids go round the eight XCDs, each with an L2 of its own, so an XCD's blocks are given an eighth of the tiles in
+    // patches of 4 x 8 (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them), a patch's tiles side by side.
+    const int total = ntt * net, xcd = (int) blockIdx.x % 8, per = (int) gridDim.x / 8;
+    int L = (int) ((long) total * xcd / 8) + (int) blockIdx.x / 8;
+    const int Lend = (int) ((long) total * (xcd + 1) / 8);
+    int t0 = 0, e0 = 0;
+    auto tile_of = [&](int l) {
+        const int p = l / (8 * ntt), w = min(8, net - 8 * p), i = l - 8 * ntt * p, q = i / (4 * w), r = i - 4 * w * q;
+        t0 = (4 * q + r / w) * RM_TILE, e0 = (8 * p + r % w) * RM_TILE;
+    };
+    const bool any = L < Lend;   // (a block without a tile helps with the items)
+    tile_of(any ? L : 0);
     const int half = n / 256, S = 2 * half;   // steps: a multiple of 16
     uint8_t* ring = lds + wave * (RM_RING * RM_STEP);
     const uint32_t ring_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) ring;
     uint32_t xoff[4], woff[4];   // instruction g: rows 8 g .. 8 g + 7, this lane's piece
-    {
+    auto point = [&]() {
         const int r7 = (lane >> 2) & 7, b = lane >> 5;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
@@ -420,37 +430,47 @@ __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu
             xoff[g] = (uint32_t) min(t0 + 8 * g + r7, T - 1) * (uint32_t) n * 4u + piece;
             woff[g] = (uint32_t) (e0 + 8 * g + r7) * (uint32_t) n * 4u + piece;
         }
-    }
+    };
+    point();
     auto from_of = [&](int s) { return 64 * wave + (s >= half ? 256 + 1024 * (s - half) : 1024 * s); };
     auto fetch = [&](int op, int from, int slot) {   // one of a step's eight instructions
         const int g = op & 3;
         if (op < 4) lds_load16(reinterpret_cast<const uint8_t*>(x) + from, xoff[g], ring_at + slot * RM_STEP + g * 1024);
         else lds_load16(reinterpret_cast<const uint8_t*>(W) + from, woff[g], ring_at + slot * RM_STEP + 4096 + g * 1024);
     };
+    if (any) {
 #pragma unroll
-    for (int s = 0; s < RM_RING; ++s)   // (S >= 16)
+        for (int s = 0; s < RM_RING; ++s)   // (S >= 16)
 #pragma unroll
-        for (int op = 0; op < 8; ++op) fetch(op, from_of(s), s);
-    if (along && 4 * et + wave < RM_TILE * (rows - net * RM_TILE)) {
-        const int item = 4 * et + wave, irow = net * RM_TILE + item / RM_TILE, it = t0 + item % RM_TILE;
-        const float4 *wp = reinterpret_cast<const float4*>(W + (size_t) irow * n) + lane, *xp = reinterpret_cast<const float4*>(x + (size_t) min(it, T - 1) * n) + lane;
-        float v = 0.f;
-        for (int c0 = 0; c0 < n / 4; c0 += 8 * 64) {
-            float4 wv[8], xv[8];
+            for (int op = 0; op < 8; ++op) fetch(op, from_of(s), s);
+    }
+    // The weight rows past the last full tile: items of such a row against one row of x. Spread: all of them over the waves of the grid;
+    // else a row of tiles' items go to its waves, whose x the L2 has.
+    if (items > 0) {
+        const int left = rows - net * RM_TILE, first = spread ? (int) blockIdx.x * RM_WAVES + wave : RM_WAVES * (e0 / RM_TILE) + wave;
+        const int count = spread ? items : any ? min(RM_TILE, T - t0) * left : 0, by = spread ? (int) gridDim.x * RM_WAVES : RM_WAVES * net;
+        for (int item = first; item < count; item += by) {
+            const int at = left == 1 ? item : item / left, it = spread ? at : t0 + at, irow = net * RM_TILE + item - at * left;
+            const float4 *wp = reinterpret_cast<const float4*>(W + (size_t) irow * n) + lane, *xp = reinterpret_cast<const float4*>(x + (size_t) it * n) + lane;
+            float v = 0.f;
+            for (int c0 = 0; c0 < n / 4; c0 += 8 * 64) {
+                float4 wv[8], xv[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) wv[k] = wp[c0 + 64 * k], xv[k] = xp[c0 + 64 * k];
+                for (int k = 0; k < 8; ++k) wv[k] = wp[c0 + 64 * k], xv[k] = xp[c0 + 64 * k];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                v = fmaf(wv[k].x, xv[k].x, v);
-                v = fmaf(wv[k].y, xv[k].y, v);
-                v = fmaf(wv[k].z, xv[k].z, v);
-                v = fmaf(wv[k].w, xv[k].w, v);
+                for (int k = 0; k < 8; ++k) {
+                    v = fmaf(wv[k].x, xv[k].x, v);
+                    v = fmaf(wv[k].y, xv[k].y, v);
+                    v = fmaf(wv[k].z, xv[k].z, v);
+                    v = fmaf(wv[k].w, xv[k].w, v);
+                }
             }
+            v = group_sum<64>(v);
+            if (lane == 0) y[(size_t) it * rows + irow] = v;
         }
-        v = group_sum<64>(v);
-        if (lane == 0 && it < T) y[(size_t) it * rows + irow] = v;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the counts below are of the steps' loads alone)
     }
+    if (!any) return;   // the same for the whole block
     const int i = lane & 31, b = lane >> 5;
     const int rd = (i >> 3) * 1024 + 64 * ((i & 7) + 8 * b), f = ((i & 7) >> 2) | (((i >> 3) & 1) << 1);
     const uint8_t* at[4];   // this lane's pieces of a step: row i of x (of W: 4 KiB on), chunk j of its block
@@ -498,6 +518,11 @@ __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    auto meet = [] {   // (the loads on their way stay there)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
     using std::integral_constant;
     constexpr integral_constant<bool, true> yes{};
     constexpr integral_constant<bool, false> no{};
@@ -508,51 +533,76 @@ __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu
         B[0][j] = *reinterpret_cast<const float4*>(at[j] + 4096);
     }
     // step k reads step k + 1's operands and fetches step k + RM_RING; RM_RING steps a trip, so that the ring's places are constants
-    auto trip = [&](int k, auto first_c, auto fold_c, auto fetch_c, auto last_c) {
+    auto trip = [&](int k, auto first_c, auto fold_c, auto last_c) {
         constexpr bool LAST = decltype(last_c)::value;
+        constexpr integral_constant<bool, !LAST> on{};
         wait(2);
-        step(A[0], B[0], A[1], B[1], 1, from_of(k + 4), first_c, fold_c, yes, fetch_c);
+        step(A[0], B[0], A[1], B[1], 1, from_of(k + 4), first_c, fold_c, yes, on);
         wait(LAST ? 1 : 2);
-        step(A[1], B[1], A[0], B[0], 2, from_of(k + 5), no, no, yes, fetch_c);
+        step(A[1], B[1], A[0], B[0], 2, from_of(k + 5), no, no, yes, on);
         wait(LAST ? 0 : 2);
-        step(A[0], B[0], A[1], B[1], 3, from_of(k + 6), no, no, yes, fetch_c);
+        step(A[0], B[0], A[1], B[1], 3, from_of(k + 6), no, no, yes, on);
         if constexpr (!LAST) wait(2);
-        step(A[1], B[1], A[0], B[0], 0, from_of(k + 7), no, no, integral_constant<bool, !LAST>{}, fetch_c);
+        step(A[1], B[1], A[0], B[0], 0, from_of(k + 7), no, no, on, on);
     };
-    trip(0, yes, no, yes, no);
-    for (int k = RM_RING; k < half; k += RM_RING) trip(k, no, no, yes, no);
-    trip(half, yes, yes, yes, no);
-    for (int k = half + RM_RING; k + RM_RING < S; k += RM_RING) trip(k, no, no, yes, no);
-    trip(S - RM_RING, no, no, no, yes);
-    // levels 32 and 16 here, 8 and 4 over the waves, 2 and 1 over the chains: wave w the accumulator's registers 4 w .. 4 w + 3, the
-    // sums through the waves' own rings (each has been read by its wave)
-    static_assert(4 * 4 * 64 * 16 <= RM_RING * RM_STEP, "a wave's sums fit its ring");
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float u[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) u[v] = held[j][4 * q + v] + (acc[j][4 * q + v] + acc[j][16 + 4 * q + v]);
-            *reinterpret_cast<float4*>(ring + ((j * 4 + q) * 64 + lane) * 16) = make_float4(u[0], u[1], u[2], u[3]);
+    while (true) {
+        const int tt0 = t0, te0 = e0;
+        const bool more = MANY && L + per < Lend;
+        trip(0, yes, no, no);
+        for (int k = RM_RING; k < half; k += RM_RING) trip(k, no, no, no);
+        trip(half, yes, yes, no);
+        for (int k = half + RM_RING; k + RM_RING < S; k += RM_RING) trip(k, no, no, no);
+        if constexpr (MANY) {   // the next tile's first steps come in behind this one's last (after the last tile its own again: no form without them)
+            L += more ? per : 0;
+            tile_of(L);
+            point();
+            trip(-RM_RING, no, no, no);
+        } else {
+            trip(0, no, no, yes);
         }
-    __syncthreads();
-    float s[4][4];
+        // levels 32 and 16 here, 8 and 4 over the waves, 2 and 1 over the chains: wave w the accumulator's registers 4 w .. 4 w + 3. The sums
+        // go through the waves' own rings (each has been read by its wave), or, where the next tile's steps are coming in there, two chains at a time
+        // through a place of their own.
+        constexpr int CH = MANY ? 2 : 4;
+        uint8_t* const to = MANY ? red + wave * RM_PART : ring;
+        const uint8_t* const from = MANY ? red : lds;
+        constexpr int part = MANY ? RM_PART : RM_RING * RM_STEP;
+        static_assert(CH * 4 * 64 * 16 <= part, "a wave's sums fit their place");
+        float s[4][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        float4 u[4];
+        for (int j0 = 0; j0 < 4; j0 += CH) {
+            if (j0) meet();   // the sums before have been read
 #pragma unroll
-        for (int w = 0; w < 4; ++w) u[w] = *reinterpret_cast<const float4*>(lds + w * (RM_RING * RM_STEP) + ((j * 4 + wave) * 64 + lane) * 16);
-        s[j][0] = (u[0].x + u[2].x) + (u[1].x + u[3].x);
-        s[j][1] = (u[0].y + u[2].y) + (u[1].y + u[3].y);
-        s[j][2] = (u[0].z + u[2].z) + (u[1].z + u[3].z);
-        s[j][3] = (u[0].w + u[2].w) + (u[1].w + u[3].w);
+            for (int j = j0; j < j0 + CH; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float u[4];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) u[v] = held[j][4 * q + v] + (acc[j][4 * q + v] + acc[j][16 + 4 * q + v]);
+                    *reinterpret_cast<float4*>(to + (((j - j0) * 4 + q) * 64 + lane) * 16) = make_float4(u[0], u[1], u[2], u[3]);
+                }
+            meet();
+#pragma unroll
+            for (int j = j0; j < j0 + CH; ++j) {
+                float4 u[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) u[w] = *reinterpret_cast<const float4*>(from + w * part + (((j - j0) * 4 + wave) * 64 + lane) * 16);
+                s[j][0] = (u[0].x + u[2].x) + (u[1].x + u[3].x);
+                s[j][1] = (u[0].y + u[2].y) + (u[1].y + u[3].y);
+                s[j][2] = (u[0].z + u[2].z) + (u[1].z + u[3].z);
+                s[j][3] = (u[0].w + u[2].w) + (u[1].w + u[3].w);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = tt0 + 8 * wave + 4 * b + v;
+            if (t < T) y[(size_t) t * rows + te0 + i] = (s[0][v] + s[2][v]) + (s[1][v] + s[3][v]);
+        }
+        if (!more) break;
+        meet();   // (the next tile's sums go to the same place)
     }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int t = t0 + 8 * wave + 4 * b + v;
-        if (t < T) y[(size_t) t * rows + e0 + i] = (s[0][v] + s[2][v]) + (s[1][v] + s[3][v]);
-    }
+    if constexpr (MANY) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing is on its way into LDS when the block leaves
+
 }
 
 // ---------------------------------------------------------------- the routed experts on the matrix cores

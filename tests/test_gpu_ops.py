@@ -85,6 +85,13 @@ def test_gemv_f32_narrow_rows_bit_exact(dev, oracle, rows, n, T):
     test_gemv_f32_short_chunks_bit_exact(dev, oracle, rows, n, T)
 
 
+# left weight rows dealt to the waves of all CUs: fewer tiles than blocks and several a block, one to four items a wave, several left rows,
+# ragged last tiles, one row of tiles and one column of them, rows of 4,096
+@pytest.mark.parametrize("rows,n,T", [(33, 2048, 2803), (129, 2048, 918), (129, 2048, 2055), (258, 2048, 500), (45, 2048, 300), (1000, 2048, 129), (130, 4096, 920)])
+def test_gemv_f32_left_rows_spread_bit_exact(dev, oracle, rows, n, T):
+    test_gemv_f32_short_chunks_bit_exact(dev, oracle, rows, n, T)
+
+
 def test_gemv_f32_sum_does_not_depend_on_T(dev):
     """A size-independent property at a size the oracle takes long for: a sum's bits do not depend on how many rows of x a
     call brings, so 4,099 rows in one call (the matrix cores' tiles, several patches of them, a ragged last tile, the 513th
