@@ -6,7 +6,7 @@
 // columns of f16, 64 KiB - is put in LDS once (by loads that write LDS directly, a token's row per wave instruction), and
 // after that a wave needs nothing from the others: it takes tiles of 16 rows, a lane decodes its four sub-blocks of its
 // row from one contiguous load of the tile16 layout, and the sixteen waves of a block (four a SIMD) meet only where the
-// block goes from one job to the next. The blocks split the (job, sixteen tiles) units of all jobs by cost - a tile's
+// block goes from one phase of jobs to the next. The blocks split the (job, sixteen tiles) units of all jobs by cost - a tile's
 // decode and its job's token tiles of multiplications - into contiguous runs.
 // part[job.out[t]][row] = W[job.w][row] . h16[job.y[t]] as kernels.hpp:330 (moe_down_mma) defines it, with the weights as
 // f16 (d (1 + 2 s) g, the f32 value rounded once, as k_moe_mma rounds it) and a row's sub-blocks accumulated super-step by
@@ -147,6 +147,7 @@ struct W16Tile16 {
     static constexpr int PS = 4;
     int nsuper;
     __device__ __forceinline__ W16Tile16(int ncols) : nsuper(ncols >> 9) {}
+    __device__ __forceinline__ int tile_size() const { return nsuper * TILE16_BYTES; }
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t tiles(const uint8_t* we, int t) const { return tile16_rsrc(we, t, nsuper); }
     __device__ __forceinline__ SuperFields load(__amdgpu_buffer_rsrc_t m, int S) const { return tile16_load_buf(m, S); }
 };
@@ -161,6 +162,7 @@ struct W16Unit64 {
         const int lane = threadIdx.x & 63, at = (lane & 15) * (ncols >> 5) + STEPS * (lane >> 4), u = (at >> 6) * UNIT_BYTES, l = at & 63;
         a = u + 8 * l, b = u + UNIT_B_AT + 4 * l, c = u + UNIT_C_AT + l, sc = u + UNIT_SCALES_AT + (l >> 1), d = u + UNIT_D_AT + 2 * (l >> 3);
     }
+    __device__ __forceinline__ int tile_size() const { return tile_bytes; }
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t tiles(const uint8_t* we, int t) const {
         return __builtin_amdgcn_make_buffer_rsrc((void*) uniform_ptr(we + (size_t) t * tile_bytes), 0, -1, 0x00020000);
     }
@@ -289,82 +291,137 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16(const MmaArgs a)
     const uint32_t xt_at = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) L.xt;
     const LY ly(a.ncols);
     const uint8_t* xlane = L.xt + r * W16_XROW + 64 * PS * grp;   // token r of a tile, this lane group's four sub-blocks of a super-step
-    int yahead[MB_TP] = {0, 0, 0, 0}, ahead = -1;
-    for (int j = jA; j <= jB && j < njall; ++j) {
-        const int g0 = j == jA ? tA : 0, g1 = j == jB ? min(tB, gpj) : gpj;
-        const fnx_bigjob* jb = job_at(j);
-        const int n = uniform(n_of(j));
-        if (n < 1 || g0 >= g1) continue;   // the same for the whole block
-        const int nt = (n + 15) >> 4, e = j >= nj ? 0 : uniform(j < W16_HELD ? L.jw[j] : jb->w);
-        const uint8_t* we = j >= nj ? a.w2 : a.ep ? uniform_ptr((const uint8_t*) a.ep[e]) : a.w + (size_t) e * a.stride;
-        // the wave's tokens' rows, tokens wave, wave + 16, .. (past the job's last: that one again): asked for while the job
-        // before was multiplied, if that was the list's job before this one
-        int y[MB_TP];
-#pragma unroll
-        for (int i = 0; i < MB_TP; ++i) y[i] = ahead == j ? yahead[i] : uniform(jb->y[min(wave + 16 * i, n - 1)]);
-        __syncthreads();   // the job before has been read
-#pragma unroll
-        for (int i = 0; i < MB_TP; ++i)   // a token's row a wave instruction, 16 bytes a lane
-            if (i < nt) lds_load16(a.x + (size_t) y[i] * a.ldx, 16u * (lane & (16 * PS - 1)), xt_at + (wave + 16 * i) * W16_XROW);
-        if (j + 1 <= jB && j + 1 < njall) {
-            const int nn = uniform(n_of(j + 1));
-            const fnx_bigjob* jn = job_at(j + 1);
-#pragma unroll
-            for (int i = 0; i < MB_TP; ++i) yahead[i] = uniform(jn->y[max(0, min(wave + 16 * i, nn - 1))]);
-            ahead = j + 1;
+    // The run goes in phases: the jobs of it, one after another, whose token tiles find room together in the four that LDS has. A
+    // phase's activations come in at once and the waves meet only where it ends; the next one's rows are looked up while they are on
+    // their way, and the first weights of a wave's next job, in this phase or the next, asked for behind its last tile of this one. With
+    // a job at a time the memory stood still wherever a block went from one to the next (us a launch of 2,048 rows: 512 jobs of two
+    // tokens 51.0 -> 47.5, 768 of four 75.5 -> 70.5, 256 of eight 28.1 -> 27.3, 512 of 64 152.3 -> 148.6; a chunk of 29 rows, 8 of 512
+    // experts, 93.5 -> 90.5, of 77, 10 picks, 159.5 -> 156.1). The weights are asked for ahead of the rows, which wait for them: behind the rows
+    // 0.4 us a launch more; the phase's rows looked up in one place of the code, not two: 0.4 us of cold code.
+    auto first_of = [&](int j) { return j == jA ? tA : 0; };   // job j's items of the run
+    auto last_of = [&](int j) { return j == jB ? min(tB, gpj) : gpj; };
+    struct Job {
+        int j, n;
+    };
+    auto next_job = [&](int j) {   // the first job from j on that has items in the run, and its tokens; past the run: the end
+        for (const int end = min(jB, njall - 1); j <= end; ++j) {
+            const int n = uniform(n_of(j));
+            if (n >= 1 && first_of(j) < last_of(j)) return Job{j, n};
         }
-        int orow[MB_TP];
+        return Job{njall, 0};
+    };
+    auto matrix_of = [&](int j) {
+        const int e = j >= nj ? 0 : uniform(j < W16_HELD ? L.jw[j] : job_at(j)->w);
+        return j >= nj ? a.w2 : a.ep ? uniform_ptr((const uint8_t*) a.ep[e]) : a.w + (size_t) e * a.stride;
+    };
+    // the phase that begins with a job: where the next one begins; this wave's tokens (tokens wave, wave + 16, .. of every job, past its
+    // last that one again) and this lane's place in the output, a token tile each
+    auto phase_at = [&](Job c, int (&y)[MB_TP], int (&orow)[MB_TP]) {
+        int used = 0, rows[MB_TP];
 #pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) orow[tt] = tt * 16 + r < n ? jb->out[tt * 16 + r] : -1;
-        int g = g0 + wave;
-        SuperFields f = ly.load(ly.tiles(we, min(g, g1 - 1)), 0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        // A tile's results go out as buffer stores that every path issues (a lane without a token: past the buffer's end, where
-        // a store is dropped): stores under a condition of their own cannot be counted, and the wait for the next tile's weights,
-        // asked for before them, was a wait for the stores too (77 rows, some 400 jobs of two tokens: 59.1 -> 56.7 us a launch, 512 rows
-        // 36.0 -> 35.2, 4,096 rows the same 186). The loop stands once for each number of token tiles, so that their stores are counted too.
-        // A job with a row past what 32-bit offsets reach stores under the condition, in one loop for all numbers: with four of
-        // them the kernel was 32.7 KB of code instead of 24.9, at the same speed (8 picks of 512 experts, 29 rows 29.7 / 29.1 us a launch).
-        const uint32_t rowb = (uint32_t) a.nrows * 4u, end = 0xE0000000u, none = 0xF0000000u;   // (none and a row's bytes: no wrap)
-        const int reach = (int) (end / rowb);
-        uint32_t at[MB_TP];
+        for (int p = 0; p < MB_TP; ++p) rows[p] = orow[p] = -1;
+        while (c.j < njall) {
+            const int nt = (c.n + 15) >> 4;
+            if (used + nt > MB_TP) break;
+            const fnx_bigjob* jb = job_at(c.j);
+#pragma unroll
+            for (int p = 0; p < MB_TP; ++p)
+                if (p >= used && p < used + nt) {
+                    const int t0 = 16 * (p - used);
+                    rows[p] = jb->y[min(wave + t0, c.n - 1)];
+                    if (t0 + r < c.n) orow[p] = jb->out[t0 + r];
+                }
+            used += nt;
+            c = next_job(c.j + 1);
+        }
+#pragma unroll
+        for (int p = 0; p < MB_TP; ++p) y[p] = uniform(rows[p]);   // (waited for together)
+        return c;
+    };
+    Job cur = next_job(jA);
+    if (cur.j >= njall) return;   // (the same for the whole block)
+    int g = first_of(cur.j) + wave;
+    const uint8_t* we = matrix_of(cur.j);
+    SuperFields f = ly.load(ly.tiles(we, min(g, last_of(cur.j) - 1)), 0);
+    int yn[MB_TP], on[MB_TP];
+    uint32_t at[MB_TP] = {0, 0, 0, 0};   // this lane's tokens' places in the output
+    bool all_near = true;
+    // A tile's results go out as buffer stores that every path issues (a lane without a token: past the buffer's end, where
+    // a store is dropped): stores under a condition of their own cannot be counted, and the wait for the next tile's weights,
+    // asked for before them, was a wait for the stores too (77 rows, some 400 jobs of two tokens: 59.1 -> 56.7 us a launch, 512 rows
+    // 36.0 -> 35.2, 4,096 rows the same 186). The loop stands once for each number of token tiles, so that their stores are counted too.
+    // A phase with a row past what 32-bit offsets reach stores under the condition, in one loop for all numbers: with four of
+    // them the kernel was 32.7 KB of code instead of 24.9, at the same speed (8 picks of 512 experts, 29 rows 29.7 / 29.1 us a launch).
+    const uint32_t rowb = (uint32_t) a.nrows * 4u, end = 0xE0000000u, none = 0xF0000000u;   // (none and a row's bytes: no wrap)
+    const int reach = (int) (end / rowb);
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*) a.out, 0, (int) end, 0x00020000);
+    for (Job pend = cur;;) {   // the phase up to pend is on its way to LDS (at first none)
+        const Job begin = pend;
+        pend = phase_at(begin, yn, on);
+        if (cur.j < begin.j) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+        for (const uint8_t* xl = xlane; cur.j < begin.j;) {
+            const int nt = (cur.n + 15) >> 4, g1 = last_of(cur.j);
+            // the next job's first tile of this wave (no job: a tile of its own again)
+            const Job then = next_job(cur.j + 1);
+            const bool any = then.j < njall;
+            const int gn = any ? first_of(then.j) + wave : 0, gl = any ? min(gn, last_of(then.j) - 1) : 0;
+            const uint8_t* wn = any ? matrix_of(then.j) : we;
+            if (g >= g1) f = ly.load(ly.tiles(wn, gl), 0);   // (no tile for this wave)
+            int left = (g1 - g + W16_WAVES - 1) / W16_WAVES;   // this wave's tiles
+            const uint8_t *tile = we + (size_t) g * ly.tile_size(), *then_tile = any ? wn + (size_t) gl * ly.tile_size() : tile;
+            auto rounds = [&](auto ntiles, auto near_tag) {   // (ntiles: a constant, or nt)
+                for (; left > 0; --left, g += W16_WAVES) {
+                    // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the phase's end
+                    // for the last: every wave takes every priority in turn, a tile each
+                    switch (((wave >> 2) + left) & 3) {
+                        case 0: __builtin_amdgcn_s_setprio(0); break;
+                        case 1: __builtin_amdgcn_s_setprio(1); break;
+                        case 2: __builtin_amdgcn_s_setprio(2); break;
+                        default: __builtin_amdgcn_s_setprio(3); break;
+                    }
+                    tile = left > 1 ? tile + (size_t) W16_WAVES * ly.tile_size() : then_tile;
+                    const SuperFields nf = ly.load(ly.tiles(tile, 0), 0);
+                    __builtin_amdgcn_sched_barrier(0);   // (left to itself the compiler asks for them behind the products)
+                    v4f acc[MB_TP];
+#pragma unroll
+                    for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+                    w16_super_step<PS>(L.tab, xl, f, ntiles, acc);
+                    // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
+#pragma unroll
+                    for (int tt = 0; tt < MB_TP; ++tt) {
+                        if constexpr (decltype(near_tag)::value) {
+                            if (tt < ntiles) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[tt]), to, at[tt], 64u * g, 0);
+                        } else if (16 * tt + r < cur.n && job_at(cur.j)->out[16 * tt + r] >= 0)
+                            *reinterpret_cast<float4*>(a.out + (size_t) job_at(cur.j)->out[16 * tt + r] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
+                    }
+                    f = nf;
+                }
+            };
+            if (!all_near) rounds(nt, std::false_type{});
+            else if (nt == 4) rounds(std::integral_constant<int, 4>{}, std::true_type{});
+            else if (nt == 3) rounds(std::integral_constant<int, 3>{}, std::true_type{});
+            else if (nt == 2) rounds(std::integral_constant<int, 2>{}, std::true_type{});
+            else rounds(std::integral_constant<int, 1>{}, std::true_type{});
+            // the next job's token tiles to the front
+            for (int i = 0; i < nt && then.j < begin.j; ++i) {
+#pragma unroll
+                for (int tt = 0; tt + 1 < MB_TP; ++tt) at[tt] = at[tt + 1];
+            }
+            xl += 16 * nt * W16_XROW;
+            cur = then, g = gn, we = wn;
+        }
+        if (begin.j >= njall) break;
+        __syncthreads();   // the phase before has been read
+#pragma unroll
+        for (int p = 0; p < MB_TP; ++p)   // a token's row a wave instruction, 16 bytes a lane
+            if (yn[p] >= 0) lds_load16(a.x + (size_t) yn[p] * a.ldx, 16u * (lane & (16 * PS - 1)), xt_at + (wave + 16 * p) * W16_XROW);
         bool near = true;
 #pragma unroll
-        for (int tt = 0; tt < MB_TP; ++tt) near = near && orow[tt] < reach, at[tt] = orow[tt] >= 0 ? (uint32_t) orow[tt] * rowb + 16u * grp : none;
-        const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc((void*) a.out, 0, (int) end, 0x00020000);
-        auto rounds = [&](auto ntiles, auto near_tag) {   // (ntiles: a constant, or nt)
-            for (; g < g1; g += W16_WAVES) {
-                // The oldest wave of a SIMD goes first, so a block's waves drift apart and the first ones wait at the job's end
-                // for the last: every wave takes every priority in turn, a tile each
-                switch (((wave >> 2) + ((g - g0) >> 4)) & 3) {
-                    case 0: __builtin_amdgcn_s_setprio(0); break;
-                    case 1: __builtin_amdgcn_s_setprio(1); break;
-                    case 2: __builtin_amdgcn_s_setprio(2); break;
-                    default: __builtin_amdgcn_s_setprio(3); break;
-                }
-                const SuperFields nf = ly.load(ly.tiles(we, g + W16_WAVES < g1 ? g + W16_WAVES : g), 0);
-                __builtin_amdgcn_sched_barrier(0);   // (left to itself the compiler asks for them behind the products)
-                v4f acc[MB_TP];
-#pragma unroll
-                for (int tt = 0; tt < MB_TP; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-                w16_super_step<PS>(L.tab, xlane, f, ntiles, acc);
-                // lane: token r of each tile, rows 4 grp .. 4 grp + 3 of the tile
-#pragma unroll
-                for (int tt = 0; tt < MB_TP; ++tt) {
-                    if constexpr (decltype(near_tag)::value) {
-                        if (tt < ntiles) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[tt]), to, at[tt], 64u * g, 0);
-                    } else if (orow[tt] >= 0)
-                        *reinterpret_cast<float4*>(a.out + (size_t) orow[tt] * a.nrows + 16 * g + 4 * grp) = make_float4(acc[tt].x, acc[tt].y, acc[tt].z, acc[tt].w);
-                }
-                f = nf;
-            }
-        };
-        if (!__all(near)) rounds(nt, std::false_type{});
-        else if (nt == 4) rounds(std::integral_constant<int, 4>{}, std::true_type{});
-        else if (nt == 3) rounds(std::integral_constant<int, 3>{}, std::true_type{});
-        else if (nt == 2) rounds(std::integral_constant<int, 2>{}, std::true_type{});
-        else rounds(std::integral_constant<int, 1>{}, std::true_type{});
+        for (int p = 0; p < MB_TP; ++p) near = near && on[p] < reach, at[p] = on[p] >= 0 ? (uint32_t) on[p] * rowb + 16u * grp : none;
+        all_near = __all(near);
     }
 }
 

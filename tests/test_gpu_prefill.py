@@ -211,6 +211,31 @@ def test_moe_mma_over_unit64_rows(dev, oracle, nrows, ncols, sizes):
         assert np.array_equal(got[at].view(np.uint32), out_of(jobs[j:j + 1])[at].view(np.uint32)), f"job {j} of {jobs[j][1]} rows"
 
 
+# Lists of several jobs a block: phases of up to four token tiles, with jobs that fill one alone, jobs without tokens between them, and
+# (18 tiles a job) second units of two tiles, where most waves have none.
+@pytest.mark.parametrize("nrows,ncols,tile16", [(288, 512, True), (288, 512, False), (96, 256, False), (2048, 512, True)])
+def test_moe_mma_phases_of_several_jobs_a_block(dev, oracle, nrows, ncols, tile16):
+    """a row's bits do not depend on the jobs that share its phase: a long list against the same jobs in lists of one a block at most"""
+    print(f"case moe_mma phases nrows={nrows} ncols={ncols} tile16={tile16}", flush=True)
+    sizes = ([1, 16, 17, 0, 2, 64, 3, 3, 33, 0, 0, 5, 48, 9, 1, 32, 15, 31, 2, 8] * 60)[:1190 if nrows < 2048 else 610]
+    rng = np.random.default_rng(757 + nrows + ncols)
+    nexp, stride = 5, nrows * ncols // 256 * 110
+    w = random_iq3s(rng, nexp * nrows * ncols // 256, dmax=2e-2)
+    x16 = rng.standard_normal((400, ncols)).astype(np.float16)
+    jobs, total = make_jobs(rng, nexp, 400, sizes)
+
+    def out_of(some):
+        return dev.moe_mma(w, stride, nrows, ncols, some, x16, total, packed=True, down=True, cap=len(some), tile16=tile16)
+
+    got = out_of(jobs)
+    few = 60
+    for j0 in (0, len(jobs) // 2, len(jobs) - few):
+        at = np.concatenate([j[2 + PF:2 + PF + int(j[1])] for j in jobs[j0:j0 + few]])
+        assert np.array_equal(got[at].view(np.uint32), out_of(jobs[j0:j0 + few])[at].view(np.uint32)), f"jobs {j0} .. {j0 + few}"
+    n = sum(sizes[:8])
+    assert rel_l2(got[:n], oracle.moe_mma(w, stride, nrows, ncols, jobs[:8], PF, x16, total)[:n]) <= 1e-5, "f16 operands are the oracle's"
+
+
 # More than 524,288 columns of all rows (on 256 CUs): a thread of the combine takes four columns, unless the rows are no whole
 # 16-byte pieces or a buffer is not aligned to them (`off`: by how many floats part, sh and out are shifted).
 @pytest.mark.parametrize("T,n,topk,off", [(257, 2048, 10, (0, 0, 0)), (300, 2048, 1, (0, 0, 0)), (410, 1300, 3, (0, 0, 0)), (140, 3844, 16, (0, 0, 0)), (1100, 512, 8, (0, 0, 0)),
