@@ -1059,11 +1059,12 @@ static int layer_fused(const fnx_moe_layer* L, const float* x, int T, float* out
     prof_mark(1, s);
     // a wait for another block gives up after this many ticks of the 100 MHz wall clock (FNX_WINDOW_WAIT_TICKS: for tests of the error path)
     static const long long wait_ticks = env_int("FNX_WINDOW_WAIT_TICKS", 20000000, 0, 2000000000);
+    const int nb = cu_count();   // one block a CU; a row has at least sixteen (moe_window_plan.h)
     WindowArgs wa{ff, L->nexp, L->topk, T, n, x, L->router, L->router_bf16,
                         (const uint8_t*) L->gu.p, L->gu_stride, (const uint8_t* const*) L->gu.ep, q8sh ? nullptr : (const uint8_t*) L->sh_gu.p,
                         (const uint8_t*) L->down.p, L->down_stride, (const uint8_t* const*) L->down.ep, q8sh ? nullptr : (const uint8_t*) L->sh_down.p,
                         sh_part, ws->logits, ws->topi, ws->topw, (uint8_t*) ws->xq, (uint32_t*) ws->gu, out, ws->sync, live,
-                        ws->jobs_gu, ws->jobs_dn, ws->njobs, wait_ticks};
+                        ws->jobs_gu, ws->jobs_dn, ws->njobs, wait_ticks, win_work(nb, T, L->nexp, L->topk, !q8sh, ff)};
     if (next && next->x) {
         wa.next_x = next->x;
         wa.next_w = next->w;
@@ -1073,8 +1074,6 @@ static int layer_fused(const fnx_moe_layer* L, const float* x, int T, float* out
         wa.pre_o = next->pre_o;
         wa.pre_w = next->pre_w;
     }
-    // one block a CU; a row's blocks are a power of two of at least sixteen (moe_window_plan.h)
-    const int nb = cu_count();
     const auto launch = [&](auto sbr, auto dec) {
         constexpr int SBR = decltype(sbr)::value;
         constexpr bool DEC = decltype(dec)::value;

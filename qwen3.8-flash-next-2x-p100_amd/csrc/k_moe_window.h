@@ -3,12 +3,12 @@
 // combine's chains. The reference runs these as operators of their own inside a captured graph; on this GPU every
 // kernel boundary costs the start and the drain of a launch that streams ~100 MB (a fifth of its time), and the
 // dependencies between the phases are local to a window row: a row's router logits are needed by that row's blocks only,
-// and a row's h (8 KB) is made and used by the same sixteen blocks. So a block belongs to one row for the whole launch
+// and a row's h (8 KB) is made and used by the same blocks (sixteen or more). So a block belongs to one row for the whole launch
 // and the row's blocks hand over through two arrival counters in the workspace - never the whole grid.
 //
 //   phase R   block (t, g) computes row t's logits of its slice of the router (slice g is read by the blocks g of all
 //             rows, which share an XCD and its L2: the router leaves HBM once) and the q8_1 blocks of x[t] (kept in LDS),
-//             then arrives on the row's first counter; the shared expert's gate|up item, which needs no pick, runs
+//             then arrives on the row's first counter; the shared expert's gate|up items, which need no pick, run
 //             while the row's logits gather.
 //   phase G   every block ranks its row itself (slices of 64 experts a wave, one wave merges) and sweeps its gate|up
 //             items - (32 values of h) x (matrix), sixteen waves x four units (gate rows 2 i, 2 i + 1 and their up rows) a
@@ -80,6 +80,7 @@ struct WindowArgs {
     fnx_job* jobs_dn;
     int* njobs;
     long long wait_ticks;     // budget of a wait for another block, in ticks of the 100 MHz wall clock
+    WinWork work;             // win_work of the grid and all T rows
     // What follows the window in a decoder, done here by the row's last block instead of by a launch of its own
     // (fnx_add_norm_q8's pass: the residual add, the next RMS norm, its q8_1 rows). next_x null: not wanted.
     float* next_x = nullptr;            // [T][rows]: x[t] += out[t] for the rows that count
@@ -249,11 +250,19 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     const int T = a.T, topk = a.topk, nexp = a.nexp, LS = nexp + 1, P = T * topk;
     const int Tl = a.live ? uniform(max(0, min(*a.live, T))) : T;
     if (Tl <= 0) return;
-    const WinPlan pl = win_plan((int) gridDim.x, Tl, nexp, topk, a.gu_shared != nullptr, a.ff);
-    const int t = (int) blockIdx.x / pl.G, g = (int) blockIdx.x - t * pl.G;
+    // the launch's plan where all of its rows count; asked for again where a later phase wants it: kept, its dozen values cost the
+    // launch's other scalars their registers, and worked out by every block they cost it half a microsecond before its first load
+    auto work = [&]() -> WinWork {
+        int rows = Tl;
+        asm volatile("" : "+s"(rows));
+        if (rows == T) return a.work;
+        return win_work((int) gridDim.x, rows, nexp, topk, a.gu_shared != nullptr, a.ff);
+    };
+    const WinWork pl = work();
+    const int t = win_row(pl, (int) blockIdx.x), g = (int) blockIdx.x - t * pl.G;
     if (t >= Tl) return;
     WIN_TS(0);
-    const int k0 = pl.k0, nk = pl.nk, qpp = pl.qpp;
+    const int qpp = a.ff / 32;   // blocks of 32 h values a pair
     unsigned* const srow = a.sync + WS_ROW0 + t * win_lines(Tl) * WS_ROW_STRIDE;   // the row's first line
     // the line this block arrives on (worked out where it is wanted: one value fewer to keep through the launch)
     auto arrival_line = [&] { return srow + (g & (win_lines(Tl) - 1)) * WS_ROW_STRIDE; };
@@ -402,21 +411,24 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     // ---------------------------------------------------------------- phase G
     // the lane's sub-block of the row's activations
     const typename F::Act xa = F::act_x(S.xq, lane);
-    const int I0 = g * pl.ipb, I1 = min(pl.per_row, I0 + pl.ipb), nsweep = max(I1 - I0, 0);   // this block's items of its row
+    // this block's items of its row: the shared expert's first, which need no pick
+    const int s0 = win_shared_first(pl, g), nsh = max(min(pl.shared - s0, pl.spb), 0), I0 = win_routed_first(pl, g);
+    const int nsweep = nsh + pl.ipb + (g < pl.more);
     const typename F::Offs o = F::offs(lane);
     const int uo_g = wave * 2 * F::UNIT, uo_u = uo_g + a.ff * F::UNIT;   // the wave's gate units and up units from an item's first gate unit
     struct Item {
         int j, k;   // block of 32 h values, matrix (0: the shared expert's, k: pick k - 1's)
     };
-    auto item_of = [&](int I) {
+    auto item_of = [&](int q) {   // the block's q-th
+        const int I = I0 + q - nsh;
         Item m;
-        m.j = uniform(I / nk);
-        m.k = k0 + I - m.j * nk;
+        m.j = q < nsh ? s0 + q : uniform(I / topk);
+        m.k = q < nsh ? 0 : 1 + I - m.j * topk;
         return m;
     };
-    auto step = [&](Item& m) {
+    auto step = [&](Item& m) {   // (routed items)
         if (++m.k > topk) {
-            m.k = k0;
+            m.k = 1;
             ++m.j;
         }
     };
@@ -445,9 +457,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         }
         return true;
     };
-    Item ma = item_of(I0);
-    const bool early = nsweep > 0 && ma.k == 0;   // the run starts with a shared expert's item: no pick needed to ask for it
-    if (early) issue_from(a.gu_shared, ma.j);
+    if (nsh > 0) issue_from(a.gu_shared, s0);
     const int sc_shift = 4 * (lane & 1);
     // where a lane's sum goes after reduce4_units: the 16-lane rows hold gate 2 i, up 2 i, gate 2 i + 1, up 2 i + 1
     const int zidx = (lane & 16 ? 32 : 0) + 2 * wave + (lane >> 5);
@@ -473,7 +483,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
                 return __ballot(f < q + 1) == 0ull;
             }))
             return false;
-        const Item m = item_of(I0 + q);
+        const Item m = item_of(q);
         const int pair = m.k > 0 ? t * topk + m.k - 1 : P + t;
         if (lane < 32) {
             const float h = silu_f(S.hgu[slot][lane]) * S.hgu[slot][32 + lane];
@@ -501,9 +511,9 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         return true;
     };
     int sw = 0;
-    if (early) {   // the shared expert's item while the row's logits gather
-        if (!decode(0)) return;
-        sw = 1;
+    for (; sw < nsh; ++sw) {   // the shared expert's items while the row's logits gather
+        if (!decode(sw)) return;
+        if (sw + 1 < nsh) issue_from(a.gu_shared, s0 + sw + 1);
     }
     WIN_TS(13);
     // The row's picks (moe.cuh:382-411: greater value first, the lower index on a tie; w_k = exp(l_k - l_0) / sum in pick
@@ -650,12 +660,9 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     // Every wave of the block makes the same sweeps: each slot sees all sixteen arrive. An item's loads are asked for when
     // the item before it has been decoded; two sweeps later the wave whose turn it is makes the sweep's q8_1 block.
     if (nsweep > 0) {
-        if (early) {
-            if (nsweep > 1) {
-                step(ma);
-                if (!issue(ma)) return;
-            }
-        } else if (!issue(ma)) return;
+        Item ma = item_of(nsh);
+        if (nsh < nsweep)
+            if (!issue(ma)) return;
         for (; sw < nsweep; ++sw) {
             // the oldest wave of a SIMD issues first, so a block's waves drift apart sweep by sweep: every wave takes each of
             // the four priorities in turn
@@ -690,7 +697,8 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     // w % dwaves and, of the row's trips, every TG-th from trip w / dwaves on; the sums meet in LDS and the units' first
     // waves run the combine's chain over them in the picks' order (the same operations on the same values).
     // (Only where a wave has one unit: the other forms of the phase are compiled without it.)
-    const int R = pl.R;
+    const WinWork pd = work();
+    const int R = pd.R;
     const int kb = lane % SBR, gl = lane / SBR;
     // trip 0 is the shared expert's, trips 1 .. topk the picks in order
     auto down_matrix = [&](int trip) -> const uint8_t* {
@@ -705,10 +713,11 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     auto down_phase = [&](auto RC) -> bool {
     constexpr int RALL = decltype(RC)::value, RR = RALL < F::MAXR ? RALL : F::MAXR;   // the wave's units, and of them a pass over the row's trips
     int TG = 1;
-    if constexpr (RALL == 1) TG = pl.dwaves <= WN_WAVES / 2 && WN_WAVES % pl.dwaves == 0 ? WN_WAVES / pl.dwaves : 1;
-    const bool dwave = TG > 1 || wave < pl.dwaves;
-    const int tgrp = TG > 1 ? wave / pl.dwaves : 0, uw = TG > 1 ? wave - tgrp * pl.dwaves : wave;
-    int u0 = g * pl.upb + uw * RALL;   // this wave's units of every matrix
+    if constexpr (RALL == 1) TG = pd.dwaves <= WN_WAVES / 2 && WN_WAVES % pd.dwaves == 0 ? WN_WAVES / pd.dwaves : 1;
+    const int tgrp = TG > 1 ? wave / pd.dwaves : 0, uw = TG > 1 ? wave - tgrp * pd.dwaves : wave;
+    const int uat = g * pd.upb + uw * RALL;
+    const bool dwave = TG > 1 || (wave < pd.dwaves && uat < a.ff);
+    int u0 = min(uat, a.ff - RALL);   // this wave's units of every matrix (inside it, whatever the plan's last block has)
     auto trip_of = [&](int i) { return first + tgrp + i * TG; };   // the wave's i-th trip
     typename F::Raw B[NB][RR];
     auto issue_trip = [&](typename F::Raw(&buf)[RR], int trip) {
@@ -779,7 +788,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     };
     if (dwave && wave != 0) first_trips();
     if (wave == 0) {
-        const bool ok = win_wait_lines(&srow[1], win_lines(Tl), (unsigned) pl.nbi, a.wait_ticks, serr);
+        const bool ok = win_wait_lines(&srow[1], win_lines(Tl), (unsigned) pd.nbi, a.wait_ticks, serr);
         if (lane == 0) __hip_atomic_store(&S.hready, ok ? 1 : -1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (dwave) first_trips();
     }
@@ -932,7 +941,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     __syncthreads();
     if (tid == 0) {
         const unsigned done = __hip_atomic_fetch_add(&srow[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (done == (unsigned) pl.G - 1) {
+        if (done == (unsigned) work().G - 1) {
             for (int l = 0; l < win_lines(Tl); ++l) __hip_atomic_store(&srow[l * WS_ROW_STRIDE + 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&srow[2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             S.fin = (int) __hip_atomic_fetch_add(&a.sync[WS_FIN], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

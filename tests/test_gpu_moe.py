@@ -88,6 +88,13 @@ def test_moe_verify_layer_shapes(dev, oracle, n, ff, nexp, topk, T, packed):
     check_layer(dev, oracle, n, ff, nexp, topk, T, 910 + T, packed)
 
 
+# rows that a power of two of blocks a row would leave part of the grid without: blocks a row in fours, units of the down matrices that do not
+# divide among them (on 256 CUs 48, 36, 28, 24 and 20 blocks a row; units of two and of four a wave, and one)
+@pytest.mark.parametrize("ff,nexp,topk,T", [(512, 64, 10, 5), (512, 512, 16, 7), (512, 40, 10, 9), (512, 24, 10, 12), (1024, 16, 4, 9), (1024, 24, 14, 11), (256, 24, 8, 10)])
+def test_moe_window_over_all_blocks(dev, oracle, ff, nexp, topk, T):
+    check_layer(dev, oracle, 2048, ff, nexp, topk, T, 930 + T + ff, True)
+
+
 @pytest.mark.parametrize("packed", [False, True])
 def test_moe_verify_layer_with_experts_from_pointer_tables(dev, oracle, packed):
     """fnx_dw.ep: an expert's matrix by a table of device pointers instead of base + e * stride (an engine whose experts

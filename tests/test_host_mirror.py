@@ -50,6 +50,16 @@ def test_window_plan(tmp_path):
     assert r.stdout.startswith("ok "), r.stdout
 
 
+def test_window_work(tmp_path):
+    """the window's work as its kernel deals it, over any number of blocks a row: every router row and item once, every unit of the down
+    matrices, and the h hand-over waits for exactly the blocks that arrive"""
+    exe = str(tmp_path / "moe_window_work_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I", os.path.join(fnx_gpu.PKG_DIR, "csrc"), "-o", exe,
+                    os.path.join(HERE, "moe_window_work_check.cpp")], check=True, capture_output=True, text=True)
+    r = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120)
+    assert r.stdout.startswith("ok "), r.stdout
+
+
 def test_q8s_split(tmp_path):
     """the dense Q8_0 mat-vec's walk of a quarter of the columns, compiled for the host: no load leaves the quarter and every
     double step is taken once, in order, for every width of 256s (1,280 and 2,560 have a short last batch)"""
