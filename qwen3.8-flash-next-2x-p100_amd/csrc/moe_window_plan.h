@@ -52,8 +52,9 @@ FNX_HOST_DEVICE inline WinPlan win_plan(int nb, int Tl, int nexp, int topk, bool
     return p;
 }
 // The work as the window deals it. Two things of the cut above cost time. A power of two of blocks a row leaves up to 44 % of the grid
-// without work at 5 .. 7 and 9 .. 15 rows: blocks are taken in fours up to nb / Tl where that makes a block's routed items a fifth
-// fewer and the even cut leaves it more than half a unit of the down matrices a wave (in fours: the blocks that take the same router
+// without work at 5 .. 7 and 9 .. 15 rows: blocks are taken in fours up to nb / Tl where that makes a block's routed items fewer
+// (only where a fifth fewer, 8 of 256 experts of width 1,024 at 11 rows IQ3_S 64.8 us / this 59.7, Q8_0 182.7 / 166.2, 512 wide 83.9 / 73.8, but Q5_K 12
+// rows 46.3 / 47.9; where they stay as many, Q8_0 3 to 8 % faster and Q4_K 1 to 4 % slower) and the even cut leaves it more than half a unit of the down matrices a wave (in fours: the blocks that take the same router
 // rows and shared items then lie on one or two of the eight XCDs, whose L2 they share; 252 blocks at 21 a row were slower than 192
 // at 16: q4_k, 12 rows 47.1 -> 51.0 us, at 20 a row 47.2). And the shared expert's items need no pick, so they are dealt apart from the routed ones, to
 // run while the row's logits gather: to the row's last blocks where there are more blocks than items, which have the fewest
@@ -77,7 +78,7 @@ FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool
     const WinPlan e = win_plan(nb, Tl, nexp, topk, shared, ff);
     const int lg = win_log2(e.G), all = nb / Tl / 4 * 4, routed = e.qpp * topk;
     WinWork p{Tl, e.G, routed, routed >> lg, 0, shared ? e.qpp : 0, 0, 0, e.rpb, e.upb, e.R, e.dwaves};
-    if (all > e.G && e.upb > WN_WAVES / 2 && 5 * ((routed + all - 1) / all) <= 4 * ((routed + e.G - 1) >> lg)) {
+    if (all > e.G && e.upb > WN_WAVES / 2 && (routed + all - 1) / all < (routed + e.G - 1) >> lg) {
         p.G = all;
         p.ipb = routed / all;
         p.rpb = (nexp + all - 1) / all;
