@@ -81,7 +81,6 @@ struct WindowArgs {
     int* njobs;
     long long wait_ticks;     // budget of a wait for another block, in ticks of the 100 MHz wall clock
     WinWork work;             // win_work of the grid and all T rows
-    WinWork fewer[FNX_MAXT - 1];   // and, with live, of 1 .. T - 1 of them
     // What follows the window in a decoder, done here by the row's last block instead of by a launch of its own
     // (fnx_add_norm_q8's pass: the residual add, the next RMS norm, its q8_1 rows). next_x null: not wanted.
     float* next_x = nullptr;            // [T][rows]: x[t] += out[t] for the rows that count
@@ -251,13 +250,13 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
     const int T = a.T, topk = a.topk, nexp = a.nexp, LS = nexp + 1, P = T * topk;
     const int Tl = a.live ? uniform(max(0, min(*a.live, T))) : T;
     if (Tl <= 0) return;
-    // the plan of the rows that count, as the launch brings it; asked for again where a later phase wants it: kept, its dozen values cost
-    // the launch's other scalars their registers, and worked out by every block they cost it half a microsecond before its first load
+    // the launch's plan where all of its rows count; asked for again where a later phase wants it: kept, its dozen values cost the
+    // launch's other scalars their registers, and worked out by every block they cost it half a microsecond before its first load
     auto work = [&]() -> WinWork {
         int rows = Tl;
         asm volatile("" : "+s"(rows));
         if (rows == T) return a.work;
-        return a.fewer[rows - 1];
+        return win_work((int) gridDim.x, rows, nexp, topk, a.gu_shared != nullptr, a.ff);
     };
     const WinWork pl = work();
     const int t = win_row(pl, (int) blockIdx.x), g = (int) blockIdx.x - t * pl.G;
