@@ -45,12 +45,14 @@ struct JmOneLds {   // for one group of 16 units: 71 to 74 KB, two blocks a CU
 
 // the job's activations of a wave's four sub-blocks: token col's bytes 8 kg .. 8 kg + 7 and its block scale. A lane past the job's tokens
 // loads the first one's, and its column of the products is thrown away: loads under a condition go out one by one, a trip to
-// memory each
+// memory each. (The first one's row is taken by the whole wave: read under the condition it would be the first lane's past the job's
+// tokens, and what an entry past a job's rows holds names no row)
 struct JmActs {
     uint32_t lo[4], hi[4], dh[4];
     template <int SBR = 64>
     __device__ __forceinline__ void load(const uint8_t* __restrict__ y, int yi, bool on, int sb0, int kg) {
-        const uint8_t* yr = y + ((size_t) (on ? yi : uniform(yi)) * SBR + sb0) * FNX_Q8_1_BLOCK;
+        const int first = uniform(yi);
+        const uint8_t* yr = y + ((size_t) (on ? yi : first) * SBR + sb0) * FNX_Q8_1_BLOCK;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const uint8_t* yb = yr + s * FNX_Q8_1_BLOCK;

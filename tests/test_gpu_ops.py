@@ -365,6 +365,29 @@ def test_mmvq_lone_calls_over_shorter_rows(dev, oracle, ncols, units, counts):
         assert np.array_equal(got[o], dev.mmvq(w, nrows * ncols // 256 * 110, nrows, ncols, jobs[j:j + 1], yq, at, packed=True)[o])
 
 
+# what a job holds past its rows names no row: nothing is read or written through it (2,048 columns: a group of 16 rows a block, blocks that
+# stream; shorter rows: whole groups of units and one that ends early)
+@pytest.mark.parametrize("nrows,ncols", [(1024, 2048), (8192, 2048), (1024, 512), (2080, 256), (48, 1024)])
+def test_mmvq_entries_past_a_jobs_rows_mean_nothing(dev, oracle, nrows, ncols):
+    print(f"case entries past the rows nrows={nrows} ncols={ncols}", flush=True)
+    rng = np.random.default_rng(424 + nrows + ncols)
+    counts, stride = [3, 1, 16, 2, 9], nrows * ncols // 256 * 110
+    w = random_iq3s(rng, 2 * nrows * ncols // 256)
+    yq = oracle.quantize_q8_1(rng.standard_normal((16, ncols)).astype(np.float32))
+    jobs = np.zeros(len(counts), dtype=JOB_DTYPE)
+    at = 0
+    for j, n in enumerate(counts):
+        jobs["w"][j], jobs["n"][j] = j % 2, n
+        jobs["y"][j, :n] = rng.permutation(16)[:n]
+        jobs["out"][j, :n] = np.arange(at, at + n)
+        at += n
+    want = dev.mmvq(w, stride, nrows, ncols, jobs, yq, at, packed=True)
+    assert rel_l2(want, oracle.mmvq(w, stride, nrows, ncols, jobs, yq, at)) <= 1e-6, "a row's terms in another order"
+    for j, n in enumerate(counts):
+        jobs["y"][j, n:] = jobs["out"][j, n:] = (1 << 30, -1 << 31)[j % 2]
+    assert np.array_equal(dev.mmvq(w, stride, nrows, ncols, jobs, yq, at, packed=True), want)
+
+
 # ---------------------------------------------------------------- head, drafting, acceptance
 def test_argmax_full_vocabulary(dev, oracle):
     rng = np.random.default_rng(500)
