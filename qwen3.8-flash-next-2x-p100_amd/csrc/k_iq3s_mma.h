@@ -49,13 +49,14 @@ struct JmOneLds {   // for one group of 16 units: 71 to 74 KB, two blocks a CU
 // tokens, and what an entry past a job's rows holds names no row)
 struct JmActs {
     uint32_t lo[4], hi[4], dh[4];
+    // (sub-blocks sb0, sb0 + step, ..)
     template <int SBR = 64>
-    __device__ __forceinline__ void load(const uint8_t* __restrict__ y, int yi, bool on, int sb0, int kg) {
+    __device__ __forceinline__ void load(const uint8_t* __restrict__ y, int yi, bool on, int sb0, int kg, int step = 1) {
         const int first = uniform(yi);
         const uint8_t* yr = y + ((size_t) (on ? yi : first) * SBR + sb0) * FNX_Q8_1_BLOCK;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const uint8_t* yb = yr + s * FNX_Q8_1_BLOCK;
+            const uint8_t* yb = yr + s * step * FNX_Q8_1_BLOCK;
             lo[s] = *reinterpret_cast<const uint32_t*>(yb + 4 + 8 * kg);
             hi[s] = *reinterpret_cast<const uint32_t*>(yb + 8 + 8 * kg);
             dh[s] = *reinterpret_cast<const unsigned short*>(yb);
@@ -75,18 +76,44 @@ __device__ __forceinline__ void jm_decode(Lds& L, int i, int wave, int lane, con
     uint8_t* dst = L.tile[i] + row * (32 * SBR + 32) + sb * 32;
     *reinterpret_cast<v4u*>(dst) = lo;
     *reinterpret_cast<v4u*>(dst + 16) = hi;
-    L.sw[i][row / JM_ROWS * SBR + sb][row % JM_ROWS] = half_bits_to_float(cur.d) * (float) (int) (1u + 2u * ((cur.sc >> (4 * (lane & 1))) & 0xFu));
+    const uint32_t sc = 1u + 2u * ((cur.sc >> (4 * (lane & 1))) & 0xFu);
+    float* sw = &L.sw[i][row / JM_ROWS * SBR + sb][row % JM_ROWS];
+    if constexpr (SBR < 64) *reinterpret_cast<uint32_t*>(sw) = (uint32_t) (unsigned short) cur.d | sc << 16;
+    else *sw = half_bits_to_float(cur.d) * (float) (int) sc;
 }
-// 2. this wave's four sub-blocks of group i's 16 rows against the tokens (shorter rows: of the 16 rows that SBR / 4 waves share)
+// 2. this wave's four sub-blocks of group i's 16 rows against the tokens. Shorter rows: of the 16 rows that W = SBR / 4 waves share, sub-blocks
+// w, w + W, w + 2 W, w + 3 W, whose terms, formed as the mat-vec kernels form them, meet in the first two levels of the butterfly over a row;
+// jm_store goes through the others. A row's bits are then those of the kernels for jobs of one and two rows and of the streaming ones,
+// whatever the job's length. (In the order that the rows of 2,048 columns have they depended on it, at the same speed.)
 template <int SBR = 64, class Lds>
 __device__ __forceinline__ void jm_multiply(Lds& L, int i, int wave, int lane, const JmActs& x, const float (&dx)[4]) {
     const int col = lane & 15, kg = lane >> 4;
+    if constexpr (SBR < 64) {
+        constexpr int W = SBR / 4;
+        const int rg = wave / W;
+        float term[4][4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int sb = wave % W + s * W;
+            const long a = *reinterpret_cast<const long*>(L.tile[i] + (JM_ROWS * rg + col) * (32 * SBR + 32) + sb * 32 + 8 * kg);
+            const v4u f = *reinterpret_cast<const v4u*>(&L.sw[i][rg * SBR + sb][4 * kg]);
+            const long xb = (long) ((unsigned long) x.lo[s] | (unsigned long) x.hi[s] << 32);
+            const jm_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, xb, jm_v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) term[s][v] = (half_bits_to_float(f[v]) * dx[s]) * (float) __mul24(d[v], (int) (f[v] >> 16));
+        }
+        float z[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) z[v] = (term[0][v] + term[2][v]) + (term[1][v] + term[3][v]);
+        *reinterpret_cast<float4*>(L.red[i][wave][lane]) = make_float4(z[0], z[1], z[2], z[3]);
+        return;
+    }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const int rg = wave / (SBR / 4), sb = 4 * (wave % (SBR / 4)) + s;
-        const long a = *reinterpret_cast<const long*>(L.tile[i] + (JM_ROWS * rg + col) * (32 * SBR + 32) + sb * 32 + 8 * kg);
-        const float4 f = *reinterpret_cast<const float4*>(&L.sw[i][rg * SBR + sb][4 * kg]);
+        const int sb = 4 * wave + s;
+        const long a = *reinterpret_cast<const long*>(L.tile[i] + col * JM_ROWLD + sb * 32 + 8 * kg);
+        const float4 f = *reinterpret_cast<const float4*>(&L.sw[i][sb][4 * kg]);
         const long xb = (long) ((unsigned long) x.lo[s] | (unsigned long) x.hi[s] << 32);
         const jm_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, xb, jm_v4i{0, 0, 0, 0}, 0, 0, 0);
         // a term is d_w (1 + 2 s) d_x sumi: the reference's (d_w d_x) (float) (sumi (1 + 2 s)) with the factors taken in another order
@@ -97,14 +124,26 @@ __device__ __forceinline__ void jm_multiply(Lds& L, int i, int wave, int lane, c
     }
     *reinterpret_cast<float4*>(L.red[i][wave][lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
 }
-// 3. one wave adds group i's sums of the sixteen (shorter rows: of the SBR / 4 from wave w0 on) in wave order and stores the tile
+// 3. one wave adds group i's sums of the sixteen in wave order (shorter rows: of the SBR / 4 from wave w0 on, in the butterfly's) and stores the tile
 template <int SBR = 64, class Lds>
 __device__ __forceinline__ void jm_store(const Lds& L, int i, int lane, float* op, int w0 = 0) {
-    float4 z = *reinterpret_cast<const float4*>(L.red[i][w0][lane]);
+    constexpr int W = SBR / 4;
+    auto sum_of = [&](int w) { return *reinterpret_cast<const float4*>(L.red[i][w0 + w][lane]); };
+    auto plus = [](float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+    float4 z;
+    if constexpr (SBR == 64) {
+        z = sum_of(0);
 #pragma unroll
-    for (int w = 1; w < SBR / 4; ++w) {
-        const float4 p = *reinterpret_cast<const float4*>(L.red[i][w0 + w][lane]);
-        z.x += p.x, z.y += p.y, z.z += p.z, z.w += p.w;
+        for (int w = 1; w < W; ++w) z = plus(z, sum_of(w));
+    } else {
+        float4 p[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) p[w] = sum_of(w);
+#pragma unroll
+        for (int o = W / 2; o >= 1; o /= 2)
+#pragma unroll
+            for (int w = 0; w < o; ++w) p[w] = plus(p[w], p[w + o]);
+        z = p[0];
     }
     op[0] = z.x, op[1] = z.y, op[2] = z.z, op[3] = z.w;
 }
@@ -155,7 +194,7 @@ __device__ __forceinline__ void jm_segment(JmLds& L, const uint8_t* __restrict__
 
 // 16 units of a matrix of nunits (16 rows, or 64 / SBR times as many shorter ones) against the job's tokens, and nothing after them: a wave
 // decodes one, no ring and no second group. Past the last unit: that one again, its rows not stored. Over rows of 2,048 columns the sums are
-// jm_segment's, bit for bit.
+// jm_segment's bit for bit, over shorter ones butterfly_sum's.
 template <int SBR, class Between>
 __device__ __forceinline__ void jm_group(JmOneLds<SBR>& L, const uint8_t* __restrict__ we, int g, int nunits, const fnx_job* jb, int n, const uint8_t* __restrict__ y,
                                          float* __restrict__ out, int out_stride, Between between) {
@@ -164,7 +203,8 @@ __device__ __forceinline__ void jm_group(JmOneLds<SBR>& L, const uint8_t* __rest
     const int yi = jb->y[col], oi = jb->out[col];
     const PackedSub cur = load_packed_buf(matrix_rsrc(we), min(16 * g + wave, nunits - 1) * UNIT_BYTES, packed_voffs(lane));
     JmActs x;
-    x.load<SBR>(y, yi, col < n, 4 * (wave % (SBR / 4)), kg);
+    if constexpr (SBR < 64) x.load<SBR>(y, yi, col < n, wave % (SBR / 4), kg, SBR / 4);
+    else x.load<SBR>(y, yi, col < n, 4 * wave, kg);
     between();
     jm_decode<SBR>(L, 0, wave, lane, cur);
     __syncthreads();   // the rows are in LDS

@@ -365,6 +365,36 @@ def test_mmvq_lone_calls_over_shorter_rows(dev, oracle, ncols, units, counts):
         assert np.array_equal(got[o], dev.mmvq(w, nrows * ncols // 256 * 110, nrows, ncols, jobs[j:j + 1], yq, at, packed=True)[o])
 
 
+# the same kernel at row counts that are multiples of 16 but not of a group of sixteen units: whole groups and one that ends early, jobs of no,
+# one, two and more rows. A row's terms are added in the butterfly's order whatever the job's length: the oracle's bits, and those of the
+# same rows in a job of their own and over ggml's blocks
+@pytest.mark.parametrize("ncols,units", [(256, 2), (256, 18), (256, 34), (512, 4), (512, 20), (512, 36), (1024, 8), (1024, 24), (1024, 40)])
+@pytest.mark.parametrize("counts", [[2, 0, 9], [5], [16], [3, 1, 16, 7, 1, 0, 2, 4]])
+def test_mmvq_shorter_rows_add_up_in_one_order(dev, oracle, ncols, units, counts):
+    nrows = units * (2048 // ncols)
+    assert nrows % 16 == 0 and units % 16, "a case for the kernel of sixteen units a block, its last group not whole"
+    print(f"case shorter rows' order nrows={nrows} ncols={ncols} counts={counts}", flush=True)
+    rng = np.random.default_rng(425 + units + ncols)
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, 2 * nrows * ncols // 256)
+    yq = oracle.quantize_q8_1(rng.standard_normal((16, ncols)).astype(np.float32))
+    jobs = np.zeros(len(counts), dtype=JOB_DTYPE)
+    at = 0
+    for j, n in enumerate(counts):
+        jobs["w"][j], jobs["n"][j] = j % 2, n
+        jobs["y"][j, :n] = rng.permutation(16)[:n]
+        jobs["out"][j, :n] = np.arange(at, at + n)
+        at += n
+    got = dev.mmvq(w, stride, nrows, ncols, jobs, yq, at, packed=True)
+    assert np.array_equal(got.view(np.uint32), oracle.mmvq(w, stride, nrows, ncols, jobs, yq, at).view(np.uint32))
+    assert np.array_equal(got.view(np.uint32), dev.mmvq(w, stride, nrows, ncols, jobs, yq, at).view(np.uint32)), "ggml's blocks"
+    for j, n in enumerate(counts):   # the job's last row alone
+        if n > 1:
+            one = jobs[j:j + 1].copy()
+            one["n"], one["y"][0, 0], one["out"][0, 0] = 1, jobs["y"][j, n - 1], 0
+            assert np.array_equal(got[jobs["out"][j, n - 1]].view(np.uint32), dev.mmvq(w, stride, nrows, ncols, one, yq, 1, packed=True)[0].view(np.uint32))
+
+
 # what a job holds past its rows names no row: nothing is read or written through it (2,048 columns: a group of 16 rows a block, blocks that
 # stream; shorter rows: whole groups of units and one that ends early)
 @pytest.mark.parametrize("nrows,ncols", [(1024, 2048), (8192, 2048), (1024, 512), (2080, 256), (48, 1024)])
