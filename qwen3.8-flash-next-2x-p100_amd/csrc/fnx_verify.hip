@@ -1153,8 +1153,9 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
         const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE, most = 8 * std::max(1, cu_count() / 8);
         const bool along = form == GemvRows::large_tiles || spread;
         const int blocks = spread ? most : std::min((ntt * net + 7) / 8 * 8, most), items = along ? left * T : 0;
-        if (blocks >= ntt * net) k_gemv_rows_mfma<false><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items, spread);
-        else k_gemv_rows_mfma<true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items, 1);
+        if (blocks < ntt * net) k_gemv_rows_mfma<true, true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items);
+        else if (spread) k_gemv_rows_mfma<false, true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items);
+        else k_gemv_rows_mfma<false, false><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items);
         if (along) return launch_status(who);
         const dim3 gm((left + GM_WAVES * GR_ROWS - 1) / (GM_WAVES * GR_ROWS), (T + FNX_MAXT - 1) / FNX_MAXT);
         k_gemv_rows_many<false><<<gm, GM_WAVES * 64, 0, s>>>(W, x, y, rows, n, T, net * RM_TILE);

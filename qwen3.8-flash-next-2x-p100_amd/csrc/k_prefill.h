@@ -392,31 +392,43 @@ __global__ void __launch_bounds__(RS_THREADS) k_gemv_rows_mfma16(const float* __
 // A CU has one block (its rings fill the LDS), which takes its tiles one after another (MANY): the next tile's first steps come in
 // behind the last ones of the tile before, and its sums go through a place of their own, so that a tile's start is not waited for and
 // its end is the exchange alone. With a block a tile the CU stood still from one tile's last MFMA to the next one's first: 513 rows of 2,048
-// columns, 4,096 rows of x 95 -> 88 us over weights in turn, 1,900 50.5 -> 46.6; two tiles a block the same (700: 24.4), and where every block
-// has one tile that form is 4 % behind the plain one (its sums in the ring, nothing asked for past the end).
-// Bound by the MFMAs and the loads behind them: some 10.5 us a tile where the MFMAs alone take 6.8, the operands' reads 0.7.
+// columns, 4,096 rows of x 95 -> 88 us over weights in turn, 1,900 51.5 -> 45.1 (the launch alone); two tiles a block the same (700: 24.4), and where
+// every block has one tile that form is 4 % behind the plain one (its sums in the ring, nothing asked for past the end).
+// Bound by the MFMAs and the loads behind them: of a chain of tiles some 11 us each (eight a CU: 88), where the MFMAs alone take 6.8, the operands'
+// reads 0.7; a tile alone 14.9 with the launch's start and end.
 // The weight rows past the last full 32 (the router's 513th) are items of such a row against one row of x, added up while the first
-// steps are on their way: where a row of tiles has a wave for each of its items, and a block one tile, those; else dealt to all waves of the grid.
+// steps are on their way: where a row of tiles has a wave for each of its items, and a block one tile, those, one a wave at most; else dealt to all
+// waves of the grid (SPREAD), T / 1,024 a wave for the router's one row: 8,192 rows of x 195 -> 176 us against a launch of a block a tile, 65,535 1,516 -> 1,401.
 typedef float v32f __attribute__((ext_vector_type(32)));
 constexpr int RM_WAVES = 4, RM_THREADS = RM_WAVES * 64, RM_STEP = 8 * 1024, RM_RING = 4, RM_PART = 2 * 4 * 64 * 16;   // (RM_PART: a wave's sums of two chains)
-template <bool MANY>
+template <bool MANY, bool SPREAD>
 __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) k_gemv_rows_mfma(const float* __restrict__ W, const float* __restrict__ x,
                                                                                                          float* __restrict__ y, int rows, int n, int T, int ntt,
-                                                                                                         int net, int items, int spread) {
+                                                                                                         int net, int items) {
     __shared__ __align__(16) uint8_t lds[RM_WAVES * RM_RING * RM_STEP];
     __shared__ __align__(16) uint8_t red[MANY ? RM_WAVES * RM_PART : 16];   // the waves' sums of two chains at a tile's end
     const int wave = uniform((int) (threadIdx.x >> 6)), lane = threadIdx.x & 63;
     // Which tiles: block ids go round the eight XCDs, each with an L2 of its own, so an XCD's blocks are given an eighth of the tiles in
-    // patches of 4 x 8 (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them), a patch's tiles side by side.
+    // patches of 4 x 8 (1 MB of x and 2 MB of W for rows of 2048: its L2 holds them), a patch's tiles side by side. Several tiles a block: the patches
+    // go along x, so that an XCD keeps its rows of W. A block a tile: along W (513 x 512 along x 15.2 us, along W 14.9, as with a grid of whole patches,
+    // whose blocks without a tile left most CUs idle where W has few rows: 33 weight rows, 8,192 of x 71 us, 35 without them).
     const int total = ntt * net, xcd = (int) blockIdx.x % 8, per = (int) gridDim.x / 8;
-    int L = (int) ((long) total * xcd / 8) + (int) blockIdx.x / 8;
-    const int Lend = (int) ((long) total * (xcd + 1) / 8);
+    int L = (total * xcd >> 3) + (int) blockIdx.x / 8;   // (total < 2^28: x and W lie below 4 GiB each)
+    const int Lend = total * (xcd + 1) >> 3;
     int t0 = 0, e0 = 0;
-    auto tile_of = [&](int l) {
-        const int p = l / (8 * ntt), w = min(8, net - 8 * p), i = l - 8 * ntt * p, q = i / (4 * w), r = i - 4 * w * q;
-        t0 = (4 * q + r / w) * RM_TILE, e0 = (8 * p + r % w) * RM_TILE;
+    auto tile_of = [&](int l) {   // (no divisions where a patch is a whole one: a block does this before its first load)
+        if (!MANY && net % 8 == 0 && ntt % 4 == 0) {
+            const int a = (l >> 5) / (net >> 3);
+            t0 = (4 * a + ((l & 31) >> 3)) * RM_TILE, e0 = (8 * ((l >> 5) - a * (net >> 3)) + (l & 7)) * RM_TILE;
+            return;
+        }
+        int p = 0;
+        for (; l >= 8 * ntt; l -= 8 * ntt) ++p;
+        const int w = min(8, net - 8 * p), q = w == 8 ? l >> 5 : l / (4 * w), r = l - 4 * w * q, d = w == 8 ? r >> 3 : r / w;
+        t0 = (4 * q + d) * RM_TILE, e0 = (8 * p + r - w * d) * RM_TILE;
     };
-    const bool any = L < Lend;   // (a block without a tile helps with the items)
+    const bool any = L < Lend;   // (a block without a tile helps with the items where they are spread)
+    if (!SPREAD && !any) return;
     tile_of(any ? L : 0);
     const int half = n / 256, S = 2 * half;   // steps: a multiple of 16
     uint8_t* ring = lds + wave * (RM_RING * RM_STEP);
@@ -444,31 +456,39 @@ __global__ void __launch_bounds__(RM_THREADS) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int op = 0; op < 8; ++op) fetch(op, from_of(s), s);
     }
-    // The weight rows past the last full tile: items of such a row against one row of x. Spread: all of them over the waves of the grid;
-    // else a row of tiles' items go to its waves, whose x the L2 has.
-    if (items > 0) {
-        const int left = rows - net * RM_TILE, first = spread ? (int) blockIdx.x * RM_WAVES + wave : RM_WAVES * (e0 / RM_TILE) + wave;
-        const int count = spread ? items : any ? min(RM_TILE, T - t0) * left : 0, by = spread ? (int) gridDim.x * RM_WAVES : RM_WAVES * net;
-        for (int item = first; item < count; item += by) {
-            const int at = left == 1 ? item : item / left, it = spread ? at : t0 + at, irow = net * RM_TILE + item - at * left;
-            const float4 *wp = reinterpret_cast<const float4*>(W + (size_t) irow * n) + lane, *xp = reinterpret_cast<const float4*>(x + (size_t) it * n) + lane;
-            float v = 0.f;
-            for (int c0 = 0; c0 < n / 4; c0 += 8 * 64) {
-                float4 wv[8], xv[8];
+    // The weight rows past the last full tile: items of such a row against one row of x. SPREAD: all of them over the waves of the grid;
+    // else a row of tiles' items go to its waves, one at most, whose x the L2 has.
+    auto item_of = [&](int it, int irow, bool on) {
+        const float4 *wp = reinterpret_cast<const float4*>(W + (size_t) irow * n) + lane, *xp = reinterpret_cast<const float4*>(x + (size_t) it * n) + lane;
+        float v = 0.f;
+        for (int c0 = 0; c0 < n / 4; c0 += 8 * 64) {
+            float4 wv[8], xv[8];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) wv[k] = wp[c0 + 64 * k], xv[k] = xp[c0 + 64 * k];
+            for (int k = 0; k < 8; ++k) wv[k] = wp[c0 + 64 * k], xv[k] = xp[c0 + 64 * k];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    v = fmaf(wv[k].x, xv[k].x, v);
-                    v = fmaf(wv[k].y, xv[k].y, v);
-                    v = fmaf(wv[k].z, xv[k].z, v);
-                    v = fmaf(wv[k].w, xv[k].w, v);
-                }
+            for (int k = 0; k < 8; ++k) {
+                v = fmaf(wv[k].x, xv[k].x, v);
+                v = fmaf(wv[k].y, xv[k].y, v);
+                v = fmaf(wv[k].z, xv[k].z, v);
+                v = fmaf(wv[k].w, xv[k].w, v);
             }
-            v = group_sum<64>(v);
-            if (lane == 0) y[(size_t) it * rows + irow] = v;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the counts below are of the steps' loads alone)
+        v = group_sum<64>(v);
+        if (lane == 0 && on) y[(size_t) it * rows + irow] = v;
+    };
+    if constexpr (SPREAD) {
+        const int left = rows - net * RM_TILE;
+        if (items > 0) {
+            for (int item = (int) blockIdx.x * RM_WAVES + wave; item < items; item += (int) gridDim.x * RM_WAVES) {
+                const int it = left == 1 ? item : item / left;
+                item_of(it, net * RM_TILE + item - it * left, true);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the counts below are of the steps' loads alone)
+        }
+    } else if (const int item = RM_WAVES * (e0 / RM_TILE) + wave; items > 0 && item < RM_TILE * (rows - net * RM_TILE)) {
+        const int it = t0 + item % RM_TILE;
+        item_of(min(it, T - 1), net * RM_TILE + item / RM_TILE, it < T);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     if (!any) return;   // the same for the whole block
     const int i = lane & 31, b = lane >> 5;

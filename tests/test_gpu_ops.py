@@ -69,6 +69,13 @@ def test_gemv_f32_many_rows_bit_exact(dev, oracle, rows, n, T):
     assert np.array_equal(dev.gemv(W, x).view(np.uint32), oracle.gemv_f32(W, x).view(np.uint32))
 
 
+# large tiles a block each: whole patches of 4 x 8 tiles with a last tile of few rows of x, patches cut short either way, one column of
+# tiles, its left row in a launch of its own and spread over the waves of all CUs
+@pytest.mark.parametrize("rows,n,T", [(257, 2048, 499), (513, 2048, 393), (290, 2048, 640), (33, 2048, 8191), (33, 2048, 4096)])
+def test_gemv_f32_patches_of_large_tiles_bit_exact(dev, oracle, rows, n, T):
+    test_gemv_f32_bit_exact(dev, oracle, rows, n, T)
+
+
 @pytest.mark.parametrize("rows,n,T", [(513, 2048, 17), (513, 2048, 77), (1, 512, 18), (15, 1024, 33), (48, 4096, 31), (130, 512, 250)])
 def test_gemv_f32_short_chunks_bit_exact(dev, oracle, rows, n, T):
     print(f"case short chunk rows={rows} n={n} T={T}", flush=True)
