@@ -1142,16 +1142,15 @@ static int gemv_any(const void* W, bool bf, const float* x, float* y, int rows, 
     hipStream_t s = (hipStream_t) st;
     // f32 weights against more rows than a window's: tiles on the matrix cores, or none (gemv_rows_plan.h)
     const bool tiles = !bf && T > FNX_MAXT && (((uintptr_t) W | (uintptr_t) x) & 15) == 0;
-    const GemvRows form = tiles ? gemv_rows_form(rows, n, T, cu_count()) : GemvRows::many;
-    const bool spread = tiles && gemv_rest_spread(rows, n, T, cu_count());
-    if (form == GemvRows::small_tiles && !spread) {
+    const GemvRows form = tiles ? gemv_rows_route(rows, n, T, cu_count()) : GemvRows::many;
+    if (form == GemvRows::small_tiles) {
         const int ntt = (T + RS_TILE - 1) / RS_TILE, net = (rows + RS_TILE - 1) / RS_TILE;
         k_gemv_rows_mfma16<<<(unsigned) ((gemv_small_tiles(rows, T) + 7) / 8 * 8), RS_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net);
         return launch_status(who);
     }
     if (form != GemvRows::many) {
         const int ntt = (T + RM_TILE - 1) / RM_TILE, net = rows / RM_TILE, left = rows - net * RM_TILE, most = 8 * std::max(1, cu_count() / 8);
-        const bool along = form == GemvRows::large_tiles || spread;
+        const bool spread = form == GemvRows::large_spread, along = form != GemvRows::large_rest;
         const int blocks = spread ? most : std::min((ntt * net + 7) / 8 * 8, most), items = along ? left * T : 0;
         if (blocks < ntt * net) k_gemv_rows_mfma<true, true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items);
         else if (spread) k_gemv_rows_mfma<false, true><<<blocks, RM_THREADS, 0, s>>>((const float*) W, x, y, rows, n, T, ntt, net, items);

@@ -12,7 +12,8 @@ enum class GemvRows {
     many,         // k_gemv_rows_many: no tiles
     small_tiles,
     large_tiles,
-    large_rest    // the large tiles, and a second launch (k_gemv_rows_many) for the weight rows past the last full tile
+    large_rest,   // the large tiles, and a second launch (k_gemv_rows_many) for the weight rows past the last full tile
+    large_spread  // the large tiles, those weight rows' items (such a row x a row of x) over the waves of all CUs
 };
 inline long gemv_small_tiles(int rows, int T) { return (long) ((T + RS_TILE - 1) / RS_TILE) * ((rows + RS_TILE - 1) / RS_TILE); }
 // The weight rows past the last full large tile ride with the tiles' blocks, an item (such a row x a row of x) a wave of the four, as
@@ -37,9 +38,12 @@ inline bool gemv_rest_along(int rows) { return 8 * (rows % RM_TILE) <= rows / RM
 // 5.1 / 9.7, 1000 30.4 / 31.8, 1500 48.6 / 41.6; 1536 wide, 64 5.7 / 12.4, 1000 42.8 / 43.5, 1500 60.9 / 57.5; 2560 wide, 64 7.3 / 17.8,
 // 3000 163 / 185; 2048 weight rows of 1024, 300 32.5 / 32.6, 450 47.0 / 46.2; of 3072, 3000 647 / 750.
 // T: more than a window's; cus: the device's. The pointers are 16-byte aligned (else: many).
-inline GemvRows gemv_rows_form(int rows, int n, int T, int cus) {
-    const bool large = T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (unsigned long long) T * n * 4 < (1ull << 32) &&
-                       (unsigned long long) rows * n * 4 < (1ull << 32);
+inline bool gemv_large_fits(int rows, int n, int T) {   // the large tiles can be had
+    return T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (unsigned long long) T * n * 4 < (1ull << 32) &&
+           (unsigned long long) rows * n * 4 < (1ull << 32);
+}
+inline GemvRows gemv_rows_form(int rows, int n, int T, int cus) {   // where no items are spread (below)
+    const bool large = gemv_large_fits(rows, n, T);
     const long tiles = gemv_small_tiles(rows, T), most = 1l << 24;
     const long upto = large ? (gemv_rest_along(rows) ? 2l : 4l) * cus : n == 512 ? 5l * cus / 2 : n == 1024 ? 8l * cus : n == 1536 ? 12l * cus : most;
     if (n % (2 * RS_COLS) == 0 && tiles < most && tiles <= upto) return GemvRows::small_tiles;
@@ -51,9 +55,10 @@ inline GemvRows gemv_rows_form(int rows, int n, int T, int cus) {
 // form says / so): 33 weight rows, 2,900 rows of x 18.0 / 16.8; 65, 1,633 17.4 / 14.9, 4,000 36.3 / 18.4; 97, 2,330 25.3 / 16.2; 129, 918 17.7 / 13.7, 1,820
 // 25.0 / 15.4, 4,096 37.9 / 29.3; 161, 770 17.2 / 13.4; 258, 500 16.3 / 13.6, 1,500 35.5 / 26.1; 1,000, 500 36.9 / 27.5.
 inline bool gemv_rest_spread(int rows, int n, int T, int cus) {
-    const bool large = T >= 2 * RM_TILE && rows >= RM_TILE && n % 2048 == 0 && (unsigned long long) T * n * 4 < (1ull << 32) &&
-                       (unsigned long long) rows * n * 4 < (1ull << 32);
-    return large && rows % RM_TILE && !gemv_rest_along(rows) && gemv_small_tiles(rows, T) > 2l * cus && (long) (rows % RM_TILE) * T <= 16l * cus;
+    return gemv_large_fits(rows, n, T) && rows % RM_TILE && !gemv_rest_along(rows) && gemv_small_tiles(rows, T) > 2l * cus && (long) (rows % RM_TILE) * T <= 16l * cus;
+}
+inline GemvRows gemv_rows_route(int rows, int n, int T, int cus) {   // the kernel that runs
+    return gemv_rest_spread(rows, n, T, cus) ? GemvRows::large_spread : gemv_rows_form(rows, n, T, cus);
 }
 
 }  // namespace fnx

@@ -60,6 +60,16 @@ def test_window_work(tmp_path):
     assert r.stdout.startswith("ok "), r.stdout
 
 
+def test_gemv_rows_route(tmp_path):
+    """which kernel a router's product over a chunk runs, compiled for the host: the left weight rows' items spread over all waves where that
+    was measured to be faster, four a wave at most, and the form of test_gemv_rows_plan everywhere else"""
+    exe = str(tmp_path / "gemv_rows_route_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I", os.path.join(fnx_gpu.PKG_DIR, "csrc"), "-o", exe,
+                    os.path.join(HERE, "gemv_rows_route_check.cpp")], check=True, capture_output=True, text=True)
+    r = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120)
+    assert r.stdout.startswith("ok "), r.stdout
+
+
 def test_q8s_split(tmp_path):
     """the dense Q8_0 mat-vec's walk of a quarter of the columns, compiled for the host: no load leaves the quarter and every
     double step is taken once, in order, for every width of 256s (1,280 and 2,560 have a short last batch)"""
