@@ -95,6 +95,34 @@ def test_moe_window_over_all_blocks(dev, oracle, ff, nexp, topk, T):
     check_layer(dev, oracle, 2048, ff, nexp, topk, T, 930 + T + ff, True)
 
 
+# the same for a split-Q8_0 shared expert (no items of it in the launch), a bf16 router, blocks in eights (80 a row) and a window whose deal
+# changes with its picks (seven rows of width 512, 9 picks)
+@pytest.mark.parametrize("ff,nexp,topk,T,q8", [(512, 24, 10, 9, True), (1024, 12, 6, 12, True), (1024, 12, 9, 3, False), (1024, 10, 5, 3, True), (512, 32, 9, 7, False),
+                                              (256, 20, 7, 11, False), (1024, 16, 12, 6, False)])
+def test_moe_window_over_all_blocks_in_other_forms(dev, oracle, ff, nexp, topk, T, q8):
+    print(f"case window over all blocks ff={ff} topk={topk} T={T} q8={q8}", flush=True)
+    rng = np.random.default_rng(935 + T + ff)
+    n = 2048
+    router, gu, down, sh_gu, sh_down = make_layer(rng, n, ff, nexp)
+    router = (router.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)   # what bf16 holds
+    sh_q8 = (q8_split(oracle, rng, 2 * ff, n, 0.02), q8_split(oracle, rng, n, ff, 0.02)) if q8 else None
+    layer = fnx_gpu.MoeLayerDev(dev, n, ff, nexp, topk, router, gu, down, sh_gu, sh_down, packed=True, sh_q8=sh_q8)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    want = oracle.moe_verify_layer(n, ff, nexp, topk, router, gu, down, None if q8 else sh_gu, None if q8 else sh_down, x, sh_q8=sh_q8)
+    bits = dev.up((router.view(np.uint32) >> 16).astype(np.uint16))
+    for bf16 in (False, True):
+        if bf16:
+            layer.L.router, layer.L.router_bf16 = bits.data_ptr(), 1
+        got = layer.run(x)
+        assert not got["sync"].any()
+        assert np.array_equal(got["logits"].view(np.uint32), want["logits"].view(np.uint32))
+        assert np.array_equal(got["topi"], want["topi"]) and got["njobs"] == want["njobs"]
+        if q8:
+            assert rel_l2(got["out"], want["out"]) <= 1e-3
+        else:
+            assert np.array_equal(got["out"].view(np.uint32), want["out"].view(np.uint32))
+
+
 @pytest.mark.parametrize("packed", [False, True])
 def test_moe_verify_layer_with_experts_from_pointer_tables(dev, oracle, packed):
     """fnx_dw.ep: an expert's matrix by a table of device pointers instead of base + e * stride (an engine whose experts

@@ -238,3 +238,22 @@ def test_window_over_other_types_in_other_forms(dev, oracle, qtype, ff, T, nexp,
     assert np.array_equal(w["logits"].cpu().numpy().view(np.uint32), want["logits"].view(np.uint32)) and np.array_equal(w["topi"].cpu().numpy(), want["topi"])
     assert int(w["njobs"][0].item()) == want["njobs"]
     assert rel_l2(out.cpu().numpy(), want["out"]) <= 1e-6
+
+
+# rows whose blocks are no power of two (on 256 CUs 28, 20, 80, 24, 36 and 40 a row): units of the down matrices that do not divide among them, at
+# width 1024 four units a wave in two passes, a unit that two waves make, items of the shared expert dealt apart from the picks'
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("ff,T,nexp,topk,tables,shared_q8", [(512, 9, 12, 10, False, False), (1024, 11, 8, 4, True, False), (1024, 3, 12, 9, False, True),
+                                                            (256, 10, 14, 8, True, True), (512, 7, 12, 9, False, False), (1024, 6, 9, 6, False, False)])
+def test_window_over_other_types_over_all_blocks(dev, oracle, qtype, ff, T, nexp, topk, tables, shared_q8):
+    print(f"case window over all blocks type={qtype} ff={ff} T={T} topk={topk} tables={tables} q8={shared_q8}", flush=True)
+    L, ws, w, x, keep, want = typed_layer(dev, oracle, qtype, ff, T, nexp, topk, 75 * qtype + ff + T, shared_q8=shared_q8, tables=tables)
+    dx, out = dev.up(x), dev.zeros((T, 2048), dev.torch.float32)
+    for _ in range(2):   # the second over the workspace as the first left it
+        out.fill_(7.5)
+        dev.ok(dev.lib.fnx_moe_verify_layer(C.byref(L), dx.data_ptr(), T, out.data_ptr(), C.byref(ws), dev.st()))
+        dev.sync()
+        assert not w["sync"].cpu().numpy().any(), "every wait ended and the counters are back at zero"
+        assert np.array_equal(w["logits"].cpu().numpy().view(np.uint32), want["logits"].view(np.uint32)) and np.array_equal(w["topi"].cpu().numpy(), want["topi"])
+        assert int(w["njobs"][0].item()) == want["njobs"]
+        assert rel_l2(out.cpu().numpy(), want["out"]) <= 1e-6

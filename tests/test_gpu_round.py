@@ -259,3 +259,42 @@ def test_rounds_stop_before_the_cache_is_full(dev, oracle, cyclic_model, chain, 
     assert all(np.array_equal(v, before[k]) for k, v in words().items())
     out_h, _ = host_loop(dev, model, prompt, len(out), K=max(1, chain), lk=lk)
     assert out == out_h
+
+
+# experts of width 512, ten picks a row: windows whose rows have no power of two of blocks (on 256 CUs 48, 28 and 20 a row), with the passes either side
+# of them in the launch and, in the rounds, the row count on the device
+@pytest.fixture(scope="module")
+def wide_model(oracle):
+    return td.TinyDecoder(oracle, seed=37, n=2048, nq=4, nkv=2, nlayers=1, vocab=256, max_ctx=512, nexp=24, topk=10, ff=512, cyclic=True)   # (its greedy tokens end in a cycle of fifteen)
+
+
+def test_verify_windows_over_all_blocks_match_the_oracle(dev, oracle, wide_model):
+    o, d = td.OracleSession(wide_model), fnx_gpu.DecoderDev(dev, wide_model)
+    pos = 0
+    for T in (9, 12, 5):
+        print(f"case decoder_verify over all blocks T={T} pos={pos}", flush=True)
+        toks = [int(t) for t in np.random.default_rng(36 + T).integers(0, 256, T)]
+        a, b = o.verify(toks, pos), d.verify(toks, pos)
+        assert b["err"] == 0
+        assert np.array_equal(a["best"], b["best"])
+        chain_close(b["hidden"], a["hidden"], pos == 0)
+        chain_close(b["logits"], a["logits"], pos == 0)
+        nxt = toks[1:] + [int(a["best"][-1])]
+        da, db = o.draft(a["hidden"], nxt, pos), d.draft(a["hidden"], nxt, pos)
+        assert np.array_equal(da["best"], db["best"])
+        chain_close(db["logits"], da["logits"], pos == 0)
+        pos += T
+
+
+@pytest.mark.parametrize("lk,chain", [(8, 0), (4, 0), (11, 2)])
+def test_rounds_over_all_blocks_equal_the_host_driven_rounds(dev, oracle, wide_model, lk, chain):
+    prompt = [t % 256 for t in repeating_prompt(12)]
+    r = RoundDev(dev, wide_model, prompt, lk=lk, chain=chain)
+    print(f"case decode_round over all blocks lk={lk} chain={chain}", flush=True)
+    for _ in range(30):   # (the cycle is entered after some twenty tokens, two a round)
+        r.launch()
+    out, log, st = r.result()
+    print("rounds", log, flush=True)
+    assert st[dev.pkg.RS_STOP] == 0 and st[dev.pkg.RS_ROUNDS] == 30 and int(r.d.b["err"].item()) == 0
+    assert max(dr for dr, _ in log) == lk, "windows of 1 + lk rows that count"
+    assert (out, log) == host_loop(dev, wide_model, prompt, len(out), K=max(chain, 1), lk=lk)
