@@ -1064,7 +1064,7 @@ static int layer_fused(const fnx_moe_layer* L, const float* x, int T, float* out
                         (const uint8_t*) L->gu.p, L->gu_stride, (const uint8_t* const*) L->gu.ep, q8sh ? nullptr : (const uint8_t*) L->sh_gu.p,
                         (const uint8_t*) L->down.p, L->down_stride, (const uint8_t* const*) L->down.ep, q8sh ? nullptr : (const uint8_t*) L->sh_down.p,
                         sh_part, ws->logits, ws->topi, ws->topw, (uint8_t*) ws->xq, (uint32_t*) ws->gu, out, ws->sync, live,
-                        ws->jobs_gu, ws->jobs_dn, ws->njobs, wait_ticks, win_work(nb, T, L->nexp, L->topk, !q8sh, ff)};
+                        ws->jobs_gu, ws->jobs_dn, ws->njobs, wait_ticks, win_work(nb, T, L->nexp, L->topk, !q8sh, ff, win_least_growth(L->gu.type))};
     if (next && next->x) {
         wa.next_x = next->x;
         wa.next_w = next->w;

@@ -17,7 +17,18 @@ namespace fnx {
 // q8_1 block's own sum field (Q4_0's offset, Q5_1's minimum)
 enum { WIN_SUM_NONE = 0, WIN_SUM_CODES = 1, WIN_SUM_FIELD = 2 };
 
+// win_work's least growth of a row's blocks, by type: what a type's loads draw with seven CUs of eight (7 rows at 32 blocks a row; 36 take the rest)
+// or three of four (6 rows, 32 or 40). Q8_0 and the 4-bit types without a minimum draw 3.0 to 3.9 TB/s there and want every CU; IQ3_S, the K-quants and
+// Q5_1, at 3.7 to 4.6, lose to the second XCD that 36 blocks a row spread a slice over, Q5_1 to the 40 too. us a window, 512 experts of width 1,024,
+// 7 rows, at 32 / 36 blocks, 9 picks and 16: Q8_0 124.4 / 119.9, 198.2 / 195.1; Q4_0 75.3 / 73.1, 117.7 / 116.4; IQ4_NL 75.6 / 74.0, 119.3 / 118.3; IQ4_XS 58.1 / 58.5,
+// 87.4 / 88.7, but of 256 experts, 10 picks, 60.2 / 59.8; IQ3_S 49.7 / 49.2, 75.4 / 76.4; Q4_K 54.5 / 56.8, 82.9 / 89.3; Q5_K 65.3 / 66.9, 99.7 / 104.0; Q5_1 67.0 /
+// 69.7, 103.6 / 109.4. 6 rows, 10 picks, at 32 / 40: Q5_1 66.6 / 68.8, Q4_K 54.2 / 54.7, Q5_K 66.6 / 65.2, IQ3_S 52.8 / 50.3, Q8_0 130.0 / 118.2.
+constexpr int win_least_growth(uint32_t type) {
+    return type == QT_Q5_1 ? 2 : type == QT_Q8_0 || type == QT_Q4_0 || type == QT_IQ4_NL || type == QT_IQ4_XS ? 0 : 1;
+}
+
 struct WinUnit64 {
+    static constexpr uint32_t GGML = FNX_T_IQ3S_UNIT64;
     static constexpr int UNIT = UNIT_BYTES, SUM = WIN_SUM_NONE;
     static constexpr bool TAB = true;   // decodes through the signed codebook in LDS
     static constexpr int MAXR = 4, NBUF = 3;   // units a wave's trip holds at most; trips' buffers where a trip holds one or two
@@ -64,6 +75,7 @@ typedef __attribute__((address_space(1), aligned(2))) const unsigned short g_u16
 
 template <uint32_t TYPE>
 struct WinQt {
+    static constexpr uint32_t GGML = TYPE;
     static constexpr bool K = TYPE == QT_Q4_K || TYPE == QT_Q5_K;
     static constexpr int BLOCK = TYPE == QT_Q4_0 || TYPE == QT_IQ4_NL ? 18 : TYPE == QT_Q5_1 ? 24 : TYPE == QT_Q8_0 ? 34 : TYPE == QT_IQ4_XS ? 136 : TYPE == QT_Q4_K ? 144 : 176;
     static constexpr int UNIT = TYPE == QT_IQ4_XS || K ? 8 * BLOCK : 64 * BLOCK;

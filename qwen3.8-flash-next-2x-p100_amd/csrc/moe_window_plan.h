@@ -53,10 +53,11 @@ FNX_HOST_DEVICE inline WinPlan win_plan(int nb, int Tl, int nexp, int topk, bool
 }
 // The work as the window deals it. Two things of the cut above cost time. A power of two of blocks a row leaves up to 44 % of the grid
 // without work at 5 .. 7 and 9 .. 15 rows: blocks are taken in fours up to nb / Tl where that makes a block's routed items fewer
-// (only where a fifth fewer, 8 of 256 experts of width 1,024 at 11 rows IQ3_S 64.8 us / this 59.7, Q8_0 182.7 / 166.2, 512 wide 83.9 / 73.8, but Q5_K 12
-// rows 46.3 / 47.9; where they stay as many, Q8_0 3 to 8 % faster and Q4_K 1 to 4 % slower) and the even cut leaves it more than half a unit of the down matrices a wave (in fours: the blocks that take the same router
-// rows and shared items then lie on one or two of the eight XCDs, whose L2 they share; 252 blocks at 21 a row were slower than 192
-// at 16: q4_k, 12 rows 47.1 -> 51.0 us, at 20 a row 47.2). And the shared expert's items need no pick, so they are dealt apart from the routed ones, to
+// and the even cut leaves it more than half a unit of the down matrices a wave. In fours, since the blocks that take the same router rows and
+// shared items then lie on one or two of the eight XCDs, whose L2 they share (252 blocks at 21 a row were slower than 192 at 16: Q4_K, 12 rows
+// 47.1 -> 51.0 us, at 20 a row 47.2), and in eights, on one, where those are nearly as many (3 rows of 5 of 512 experts of width 1,024, us at 64 / 84 /
+// 80 blocks a row: IQ3_S 28.2 / 28.4 / 27.9, Q4_K 27.6 / 27.8 / 27.2; of 10 IQ3_S 37.4 / 36.5 / 36.2, but Q8_0 74.7 / 69.7 / 70.5). Not where a row gets
+// only a few blocks more, by the type (win_least_growth, k_window_formats.h). And the shared expert's items need no pick, so they are dealt apart from the routed ones, to
 // run while the row's logits gather: to the row's last blocks where there are more blocks than items, which have the fewest
 // routed ones; the routed ones as evenly as they go, since they are what a block does once its picks are known. us a window, 10 of 512
 // experts of width 512 (the even cut in runs of [shared, picks ..] / this): IQ3_S 2 rows 26.8 / 25.8, 7 rows 37.2 / 34.9, 9 rows 46.6 / 38.9, 12 rows
@@ -74,11 +75,12 @@ struct WinWork {
 FNX_HOST_DEVICE inline int win_row(const WinWork& p, int b) { return (p.G & (p.G - 1)) == 0 ? b >> win_log2(p.G) : b / p.G; }   // block b's
 FNX_HOST_DEVICE inline int win_routed_first(const WinWork& p, int g) { return g * p.ipb + (g < p.more ? g : p.more); }
 FNX_HOST_DEVICE inline int win_shared_first(const WinWork& p, int g) { return (p.G > p.shared ? p.G - 1 - g : g) * p.spb; }
-FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool shared, int ff) {
+// least: a row's blocks are taken in fours where that makes them more by over `least` eighths
+FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool shared, int ff, int least = 0) {
     const WinPlan e = win_plan(nb, Tl, nexp, topk, shared, ff);
-    const int lg = win_log2(e.G), all = nb / Tl / 4 * 4, routed = e.qpp * topk;
+    const int lg = win_log2(e.G), f4 = nb / Tl / 4 * 4, f8 = nb / Tl / 8 * 8, all = 16 * f8 >= 15 * f4 ? f8 : f4, routed = e.qpp * topk;
     WinWork p{Tl, e.G, routed, routed >> lg, 0, shared ? e.qpp : 0, 0, 0, e.rpb, e.upb, e.R, e.dwaves};
-    if (all > e.G && e.upb > WN_WAVES / 2 && (routed + all - 1) / all < (routed + e.G - 1) >> lg) {
+    if (8 * (all - e.G) > least * e.G && e.upb > WN_WAVES / 2 && (routed + all - 1) / all < (routed + e.G - 1) >> lg) {
         p.G = all;
         p.ipb = routed / all;
         p.rpb = (nexp + all - 1) / all;

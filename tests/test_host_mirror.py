@@ -60,6 +60,16 @@ def test_window_work(tmp_path):
     assert r.stdout.startswith("ok "), r.stdout
 
 
+def test_window_work_least_growth(tmp_path):
+    """the window's work for the types whose rows take blocks in fours only where they get more by over an eighth or a quarter, compiled for the
+    host: the deal of the other types, or every item once over a power of two of blocks and the hand-over's count"""
+    exe = str(tmp_path / "moe_window_least_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I", os.path.join(fnx_gpu.PKG_DIR, "csrc"), "-o", exe,
+                    os.path.join(HERE, "moe_window_least_check.cpp")], check=True, capture_output=True, text=True)
+    r = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120)
+    assert r.stdout.startswith("ok "), r.stdout
+
+
 def test_gemv_rows_route(tmp_path):
     """which kernel a router's product over a chunk runs, compiled for the host: the left weight rows' items spread over all waves where that
     was measured to be faster, four a wave at most, and the form of test_gemv_rows_plan everywhere else"""
