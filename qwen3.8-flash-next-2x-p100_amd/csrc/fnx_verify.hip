@@ -1576,8 +1576,9 @@ static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const 
     if (njobs_cap < 1) return fail(std::string(who) + ": no jobs");
     MmaArgs a{(const uint8_t*) A->p, sa, A->ep, A->n_out, A->n_in, jobs, njobs, njobs_cap, x, A->n_in, out};
     const bool tile16 = A->type == FNX_T_IQ3S_TILE16;
-    // unit64 rows that the wave forms take: whole units a tile of 16 rows, a lane's sub-blocks of a super-step inside one unit
-    const bool unit64 = A->type == FNX_T_IQ3S_UNIT64 && (A->n_in == 256 || A->n_in == 512 || A->n_in == 1024 || A->n_in % 2048 == 0);
+    // unit64 rows that the wave forms take: whole units a tile of 16 rows, a lane's sub-blocks of a super-step inside one unit; rows of x that
+    // loads of 16 bytes straight into LDS find aligned (others keep the kernel without such loads)
+    const bool unit64 = A->type == FNX_T_IQ3S_UNIT64 && ((uintptr_t) x & 15) == 0 && (A->n_in == 256 || A->n_in == 512 || A->n_in == 1024 || A->n_in % 2048 == 0);
     // the wave forms take the second list - the shared expert's matrix - in the same launch
     const bool merged = A2 && (tile16 || unit64) && A2->p && A2->type == A->type && A2->n_in == A->n_in && A2->n_out == A->n_out;
     if (A2 && !merged) {   // two launches
@@ -1630,7 +1631,7 @@ static int mma_launch(const fnx_dw* A, size_t sa, const fnx_bigjob* jobs, const 
         return launch_status(who);
     }
     if (tile16) return fail(std::string(who) + ": tile16 matrices are the prompt path's two: stacked gate|up leaving h, and rows of 512 columns");
-    // raw blocks, and unit64 rows of other widths: a wave a task of 32 rows x 32 tokens
+    // raw blocks, and unit64 rows of other widths or over unaligned x: a wave a task of 32 rows x 32 tokens
     static const int per_cu = env_int("FNX_MMA_BLOCKS_PER_CU", 2, 1, 8);
     const long tasks = (long) njobs_cap * (A->n_out / 32) * (MM_TT / MM_TP);
     const int grid = (int) std::max(1l, std::min<long>((long) per_cu * cu_count(), (tasks + MM_WAVES - 1) / MM_WAVES));

@@ -5,6 +5,8 @@ Bar: bit-exact for picks, counts, job bases and job lists (integers), and for f3
 for the matrix-core products (f16 operands identical to the oracle's, only the fp32 summation order differs: ~1e-6
 measured); SwiGLU f16 codes within one step in a small share of places (device expf).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -209,6 +211,26 @@ def test_moe_mma_over_unit64_rows(dev, oracle, nrows, ncols, sizes):
     for j in {0, len(jobs) // 2, len(jobs) - 1}:
         at = jobs[j][2 + PF:2 + PF + int(jobs[j][1])]
         assert np.array_equal(got[at].view(np.uint32), out_of(jobs[j:j + 1])[at].view(np.uint32)), f"job {j} of {jobs[j][1]} rows"
+
+
+@pytest.mark.parametrize("nrows,ncols", [(64, 256), (96, 512), (32, 1024), (64, 2048)])
+def test_moe_mma_over_unit64_rows_and_unaligned_activations(dev, oracle, nrows, ncols):
+    """rows of x that begin four bytes past a multiple of sixteen: the form without 16-byte loads into LDS, as for raw blocks"""
+    print(f"case moe_mma unit64 unaligned nrows={nrows} ncols={ncols}", flush=True)
+    rng = np.random.default_rng(752 + nrows + ncols)
+    stride = nrows * ncols // 256 * 110
+    w = random_iq3s(rng, 3 * nrows * ncols // 256, dmax=2e-2)
+    x16 = rng.standard_normal((80, ncols)).astype(np.float16)
+    jobs, total = make_jobs(rng, 3, 80, [5, 64, 17, 1, 40])
+    want = oracle.moe_mma(w, stride, nrows, ncols, jobs, PF, x16, total)
+    dw_, dj = dev.up(w), dev.up(jobs)
+    dx = dev.up(np.concatenate([np.zeros(2, np.float16), x16.reshape(-1)]))
+    assert dx.data_ptr() % 16 == 0
+    dev.ok(dev.lib.fnx_iq3s_repack(dw_.data_ptr(), dw_.data_ptr(), w.size // 110 * 256, dev.st()))
+    W, nj, out = dev.pkg.dw(dw_, ncols, nrows, packed=True), dev.up(np.array([len(jobs)], np.int32)), dev.zeros((total, nrows), dev.torch.float32)
+    dev.ok(dev.lib.fnx_moe_down_mma(C.byref(W), stride, dj.data_ptr(), nj.data_ptr(), len(jobs), dx.data_ptr() + 4, out.data_ptr(), dev.st()))
+    dev.sync()
+    assert rel_l2(out.cpu().numpy(), want) <= 1e-5, "f16 operands are the oracle's: only the summation order may differ"
 
 
 # Lists of several jobs a block: phases of up to four token tiles, with jobs that fill one alone, jobs without tokens between them, and
