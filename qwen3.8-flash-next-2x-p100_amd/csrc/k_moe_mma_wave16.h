@@ -110,7 +110,7 @@ __device__ __forceinline__ void w16_super_step(const uint2* tab, const uint8_t* 
 // the registers that one tile's whole sub-block takes above. between: run between the second and the third of the four
 // steps, where the first half of the fields is dead (loads of what comes next find registers there). Every sum is
 // accumulated as w16_super_step does it.
-template <int NT, int PS, class Between>
+template <int NT, class Between>
 __device__ __forceinline__ void w16_super_pair(const uint2* tab, const uint8_t* xlane, const SuperFields& f0, const SuperFields& f1, v4f (&acc0)[NT],
                                                v4f (&acc1)[NT], Between between) {
     auto step = [&](auto p_c) {
@@ -135,11 +135,11 @@ __device__ __forceinline__ void w16_super_pair(const uint2* tab, const uint8_t* 
         }
     };
     step(std::integral_constant<int, 0>{});
-    if constexpr (PS == 4) step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 1>{});
     __builtin_amdgcn_sched_barrier(0);
     between();
-    step(std::integral_constant<int, PS == 4 ? 2 : 1>{});
-    if constexpr (PS == 4) step(std::integral_constant<int, 3>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
 }
 
 // Where a lane finds its sub-blocks of a tile of 16 rows: PS of them a super-step of 128 PS columns, PS (lane / 16) .. of its row.
@@ -471,6 +471,7 @@ struct Wave16GuLds {
 template <bool GU, class LY>
 __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_pairs(const MmaArgs a) {
     constexpr int PS = LY::PS;
+    static_assert(PS == 4, "whole super-steps");
     // the block's place in the plan: blocks with neighbouring places run on one XCD (workgroups go to the eight XCDs in turn), so
     // the units of one expert, which the plan deals to neighbouring places, find the expert's weights in that XCD's L2
     const unsigned vb = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
@@ -695,7 +696,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_pairs(const MmaA
                 turn(S0 + s);
                 const int Sn = min(S0 + s + 1, nsuper - 1);
                 SuperFields nf, nfu;
-                w16_super_pair<NT, PS>(L.tab, xlane + 16 * NT * s * W16_XROW, f, fu, accg, accu, [&] { nf = ly.load(mg, Sn), nfu = ly.load(mu, Sn); });
+                w16_super_pair<NT>(L.tab, xlane + 16 * NT * s * W16_XROW, f, fu, accg, accu, [&] { nf = ly.load(mg, Sn), nfu = ly.load(mu, Sn); });
                 f = nf, fu = nfu;
             }
         }
@@ -801,7 +802,7 @@ __global__ void __launch_bounds__(W16_THREADS) k_moe_mma_wave16_pairs(const MmaA
             for (int S = 0; S < nsuper; ++S) {
                 turn(S);
                 SuperFields nf, nfu;
-                w16_super_pair<1, PS>(L.tab, xk + S * 16 * W16_XROW, f, fu, accg, accu, [&] {
+                w16_super_pair<1>(L.tab, xk + S * 16 * W16_XROW, f, fu, accg, accu, [&] {
                     if (S + 1 == nsuper) tiles_of(min(pn, pe - 1));
                     const int Sn = S + 1 < nsuper ? S + 1 : 0;
                     nf = ly.load(mg, Sn), nfu = ly.load(mu, Sn);
