@@ -55,7 +55,7 @@ FNX_HOST_DEVICE inline WinPlan win_plan(int nb, int Tl, int nexp, int topk, bool
 // without work at 5 .. 7 and 9 .. 15 rows: blocks are taken in fours up to nb / Tl where that makes a block's routed items fewer
 // and the even cut leaves it more than half a unit of the down matrices a wave. In fours, since the blocks that take the same router rows and
 // shared items then lie on one or two of the eight XCDs, whose L2 they share (252 blocks at 21 a row were slower than 192 at 16: Q4_K, 12 rows
-// 47.1 -> 51.0 us, at 20 a row 47.2), and in eights, on one, where those are nearly as many (3 rows of 5 of 512 experts of width 1,024, us at 64 / 84 /
+// 47.1 -> 51.0 us, at 20 a row 47.2), and in eights, on one, where that leaves out a block in sixteen at most (3 rows of 5 of 512 experts of width 1,024, us at 64 / 84 /
 // 80 blocks a row: IQ3_S 28.2 / 28.4 / 27.9, Q4_K 27.6 / 27.8 / 27.2; of 10 IQ3_S 37.4 / 36.5 / 36.2, but Q8_0 74.7 / 69.7 / 70.5). Not where a row gets
 // only a few blocks more, by the type (win_least_growth, k_window_formats.h). And the shared expert's items need no pick, so they are dealt apart from the routed ones, to
 // run while the row's logits gather: to the row's last blocks where there are more blocks than items, which have the fewest
@@ -78,7 +78,7 @@ FNX_HOST_DEVICE inline int win_shared_first(const WinWork& p, int g) { return (p
 // least: a row's blocks are taken in fours where that makes them more by over `least` eighths
 FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool shared, int ff, int least = 0) {
     const WinPlan e = win_plan(nb, Tl, nexp, topk, shared, ff);
-    const int lg = win_log2(e.G), f4 = nb / Tl / 4 * 4, f8 = nb / Tl / 8 * 8, all = 16 * f8 >= 15 * f4 ? f8 : f4, routed = e.qpp * topk;
+    const int lg = win_log2(e.G), per = nb / Tl, all = per >= 64 ? per & ~7 : per & ~3, routed = e.qpp * topk;
     WinWork p{Tl, e.G, routed, routed >> lg, 0, shared ? e.qpp : 0, 0, 0, e.rpb, e.upb, e.R, e.dwaves};
     if (8 * (all - e.G) > least * e.G && e.upb > WN_WAVES / 2 && (routed + all - 1) / all < (routed + e.G - 1) >> lg) {
         p.G = all;
