@@ -316,8 +316,8 @@ __device__ __forceinline__ void jm_two(const uint32_t* tab, const uint8_t* we, i
 // others: every block fetches its job's activations, 8,192 rows, sixteen rows of one job 9.7 / 11.7; 1,024 rows, twenty jobs 19.4 / 24.1.
 // SBR < 64: a mat-vec call of up to eight jobs over shorter rows, 16 64 / SBR of them a block. The vector-ALU kernel that took them loads and
 // decodes a weight once for every two rows of a job, or four. Us a call with its quantisation, before / now, jobs of 1 row, 5, 16: 8,192
-// rows of 512 columns 8.5 / 6.8, 11.0 / 7.4, 15.8 / 8.4, of 1,024 columns 8.3 / 7.1, 11.4 / 7.9, 17.6 / 9.4; two blocks on some CUs: 12,288
-// rows of 1,024 columns 7.9 / 7.4, 11.4 / 9.8, 18.0 / 13.6. Past two blocks a CU the streaming kernel's runs stay.
+// rows of 512 columns 7.5 / 7.4, 10.5 / 7.4, 15.6 / 8.3, of 1,024 columns 7.8 / 7.4, 11.1 / 7.7, 16.8 / 9.1; two blocks on some CUs: 12,288
+// rows of 1,024 columns 8.0 / 7.3, 11.4 / 9.8, 17.7 / 13.2. Past two blocks a CU the streaming kernel's runs stay.
 template <int SBR>
 __global__ void __launch_bounds__(JM_THREADS) k_iq3s_jobs_mma_one(const RowsArgs a) {
     __shared__ JmOneLds<SBR> L;

@@ -16,6 +16,8 @@ namespace fnx {
 
 constexpr int WN_WAVES = 16;   // waves a block
 
+// The even cut. (nk, k0, per_row, ipb, nbi: its gate|up items in runs of [shared, picks ..]. The window deals them otherwise, win_work below, and
+// these are for the host check of the cut alone.)
 struct WinPlan {
     int Tl;        // rows of the window that count
     int G;         // blocks a row, a power of two (win_work below: not always); block b belongs to row b / G and is the row's block b % G
