@@ -98,7 +98,7 @@ int fnx_quantize_q8_1(const float* x, void* q, int n, int rows, void* st);
  * (njobs null: njobs_max jobs). y: q8_1 rows of W->n_in. W (here and in fnx_moe_gate_up / fnx_moe_down): IQ3_S as ggml
  * blocks, as unit64, or as tile16 (rows in 16s, 512 .. 2048 columns in 512s; w_stride then counts that layout's bytes):
  * tile16 is the layout for jobs of many rows, whose weights go decoded straight into matrix-core operands, unit64 the
- * one for jobs of one or two rows. What a job holds past its n rows is not read. Over ggml blocks, and over unit64 rows of up to 1,024 columns,
+ * one for jobs of one or two rows. What a job holds past its n rows names nothing. Over ggml blocks, and over unit64 rows of up to 1,024 columns,
  * an output's bits do not depend on the job's other rows; over unit64 rows of 2,048 columns a job of one row adds in another order than longer ones. */
 int fnx_mmvq(const fnx_dw* W, size_t w_stride, const fnx_job* jobs, const int* njobs, int njobs_max, const void* y,
              float* out, int out_stride, void* st);
