@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(WN_THREADS) k_moe_window(const WindowArgs a) {
         int rows = Tl;
         asm volatile("" : "+s"(rows));
         if (rows == T) return a.work;
-        return win_work((int) gridDim.x, rows, nexp, topk, a.gu_shared != nullptr, a.ff, win_least_growth(F::GGML));
+        return win_work((int) gridDim.x, rows, nexp, topk, a.gu_shared != nullptr, a.ff, 0, false);
     };
     const WinWork pl = work();
     const int t = win_row(pl, (int) blockIdx.x), g = (int) blockIdx.x - t * pl.G;

@@ -28,7 +28,6 @@ constexpr int win_least_growth(uint32_t type) {
 }
 
 struct WinUnit64 {
-    static constexpr uint32_t GGML = FNX_T_IQ3S_UNIT64;
     static constexpr int UNIT = UNIT_BYTES, SUM = WIN_SUM_NONE;
     static constexpr bool TAB = true;   // decodes through the signed codebook in LDS
     static constexpr int MAXR = 4, NBUF = 3;   // units a wave's trip holds at most; trips' buffers where a trip holds one or two
@@ -75,7 +74,6 @@ typedef __attribute__((address_space(1), aligned(2))) const unsigned short g_u16
 
 template <uint32_t TYPE>
 struct WinQt {
-    static constexpr uint32_t GGML = TYPE;
     static constexpr bool K = TYPE == QT_Q4_K || TYPE == QT_Q5_K;
     static constexpr int BLOCK = TYPE == QT_Q4_0 || TYPE == QT_IQ4_NL ? 18 : TYPE == QT_Q5_1 ? 24 : TYPE == QT_Q8_0 ? 34 : TYPE == QT_IQ4_XS ? 136 : TYPE == QT_Q4_K ? 144 : 176;
     static constexpr int UNIT = TYPE == QT_IQ4_XS || K ? 8 * BLOCK : 64 * BLOCK;

@@ -77,10 +77,12 @@ struct WinWork {
 FNX_HOST_DEVICE inline int win_row(const WinWork& p, int b) { return (p.G & (p.G - 1)) == 0 ? b >> win_log2(p.G) : b / p.G; }   // block b's
 FNX_HOST_DEVICE inline int win_routed_first(const WinWork& p, int g) { return g * p.ipb + (g < p.more ? g : p.more); }
 FNX_HOST_DEVICE inline int win_shared_first(const WinWork& p, int g) { return (p.G > p.shared ? p.G - 1 - g : g) * p.spb; }
-// least: a row's blocks are taken in fours where that makes them more by over `least` eighths
-FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool shared, int ff, int least = 0) {
+// least: a row's blocks are taken in fours where that makes them more by over `least` eighths; eights: in eights where the above says so. (The window itself,
+// where a row count on the device makes every block work this out before its first load, goes without both: with them eight rounds with a chain of three
+// drafts took 6,682 us, 6,652 without, and a window of two rows, whose code only shares its registers with that, 25.98 and 25.85.)
+FNX_HOST_DEVICE inline WinWork win_work(int nb, int Tl, int nexp, int topk, bool shared, int ff, int least = 0, bool eights = true) {
     const WinPlan e = win_plan(nb, Tl, nexp, topk, shared, ff);
-    const int lg = win_log2(e.G), per = nb / Tl, all = per >= 64 ? per & ~7 : per & ~3, routed = e.qpp * topk;
+    const int lg = win_log2(e.G), per = nb / Tl, all = eights && per >= 64 ? per / 8 * 8 : per / 4 * 4, routed = e.qpp * topk;
     WinWork p{Tl, e.G, routed, routed >> lg, 0, shared ? e.qpp : 0, 0, 0, e.rpb, e.upb, e.R, e.dwaves};
     if (8 * (all - e.G) > least * e.G && e.upb > WN_WAVES / 2 && (routed + all - 1) / all < (routed + e.G - 1) >> lg) {
         p.G = all;
